@@ -1,0 +1,68 @@
+"""Prompt steps of the mixers' attention on the bf16 matrix cores against the general kernel.
+
+The general kernel takes a call whose queries do not lie on 16 bytes, so the same step with its queries moved by one float
+is the reference.  Both keep scores, weights and sums in fp32 (an error of about 1e-5 of the largest value) and round once to
+bf16: two results are at most one unit in the last place, 2^-7 of the value at most, apart."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _step(lengths, page):
+    starts, owner, tables, used = [0], [], [], 2
+    width = max(-(-(c + n) // page) for c, n in lengths)
+    for i, (c, n) in enumerate(lengths):
+        starts.append(starts[-1] + n)
+        owner += [i] * n
+        need = -(-(c + n) // page)
+        tables.append([used + (j * 7 + 3) % need if need % 7 else used + need - 1 - j for j in range(need)] + [0] * (width - need))
+        used += need
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
+    return SimpleNamespace(q_start=i32(starts), ctx_len=i32([c for c, _ in lengths]), token_seq=i32(owner),
+                           state_slot=i32(list(range(len(lengths)))), block_tables=i32(tables), num_seqs=len(lengths),
+                           max_query_len=max(n for _, n in lengths), max_pages_used=width, max_page_id=used - 1,
+                           max_state_slot=len(lengths) - 1), used
+
+
+@pytest.mark.parametrize("H,G,d,dv,page", [(4, 4, 128, 128, 16), (8, 2, 64, 96, 16), (6, 2, 40, 24, 8), (32, 1, 16, 8, 32),
+                                           (3, 1, 104, 128, 12)])
+@pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "sink", "learned sink", "sigmoid", "values in the keys"])
+def test_prompt_steps_agree_with_the_general_kernel(H, G, d, dv, page, option):
+    from splitwise_amd import _C
+    per_wg = 4 * (32 // (H // G))                            # tokens of a workgroup
+    lengths = [(0, per_wg), (5, per_wg + 1), (0, 1), (31, max(1, per_wg - 1)), (0, 2 * per_wg + 33), (200, 32), (64, 1)]
+    batch, pages = _step(lengths, page)
+    g = torch.Generator(device=DEV).manual_seed(H * 100 + d)
+    rows = sum(n for _, n in lengths)
+    if option == "values in the keys" and G > 1:
+        dv = d
+    kc = torch.randn(pages, page, G * d, generator=g, device=DEV).to(torch.bfloat16)
+    vc = torch.randn(pages, page, G * dv, generator=g, device=DEV).to(torch.bfloat16)
+    kc[:2], vc[:2] = float("nan"), float("nan")              # pages that no table names
+    if option == "values in the keys":
+        dv, vc = min(d, dv) // 8 * 8, None
+    else:                                                    # slots behind a sequence's end have never been written
+        for i, (c, n) in enumerate(lengths):
+            if (c + n) % page:
+                last = int(batch.block_tables[i, (c + n) // page])
+                kc[last, (c + n) % page:], vc[last, (c + n) % page:] = float("nan"), float("nan")
+    q = torch.randn(rows * H * d + 4, generator=g, device=DEV) * 2
+    gate = torch.randn(rows, H * dv + 3, generator=g, device=DEV).to(torch.bfloat16)[:, 3:]
+    kw = {"cap": dict(softcap=4.0), "window": dict(window=37), "chunk": dict(chunk=48), "sink": dict(sink=True),
+          "learned sink": dict(sink=torch.linspace(-3.0, 9.0, H, device=DEV)),
+          "sigmoid": dict(score_bias=torch.linspace(-2.0, 1.0, H, device=DEV))}.get(option, {})
+    outs = []
+    for lead in (0, 1):                                      # aligned queries, then the same ones a float further on
+        at = torch.empty(rows * H * d + 1, device=DEV)[lead:lead + rows * H * d].view(rows, H * d)
+        at.copy_(q[:rows * H * d].view(rows, H * d))
+        assert at.data_ptr() % 16 == 4 * lead
+        out = torch.full((rows, H * dv), float("nan"), dtype=torch.bfloat16, device=DEV)
+        _C.mixer_ops.capped_attention(out, at, kc, vc, gate if option != "plain" else None, batch, H, G, d, dv, d ** -0.5,
+                                      **kw)
+        outs.append(out.float())
+    torch.testing.assert_close(outs[0], outs[1], atol=2e-4, rtol=2.0 ** -7)
+    assert outs[0].isfinite().all() and outs[0].abs().max() > 0.1

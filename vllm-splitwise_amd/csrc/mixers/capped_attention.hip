@@ -6,7 +6,8 @@
 // query head the same kernels run WITHOUT a softmax: a seen key weighs sigmoid(score + bias), nothing is normalised over
 // the keys, and parts are joined by plain addition.
 // Scores, softmax weights and the weighted sum of values are fp32: both products run on the matrix cores in
-// fp32 (v_mfma_f32_32x32x2_f32), keys and values are widened when they come from a bf16 cache.
+// fp32 (v_mfma_f32_32x32x2_f32), keys and values are widened when they come from a bf16 cache.  Prompt steps over a bf16 cache
+// have a kernel of their own (prompt_attention.hip); what is here serves decode steps, fp32 caches and larger heads.
 //
 // Work split.  A tile is 32 query rows of ONE sequence and ONE key/value head: the R = heads / kv_heads query heads
 // of that group for 32 / R consecutive new tokens (row = token * R + head), so a decode step keeps all heads of a
@@ -22,7 +23,7 @@
 //                 its partner lane l ^ 32 the other 16.
 //   O^T = V^T P^T: A = values (channel l % 32 of key (r, hl)), B = the lane's own weights p[r]: no shuffle between
 //                 the two products.  C element r is channel 8 (r / 4) + 4 hl + r % 4 of the lane's query.
-#include "mixers_common.cuh"
+#include "prompt_attention.cuh"
 
 namespace swm {
 
@@ -652,6 +653,25 @@ int launch_capped_attention(void* out, int64_t out_stride, const float* q, const
                            chunk, sink, sink_logit, score_bias, k_stride, v_stride, stream))
       return status;
   }
+  int page_shift = -1;
+  if ((page_size & (page_size - 1)) == 0)
+    for (page_shift = 0; (1 << page_shift) < page_size; ++page_shift) {}
+  if constexpr (std::is_same<T, bf16_t>::value && NB <= 4) {
+    if (!split && prompt_attention_fits(q, key_cache, value_cache, dim, vdim, k_stride, v_stride)) {
+      PromptAttention a;
+      a.out = out; a.q = q;
+      a.key_cache = static_cast<const uint16_t*>(key_cache);
+      a.value_cache = static_cast<const uint16_t*>(value_cache);
+      a.gate = static_cast<const uint16_t*>(gate);
+      a.block_tables = block_tables; a.q_start = q_start; a.ctx_len = ctx_len;
+      a.sink_logit = sink_logit; a.score_bias = score_bias;
+      a.out_stride = out_stride; a.gate_stride = gate_stride; a.k_stride = k_stride; a.v_stride = v_stride;
+      a.table_width = table_width; a.num_seqs = num_seqs; a.heads = heads; a.kv_heads = kv_heads; a.dim = dim;
+      a.vdim = vdim; a.page_size = page_size; a.page_shift = page_shift; a.window = window; a.chunk = chunk;
+      a.sink = sink; a.tpt = tpt; a.scale = scale; a.softcap = softcap;
+      return launch_prompt_attention(a, rows, stream);
+    }
+  }
   auto lds_bytes = [&](int nw) {
     const size_t floats = split ? (size_t)kQT * qstride + (size_t)nw * kQT * 2 + (size_t)nw * rows_used * ostride
                                 : (size_t)nw * kQT * std::max(qstride, ostride);
@@ -667,9 +687,6 @@ int launch_capped_attention(void* out, int64_t out_stride, const float* q, const
   SW_CHECK_ARG(lds_bytes(nw) <= 160 * 1024, "capped_attention: key size %d with value size %d needs too much LDS", dim,
                vdim);
   auto kernel = capped_attention_kernel<T, NB>;
-  int page_shift = -1;
-  if ((page_size & (page_size - 1)) == 0)
-    for (page_shift = 0; (1 << page_shift) < page_size; ++page_shift) {}
   static size_t allowed = 0;                                 // per instantiation
   if (lds_bytes(nw) > allowed) {
     SW_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,

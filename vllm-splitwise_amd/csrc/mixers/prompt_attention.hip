@@ -1,0 +1,361 @@
+// Prompt steps of the paged attention in capped_attention.hip over a bf16 cache, on the bf16 matrix cores without giving up
+// fp32 scores and weights.
+//
+// What bounds it: matrix work.  The fp32 instructions (v_mfma_f32_32x32x2_f32) reach 154 TFLOP/s on this GPU, the bf16 ones
+// nine times that.  Keys and values ARE bf16 numbers; queries and softmax weights are fp32 and are taken apart into three
+// bf16 numbers each by truncation, x = h + m + l with 8 + 8 + 8 significant bits: the parts are exact, a bf16 x bf16 product
+// is exact in fp32, so three bf16 products accumulated in fp32 are the fp32 product with its sums reordered -- at three
+// times the work on units nine times as fast.
+//
+// Tile: a workgroup of 4 waves owns 4 x 32 query rows of one sequence and key/value head (row = token * R + head of the
+// group, 32 / R tokens a wave) and walks the keys it sees in stages of 32 that the waves share through LDS: global -> registers
+// two stages ahead, registers -> LDS one stage ahead, one barrier a stage.  (In the loop that it replaces every wave fetched
+// every key and value itself.)
+//   S^T = K Q^T : A = keys (row l % 32, 8 neighbouring coordinates per lane), B = the query parts, kept in registers;
+//                 C element r of lane l: key 8 (r / 4) + 4 (l / 32) + r % 4, query l % 32.
+//   O^T = V^T P^T: the score accumulator's layout is the B operand's, two runs of 4 keys per lane; A is read from the
+//                 row-major value stage by the transposing ds_read_b64_tr_b16.
+// The output is referred to a new running maximum only when some lane's has grown by more than 2^8 (weights are then below
+// 2^8, sums stay in fp32 range, the factor cancels in the division).
+// Workgroups are numbered latest tile of a sequence first: under a causal mask those have the longest walks.
+//
+// Measured, two prompts of 4324 tokens together, 16 query heads on 4 of size 128, capped scores and a gate: 989 us with the
+// fp32 instructions (39 TFLOP/s), 169 us here (231 TFLOP/s; the matrix units do three times that).  Error against 64 bits
+// before the rounding to bf16: 1.3e-6 there, 1.2e-6 here (without a cap 6.7e-7 and 3.6e-7).
+#include "prompt_attention.cuh"
+
+#include <algorithm>
+
+namespace swm {
+
+using pa_bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
+using pa_f32x16 = __attribute__((ext_vector_type(16))) float;
+using pa_u32x4 = __attribute__((ext_vector_type(4))) uint32_t;
+using pa_i16x4 = __attribute__((ext_vector_type(4))) short;
+using pa_lds_i16x4 = __attribute__((address_space(3))) pa_i16x4*;
+
+constexpr int kPaKeys = 32, kPaWaves = 4;
+constexpr float kLog2e = 1.4426950408889634f;
+
+// one 16-byte fragment: 8 neighbouring bf16 numbers
+union PaFrag {
+  uint32_t w[4];
+  pa_bf16x8 v;
+};
+
+// x = h + m + l, truncated to bf16 one after the other (exact); an infinity or NaN stays whole in h
+__device__ __forceinline__ void split3(float x, uint32_t& h, uint32_t& m, uint32_t& l) {
+  h = __float_as_uint(x) & 0xffff0000u;
+  const float r1 = (h & 0x7f800000u) == 0x7f800000u ? 0.0f : x - __uint_as_float(h);
+  m = __float_as_uint(r1) & 0xffff0000u;
+  l = __float_as_uint(r1 - __uint_as_float(m));
+}
+// the upper halves of two words, `lo` in the lower half
+__device__ __forceinline__ uint32_t upper_halves(uint32_t hi, uint32_t lo) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); }
+
+__host__ __device__ constexpr int pa_kstride(int nb) { return nb * 64 + 16; }                          // bytes per key row
+__host__ __device__ constexpr int pa_vstride(int nb) { return (nb * 64 + 255) / 256 * 256 + 64; }      // bytes per value row
+__host__ __device__ constexpr int pa_lds_bytes(int nb) { return 2 * kPaKeys * (pa_kstride(nb) + pa_vstride(nb)); }
+
+// NB: blocks of 32 coordinates of the larger of key and value size.
+template <int NB>
+__global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attention_kernel(const PromptAttention a) {
+  constexpr int KS = 2 * NB, CPR = 4 * NB, CHUNKS = kPaKeys * CPR, THREADS = 64 * kPaWaves;
+  constexpr int LOADS = (CHUNKS + THREADS - 1) / THREADS;
+  constexpr int KSTRIDE = pa_kstride(NB), VSTRIDE = pa_vstride(NB);
+  extern __shared__ __attribute__((aligned(16))) char pa_lds[];
+  char* k_img = pa_lds;                                      // [2][32][KSTRIDE]
+  char* v_img = pa_lds + 2 * kPaKeys * KSTRIDE;              // [2][32][VSTRIDE]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qi = lane & 31, hl = lane >> 5;
+  const int R = a.heads / a.kv_heads, g = blockIdx.x % a.kv_heads;
+
+  // ---- this workgroup's tile: sequences from the last, each one's tiles from its latest
+  const int per_wg = kPaWaves * a.tpt;
+  int tile = blockIdx.x / a.kv_heads, seq = -1, tok0 = 0, ntok = 0;
+  for (int s = a.num_seqs - 1; s >= 0; --s) {
+    const int n = a.q_start[s + 1] - a.q_start[s], tiles = (n + per_wg - 1) / per_wg;
+    if (tile < tiles) {
+      seq = s;
+      tok0 = (tiles - 1 - tile) * per_wg;
+      ntok = min(per_wg, n - tok0);
+      break;
+    }
+    tile -= tiles;
+  }
+  if (seq < 0) return;                                       // the whole workgroup
+  const int ctx = a.ctx_len[seq];
+  const int32_t* table = a.block_tables + (int64_t)seq * a.table_width;
+  // this wave's rows; a wave without tokens stages keys and meets barriers
+  const int wtok = wave * a.tpt, nw = max(0, min(a.tpt, ntok - wtok));
+  const int64_t row0 = (int64_t)a.q_start[seq] + tok0 + wtok;
+  const int wfirst = ctx + tok0 + wtok, wlast = wfirst + nw - 1;
+  const int tt = qi / R, hh = qi - tt * R;
+  const bool row_ok = tt < nw;
+  // rows without a token behave like the wave's last token and are never stored
+  const int pos_q = wfirst + min(tt, max(nw - 1, 0));
+  const int low_q = a.chunk > 0 ? pos_q / a.chunk * a.chunk : a.window > 0 ? pos_q - a.window + 1 : 0;
+  auto lowest_of = [&](int first) {
+    return a.chunk > 0 ? first / a.chunk * a.chunk : a.window > 0 ? max(0, first - a.window + 1) : 0;
+  };
+  const int wlow = lowest_of(wfirst);                                              // the wave's first key
+  const int wlow_last = a.chunk > 0 ? wlast / a.chunk * a.chunk : a.window > 0 ? wlast - a.window + 1 : 0;   // its last row's
+  const int last_pos = ctx + tok0 + ntok - 1;
+  const int s_lo = lowest_of(ctx + tok0) / kPaKeys, s_hi = last_pos / kPaKeys;     // stages
+
+  // ---- the queries' parts, scaled; scores live in the log2 domain unless a cap is applied to them first
+  const bool sig = a.score_bias != nullptr, capped = a.softcap > 0.0f;
+  const float qscale = capped ? a.scale : a.scale * kLog2e;
+  const float cap2 = a.softcap * kLog2e, cap_in = capped ? 2.0f * kLog2e / a.softcap : 0.0f;
+  const float bias2 = sig ? a.score_bias[g * R + hh] * kLog2e : 0.0f;
+  PaFrag qh[KS], qm[KS], ql[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    float x[8];
+    const int c = 16 * ks + 8 * hl;
+    const bool ok = row_ok && c < a.dim;
+    const float* p = a.q + (row0 + tt) * (int64_t)a.heads * a.dim + (int64_t)(g * R + hh) * a.dim + c;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float4 v = ok ? *reinterpret_cast<const float4*>(p + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
+      x[4 * j] = v.x * qscale; x[4 * j + 1] = v.y * qscale; x[4 * j + 2] = v.z * qscale; x[4 * j + 3] = v.w * qscale;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint32_t h0, m0, l0, h1, m1, l1;
+      split3(x[2 * j], h0, m0, l0);
+      split3(x[2 * j + 1], h1, m1, l1);
+      qh[ks].w[j] = upper_halves(h1, h0);
+      qm[ks].w[j] = upper_halves(m1, m0);
+      ql[ks].w[j] = upper_halves(l1, l0);
+    }
+  }
+
+  // ---- staging: this thread's 16-byte pieces of a stage (key row c / CPR, piece c % CPR)
+  int page_of[LOADS];
+  pa_u32x4 kreg[LOADS], vreg[LOADS];
+  auto key_of = [&](int it, int stage) { return min(stage * kPaKeys + (it * THREADS + tid) / CPR, last_pos); };
+  auto tfetch = [&](int stage) {                             // page numbers, a stage before the pieces that they address
+    sw::static_for<LOADS>([&](auto IT) {
+      constexpr int it = decltype(IT)::value;
+      const int key = key_of(it, stage);
+      page_of[it] = table[a.page_shift >= 0 ? key >> a.page_shift : key / a.page_size];
+    });
+  };
+  auto fetch = [&](int stage) {
+    sw::static_for<LOADS>([&](auto IT) {
+      constexpr int it = decltype(IT)::value;
+      const int c = it * THREADS + tid, ch = c % CPR, key = key_of(it, stage);
+      const int64_t slot = (int64_t)page_of[it] * a.page_size + (a.page_shift >= 0 ? key & (a.page_size - 1) : key % a.page_size);
+      pa_u32x4 kv = {0u, 0u, 0u, 0u}, vv = {0u, 0u, 0u, 0u};
+      if ((CHUNKS % THREADS == 0 || c < CHUNKS)) {
+        if (ch * 8 < a.dim)
+          kv = *reinterpret_cast<const pa_u32x4*>(a.key_cache + slot * a.k_stride + (int64_t)g * a.dim + ch * 8);
+        if (ch * 8 < a.vdim)
+          vv = *reinterpret_cast<const pa_u32x4*>(a.value_cache + slot * a.v_stride + (int64_t)g * a.vdim + ch * 8);
+      }
+      kreg[it] = kv;
+      vreg[it] = vv;
+    });
+  };
+  auto commit = [&](int buf) {
+    sw::static_for<LOADS>([&](auto IT) {
+      constexpr int it = decltype(IT)::value;
+      const int c = it * THREADS + tid, key = c / CPR, ch = c % CPR;
+      if (CHUNKS % THREADS == 0 || c < CHUNKS) {
+        *reinterpret_cast<pa_u32x4*>(k_img + (buf * kPaKeys + key) * KSTRIDE + ch * 16) = kreg[it];
+        *reinterpret_cast<pa_u32x4*>(v_img + (buf * kPaKeys + key) * VSTRIDE + ch * 16) = vreg[it];
+      }
+    });
+  };
+  // (one v_permlane32_swap; a shuffle through LDS would wait for an LDS round trip in every stage)
+  auto other_half = [&](float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(hl ? r[0] : r[1]);
+  };
+
+  pa_f32x16 o[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[b][r] = 0.0f;
+  float m_run = sig ? 0.0f : -INFINITY, l_part = 0.0f;
+  // transposing reads: lane 4 i + p of a group of 16 names value row i, channels 4 p .. 4 p + 3 of a 4 x 16 block; the
+  // wave's four groups are channels 0 / 16 of keys 0 / 4
+  const int tr_off = (4 * (lane >> 5) + ((lane & 15) >> 2)) * VSTRIDE + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+  const int k_off = qi * KSTRIDE + hl * 16;
+
+  const int stages = s_hi - s_lo + 1;
+  tfetch(s_lo);
+  fetch(s_lo);
+  if (stages > 1) tfetch(s_lo + 1);
+  commit(0);
+  if (stages > 1) fetch(s_lo + 1);
+  if (stages > 2) tfetch(s_lo + 2);
+  __syncthreads();
+  int buf = 0;
+#pragma unroll 1
+  for (int t = 0; t < stages; ++t, buf ^= 1) {               // uniform over the workgroup: every wave meets every barrier
+    const int k0 = (s_lo + t) * kPaKeys;
+    if (t + 1 < stages) commit(buf ^ 1);
+    if (t + 2 < stages) fetch(s_lo + t + 2);
+    if (t + 3 < stages) tfetch(s_lo + t + 3);
+    if (nw > 0 && k0 <= wlast && k0 + kPaKeys > wlow) {      // wave-uniform
+      // ---- S^T = K Q^T: the leading parts in one sum, the others in a second
+      pa_f32x16 s, s2;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = s2[r] = 0.0f;
+      const char* kb = k_img + buf * kPaKeys * KSTRIDE + k_off;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const pa_bf16x8 kf = *reinterpret_cast<const pa_bf16x8*>(kb + 32 * ks);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qh[ks].v, s, 0, 0, 0);
+        s2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, ql[ks].v, s2, 0, 0, 0);
+        s2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qm[ks].v, s2, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] += s2[r];
+      // ---- cap, mask, running softmax (this lane: query qi, keys (r, hl))
+      if (capped) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)                         // cap * tanh(s / cap) = cap (1 - 2 / (1 + e^(2 s / cap)))
+          s[r] = cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s[r] * cap_in));
+      }
+      if (k0 + kPaKeys - 1 > wfirst || k0 < wlow_last) {     // wave-uniform: something to mask
+        const int hi = pos_q - k0 - 4 * hl, lo = low_q - k0 - 4 * hl;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int j = 8 * (r / 4) + r % 4;
+          s[r] = j <= hi && j >= lo ? s[r] : -INFINITY;
+        }
+      }
+      if (sig) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)                         // a hidden key: 1 / (1 + e^inf) = 0
+          s[r] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-(s[r] + bias2)));
+      } else {
+        float tmax = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
+        const float m_new = fmaxf(m_run, fmaxf(tmax, other_half(tmax)));
+        if (__builtin_amdgcn_ballot_w64(m_new > m_run + 8.0f) != 0) {
+          const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
+          l_part *= alpha;
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[b][r] *= alpha;
+          m_run = m_new;
+        }
+        const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+        float sum0 = 0.0f, sum1 = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+          s[r] = __builtin_amdgcn_exp2f(s[r] - m_use);
+          s[r + 1] = __builtin_amdgcn_exp2f(s[r + 1] - m_use);
+          sum0 += s[r];
+          sum1 += s[r + 1];
+        }
+        l_part += sum0 + sum1;
+      }
+      // ---- O^T += V^T P^T, 16 keys at a time; B element j of a lane is key 16 st + 8 (j / 4) + 4 hl + j % 4
+      const char* vb = v_img + buf * kPaKeys * VSTRIDE + tr_off;
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        PaFrag ph, pm, pl;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          // (no infinity to look out for: a weight is at most 2^8)
+          const float x0 = s[8 * st + 2 * j], x1 = s[8 * st + 2 * j + 1];
+          const uint32_t h0 = __float_as_uint(x0) & 0xffff0000u, h1 = __float_as_uint(x1) & 0xffff0000u;
+          const float r0 = x0 - __uint_as_float(h0), r1 = x1 - __uint_as_float(h1);
+          const uint32_t m0 = __float_as_uint(r0) & 0xffff0000u, m1 = __float_as_uint(r1) & 0xffff0000u;
+          ph.w[j] = upper_halves(h1, h0);
+          pm.w[j] = upper_halves(m1, m0);
+          pl.w[j] = upper_halves(__float_as_uint(r1 - __uint_as_float(m1)), __float_as_uint(r0 - __uint_as_float(m0)));
+        }
+        pa_bf16x8 vf[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const char* base = vb + 16 * st * VSTRIDE + b * 64;
+          union { pa_i16x4 half[2]; pa_bf16x8 f; } u;
+          u.half[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pa_lds_i16x4)(base));
+          u.half[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pa_lds_i16x4)(base + 8 * VSTRIDE));
+          vf[b] = u.f;
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[b], pl.v, o[b], 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[b], pm.v, o[b], 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[b], ph.v, o[b], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
+  if (!row_ok) return;
+
+  // ---- normalise, gate, store: this lane holds query qi, channels 32 b + 8 (r / 4) + 4 hl + r % 4
+  const float l_run = l_part + other_half(l_part);
+  float inv = 1.0f;
+  if (!sig) {
+    // the sink: one more term that carries no value, of score 0 or of the head's learned score
+    const float sk = a.sink_logit != nullptr ? a.sink_logit[g * R + hh] * kLog2e : 0.0f;
+    const float m_fin = a.sink ? fmaxf(m_run, sk) : m_run;
+    const float fin = a.sink ? __builtin_amdgcn_exp2f(m_run - m_fin) : 1.0f;
+    inv = fin / (l_run * fin + (a.sink ? __builtin_amdgcn_exp2f(sk - m_fin) : 0.0f));
+  }
+  const int64_t col0 = (int64_t)(g * R + hh) * a.vdim;
+  uint16_t* op = static_cast<uint16_t*>(a.out) + (row0 + tt) * a.out_stride + col0;
+  const uint16_t* gp = a.gate != nullptr ? a.gate + (row0 + tt) * a.gate_stride + col0 : nullptr;
+  const bool quads = a.out_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.out) % 8 == 0;
+  const bool gquads = a.gate_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.gate) % 8 == 0;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+      const int c = 32 * b + 8 * r4 + 4 * hl;
+      if (c >= a.vdim) continue;
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = o[b][4 * r4 + j] * inv;
+      if (gp != nullptr) {
+        float gv[4];
+        if (gquads) {
+          ld_vec<bf16_t, 4>(gv, gp, c);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) gv[j] = ld<bf16_t>(gp, c + j);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] *= sigmoidf_(gv[j]);
+      }
+      if (quads) {
+        st_vec<bf16_t, 4>(op, c, v);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) st<bf16_t>(op, c + j, v[j]);
+      }
+    }
+}
+
+template <int NB>
+int launch_prompt_tiles(const PromptAttention& a, int64_t rows, hipStream_t stream) {
+  const int64_t per_wg = (int64_t)kPaWaves * a.tpt;
+  const int64_t groups = ((rows + per_wg - 1) / per_wg + a.num_seqs) * a.kv_heads;
+  SW_CHECK_ARG(groups < (1ll << 31), "masked_attention: too many rows");
+  hipLaunchKernelGGL(prompt_attention_kernel<NB>, dim3((unsigned)groups), dim3(64 * kPaWaves), pa_lds_bytes(NB), stream, a);
+  SW_CHECK_LAUNCH();
+  return SW_OK;
+}
+
+int launch_prompt_attention(const PromptAttention& a, int64_t rows, hipStream_t stream) {
+  switch ((std::max(a.dim, a.vdim) + 31) / 32) {
+    case 1: return launch_prompt_tiles<1>(a, rows, stream);
+    case 2: return launch_prompt_tiles<2>(a, rows, stream);
+    case 3: return launch_prompt_tiles<3>(a, rows, stream);
+    default: return launch_prompt_tiles<4>(a, rows, stream);
+  }
+}
+
+}  // namespace swm
