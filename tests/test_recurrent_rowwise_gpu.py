@@ -1,0 +1,74 @@
+"""The short convolution in runs of rows and the per-head norm in 16-byte pieces against the kernels that take one element at
+a time.  Those serve calls whose inputs do not lie on 16 bytes, so the same call with its input moved by one element is the
+reference: fp32 sums of at most 4 products, in the same order (rtol 1e-5), rounded once where the result is bf16 (2^-7)."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _tol(dtype):
+    return dict(atol=1e-5, rtol=1e-5) if dtype == torch.float32 else dict(atol=1e-4, rtol=2.0 ** -7)
+
+
+def _moved(t, lead, row):
+    """``t`` [rows, n] as a view with row stride ``row`` that begins ``lead`` elements into its storage."""
+    at = torch.empty(t.shape[0] * row + lead + 8, dtype=t.dtype, device=DEV)
+    view = at[lead:lead + t.shape[0] * row].view(t.shape[0], row)[:, :t.shape[1]]
+    view.copy_(t)
+    return view
+
+
+@pytest.mark.parametrize("lens", [[1], [1] * 5 + [2, 3, 4, 1, 7], [15, 2, 1, 16, 33, 1, 3, 17, 2, 64], [1, 1030, 2, 31, 1, 1, 3, 100]])
+@pytest.mark.parametrize("channels,taps", [(8, 4), (72, 3), (4160, 4), (264, 2)])
+@pytest.mark.parametrize("x_dtype,out_dtype", [(torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16),
+                                               (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
+def test_convolution_in_runs(lens, channels, taps, x_dtype, out_dtype):
+    from splitwise_amd import _C
+    starts, owner = [0], []
+    for i, n in enumerate(lens):
+        starts.append(starts[-1] + n)
+        owner += [i] * n
+    rows, count = starts[-1], len(lens)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
+    slots = [(i * 3 + 1) % (count + 2) if (count + 2) % 3 else i + 1 for i in range(count)]
+    batch = SimpleNamespace(q_start=i32(starts), ctx_len=i32([(0, 9)[i % 2] for i in range(count)]), token_seq=i32(owner),
+                            state_slot=i32(slots), max_state_slot=max(slots))
+    g = torch.Generator(device=DEV).manual_seed(rows + channels)
+    x = torch.randn(rows, channels, generator=g, device=DEV).to(x_dtype)
+    w = torch.randn(channels, taps, generator=g, device=DEV)
+    state = torch.randn(count + 2, taps - 1, channels, generator=g, device=DEV)
+    for silu, residual in ((True, False), (False, True)):
+        res = []
+        for lead in (0, 1):
+            s, out = state.clone(), torch.full((rows, channels), float("nan"), dtype=out_dtype, device=DEV)
+            at = _moved(x, lead, channels + 8)
+            assert at.data_ptr() % 16 == lead * x.element_size()
+            _C.mixer_ops.causal_conv(out, at, w, s, batch, silu=silu, residual=residual)
+            res.append((out, s))
+        torch.testing.assert_close(res[0][0], res[1][0], **_tol(out_dtype))
+        assert torch.equal(res[0][1], res[1][1])               # inputs are copied, nothing is rounded
+
+
+@pytest.mark.parametrize("heads,vdim", [(3, 8), (5, 40), (16, 64), (1, 72), (2, 128), (7, 200), (3, 512), (1, 520), (2, 1024), (1, 2048),
+                                        (1, 4096)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_head_norm_in_pieces(heads, vdim, dtype):
+    from splitwise_amd import _C
+    g = torch.Generator(device=DEV).manual_seed(heads * 1000 + vdim)
+    for rows in (1, 37):
+        o = torch.randn(rows, heads * vdim, generator=g, device=DEV)
+        o[0] *= 1e-3                                           # small enough for eps to count
+        gate = torch.randn(rows, heads * vdim, generator=g, device=DEV).to(dtype) * 3
+        for weight, per_head, silu in ((None, False, True), (torch.randn(vdim, generator=g, device=DEV), False, False),
+                                       (torch.randn(heads * vdim, generator=g, device=DEV), True, True)):
+            res = []
+            for lead in (0, 1):
+                out = torch.full((rows, heads * vdim), float("nan"), dtype=dtype, device=DEV)
+                _C.mixer_ops.head_norm_gate(out, o, _moved(gate, lead, heads * vdim + 16), weight, per_head, 1e-5, heads, vdim,
+                                            gate_silu=silu)
+                res.append(out)
+            torch.testing.assert_close(res[0], res[1], **_tol(dtype))
