@@ -72,3 +72,36 @@ def test_head_norm_in_pieces(heads, vdim, dtype):
                                             gate_silu=silu)
                 res.append(out)
             torch.testing.assert_close(res[0], res[1], **_tol(dtype))
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(1, 1, 4, 4), (4, 2, 24, 36), (2, 2, 64, 64), (3, 1, 100, 132), (4, 4, 128, 128),
+                                                     (2, 1, 256, 256), (1, 1, 256, 8), (2, 1, 6, 260)])
+@pytest.mark.parametrize("per_channel", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_delta_decode_step_in_one_launch(heads, kv_heads, dim, vdim, per_channel, dtype):
+    """Against the prologue and recurrence, which an output off 16 bytes goes to: sums of at most 256 products of numbers
+    around 1 in fp32, in another order."""
+    from splitwise_amd import _C
+    g = torch.Generator(device=DEV).manual_seed(heads * 1000 + dim + vdim)
+    seqs, slots = 9, [3, 0, 11, 5, 7, 1, 8, 2, 10]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
+    lens = [1, 1, 0, 2, 1, 1, 1, 1, 1]                         # as many rows as sequences, though not one each
+    starts = [sum(lens[:i]) for i in range(seqs + 1)]
+    batch = SimpleNamespace(q_start=i32(starts), ctx_len=i32([5, 0, 7, 0, 3, 9, 0, 64, 1]), max_query_len=1, max_state_slot=11,
+                            token_seq=i32([i for i, n in enumerate(lens) for _ in range(n)]), state_slot=i32(slots))
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)               # noqa: E731
+    qkv = rnd(seqs, 2 * kv_heads * dim + heads * vdim)
+    beta, dt_bias, a_log = rnd(seqs, heads + 3).to(dtype)[:, :heads], rnd(heads * (dim if per_channel else 1)), rnd(heads) * 0.3
+    decay = rnd(seqs, heads * dim if per_channel else heads).to(dtype)
+    state = rnd(12, heads, dim, vdim)
+    res = []
+    for lead in (0, 1):
+        s = state.clone()
+        out = torch.full((seqs * heads * vdim + 1,), float("nan"), device=DEV)[lead:lead + seqs * heads * vdim].view(seqs, -1)
+        op = _C.mixer_ops.channel_delta if per_channel else _C.mixer_ops.gated_delta
+        op(out, qkv, beta, decay, dt_bias, a_log, s, batch, heads, kv_heads, dim, vdim)
+        res.append((out, s))
+    torch.testing.assert_close(res[0][0], res[1][0], atol=3e-5, rtol=1e-4)
+    torch.testing.assert_close(res[0][1], res[1][1], atol=3e-5, rtol=1e-4)
+    idle = [i for i in range(12) if i not in slots] + [11]     # slots of nobody, and of the sequence without a token
+    assert torch.equal(res[0][1][idle], state[idle])

@@ -15,6 +15,12 @@
 
 namespace swm {
 
+// delta_step.hip: a decode step in one launch; false when the sizes or addresses are not for it
+bool delta_step(float* out, const float* qkv, const void* beta_pre, int64_t beta_stride, const void* decay_pre,
+                int64_t decay_stride, int decay_per_head, const float* dt_bias, const float* a_log, float* state,
+                const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot, int num_seqs, int heads, int kv_heads,
+                int dim, int vdim, int act_dtype, hipStream_t stream);
+
 constexpr int kColsPerWave = 16;
 constexpr int kPrepThreads = 256;
 
@@ -322,6 +328,12 @@ static int delta_with_decay(float* out, const float* qkv, const void* beta_pre, 
                "channel_delta: heads %d, kv heads %d, key size %d (up to 256), value size %d", heads, kv_heads, dim,
                vdim);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // as many rows as sequences: a decode step (should a sequence bring none and another two, it is right all the same)
+  if (rows <= num_seqs && delta_step(out, qkv, beta_pre, beta_stride, decay_pre, decay_stride, decay_per_head, dt_bias, a_log,
+                                     state, q_start, ctx_len, state_slot, num_seqs, heads, kv_heads, dim, vdim, act_dtype, s)) {
+    SW_CHECK_LAUNCH();
+    return SW_OK;
+  }
   float* ops = workspace;
   float* beta = workspace + rows * heads * 3 * (int64_t)((dim + 3) & ~3);
   SWM_DISPATCH_ACT(act_dtype, hipLaunchKernelGGL(channel_delta_prep_kernel<T>, dim3((unsigned)rows), dim3(kPrepThreads), 0,
