@@ -19,6 +19,8 @@
 // multiplied out by the prologue, staged in LDS behind two barriers, and 32 channels per workgroup (128 workgroups); 69 and
 // 233 us here.  Of the walk's 3.0 us a chunk 1.9 are its products, exchanges and waits alone (66 products of 32 cycles are 0.9),
 // 0.6 the operands' way through the L1 and 0.5 their way from memory.
+// L is summed in 64 bits: its differences are what counts, and where decays are strong 32 bits leave the end states an error of
+// 0.5 - 1.3e-6 (1.3 - 1.5e-7 here, for the prologue's 69 us all the same).
 // Rows of a last, shorter chunk are padded with beta = 0, k = 0, g = 1: they change nothing and are not stored.
 #include "mixers_common.cuh"
 
@@ -139,37 +141,38 @@ __global__ __launch_bounds__(kDcPrepThreads) void delta_chunk_prep_kernel(
   }
   __syncthreads();
   // ---- a wave per value head of this key head
-  float* A = red + wave * (kDcChunk * 36 + 64);  // [32][36]: row t, its even columns, then its odd ones
-  float* Ls = A + kDcChunk * 36;                 // [32] running sums of the log decays
-  float* Bs = Ls + kDcChunk;                     // [32] beta
+  float* A = red + wave * (kDcChunk * 36 + 96);  // [32][36]: row t, its even columns, then its odd ones
+  double* Ls = reinterpret_cast<double*>(A + kDcChunk * 36);  // [32] running sums of the log decays
+  float* Bs = A + kDcChunk * 36 + 64;            // [32] beta
   for (int m = wave; m < group; m += kDcPrepThreads / 64) {
     const int h = g * group + m;
     float* rec = records + ((int64_t)blockIdx.x * heads + h) * kDcRecord;
-    float beta = 0.0f, L = 0.0f;                 // of token li, in both halves
+    float beta = 0.0f;
+    double L = 0.0;                              // of token li, in both halves
     if (li < cn) {
       beta = sigmoidf_(ld<T>(beta_pre, (row0 + li) * beta_stride + h));
       L = -expf(a_log[h]) * softplusf_(ld<T>(decay_pre, (row0 + li) * decay_stride + h) + dt_bias[h]);
     }
 #pragma unroll
     for (int step = 1; step < 32; step <<= 1) {
-      const float o = __shfl_up(L, step, 32);
+      const double o = __shfl_up(L, step, 32);
       if (li >= step) L += o;
     }
-    const float Ln = __shfl(L, 31, 32);
+    const double Ln = __shfl(L, 31, 32);
     if (hl == 0) {
       Ls[li] = L;
       Bs[li] = beta;
       rec[2048 + li] = beta;
-      rec[2048 + 32 + li] = expf(L);
-      rec[2048 + 64 + li] = expf(Ln - L);
-      if (li == 0) rec[2048 + 96] = expf(Ln);
+      rec[2048 + 32 + li] = expf((float)L);
+      rec[2048 + 64 + li] = expf((float)(Ln - L));
+      if (li == 0) rec[2048 + 96] = expf((float)Ln);
     }
     __builtin_amdgcn_wave_barrier();
     __threadfence_block();
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int t = 8 * (r / 4) + 4 * hl + r % 4;
-      const float ratio = li <= t ? expf(Ls[t] - L) : 0.0f;
+      const float ratio = li <= t ? expf((float)(Ls[t] - L)) : 0.0f;
       A[t * 36 + (li & 1) * 16 + (li >> 1)] = li < t ? Bs[t] * ratio * kk[r] : 0.0f;
       rec[1024 + t * 32 + li] = ratio * qk[r];
     }
