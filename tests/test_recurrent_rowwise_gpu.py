@@ -132,3 +132,49 @@ def test_delta_chunks_agree_with_the_tokens(heads, kv_heads, dim, vdim):
     torch.testing.assert_close(res[0][0], res[1][0], atol=2e-5, rtol=1e-4)
     torch.testing.assert_close(res[0][1], res[1][1], atol=2e-5, rtol=1e-4)
     assert torch.equal(res[0][1][[5, 6]], state[[5, 6]])
+
+
+@pytest.mark.parametrize("rule", ["gla", "gla, strong decays", "lightning", "retention"])
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 32, 16), (3, 64, 17), (1, 72, 130), (2, 128, 40), (1, 160, 16), (1, 256, 33)])
+def test_linear_attention_walk_agrees_with_short_runs(rule, heads, dim, vdim):
+    """Runs that end at, before and behind the borders of a chunk and of its halves, in one step and in portions of at most 16
+    tokens, which take the kernels of decode steps.  Sums of fp32 products in another order."""
+    from splitwise_amd import _C
+    ops = _C.mixer_ops
+    lens = [17, 32, 33, 16, 1, 64, 95]
+    g = torch.Generator(device=DEV).manual_seed(dim + vdim)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)               # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
+    rows, nk, nv = sum(lens), heads * dim, heads * vdim
+    dtype = torch.float32 if rule == "retention" else torch.bfloat16
+    proj = rnd(rows, 2 * nk + nv + 8).to(dtype)
+    strong = rule == "gla, strong decays"
+    z, bias = rnd(rows, nk).to(dtype) * (6.0 if strong else 1.0), rnd(nk)
+    decay, ctx, slots = torch.linspace(0.3, 0.999, heads, device=DEV), [0, 3, 9, 0, 64, 0, 1], [4, 0, 8, 2, 1, 7, 3]
+    state = rnd(9, heads, dim, vdim) * 0.1
+
+    def step(parts, out, s):
+        """parts: (sequence, tokens before it, tokens)."""
+        first = [sum(lens[:i]) for i in range(len(lens))]
+        pick = torch.cat([torch.arange(first[i] + lo, first[i] + lo + n, device=DEV) for i, lo, n in parts])
+        starts = [sum(n for _, _, n in parts[:i]) for i in range(len(parts) + 1)]
+        batch = SimpleNamespace(q_start=i32(starts), ctx_len=i32([ctx[i] + lo for i, lo, _ in parts]), max_state_slot=8,
+                                max_query_len=max(n for _, _, n in parts), state_slot=i32([slots[i] for i, _, _ in parts]),
+                                token_seq=i32([j for j, (_, _, n) in enumerate(parts) for _ in range(n)]))
+        p, o = proj[pick], torch.empty(len(pick), nv, device=DEV)
+        q, k, v = p[:, :nk], p[:, nk:2 * nk], p[:, 2 * nk:2 * nk + nv]
+        if rule == "lightning":
+            ops.lightning(o, q, k, v, decay, s, batch, heads, dim, vdim)
+        elif rule == "retention":
+            ops.retention(o, q.contiguous(), k.contiguous() * dim ** -0.5, v, decay, s, batch, heads, dim, vdim)
+        else:
+            ops.gla(o, q, k, v, z[pick].contiguous(), bias, 0.5 if strong else 8.0, dim ** -0.5, s, batch, heads, dim, vdim)
+        out[pick] = o
+    a, b = state.clone(), state.clone()
+    whole, pieces = (torch.full((rows, nv), float("nan"), device=DEV) for _ in range(2))
+    step([(i, 0, n) for i, n in enumerate(lens)], whole, a)
+    for lo in range(0, max(lens), 13):
+        step([(i, lo, min(13, n - lo)) for i, n in enumerate(lens) if n > lo], pieces, b)
+    size = float(pieces.abs().max())
+    torch.testing.assert_close(whole, pieces, atol=1e-5 * size, rtol=1e-4)
+    torch.testing.assert_close(a, b, atol=1e-5 * float(b.abs().max()), rtol=1e-4)

@@ -16,34 +16,29 @@
 //    value channel join their halves of S^T q.  Exact for any decay (a product of decays that underflows is a state
 //    that has been forgotten), and the cheaper route for runs of a few tokens (a decoded token is a chunk of one).
 //
-// Long runs are cut into segments of kGlaSegment tokens that run side by side: a first launch takes every segment but a
-// sequence's last from the EMPTY state and leaves its end state and its summed log decays; a scan turns these into the
-// states at the segments' ends, S_end(j) = diag(e^(D_j)) S_end(j - 1) + local(j); a second launch runs every segment
-// from its true start state and writes the outputs.
-#include "mixers_common.cuh"
+// Runs of more than kGlaWalkFrom tokens are taken by linear_walk.hip.
+#include "linear_walk.cuh"
 
 namespace swm {
 
 using f32x16 = __attribute__((ext_vector_type(16))) float;
 constexpr int kGlaChunk = 32;
-constexpr int kGlaSegment = 128;       // tokens per segment of a long run (a multiple of kGlaChunk)
+// Steps whose longest run has more tokens than this go to linear_walk.hip (us here / there, with norm and gate, the host's 30 a
+// call included: 1 x 16 heads of 128, 16 tokens 32 / 34, 31 tokens 37 / 34, 64 tokens 63 / 34, 1000 tokens 921 / 75).
+constexpr int kGlaWalkFrom = 16;
 constexpr float kSafeLog = 24.0f;      // the matrix route needs every channel's summed log-decay of a chunk above -this
 constexpr int kTokenRouteBelow = 6;    // chunks shorter than this go token by token without asking
-constexpr int kGlaWhole = 0, kGlaLocal = 1, kGlaFinal = 2;
 
 // log(sigmoid(x)) = min(x, 0) - log1p(exp(-|x|))
 __device__ __forceinline__ float logsigmoidf_(float x) { return fminf(x, 0.0f) - log1pf(expf(-fabsf(x))); }
 
-// mode kGlaWhole: blockIdx.x is a sequence and its whole run goes from the slot's state to the slot's state.
-// kGlaLocal / kGlaFinal: blockIdx.x is a segment (see the head of the file); seg_state [segments, heads, dim, vdim],
-// seg_decay [segments, heads, dim].
+// blockIdx.x is a sequence; its whole run goes from the slot's state to the slot's state.
 template <typename T, int NDB>
 __global__ __launch_bounds__(512) void gla_kernel(
     float* __restrict__ out, const void* __restrict__ q, const void* __restrict__ k, const void* __restrict__ v,
     int64_t in_stride, const void* __restrict__ decay_pre, int64_t decay_stride, const float* __restrict__ decay_bias,
     float inv_tau, float q_scale, float* __restrict__ state, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int num_seqs, int heads, int dim,
-    int vdim, int mode, float* __restrict__ seg_state, float* __restrict__ seg_decay) {
+    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int dim, int vdim) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int DS = NDB * 32 + 4;                           // row stride of the staged tiles
   constexpr int CH = NDB * 32;                               // key channels, padded
@@ -54,26 +49,16 @@ __global__ __launch_bounds__(512) void gla_kernel(
   float* Gs = Ks + kGlaChunk * DS;                           // [32][DS] log decays, then their running sums or the decays
   float* Vs = Gs + kGlaChunk * DS;                           // [32][VS] values of this workgroup's channels
   float* part = Vs + kGlaChunk * VS;                         // [8][CH] sums of the log decays over groups of tokens
-  float* dsum = part + 8 * CH;                               // [CH] summed log decays of the whole segment
-  float* red = dsum + CH;                                    // [nw] workgroup minimum
+  float* red = part + 8 * CH;                                // [nw] workgroup minimum
   const int h = blockIdx.y;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 31, hl = lane >> 5;
   const int vb0 = blockIdx.z * nw;                           // first block of 32 value channels of the workgroup
-  int seq = blockIdx.x, tok0 = 0, n;
-  if (mode == kGlaWhole) {
-    n = q_start[seq + 1] - q_start[seq];
-  } else {
-    n = find_query_tile(q_start, num_seqs, blockIdx.x, kGlaSegment, &seq, &tok0);
-  }
+  const int seq = blockIdx.x, n = q_start[seq + 1] - q_start[seq];
   if (n <= 0) return;                                        // the whole workgroup
-  const int row0 = q_start[seq] + tok0;
-  const bool last_seg = tok0 + n == q_start[seq + 1] - q_start[seq];
-  if (mode == kGlaLocal && last_seg) return;
+  const int row0 = q_start[seq];
   const int vc = (vb0 + wave) * 32 + li;                     // this lane's value channel
   const bool vc_ok = vc < vdim;
   float* sp = state + ((int64_t)state_slot[seq] * heads + h) * (int64_t)dim * vdim;
-  float* seg_out = seg_state + ((int64_t)blockIdx.x * heads + h) * (int64_t)dim * vdim;      // segment modes only
-  const float* start = (mode == kGlaFinal && tok0 > 0) ? seg_out - (int64_t)heads * dim * vdim : sp;
 
   // token groups for the sums down a chunk: `groups` threads per channel, each with 32 / groups tokens
   int groups = 1;
@@ -81,29 +66,27 @@ __global__ __launch_bounds__(512) void gla_kernel(
   const int per = kGlaChunk / groups;
 
   f32x16 S[NDB];
-  const bool fresh = mode == kGlaLocal || (tok0 == 0 && ctx_len[seq] == 0);
+  const bool fresh = ctx_len[seq] == 0;
 #pragma unroll
   for (int b = 0; b < NDB; ++b)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int c = 32 * b + 8 * (r / 4) + 4 * hl + (r % 4);
-      S[b][r] = (!fresh && vc_ok && c < dim) ? start[(int64_t)c * vdim + vc] : 0.0f;
+      S[b][r] = (!fresh && vc_ok && c < dim) ? sp[(int64_t)c * vdim + vc] : 0.0f;
     }
-  if (mode == kGlaLocal)
-    for (int c = threadIdx.x; c < CH; c += blockDim.x) dsum[c] = 0.0f;
 
   const int64_t qk_col = (int64_t)h * dim, v_col = (int64_t)h * vdim;
   for (int c0 = 0; c0 < n; c0 += kGlaChunk) {
     const int cn = min(kGlaChunk, n - c0);
     const int64_t base = (int64_t)(row0 + c0) * in_stride, dbase = (int64_t)(row0 + c0) * decay_stride;
-    const bool ask = cn >= kTokenRouteBelow || mode == kGlaLocal;     // uniform over the workgroup
+    const bool ask = cn >= kTokenRouteBelow;                 // uniform over the workgroup
     const int stage_rows = ask ? kGlaChunk : cn;             // the matrix route reads all 32 rows: the rest are zeros
     __syncthreads();                                         // the last chunk's tiles have been read
     for (int e = threadIdx.x; e < stage_rows * CH; e += blockDim.x) {
       const int r = e / CH, c = e % CH;
       float qv = 0.0f, kv = 0.0f, gv = 0.0f;
       if (r < cn && c < dim) {
-        if (mode != kGlaLocal) qv = ld<T>(q, base + r * in_stride + qk_col + c) * q_scale;
+        qv = ld<T>(q, base + r * in_stride + qk_col + c) * q_scale;
         kv = ld<T>(k, base + r * in_stride + qk_col + c);
         float z = ld<T>(decay_pre, dbase + r * decay_stride + qk_col + c);
         if (decay_bias != nullptr) z += decay_bias[qk_col + c];
@@ -134,7 +117,6 @@ __global__ __launch_bounds__(512) void gla_kernel(
         float total = 0.0f;
         for (int gi = 0; gi < groups; ++gi) total += part[gi * CH + c];
         lowest = fminf(lowest, total);
-        if (mode == kGlaLocal) dsum[c] += total;
       }
 #pragma unroll
       for (int step = 32; step >= 1; step >>= 1) lowest = fminf(lowest, __shfl_xor(lowest, step, 64));
@@ -161,7 +143,7 @@ __global__ __launch_bounds__(512) void gla_kernel(
       float vt[16];
 #pragma unroll
       for (int r = 0; r < 16; ++r) vt[r] = Vs[(8 * (r / 4) + 4 * hl + (r % 4)) * VS + wave * 32 + li];
-      if (mode != kGlaLocal) {
+      {
         // ---- A^T = K~ Q~^T (rows: keys, columns: queries); this lane: token li of the chunk as key and as query
         f32x16 a;
 #pragma unroll
@@ -264,73 +246,29 @@ __global__ __launch_bounds__(512) void gla_kernel(
         }
       }
       acc += __shfl_xor(acc, 32, 64);
-      if (mode != kGlaLocal && hl == 0 && vc_ok) out[(int64_t)(row0 + c0 + j) * heads * vdim + v_col + vc] = acc;
+      if (hl == 0 && vc_ok) out[(int64_t)(row0 + c0 + j) * heads * vdim + v_col + vc] = acc;
     }
   }
-  if (mode == kGlaFinal && !last_seg) return;                // its end state is the next segment's start: known already
-  float* end = mode == kGlaLocal ? seg_out : sp;
   if (vc_ok) {
 #pragma unroll
     for (int b = 0; b < NDB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int c = 32 * b + 8 * (r / 4) + 4 * hl + (r % 4);
-        if (c < dim) end[(int64_t)c * vdim + vc] = S[b][r];
+        if (c < dim) sp[(int64_t)c * vdim + vc] = S[b][r];
       }
-  }
-  if (mode == kGlaLocal && blockIdx.z == 0) {
-    __syncthreads();
-    for (int c = threadIdx.x; c < dim; c += blockDim.x) seg_decay[((int64_t)blockIdx.x * heads + h) * dim + c] = dsum[c];
-  }
-}
-
-// seg_state[segment] (its end state from the empty state) -> the state at the segment's end:
-// S_end(j) = diag(e^(D_j)) S_end(j - 1) + local(j), S_end(-1) = the slot's state (nothing for a new sequence)
-__global__ __launch_bounds__(256) void gla_scan_kernel(
-    float* __restrict__ seg_state, const float* __restrict__ seg_decay, const float* __restrict__ state,
-    const int32_t* __restrict__ q_start, const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot,
-    int heads, int dim, int vdim) {
-  const int seq = blockIdx.x, h = blockIdx.y;
-  const int e = blockIdx.z * 256 + threadIdx.x;
-  const int size = dim * vdim;
-  if (e >= size) return;
-  const int c = e / vdim;
-  const int n = q_start[seq + 1] - q_start[seq];
-  const int segs = (n + kGlaSegment - 1) / kGlaSegment;
-  if (segs <= 1) return;
-  int first = 0;
-  for (int s = 0; s < seq; ++s) first += (q_start[s + 1] - q_start[s] + kGlaSegment - 1) / kGlaSegment;
-  float S = ctx_len[seq] == 0 ? 0.0f : state[((int64_t)state_slot[seq] * heads + h) * size + e];
-  // eight segments at a time: their loads do not wait for one another
-  const int64_t stride = (int64_t)heads * size, dstride = (int64_t)heads * dim;
-  float* p = seg_state + ((int64_t)first * heads + h) * size + e;
-  const float* d = seg_decay + ((int64_t)first * heads + h) * dim + c;
-  for (int j0 = 0; j0 + 1 < segs; j0 += 8) {
-    float local[8], keep[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      local[i] = j0 + i + 1 < segs ? p[(j0 + i) * stride] : 0.0f;
-      keep[i] = j0 + i + 1 < segs ? expf(d[(j0 + i) * dstride]) : 0.0f;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (j0 + i + 1 < segs) {
-        S = keep[i] * S + local[i];
-        p[(j0 + i) * stride] = S;
-      }
-    }
   }
 }
 
 template <typename T, int NDB>
 int launch_gla(float* out, const void* q, const void* k, const void* v, int64_t in_stride, const void* decay_pre,
                int64_t decay_stride, const float* decay_bias, float tau, float q_scale, float* state,
-               const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot, int64_t rows, int num_seqs,
-               int max_query_len, int heads, int dim, int vdim, float* workspace, hipStream_t stream) {
+               const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot, int num_seqs, int heads, int dim,
+               int vdim, hipStream_t stream) {
   const int vblocks = (vdim + 31) / 32;
   const int waves = std::min(vblocks, 8);
   const size_t lds_bytes =
-      (size_t)(3 * kGlaChunk * (NDB * 32 + 4) + kGlaChunk * waves * 32 + 9 * NDB * 32 + 16) * sizeof(float);
+      (size_t)(3 * kGlaChunk * (NDB * 32 + 4) + kGlaChunk * waves * 32 + 8 * NDB * 32 + 16) * sizeof(float);
   auto kernel = gla_kernel<T, NDB>;
   static size_t allowed = 64 * 1024;                         // per instantiation
   if (lds_bytes > allowed) {
@@ -340,26 +278,9 @@ int launch_gla(float* out, const void* q, const void* k, const void* v, int64_t 
   }
   const unsigned zgroups = (unsigned)((vblocks + waves - 1) / waves);
   const float inv_tau = 1.0f / tau;
-  if (workspace == nullptr || max_query_len <= 2 * kGlaSegment) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)num_seqs, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream,
-                       out, q, k, v, in_stride, decay_pre, decay_stride, decay_bias, inv_tau, q_scale, state, q_start,
-                       ctx_len, state_slot, num_seqs, heads, dim, vdim, kGlaWhole, (float*)nullptr, (float*)nullptr);
-    SW_CHECK_LAUNCH();
-    return SW_OK;
-  }
-  const int64_t items = rows / kGlaSegment + num_seqs;
-  float* seg_state = workspace;
-  float* seg_decay = workspace + items * heads * (int64_t)dim * vdim;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)items, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream, out,
-                     q, k, v, in_stride, decay_pre, decay_stride, decay_bias, inv_tau, q_scale, state, q_start, ctx_len,
-                     state_slot, num_seqs, heads, dim, vdim, kGlaLocal, seg_state, seg_decay);
-  SW_CHECK_LAUNCH();
-  hipLaunchKernelGGL(gla_scan_kernel, dim3((unsigned)num_seqs, (unsigned)heads, (unsigned)((dim * vdim + 255) / 256)),
-                     dim3(256), 0, stream, seg_state, seg_decay, state, q_start, ctx_len, state_slot, heads, dim, vdim);
-  SW_CHECK_LAUNCH();
-  hipLaunchKernelGGL(kernel, dim3((unsigned)items, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream, out,
-                     q, k, v, in_stride, decay_pre, decay_stride, decay_bias, inv_tau, q_scale, state, q_start, ctx_len,
-                     state_slot, num_seqs, heads, dim, vdim, kGlaFinal, seg_state, seg_decay);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)num_seqs, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream, out, q, k, v,
+                     in_stride, decay_pre, decay_stride, decay_bias, inv_tau, q_scale, state, q_start, ctx_len, state_slot, heads,
+                     dim, vdim);
   SW_CHECK_LAUNCH();
   return SW_OK;
 }
@@ -367,8 +288,8 @@ int launch_gla(float* out, const void* q, const void* k, const void* v, int64_t 
 }  // namespace swm
 
 extern "C" int64_t swm_gla_workspace_floats(int64_t rows, int num_seqs, int max_query_len, int heads, int dim, int vdim) {
-  if (max_query_len <= 2 * swm::kGlaSegment) return 0;
-  return (rows / swm::kGlaSegment + num_seqs) * (int64_t)heads * dim * ((int64_t)vdim + 1);
+  (void)vdim;
+  return max_query_len <= swm::kGlaWalkFrom ? 0 : swm::linear_walk_floats(rows, num_seqs, heads, dim);
 }
 
 extern "C" int swm_gla(float* out, const void* q, const void* k, const void* v, int64_t in_stride,
@@ -383,12 +304,16 @@ extern "C" int swm_gla(float* out, const void* q, const void* k, const void* v, 
                "gla: %d heads, key size %d (at most 256), value size %d", heads, dim, vdim);
   SW_CHECK_ARG(tau > 0.0f, "gla: tau must be positive");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (workspace != nullptr && max_query_len > kGlaWalkFrom) {
+    const LinearStep step{out, q, k, v, in_stride, in_stride, state, q_start, ctx_len, state_slot, rows, num_seqs, heads, dim, vdim,
+                          workspace};
+    return gla_walk(step, decay_pre, decay_stride, decay_bias, 1.0f / tau, q_scale, act_dtype, s);
+  }
 #define SWM_GLA_CASE(N)                                                                                             \
   case N:                                                                                                           \
     SWM_DISPATCH_ACT(act_dtype, return (launch_gla<T, N>(out, q, k, v, in_stride, decay_pre, decay_stride,          \
                                                          decay_bias, tau, q_scale, state, q_start, ctx_len,         \
-                                                         state_slot, rows, num_seqs, max_query_len, heads, dim,     \
-                                                         vdim, workspace, s)););                                    \
+                                                         state_slot, num_seqs, heads, dim, vdim, s)););             \
     break;
   switch ((dim + 31) / 32) {
     SWM_GLA_CASE(1)

@@ -14,15 +14,15 @@
 // key coordinate 32 b + 8 (r / 4) + 4 (l / 32) + r % 4).  That layout is also what the A operand of S^T q needs
 // when q is read in the same order of coordinates, so the state never moves between registers.  A decoded
 // token is a chunk of one.
-#include "mixers_common.cuh"
+#include "linear_walk.cuh"
 
 namespace swm {
 
 using f32x16 = __attribute__((ext_vector_type(16))) float;
 constexpr int kChunk = 32;
-constexpr int kWhole = 0, kLocal = 1, kFinal = 2;
-constexpr int kSegment = 128;          // tokens per segment of a long run (a multiple of kChunk)
-
+// Steps whose longest run has more tokens than this go to linear_walk.hip (us here / there, with norm and gate, the host's 30 a
+// call included: 1 x 16 heads of 128, 16 tokens 33 / 33, 31 tokens 37 / 33, 64 tokens 54 / 34, 1000 tokens 665 / 76).
+constexpr int kWalkFrom = 16;
 
 // NDB: 32-coordinate blocks of the key size.  A workgroup owns (sequence, head) and up to 8 blocks of 32 value
 // channels, one wave each; the chunk's silu(q) and silu(k) are staged once in LDS for all of them.
@@ -31,8 +31,7 @@ template <typename TQ, typename T, bool SILU, int NDB>
 __global__ __launch_bounds__(512) void lightning_kernel(
     float* __restrict__ out, const void* __restrict__ q, const void* __restrict__ k, int64_t qk_stride,
     const void* __restrict__ v, int64_t v_stride, const float* __restrict__ decay, float* __restrict__ state, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int num_seqs, int heads, int dim,
-    int vdim, int mode, int seg_len, float* __restrict__ seg_state) {
+    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int dim, int vdim) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int DS = NDB * 32 + 4;                           // row stride of the staged tiles
   float* Qs = lds;                                           // [32][DS]
@@ -41,21 +40,10 @@ __global__ __launch_bounds__(512) void lightning_kernel(
   const int h = blockIdx.y;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 31, hl = lane >> 5;
   const int vb = blockIdx.z * (blockDim.x >> 6) + wave;
-  // mode 0: blockIdx.x is a sequence and its whole run is taken from the slot's state to the slot's state.
-  // Long runs are cut into segments of seg_len tokens that run side by side: mode 1 takes every segment but a
-  // sequence's last from the EMPTY state and leaves its end state in seg_state[segment]; a scan (below) turns these
-  // into the states at the segments' ends; mode 2 then takes every segment from its true start state (the slot's for
-  // a sequence's first segment), writes the outputs, and a sequence's last segment leaves its state in the slot.
-  int seq = blockIdx.x, tok0 = 0, n;
-  if (mode == kWhole) {
-    n = q_start[seq + 1] - q_start[seq];
-  } else {
-    n = find_query_tile(q_start, num_seqs, blockIdx.x, seg_len, &seq, &tok0);
-  }
+  // blockIdx.x is a sequence; its whole run goes from the slot's state to the slot's state
+  const int seq = blockIdx.x, n = q_start[seq + 1] - q_start[seq];
   if (n <= 0) return;                                        // the whole workgroup
-  const int row0 = q_start[seq] + tok0;
-  const bool last_seg = tok0 + n == q_start[seq + 1] - q_start[seq];
-  if (mode == kLocal && last_seg) return;
+  const int row0 = q_start[seq];
   const float lam = decay[h];
   if (threadIdx.x == 0) {
     float p = 1.0f;
@@ -68,17 +56,14 @@ __global__ __launch_bounds__(512) void lightning_kernel(
   const bool vc_ok = vc < vdim;
   float* sp = state + ((int64_t)state_slot[seq] * heads + h) * (int64_t)dim * vdim;
 
-  float* seg_out = seg_state + ((int64_t)blockIdx.x * heads + h) * (int64_t)dim * vdim;      // modes 1, 2 only
-  const float* start = (mode == kFinal && tok0 > 0) ? seg_out - (int64_t)heads * dim * vdim : sp;
-
   f32x16 S[NDB];
-  const bool fresh = mode == kLocal || (tok0 == 0 && ctx_len[seq] == 0);
+  const bool fresh = ctx_len[seq] == 0;
 #pragma unroll
   for (int b = 0; b < NDB; ++b)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int c = 32 * b + 8 * (r / 4) + 4 * hl + (r % 4);
-      S[b][r] = (!fresh && vc_ok && c < dim) ? start[(int64_t)c * vdim + vc] : 0.0f;
+      S[b][r] = (!fresh && vc_ok && c < dim) ? sp[(int64_t)c * vdim + vc] : 0.0f;
     }
 
   const int64_t qk_col = (int64_t)h * dim, v_col = (int64_t)h * vdim;
@@ -170,7 +155,7 @@ __global__ __launch_bounds__(512) void lightning_kernel(
         }
       }
     }
-    if (mode != kLocal && li < cn && vb * 32 < vdim) {
+    if (li < cn && vb * 32 < vdim) {
       float* dst = out + (int64_t)(row0 + c0 + li) * heads * vdim + v_col + vb * 32;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -194,60 +179,21 @@ __global__ __launch_bounds__(512) void lightning_kernel(
       }
     }
   }
-  if (mode == kFinal && !last_seg) return;                  // its end state is the next segment's start: known already
-  float* end = mode == kLocal ? seg_out : sp;
   if (vc_ok) {
 #pragma unroll
     for (int b = 0; b < NDB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int c = 32 * b + 8 * (r / 4) + 4 * hl + (r % 4);
-        if (c < dim) end[(int64_t)c * vdim + vc] = S[b][r];
+        if (c < dim) sp[(int64_t)c * vdim + vc] = S[b][r];
       }
-  }
-}
-
-// seg_state[segment] (its end state from the empty state) -> the state at the segment's end:
-// S_end(j) = decay^seg_len S_end(j - 1) + local(j), S_end(-1) = the slot's state (nothing for a new sequence)
-__global__ __launch_bounds__(256) void lightning_scan_kernel(
-    float* __restrict__ seg_state, const float* __restrict__ state, const float* __restrict__ decay,
-    const int32_t* __restrict__ q_start, const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot,
-    int heads, int dim, int vdim, int seg_len) {
-  const int seq = blockIdx.x, h = blockIdx.y;
-  const int e = blockIdx.z * 256 + threadIdx.x;
-  const int size = dim * vdim;
-  if (e >= size) return;
-  const int n = q_start[seq + 1] - q_start[seq];
-  const int segs = (n + seg_len - 1) / seg_len;
-  if (segs <= 1) return;
-  int first = 0;
-  for (int s = 0; s < seq; ++s) first += (q_start[s + 1] - q_start[s] + seg_len - 1) / seg_len;
-  float keep = 1.0f;
-  const float lam = decay[h];
-  for (int i = 0; i < seg_len; ++i) keep *= lam;
-  float S = ctx_len[seq] == 0 ? 0.0f : state[((int64_t)state_slot[seq] * heads + h) * size + e];
-  // eight segments at a time: their loads do not wait for one another
-  const int64_t stride = (int64_t)heads * size;
-  float* p = seg_state + ((int64_t)first * heads + h) * size + e;
-  for (int j0 = 0; j0 + 1 < segs; j0 += 8) {
-    float local[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) local[i] = j0 + i + 1 < segs ? p[(j0 + i) * stride] : 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (j0 + i + 1 < segs) {
-        S = keep * S + local[i];
-        p[(j0 + i) * stride] = S;
-      }
-    }
   }
 }
 
 template <typename TQ, typename T, bool SILU, int NDB>
 int launch_lightning(float* out, const void* q, const void* k, int64_t qk_stride, const void* v, int64_t v_stride, const float* decay,
                      float* state, const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot,
-                     int64_t rows, int num_seqs, int max_query_len, int heads, int dim, int vdim, float* seg_state,
-                     hipStream_t stream) {
+                     int num_seqs, int heads, int dim, int vdim, hipStream_t stream) {
   const int vblocks = (vdim + 31) / 32;
   const int waves = std::min(vblocks, 8);
   const size_t lds_bytes = (size_t)(2 * kChunk * (NDB * 32 + 4) + kChunk + 2) * sizeof(float);
@@ -259,25 +205,8 @@ int launch_lightning(float* out, const void* q, const void* k, int64_t qk_stride
     raised = true;
   }
   const unsigned zgroups = (unsigned)((vblocks + waves - 1) / waves);
-  if (seg_state == nullptr || max_query_len <= 2 * kSegment) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)num_seqs, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream,
-                       out, q, k, qk_stride, v, v_stride, decay, state, q_start, ctx_len, state_slot, num_seqs, heads, dim, vdim,
-                       kWhole, kSegment, seg_state);
-    SW_CHECK_LAUNCH();
-    return SW_OK;
-  }
-  const unsigned items = (unsigned)(rows / kSegment + num_seqs);
-  hipLaunchKernelGGL(kernel, dim3(items, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream, out, q, k,
-                     qk_stride, v, v_stride, decay, state, q_start, ctx_len, state_slot, num_seqs, heads, dim, vdim, kLocal, kSegment,
-                     seg_state);
-  SW_CHECK_LAUNCH();
-  hipLaunchKernelGGL(lightning_scan_kernel, dim3((unsigned)num_seqs, (unsigned)heads, (unsigned)((dim * vdim + 255) / 256)),
-                     dim3(256), 0, stream, seg_state, state, decay, q_start, ctx_len, state_slot, heads, dim, vdim,
-                     kSegment);
-  SW_CHECK_LAUNCH();
-  hipLaunchKernelGGL(kernel, dim3(items, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream, out, q, k,
-                     qk_stride, v, v_stride, decay, state, q_start, ctx_len, state_slot, num_seqs, heads, dim, vdim, kFinal, kSegment,
-                     seg_state);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)num_seqs, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream, out, q, k,
+                     qk_stride, v, v_stride, decay, state, q_start, ctx_len, state_slot, heads, dim, vdim);
   SW_CHECK_LAUNCH();
   return SW_OK;
 }
@@ -286,8 +215,8 @@ int launch_lightning(float* out, const void* q, const void* k, int64_t qk_stride
 
 extern "C" int64_t swm_lightning_workspace_floats(int64_t rows, int num_seqs, int max_query_len, int heads, int dim,
                                                   int vdim) {
-  if (max_query_len <= 2 * swm::kSegment) return 0;
-  return (rows / swm::kSegment + num_seqs) * (int64_t)heads * dim * vdim;
+  (void)vdim;
+  return max_query_len <= swm::kWalkFrom ? 0 : swm::linear_walk_floats(rows, num_seqs, heads, dim);
 }
 
 extern "C" int swm_lightning(float* out, const void* q, const void* k, const void* v, int64_t in_stride,
@@ -300,12 +229,16 @@ extern "C" int swm_lightning(float* out, const void* q, const void* k, const voi
   SW_CHECK_ARG(heads > 0 && heads < 65536 && dim > 0 && dim <= 256 && vdim > 0 && (vdim + 255) / 256 < 65536,
                "lightning: %d heads, key size %d (at most 256), value size %d", heads, dim, vdim);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define SWM_LIGHTNING_CASE(N)                                                                                             \
-  case N:                                                                                                                 \
-    SWM_DISPATCH_ACT(act_dtype, return (launch_lightning<T, T, true, N>(out, q, k, in_stride, v, in_stride, decay, state, \
-                                                                        q_start, ctx_len, state_slot, rows, num_seqs,     \
-                                                                        max_query_len, heads, dim, vdim, workspace,       \
-                                                                        s)););                                            \
+  if (workspace != nullptr && max_query_len > kWalkFrom) {
+    const LinearStep step{out, q, k, v, in_stride, in_stride, state, q_start, ctx_len, state_slot, rows, num_seqs, heads, dim, vdim,
+                          workspace};
+    return lightning_walk(step, decay, true, act_dtype, act_dtype, s);
+  }
+#define SWM_LIGHTNING_CASE(N)                                                                                              \
+  case N:                                                                                                                  \
+    SWM_DISPATCH_ACT(act_dtype, return (launch_lightning<T, T, true, N>(out, q, k, in_stride, v, in_stride, decay, state,  \
+                                                                        q_start, ctx_len, state_slot, num_seqs, heads,     \
+                                                                        dim, vdim, s)););                                  \
     break;
   switch ((dim + 31) / 32) {
     SWM_LIGHTNING_CASE(1)
@@ -331,12 +264,16 @@ extern "C" int swm_retention(float* out, const float* q, const float* k, int64_t
   SW_CHECK_ARG(heads > 0 && heads < 65536 && dim > 0 && dim <= 256 && vdim > 0 && (vdim + 255) / 256 < 65536,
                "retention: %d heads, key size %d (at most 256), value size %d", heads, dim, vdim);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (workspace != nullptr && max_query_len > kWalkFrom) {
+    const LinearStep step{out, q, k, v, qk_stride, v_stride, state, q_start, ctx_len, state_slot, rows, num_seqs, heads, dim, vdim,
+                          workspace};
+    return lightning_walk(step, decay, false, SW_F32, act_dtype, s);
+  }
 #define SWM_RETENTION_CASE(N)                                                                                          \
   case N:                                                                                                              \
     SWM_DISPATCH_ACT(act_dtype, return (launch_lightning<float, T, false, N>(out, q, k, qk_stride, v, v_stride, decay, \
                                                                              state, q_start, ctx_len, state_slot,      \
-                                                                             rows, num_seqs, max_query_len, heads,     \
-                                                                             dim, vdim, workspace, s)););              \
+                                                                             num_seqs, heads, dim, vdim, s)););        \
     break;
   switch ((dim + 31) / 32) {
     SWM_RETENTION_CASE(1)

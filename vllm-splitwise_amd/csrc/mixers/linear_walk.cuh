@@ -1,0 +1,34 @@
+// Long runs of the linear-attention rules (linear_walk.hip): arguments shared with gla.hip and lightning.hip.
+#pragma once
+
+#include "mixers_common.cuh"
+
+namespace swm {
+
+constexpr int kLwChunk = 32;
+
+struct LinearStep {
+  float* out;
+  const void *q, *k, *v;
+  int64_t qk_stride, v_stride;          // elements between rows
+  float* state;
+  const int32_t *q_start, *ctx_len, *state_slot;
+  int64_t rows;
+  int num_seqs, heads, dim, vdim;
+  float* workspace;
+};
+
+// floats of scratch: per chunk of 32 tokens and head the scaled queries [32][dp], the scaled keys [dp][32], the decays [dp] and
+// the chunk's weights among its own tokens [32][32], dp = the key size in whole blocks of 32
+inline int64_t linear_walk_floats(int64_t rows, int num_seqs, int heads, int dim) {
+  const int64_t dp = (dim + 31) / 32 * 32;
+  return (rows / kLwChunk + num_seqs) * heads * (65 * dp + 1024);
+}
+
+// S <- diag(a_t) S + k v^T with a_t = sigmoid(decay_pre + bias)^(1 / tau) per key channel, o = S^T (q_scale q)
+int gla_walk(const LinearStep& a, const void* decay_pre, int64_t decay_stride, const float* decay_bias, float inv_tau, float q_scale,
+             int act_dtype, hipStream_t stream);
+// S <- decay_h S + k v^T, o = S^T q; silu: q, k and v pass a silu first.  q and k in q_dtype, v in v_dtype.
+int lightning_walk(const LinearStep& a, const float* decay, bool silu, int q_dtype, int v_dtype, hipStream_t stream);
+
+}  // namespace swm

@@ -1,0 +1,515 @@
+// Linear attention over long runs:  S_t = diag(a_t) S_(t-1) + k_t v_t^T,  o_t = S_t^T q_t,  S [key size, value size] fp32 carried
+// per sequence, with a decay per head and key channel (gla.hip) or one constant per head (lightning.hip), in chunks of 32 tokens:
+//     O = A V + Q~ S_0,   S_n = diag(d) S_0 + K~^T V,
+//     Q~_i = q_i a_1 .. a_i,   K~_j = k_j a_(j+1) .. a_n,   d = a_1 .. a_n,   A[i, j] = sum_c q_ic k_jc a_(j+1) .. a_i   (j <= i)
+// A PROLOGUE, parallel over (chunk, head), writes Q~, K~^T, d and A; a WALK goes through a sequence's chunks.
+//
+// Every factor above is a product of decays and at most 1, so nothing overflows however strong they are.  Only A, as a matrix
+// product, needs its decays taken apart: between the chunk's halves of 16 tokens at the border, where both parts are again
+// at most 1; inside a half as p_i / p_j with p the half's running products.  A half in which some channel's product falls
+// below e^-kLwSafeLog has its 16 x 16 weights worked out on the vector units instead, with the decays multiplied up token by token.
+// Products are exponentials of running SUMS of log a, from the half's border towards the token: a decay near 1 (most are) has
+// few significant digits left once it is rounded to a float, and over thousands of tokens the state would show it.
+//
+// The walk's only chain is the state itself, an accumulation: a workgroup owns (sequence, head, 16 value channels), its wave b the
+// key coordinates 32 b .. 32 b + 31 in the accumulators of v_mfma_f32_16x16x4_f32 (lane l: channel l % 16; element r of tile i:
+// coordinate 32 b + 16 i + 4 (l / 16) + r), in the layout that the B operand of the next product wants.  Operands come straight
+// from memory into the A operands' registers, a chunk ahead; the waves' shares of Q~ S_0 meet in LDS behind the one barrier
+// of a chunk.  Workgroups that read the same chunks (the channels of a head) have numbers 8 apart: one XCD, one L2.
+//
+// Measured, two prompts of 4324 tokens together, 16 heads of 128, a decay per key channel: 676 + 20 us in segments of 128 tokens
+// taken twice, from nothing and from their true states, with a scan between (560 workgroups on 512 places: the second round
+// nearly empty); 52 us prologue and 139 us walk here.  Of the walk's 1.8 us a chunk the products, the exchange and its barrier
+// alone are 1.2 (38 products of 32 cycles are 0.5), the operands' way through the L1 0.5.  The prologue took 111 us with its
+// operands staged in LDS first.  Relative error of the end states against 64 bits: 1.3e-7 here, 2.2e-7 in segments.
+#include "linear_walk.cuh"
+
+#include <type_traits>
+
+namespace swm {
+
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+constexpr int kLwThreads = 256;
+constexpr int kLwChannels = 16;
+constexpr float kLwSafeLog = 12.0f;
+
+// log(sigmoid(x)) = min(x, 0) - log(1 + t), t = e^-|x|, the logarithm on the hardware's log2 with the rounding of 1 + t put back:
+// largest relative error over [-30, 30] 2.2e-7 (with log1pf 1.3e-7), root mean square 3.5e-8 (2.8e-8), a quarter of the instructions
+__device__ __forceinline__ float log_sigmoid(float x) {
+  const float t = expf(-fabsf(x)), u = 1.0f + t;
+  return fminf(x, 0.0f) - (0.69314718055994531f * __builtin_amdgcn_logf(u) + (t - (u - 1.0f)) * __builtin_amdgcn_rcpf(u));
+}
+__device__ __forceinline__ int64_t lw_record(int dp) { return 65 * (int64_t)dp + 1024; }
+
+// the 16 x 16 weights of rows Xr (queries) against rows Yr (keys): element r of lane l is row 4 (l / 16) + r, column l % 16
+__device__ __forceinline__ f32x4 lw_block(const float* X, const float* Y, int KS, int dp) {
+  const int lane = threadIdx.x & 63, li = lane & 15, gq = lane >> 4;
+  f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;
+  for (int c = 4 * gq; c < dp; c += 32) {
+    const float4 x = *reinterpret_cast<const float4*>(X + li * KS + c), y = *reinterpret_cast<const float4*>(Y + li * KS + c);
+    const float4 x1 = *reinterpret_cast<const float4*>(X + li * KS + c + 16), y1 = *reinterpret_cast<const float4*>(Y + li * KS + c + 16);
+    s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, y.x, s0, 0, 0, 0);
+    s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x1.x, y1.x, s1, 0, 0, 0);
+    s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, y.y, s0, 0, 0, 0);
+    s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x1.y, y1.y, s1, 0, 0, 0);
+    s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, y.z, s0, 0, 0, 0);
+    s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x1.z, y1.z, s1, 0, 0, 0);
+    s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, y.w, s0, 0, 0, 0);
+    s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x1.w, y1.w, s1, 0, 0, 0);
+  }
+  return s0 + s1;
+}
+
+// 8 neighbouring numbers of row `row`, zeros where the row or the channels are not there
+template <typename T>
+__device__ __forceinline__ void lw_load8(float (&x)[8], const void* p, int64_t at, int c, int dim, bool in, bool vec) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j] = 0.0f;
+  if (!in) return;
+  if (vec && c + 8 <= dim) {
+    if constexpr (sizeof(typename Conv<T>::store_t) == 2) {
+      ld_vec<T, 8>(x, p, at + c);
+    } else {
+      float lo[4], hi[4];
+      ld_vec<T, 4>(lo, p, at + c);
+      ld_vec<T, 4>(hi, p, at + c + 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = lo[j], x[4 + j] = hi[j];
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (c + j < dim) x[j] = ld<T>(p, at + c + j);
+  }
+}
+__device__ __forceinline__ void lw_put8(float* p, const float (&x)[8]) {
+  *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]);
+  *reinterpret_cast<float4*>(p + 4) = make_float4(x[4], x[5], x[6], x[7]);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kLwThreads, 3) void gla_walk_prep_kernel(const LinearStep a, const void* __restrict__ decay_pre,
+                                                                   int64_t decay_stride, const float* __restrict__ decay_bias,
+                                                                   float inv_tau, float q_scale, int dp) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int KS = dp + 4;
+  float* Qs = lds;                               // [32][KS] queries times p
+  float* Ks = Qs + kLwChunk * KS;                // [32][KS] keys divided by p
+  float* Ko = Ks + kLwChunk * KS;                // [16][KS] the first half's keys carried to its end
+  float* total = Ko + 16 * KS;                   // [2][dp] the halves' sums of log a
+  int* unsafe = reinterpret_cast<int*>(total + 2 * dp);                  // [2]
+  int seq = 0, tok0 = 0;
+  const int cn = find_query_tile(a.q_start, a.num_seqs, blockIdx.x, kLwChunk, &seq, &tok0);
+  if (cn <= 0) return;                           // the whole workgroup
+  const int h = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int64_t row0 = a.q_start[seq] + tok0;
+  float* rec = a.workspace + ((int64_t)blockIdx.x * a.heads + h) * lw_record(dp);
+  float* Qg = rec;                               // [32][dp]
+  float* Kt = rec + 32 * (int64_t)dp;            // [dp][32]
+  float* keep = rec + 64 * (int64_t)dp;          // [dp]
+  float* A = rec + 65 * (int64_t)dp;             // [32][32]
+  if (tid < 2) unsafe[tid] = 0;
+  __syncthreads();
+  // ---- a thread per (channel, half), its 16 tokens in registers; key sizes beyond 128 take a second round
+  const int half = __builtin_amdgcn_readfirstlane(tid / (kLwThreads / 2));
+  for (int c0 = 0; c0 < dp; c0 += kLwThreads / 2) {
+    const int c = c0 + tid % (kLwThreads / 2);
+    const bool mine = c < dp, in = c < a.dim;
+    float k[16], q[16], g[16], sum = 0.0f;
+    if (mine) {
+      const int col = h * a.dim + min(c, a.dim - 1);
+      const float bias = decay_bias != nullptr ? decay_bias[col] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {             // (the rows' addresses are uniform over the wave)
+        const int64_t row = row0 + min(16 * half + i, cn - 1);
+        k[i] = ld<T>(static_cast<const typename Conv<T>::store_t*>(a.k) + row * a.qk_stride, col);
+        q[i] = ld<T>(static_cast<const typename Conv<T>::store_t*>(a.q) + row * a.qk_stride, col);
+        g[i] = ld<T>(static_cast<const typename Conv<T>::store_t*>(decay_pre) + row * decay_stride, col);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const bool there = in && 16 * half + i < cn;         // rows beyond the chunk: no key, no decay
+        k[i] = there ? k[i] : 0.0f;
+        q[i] = there ? q[i] * q_scale : 0.0f;
+        g[i] = there ? log_sigmoid(g[i] + bias) * inv_tau : 0.0f;
+        sum += g[i];
+      }
+      total[half * dp + c] = sum;
+      if (!(sum >= -kLwSafeLog)) unsafe[half] = 1;
+    }
+    __syncthreads();
+    if (mine) {                                  // (in a half that is not safe the keys may overflow: they are put back below)
+      const float before = half ? expf(total[c]) : 1.0f, after = half ? 1.0f : expf(total[dp + c]);
+      if (half == 0) keep[c] = expf(total[c] + total[dp + c]);
+      float run = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {             // towards the half's end: queries, and keys for the half's own weights
+        run += g[i];
+        const float p = expf(run);
+        q[i] *= p;
+        Qs[(16 * half + i) * KS + c] = q[i];
+        Ks[(16 * half + i) * KS + c] = k[i] / p;
+        Qg[(16 * half + i) * dp + c] = q[i] * before;
+      }
+      run = 0.0f;
+#pragma unroll
+      for (int i = 15; i >= 0; --i) {            // towards its start: keys carried to the end
+        k[i] *= expf(run);
+        run += g[i];
+        if (half == 0) Ko[i * KS + c] = k[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 16; i += 4)
+        *reinterpret_cast<float4*>(Kt + c * 32 + 16 * half + i) =
+            make_float4(k[i] * after, k[i + 1] * after, k[i + 2] * after, k[i + 3] * after);
+    }
+  }
+  __syncthreads();
+  // ---- the chunk's weights: wave 0 and 1 the halves' own, wave 2 the second half's on the first
+  const int li = lane & 15, gq = lane >> 4;
+  if (wave < 3 && !(wave < 2 && unsafe[wave] != 0)) {
+    const int bi = wave == 0 ? 0 : 1, bj = wave == 1 ? 1 : 0;
+    const f32x4 w = lw_block(Qs + bi * 16 * KS, wave == 2 ? Ko : Ks + bj * 16 * KS, KS, dp);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 16 * bi + 4 * gq + r, j = 16 * bj + li;
+      A[i * 32 + j] = j <= i ? w[r] : 0.0f;
+    }
+  }
+  if (unsafe[0] == 0 && unsafe[1] == 0) return;  // uniform over the workgroup
+  __syncthreads();
+  for (int e = tid; e < kLwChunk * dp; e += kLwThreads) {    // the decays themselves in Qs, the keys as they are in Ks
+    const int r = e / dp, c = e - r * dp;
+    float d = 1.0f, k = 0.0f;
+    if (r < cn && c < a.dim) {
+      const int64_t col = (int64_t)h * a.dim + c;
+      const float z = ld<T>(decay_pre, (row0 + r) * decay_stride + col) + (decay_bias != nullptr ? decay_bias[col] : 0.0f);
+      d = expf(log_sigmoid(z) * inv_tau);
+      k = ld<T>(a.k, (row0 + r) * a.qk_stride + col);
+    }
+    Qs[r * KS + c] = d;
+    Ks[r * KS + c] = k;
+  }
+  __syncthreads();
+  for (int part = 0; part < 2; ++part) {
+    if (unsafe[part] == 0) continue;             // uniform over the workgroup
+    // 16 lanes share a key's channels; from the key on, its weight for one query after the other
+    const int j = 16 * part + (tid >> 4);
+    float sum[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sum[i] = 0.0f;
+    for (int c = tid & 15; c < a.dim; c += 16) {
+      float kd = Ks[j * KS + c];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int t = 16 * part + i;
+        if (t < j || t >= cn) continue;
+        if (t > j) kd *= Qs[t * KS + c];
+        sum[i] += ld<T>(a.q, (row0 + t) * a.qk_stride + (int64_t)h * a.dim + c) * q_scale * kd;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float w = lanes_sum<16>(sum[i]);
+      if ((tid & 15) == i) A[(16 * part + i) * 32 + j] = w;
+    }
+  }
+}
+
+// vec: rows of q and k lie on 16 bytes
+template <typename TQ, bool SILU>
+__global__ __launch_bounds__(kLwThreads) void lightning_walk_prep_kernel(const LinearStep a, const float* __restrict__ decay, int dp,
+                                                                         int vec) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int KS = dp + 4;
+  float* Qs = lds;                               // [32][KS]
+  float* Ks = Qs + kLwChunk * KS;                // [32][KS]
+  float* pw = Ks + kLwChunk * KS;                // [33] powers of the decay, by repeated multiplication
+  int seq = 0, tok0 = 0;
+  const int cn = find_query_tile(a.q_start, a.num_seqs, blockIdx.x, kLwChunk, &seq, &tok0);
+  if (cn <= 0) return;                           // the whole workgroup
+  const int h = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int64_t row0 = a.q_start[seq] + tok0;
+  float* rec = a.workspace + ((int64_t)blockIdx.x * a.heads + h) * lw_record(dp);
+  float* Qg = rec;
+  float* Kt = rec + 32 * (int64_t)dp;
+  float* keep = rec + 64 * (int64_t)dp;
+  float* A = rec + 65 * (int64_t)dp;
+  if (tid == 0) {
+    const double lam = decay[h];                 // 64 bits: a chunk's 32 roundings would add up over a long run
+    double p = 1.0;
+    for (int e = 0; e <= kLwChunk; ++e) {
+      pw[e] = (float)p;
+      p *= lam;
+    }
+  }
+  for (int e = tid; e < kLwChunk * dp / 8; e += kLwThreads) {
+    const int r = e / (dp / 8), c = (e - r * (dp / 8)) * 8;
+    const int64_t at = (row0 + r) * a.qk_stride + (int64_t)h * a.dim;
+    float q[8], k[8];
+    lw_load8<TQ>(q, a.q, at, c, a.dim, r < cn, vec != 0);
+    lw_load8<TQ>(k, a.k, at, c, a.dim, r < cn, vec != 0);
+    if (SILU) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {              // silu(0) = 0
+        q[j] = fast_siluf_(q[j]);
+        k[j] = fast_siluf_(k[j]);
+      }
+    }
+    lw_put8(Qs + r * KS + c, q);
+    lw_put8(Ks + r * KS + c, k);
+  }
+  __syncthreads();
+  for (int e = tid; e < kLwChunk * dp / 4; e += kLwThreads) {
+    const int r = e / (dp / 4), c = (e - r * (dp / 4)) * 4;
+    const float4 q = *reinterpret_cast<const float4*>(Qs + r * KS + c);
+    const float f = pw[r + 1];
+    *reinterpret_cast<float4*>(Qg + r * (int64_t)dp + c) = make_float4(q.x * f, q.y * f, q.z * f, q.w * f);
+  }
+  for (int e = tid; e < dp * 8; e += kLwThreads) {
+    const int c = e >> 3, t = (e & 7) * 4;
+    float k[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) k[j] = Ks[(t + j) * KS + c] * pw[max(cn - 1 - t - j, 0)];    // rows beyond the chunk are zeros
+    *reinterpret_cast<float4*>(Kt + (int64_t)c * 32 + t) = make_float4(k[0], k[1], k[2], k[3]);
+  }
+  for (int c = tid; c < dp; c += kLwThreads) keep[c] = pw[cn];
+  if (wave < 3) {
+    const int li = lane & 15, gq = lane >> 4, bi = wave == 0 ? 0 : 1, bj = wave == 1 ? 1 : 0;
+    const f32x4 w = lw_block(Qs + bi * 16 * KS, Ks + bj * 16 * KS, KS, dp);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 16 * bi + 4 * gq + r, j = 16 * bj + li;
+      A[i * 32 + j] = j <= i ? w[r] * pw[max(i - j, 0)] : 0.0f;
+    }
+  }
+}
+
+// What a chunk brings to a wave, in the layouts of the A operands (16 x 4: lane l is row l % 16, reduction index l / 16)
+template <typename TV>
+struct LwOperands {
+  f32x4 q[2][2];                                 // [16 tokens][16 coordinates]: token l % 16, coordinates 4 (l / 16) ..
+  f32x4 kt[2][2];                                // [16 coordinates][16 tokens]: coordinate l % 16, tokens 4 (l / 16) ..
+  f32x4 a[3];                                    // tiles (0, 0), (1, 0), (1, 1) of A: row l % 16, columns 4 (l / 16) ..
+  f32x4 keep[2];                                 // coordinates 16 i + 4 (l / 16) ..
+  typename Conv<TV>::store_t v[2][4];            // tokens 16 i + 4 (l / 16) + r of this lane's channel
+};
+
+template <typename TV, bool SILU, int NDB>
+__global__ __launch_bounds__(64 * NDB) void linear_walk_kernel(const LinearStep a) {
+  __shared__ f32x4 red[2][NDB][2][64];           // [chunk parity][wave][token tile][lane]: shares of Q~ S_0
+  constexpr int DP = NDB * 32;
+  const int vblocks = (a.vdim + kLwChannels - 1) / kLwChannels;
+  const int unit = (blockIdx.x >> 3) / vblocks * 8 + (blockIdx.x & 7), vb = (blockIdx.x >> 3) % vblocks;
+  if (unit >= a.num_seqs * a.heads) return;      // the whole workgroup
+  const int seq = unit / a.heads, h = unit - seq * a.heads;
+  const int b = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, gq = lane >> 4;
+  const int n = a.q_start[seq + 1] - a.q_start[seq];
+  if (n <= 0) return;                            // the whole workgroup
+  const int64_t row0 = a.q_start[seq];
+  int64_t chunk0 = 0;                            // this sequence's first chunk among the step's
+  for (int s = 0; s < seq; ++s) chunk0 += (a.q_start[s + 1] - a.q_start[s] + kLwChunk - 1) / kLwChunk;
+  const int vc = vb * kLwChannels + li;          // this lane's value channel
+  const bool vc_ok = vc < a.vdim;
+  float* sp = a.state + ((int64_t)a.state_slot[seq] * a.heads + h) * (int64_t)a.dim * a.vdim;
+  f32x4 S[2];
+  const bool fresh = a.ctx_len[seq] == 0;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int c = 32 * b + 16 * i + 4 * gq + r;
+      S[i][r] = (!fresh && vc_ok && c < a.dim) ? sp[(int64_t)c * a.vdim + vc] : 0.0f;
+    }
+  const typename Conv<TV>::store_t* vsrc = static_cast<const typename Conv<TV>::store_t*>(a.v) + row0 * a.v_stride +
+                                           (int64_t)h * a.vdim + (vc_ok ? vc : a.vdim - 1);
+  const int chunks = (n + kLwChunk - 1) / kLwChunk;
+  using Ops = LwOperands<TV>;
+  auto fetch = [&](Ops& x, int ci) {
+    const float* rec = a.workspace + ((chunk0 + ci) * a.heads + h) * lw_record(DP);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        x.q[i][j] = *reinterpret_cast<const f32x4*>(rec + (16 * i + li) * DP + 32 * b + 16 * j + 4 * gq);
+        x.kt[i][j] = *reinterpret_cast<const f32x4*>(rec + 32 * DP + (32 * b + 16 * i + li) * 32 + 16 * j + 4 * gq);
+      }
+      x.keep[i] = *reinterpret_cast<const f32x4*>(rec + 64 * DP + 32 * b + 16 * i + 4 * gq);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x.v[i][r] = vsrc[min(ci * kLwChunk + 16 * i + 4 * gq + r, n - 1) * a.v_stride];
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      x.a[i] = *reinterpret_cast<const f32x4*>(rec + 65 * DP + (i == 0 ? 0 : 16 * 32) + (i == 2 ? 16 : 0) + li * 32 + 4 * gq);
+  };
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 av[2], qs[2];
+  // The outputs of a chunk: its shares of Q~ S_0 meet behind a barrier and are read while the next chunk's products run; the
+  // token tiles are finished by different waves, in turn.
+  f32x4 part[NDB], own[2];
+  auto collect = [&](int ci) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if ((2 * ci + i) % NDB != b) continue;     // wave-uniform
+      if (NDB > 1) {
+#pragma unroll
+        for (int w = 0; w < NDB; ++w) part[w] = red[ci & 1][w][i][lane];
+      } else {
+        own[i] = qs[i];
+      }
+    }
+  };
+  auto finish = [&](int ci) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if ((2 * ci + i) % NDB != b) continue;     // wave-uniform
+      f32x4 o = av[i];
+      if (NDB > 1) {
+#pragma unroll
+        for (int w = 0; w < NDB; ++w) o += part[w];
+      } else {
+        o += own[i];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = ci * kLwChunk + 16 * i + 4 * gq + r;
+        if (vc_ok && t < n) a.out[((row0 + t) * a.heads + h) * (int64_t)a.vdim + vc] = o[r];
+      }
+    }
+  };
+  auto chunk = [&](const Ops& x, int ci) {
+    if (ci > 0) collect(ci - 1);
+    f32x4 v[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {              // (the padding read some other token's value)
+        const float y = ci * kLwChunk + 16 * i + 4 * gq + r < n ? Conv<TV>::to_float(x.v[i][r]) : 0.0f;
+        v[i][r] = SILU ? fast_siluf_(y) : y;
+      }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) qs[i] = zero;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) qs[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][j][r], S[j][r], qs[i], 0, 0, 0);
+    f32x4 add[2] = {zero, zero};                 // summed by itself: the state is rounded once a chunk, not once a token
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) add[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kt[i][j][r], v[j][r], add[i], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) S[i] = S[i] * x.keep[i] + add[i];
+    if (ci > 0) finish(ci - 1);
+    if (NDB > 1) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) red[ci & 1][b][i][lane] = qs[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if ((2 * ci + i) % NDB != b) continue;     // wave-uniform
+      av[i] = zero;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        av[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.a[i][r], v[0][r], av[i], 0, 0, 0);
+        if (i == 1) av[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.a[2][r], v[1][r], av[i], 0, 0, 0);
+      }
+    }
+    if (NDB > 1) __syncthreads();                // (two buffers: nobody is more than a chunk ahead of a reader)
+  };
+  // (the barriers of the schedule keep a chunk's loads in front of the products of the chunk before it)
+  Ops x0, x1;
+  fetch(x0, 0);
+#pragma unroll 1
+  for (int ci = 0; ci < chunks; ci += 2) {       // uniform over the workgroup: every wave meets every barrier
+    fetch(x1, min(ci + 1, chunks - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    chunk(x0, ci);
+    if (ci + 1 >= chunks) break;
+    fetch(x0, min(ci + 2, chunks - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    chunk(x1, ci + 1);
+  }
+  collect(chunks - 1);
+  finish(chunks - 1);
+  if (vc_ok) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int c = 32 * b + 16 * i + 4 * gq + r;
+        if (c < a.dim) sp[(int64_t)c * a.vdim + vc] = S[i][r];
+      }
+  }
+}
+
+template <typename K>
+inline hipError_t lw_allow_lds(K kernel, size_t bytes) {
+  if (bytes <= 64 * 1024) return hipSuccess;
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
+template <typename TV, bool SILU>
+int launch_walk(const LinearStep& a, hipStream_t stream) {
+  const int64_t units = ((int64_t)a.num_seqs * a.heads + 7) / 8 * 8;
+  const int64_t groups = units * ((a.vdim + kLwChannels - 1) / kLwChannels);
+  SW_CHECK_ARG(groups < (1ll << 31), "linear attention: too many sequences and heads");
+#define SWM_LW_CASE(N)                                                                                                 \
+  case N:                                                                                                              \
+    hipLaunchKernelGGL((linear_walk_kernel<TV, SILU, N>), dim3((unsigned)groups), dim3(64 * N), 0, stream, a);         \
+    break;
+  switch ((a.dim + 31) / 32) {
+    SWM_LW_CASE(1)
+    SWM_LW_CASE(2)
+    SWM_LW_CASE(3)
+    SWM_LW_CASE(4)
+    SWM_LW_CASE(5)
+    SWM_LW_CASE(6)
+    SWM_LW_CASE(7)
+    SWM_LW_CASE(8)
+  }
+#undef SWM_LW_CASE
+  SW_CHECK_LAUNCH();
+  return SW_OK;
+}
+
+inline bool lw_aligned(const LinearStep& a, int dtype) {
+  const int per16 = dtype == SW_F32 ? 4 : 8;
+  return a.dim % 8 == 0 && a.qk_stride % per16 == 0 &&
+         (reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k)) % 16 == 0;
+}
+
+int gla_walk(const LinearStep& a, const void* decay_pre, int64_t decay_stride, const float* decay_bias, float inv_tau, float q_scale,
+             int act_dtype, hipStream_t stream) {
+  const int dp = (a.dim + 31) / 32 * 32;
+  const size_t bytes = sizeof(float) * (80 * (size_t)(dp + 4) + 2 * dp + 4);
+  const dim3 grid((unsigned)(a.rows / kLwChunk + a.num_seqs), (unsigned)a.heads);       // an upper bound of the chunks
+  SWM_DISPATCH_ACT(act_dtype, SW_CHECK_HIP(lw_allow_lds(gla_walk_prep_kernel<T>, bytes));
+                   hipLaunchKernelGGL(gla_walk_prep_kernel<T>, grid, dim3(kLwThreads), bytes, stream, a, decay_pre, decay_stride,
+                                      decay_bias, inv_tau, q_scale, dp);
+                   SW_CHECK_LAUNCH();
+                   return (launch_walk<T, false>(a, stream)););
+}
+
+int lightning_walk(const LinearStep& a, const float* decay, bool silu, int q_dtype, int v_dtype, hipStream_t stream) {
+  const int dp = (a.dim + 31) / 32 * 32;
+  const size_t bytes = sizeof(float) * (64 * (size_t)(dp + 4) + kLwChunk + 4);
+  const int vec = lw_aligned(a, q_dtype);
+  const dim3 grid((unsigned)(a.rows / kLwChunk + a.num_seqs), (unsigned)a.heads);       // an upper bound of the chunks
+  if (silu) {                                    // one projection: q, k and v of one type
+    SWM_DISPATCH_ACT(q_dtype, SW_CHECK_HIP(lw_allow_lds(lightning_walk_prep_kernel<T, true>, bytes));
+                     hipLaunchKernelGGL((lightning_walk_prep_kernel<T, true>), grid, dim3(kLwThreads), bytes, stream, a, decay, dp, vec);
+                     SW_CHECK_LAUNCH();
+                     return (launch_walk<T, true>(a, stream)););
+  }
+  SW_CHECK_HIP(lw_allow_lds(lightning_walk_prep_kernel<float, false>, bytes));
+  hipLaunchKernelGGL((lightning_walk_prep_kernel<float, false>), grid, dim3(kLwThreads), bytes, stream, a, decay, dp, vec);
+  SW_CHECK_LAUNCH();
+  SWM_DISPATCH_ACT(v_dtype, return (launch_walk<T, false>(a, stream)););
+}
+
+}  // namespace swm
