@@ -66,3 +66,49 @@ def test_prompt_steps_agree_with_the_general_kernel(H, G, d, dv, page, option):
         outs.append(out.float())
     torch.testing.assert_close(outs[0], outs[1], atol=2e-4, rtol=2.0 ** -7)
     assert outs[0].isfinite().all() and outs[0].abs().max() > 0.1
+
+
+@pytest.mark.parametrize("H,G,d,dv,page", [(4, 4, 128, 128, 16), (8, 2, 64, 96, 16), (6, 2, 40, 24, 8), (8, 1, 16, 8, 32),
+                                           (5, 1, 104, 128, 12)])
+@pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "sink", "learned sink", "sigmoid", "values in the keys"])
+@pytest.mark.parametrize("long", [0, 1, 2])
+def test_decode_steps_agree_with_the_general_kernel(H, G, d, dv, page, option, long):
+    """Few query rows per sequence and key/value head: one or two sets of four, one or several workgroups per sequence (the
+    step's longest context decides), contexts at the edges of the 32-key tiles.  Same bound as above."""
+    from splitwise_amd import _C
+    most = 8 // (H // G)                                     # tokens of a sequence
+    lengths = [[(0, 1), (5, 1), (30, 1), (31, 1), (32, most), (200, 1), (256, most)], [(900, 1), (2300, most), (31, 1)],
+               [(4001, 1)]][long]
+    batch, pages = _step(lengths, page)
+    g = torch.Generator(device=DEV).manual_seed(H * 100 + d + long)
+    rows = sum(n for _, n in lengths)
+    if option == "values in the keys" and G > 1:
+        dv = d
+    kc = torch.randn(pages, page, G * d, generator=g, device=DEV).to(torch.bfloat16)
+    vc = torch.randn(pages, page, G * dv, generator=g, device=DEV).to(torch.bfloat16)
+    kc[:2], vc[:2] = float("nan"), float("nan")              # pages that no table names
+    if option == "values in the keys":
+        dv, vc = min(d, dv) // 8 * 8, None
+    else:                                                    # slots behind a sequence's end have never been written
+        for i, (c, n) in enumerate(lengths):
+            if (c + n) % page:
+                last = int(batch.block_tables[i, (c + n) // page])
+                kc[last, (c + n) % page:], vc[last, (c + n) % page:] = float("nan"), float("nan")
+            if option == "window" and c > 3 * page + 37:     # pages behind a window may be somebody else's by now
+                batch.block_tables[i, :(c - 36) // page] = 0
+    q = torch.randn(rows * H * d + 4, generator=g, device=DEV) * 2
+    gate = torch.randn(rows, H * dv + 3, generator=g, device=DEV).to(torch.bfloat16)[:, 3:]
+    kw = {"cap": dict(softcap=4.0), "window": dict(window=37), "chunk": dict(chunk=48), "sink": dict(sink=True),
+          "learned sink": dict(sink=torch.linspace(-3.0, 9.0, H, device=DEV)),
+          "sigmoid": dict(score_bias=torch.linspace(-2.0, 1.0, H, device=DEV))}.get(option, {})
+    outs = []
+    for lead in (0, 1):                                      # aligned queries, then the same ones a float further on
+        at = torch.empty(rows * H * d + 1, device=DEV)[lead:lead + rows * H * d].view(rows, H * d)
+        at.copy_(q[:rows * H * d].view(rows, H * d))
+        out = torch.full((rows, H * dv), float("nan"), dtype=torch.bfloat16, device=DEV)
+        _C.mixer_ops.capped_attention(out, at, kc, vc, gate if option != "plain" else None, batch, H, G, d, dv, d ** -0.5,
+                                      **kw)
+        outs.append(out.float())
+    torch.testing.assert_close(outs[0], outs[1], atol=2e-4, rtol=2.0 ** -7)
+    # (a mean over up to 4002 keys of values of spread 1: 4002^-1/2 = 0.016 at least, the largest of them more)
+    assert outs[0].isfinite().all() and outs[0].abs().max() > 0.016

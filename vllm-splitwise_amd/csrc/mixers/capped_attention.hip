@@ -7,7 +7,8 @@
 // the keys, and parts are joined by plain addition.
 // Scores, softmax weights and the weighted sum of values are fp32: both products run on the matrix cores in
 // fp32 (v_mfma_f32_32x32x2_f32), keys and values are widened when they come from a bf16 cache.  Prompt steps over a bf16 cache
-// have a kernel of their own (prompt_attention.hip); what is here serves decode steps, fp32 caches and larger heads.
+// have a kernel of their own (prompt_attention.hip), and so have decode steps of few query rows (decode_attention.hip); what is
+// here serves fp32 caches, larger heads and decode steps of more rows.
 //
 // Work split.  A tile is 32 query rows of ONE sequence and ONE key/value head: the R = heads / kv_heads query heads
 // of that group for 32 / R consecutive new tokens (row = token * R + head), so a decode step keeps all heads of a
@@ -383,10 +384,10 @@ __global__ __launch_bounds__(64 * max_waves_of(NB)) void capped_attention_kernel
   }
 }
 
-// Steps of very few query rows per sequence and key/value head (a decode step: one token's R query heads) leave a
-// 32-row matrix tile mostly empty, so they run on the vector units instead: LK (8 or 16) lanes share a key, each with C
-// coordinates of the key, of every query row and of the value; a wave walks 64 / LK keys at a time, a workgroup owns
-// (sequence, key/value head).  Every lane group keeps a running softmax of its own; groups are joined by shuffles,
+// Steps of very few query rows per sequence and key/value head (a decode step: one token's R query heads) that
+// decode_attention.hip does not take leave a 32-row matrix tile mostly empty, so they run on the vector units: LK (8 or 16)
+// lanes share a key, each with C coordinates of the key, of every query row and of the value; a wave walks 64 / LK keys at a
+// time, a workgroup owns (sequence, key/value head).  Every lane group keeps a running softmax of its own; groups are joined by shuffles,
 // waves through LDS, both in a fixed order.  RQ: query rows (padded), C: coordinates per lane, U: keys in flight.
 template <typename T, int RQ, int C, int LK, int U>
 __global__ __launch_bounds__(512) void capped_attention_rows_kernel(
@@ -646,18 +647,11 @@ int launch_capped_attention(void* out, int64_t out_stride, const float* q, const
   const int qstride = (dim + 31) / 32 * 32 + 4, ostride = NB * 32 + 1;
   const bool split = max_query_len > 0 && max_query_len <= tpt;
   const int rows_used = split ? max_query_len * R : kQT;
-  if (split) {
-    int status = SW_OK;
-    if (try_capped_rows<T>(&status, rows_used, out, out_stride, q, key_cache, value_cache, gate, gate_stride, block_tables, table_width,
-                           q_start, ctx_len, num_seqs, heads, kv_heads, dim, vdim, page_size, scale, softcap, window,
-                           chunk, sink, sink_logit, score_bias, k_stride, v_stride, stream))
-      return status;
-  }
   int page_shift = -1;
   if ((page_size & (page_size - 1)) == 0)
     for (page_shift = 0; (1 << page_shift) < page_size; ++page_shift) {}
   if constexpr (std::is_same<T, bf16_t>::value && NB <= 4) {
-    if (!split && prompt_attention_fits(q, key_cache, value_cache, dim, vdim, k_stride, v_stride)) {
+    if ((!split || rows_used <= kDecodeRows) && prompt_attention_fits(q, key_cache, value_cache, dim, vdim, k_stride, v_stride)) {
       PromptAttention a;
       a.out = out; a.q = q;
       a.key_cache = static_cast<const uint16_t*>(key_cache);
@@ -669,8 +663,16 @@ int launch_capped_attention(void* out, int64_t out_stride, const float* q, const
       a.table_width = table_width; a.num_seqs = num_seqs; a.heads = heads; a.kv_heads = kv_heads; a.dim = dim;
       a.vdim = vdim; a.page_size = page_size; a.page_shift = page_shift; a.window = window; a.chunk = chunk;
       a.sink = sink; a.tpt = tpt; a.scale = scale; a.softcap = softcap;
-      return launch_prompt_attention(a, rows, stream);
+      return split ? launch_decode_attention(a, rows, max_query_len, workspace, stream)
+                   : launch_prompt_attention(a, rows, stream);
     }
+  }
+  if (split) {
+    int status = SW_OK;
+    if (try_capped_rows<T>(&status, rows_used, out, out_stride, q, key_cache, value_cache, gate, gate_stride, block_tables, table_width,
+                           q_start, ctx_len, num_seqs, heads, kv_heads, dim, vdim, page_size, scale, softcap, window,
+                           chunk, sink, sink_logit, score_bias, k_stride, v_stride, stream))
+      return status;
   }
   auto lds_bytes = [&](int nw) {
     const size_t floats = split ? (size_t)kQT * qstride + (size_t)nw * kQT * 2 + (size_t)nw * rows_used * ostride
@@ -715,7 +717,9 @@ extern "C" int64_t swm_masked_attention_workspace_floats(int64_t rows, int num_s
                                                          int kv_heads, int vdim, int page_size, int table_width,
                                                          int window, int chunk) {
   if (heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || heads / kv_heads > swm::kQT) return 0;
-  const int parts = swm::key_parts(num_seqs, max_query_len, heads, kv_heads, page_size, table_width, window, chunk);
+  const int parts = std::max(
+      swm::key_parts(num_seqs, max_query_len, heads, kv_heads, page_size, table_width, window, chunk),
+      swm::decode_attention_parts(num_seqs, max_query_len, heads, kv_heads, page_size, table_width, window, chunk));
   return parts > 1 ? (int64_t)parts * rows * heads * (vdim + 2) : 0;
 }
 

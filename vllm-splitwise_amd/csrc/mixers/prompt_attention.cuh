@@ -1,4 +1,5 @@
-// Prompt steps of capped_attention.hip that run on the bf16 matrix cores (prompt_attention.hip): arguments and dispatch.
+// Steps of capped_attention.hip that run on the bf16 matrix cores, prompts (prompt_attention.hip) and decode steps of few rows
+// (decode_attention.hip): arguments and dispatch.
 #pragma once
 
 #include "mixers_common.cuh"
@@ -16,9 +17,9 @@ struct PromptAttention {
   float scale, softcap;
 };
 
-// Whether a step that is not a decode step (see launch_capped_attention) goes there: a bf16 cache whose rows can be read in
-// 16-byte pieces, key and value sizes up to 128.  Beyond 128 the three parts of the queries (96 registers at 128) no longer
-// leave room for two waves per SIMD; fp32 caches have no exact bf16 keys.  Both keep the general kernel.
+// Whether a step goes there: a bf16 cache whose rows can be read in 16-byte pieces, key and value sizes up to 128.  Beyond 128
+// the three parts of a prompt's queries (96 registers at 128) no longer leave room for two waves per SIMD; fp32 caches have no
+// exact bf16 keys.  Both keep the general kernels.
 inline bool prompt_attention_fits(const float* q, const void* key_cache, const void* value_cache, int dim, int vdim,
                                   int64_t k_stride, int64_t v_stride) {
   const uintptr_t at = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(key_cache) |
@@ -27,5 +28,13 @@ inline bool prompt_attention_fits(const float* q, const void* key_cache, const v
 }
 
 int launch_prompt_attention(const PromptAttention& a, int64_t rows, hipStream_t stream);
+
+// Decode steps: at most this many query rows (tokens x heads of a group) per sequence and key/value head
+constexpr int kDecodeRows = 8;
+constexpr int kDecodeGroups = 256, kDecodePartKeys = 256;
+// how many workgroups share a sequence's keys, given a workspace of parts x rows x heads x (vdim + 2) floats
+int decode_attention_parts(int num_seqs, int max_query_len, int heads, int kv_heads, int page_size, int table_width, int window,
+                           int chunk);
+int launch_decode_attention(const PromptAttention& a, int64_t rows, int max_query_len, float* workspace, hipStream_t stream);
 
 }  // namespace swm
