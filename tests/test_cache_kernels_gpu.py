@@ -148,3 +148,14 @@ def test_convert_fp8_e5m2(dtype):
     nan = torch.isnan(ref)
     assert torch.equal(torch.isnan(dec.cpu()), nan)
     assert torch.equal(_bits(dec.cpu()[~nan]), _bits(ref[~nan]))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kv_cache_dtype", ["auto", "fp8_e5m2"])
+@pytest.mark.parametrize("num_heads,head_size,block_size", [(2, 64, 4), (3, 48, 12), (1, 16, 2), (2, 272, 64), (40, 128, 16)])
+@pytest.mark.parametrize("pattern", ["prompt", "decode", "padded"])
+def test_reshape_and_cache_block_sizes(dtype, kv_cache_dtype, num_heads, head_size, block_size, pattern):
+    """Blocks that hold a whole number of 16-byte value pieces, of 8-byte ones, and neither; rows of one piece and of many."""
+    if pattern == "decode" and block_size * 96 < 42 or pattern == "padded" and block_size * 56 < 35:
+        pytest.skip("the pattern needs more slots")
+    test_reshape_and_cache(dtype, kv_cache_dtype, num_heads, head_size, block_size, pattern)
