@@ -108,6 +108,12 @@ def test_gptq_gemm_shuffled(m, k, n, group):
     _close(got, quant.gptq_gemm(a, w, qzeros, scales, None, True))
 
 
+@pytest.mark.parametrize("m,k,n,group", [(33, 512, 72, 64), (64, 1536, 16648, 128), (61, 6144, 5120, 128), (47, 6656, 5128, 512)])
+def test_gptq_gemm_64_row_tiles_in_chunks_of_512(m, k, n, group):
+    """33..64 rows with k a multiple of 512: one chunk, several, and k split across workgroups (evenly and not)."""
+    test_gptq_gemm_shuffled(m, k, n, group)
+
+
 def test_gptq_gemm_tile_kernel_on_seeded_random_shapes():
     """Shapes drawn at random inside the 128-row tile kernel's domain (rows 129..256, k in multiples of 256,
     columns in multiples of 8, groups of 64 / 128 / 256 / all of k), against the CPU restatement."""

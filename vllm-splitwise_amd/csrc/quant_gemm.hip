@@ -1419,7 +1419,9 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
   // Kernel choice, from measurements on the 13B / TP2 matrices (tools/quant_exp.hip):
   //   * up to 32 rows: one row tile per workgroup, k split across its waves, A straight from memory;
   //   * tile kernels (A through LDS; they need k in multiples of 256 and groups in multiples of 64):
-  //       33..64 rows    64 x 64 tiles, the 8 waves are 8 k parts of every chunk;
+  //       33..64 rows    64 x 64 tiles, the 8 waves are 8 k parts of every chunk; chunks of 512 k where k is a multiple of
+  //                      that and can be split as often (half the barriers: 61 rows x 5120 x 15360 25.3 -> 23.1 us,
+  //                      x 27648 44.0 -> 40.4, 13824 x 5120 25.2 -> 23.4; 5120 x 5120, in 2 splits instead of 3, 15.1 -> 15.4);
   //       65..128 rows   128 x 64 tiles of the same form -- a 13824-column matrix is 216 of them, so k is not split
   //                      across workgroups and no fp32 partial tile goes through memory; with a short k (<= 3072) and
   //                      few columns two 64-row tiles per column tile, k unsplit, are faster than 128-row tiles whose
@@ -1463,7 +1465,8 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
       case 4: break;
       case 2: t_kq = 2; t_cg = 4; chunk_k = 128; break;
       case 8: t_kq = 8; t_cg = 1; break;
-      case 68: t_rows = 64; t_kq = 8; t_cg = 1; break;
+      case 68:
+      case 70: t_rows = 64; t_kq = 8; t_cg = 1; break;
       case 38: t_rows = 32; t_kq = 8; t_cg = 1; break;
       case 82: t_rows = 256; t_kq = 2; t_cg = 2; chunk_k = 128; break;
       case 84: t_rows = 256; t_kq = 4; t_cg = 1; chunk_k = 128; break;
@@ -1473,6 +1476,7 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
                  "gptq_gemm: no 128-row tile variant %d for K=%d, group size %d", t_variant, K, group_size);
     const int rt = (M + t_rows - 1) / t_rows, ct = (N + 64 * t_cg - 1) / (64 * t_cg);
     int ks = pick_ksplit(ct * rt, K / chunk_k, 4, M, N, avail, 1, 256);
+    if (t_variant == 68 && M <= 64 && K % 512 == 0 && pick_ksplit(ct * rt, K / 512, 4, M, N, avail, 1, 256) == ks) t_variant = 70;
     if (force_ks > 0 && force_ks <= K / chunk_k) ks = force_ks;
 #define SW_GPTQ_T128(MT_, KQ_, CG_, SPW_, NB_)                                                                 \
   do {                                                                                                           \
@@ -1487,6 +1491,7 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
     else if (t_variant == 2) SW_GPTQ_T128(4, 2, 4, 4, 3);
     else if (t_variant == 8) SW_GPTQ_T128(4, 8, 1, 2, 2);
     else if (t_variant == 68) SW_GPTQ_T128(2, 8, 1, 2, 2);
+    else if (t_variant == 70) SW_GPTQ_T128(2, 8, 1, 4, 2);
 #ifdef SW_QUANT_EXPERIMENT
     else if (t_variant == 38) SW_GPTQ_T128(1, 8, 1, 2, 2);    // 32-row tiles: behind the k-across-waves kernel at every shape
     else if (t_variant == 82) SW_GPTQ_T128(8, 2, 2, 4, 2);
