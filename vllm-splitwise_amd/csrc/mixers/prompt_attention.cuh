@@ -31,7 +31,7 @@ int launch_prompt_attention(const PromptAttention& a, int64_t rows, hipStream_t 
 
 // Decode steps: at most this many query rows (tokens x heads of a group) per sequence and key/value head
 constexpr int kDecodeRows = 8;
-constexpr int kDecodeGroups = 256, kDecodePartKeys = 256;
+constexpr int kDecodeGroups = 256, kDecodePartKeys = 256, kDecodeSharedKeys = 1024;
 // how many workgroups share a sequence's keys, given a workspace of parts x rows x heads x (vdim + 2) floats
 int decode_attention_parts(int num_seqs, int max_query_len, int heads, int kv_heads, int page_size, int table_width, int window,
                            int chunk);
