@@ -304,7 +304,8 @@ int swm_group_norm_add(float* residual, const void* y1, int64_t y1_stride, float
 /* The short causal convolution of swm_short_conv with the types and the form named: x of x_dtype, out of out_dtype
  * [rows, channels]; out = act(conv(x) + (residual != 0 ? x : 0)), act = silu when silu != 0.  The state holds the last
  * num_taps - 1 inputs in fp32; advance != 0: the same launch moves it past the step's tokens (else
- * swm_short_conv_advance with x's dtype does). */
+ * swm_short_conv_advance with x's dtype does).  Row t belongs to sequence s = token_seq[t], q_start[s] <= t < q_start[s + 1];
+ * the output of a row for which that does not hold (padding) is not defined, and nothing else depends on it. */
 int swm_causal_conv(void* out, int out_dtype, const void* x, int x_dtype, int64_t x_stride, const float* taps,
                     float* state, const int32_t* q_start, const int32_t* ctx_len, const int32_t* token_seq,
                     const int32_t* state_slot, int64_t rows, int channels, int num_taps, int silu, int residual,

@@ -3,6 +3,7 @@
 // carried inputs.  All arithmetic is fp32; activations are read and written in the model's dtype.
 #include <string>
 
+#include "conv_runs.h"
 #include "mixers_common.cuh"
 
 namespace sw {
@@ -295,24 +296,26 @@ __global__ __launch_bounds__(kRowThreads) void conv_run_kernel(
 #pragma unroll
     for (int j = 0; j < NT; ++j) w[v][j] = taps[(int64_t)(c + v) * NT + j];
   int64_t t = (int64_t)blockIdx.x * run;
-  const int64_t end = min(t + run, rows), begin = t;
+  const int64_t end = min(t + run, rows);
   while (t < end) {                                          // uniform over the workgroup
     const int s = token_seq[t];
     const int64_t first = q_start[s], stop = q_start[s + 1];
-    if (t == begin && t > first && t < first + KEEP) {       // the workgroup of the sequence's first row does these
-      t = min(first + KEEP, stop);
+    const ConvPiece piece = conv_piece(t, end, first, stop, KEEP);
+    if (piece.what == kRowsElsewhere) {
+      t = piece.next;
       continue;
     }
-    const bool fresh = t == first, carried = ctx_len[s] > 0;
-    const int64_t upto = min(stop, fresh ? max(end, first + KEEP) : end);
+    const int64_t upto = piece.next;
+    const bool inside = piece.what == kRowsInOrder, fresh = inside && t == first, carried = inside && ctx_len[s] > 0;
     float* carry = state + (int64_t)state_slot[s] * KEEP * channels + c;
     float past[KEEP][V];                                     // the inputs before row t, the oldest first
 #pragma unroll
     for (int j = 0; j < KEEP; ++j) {
 #pragma unroll
       for (int v = 0; v < V; ++v) past[j][v] = 0.0f;
-      if (!fresh) ld_vec<TX, V>(past[j], x, (t - KEEP + j) * x_stride + c);
-      else if (carried) {
+      if (!fresh) {                                          // (a row outside its sequence: what lies there of the sequence)
+        if (inside || t - KEEP + j >= first) ld_vec<TX, V>(past[j], x, (t - KEEP + j) * x_stride + c);
+      } else if (carried) {
 #pragma unroll
         for (int v = 0; v < V; v += 4) {
           const float4 q = *reinterpret_cast<const float4*>(carry + (int64_t)j * channels + v);
