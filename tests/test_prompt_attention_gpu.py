@@ -28,6 +28,64 @@ def _step(lengths, page):
                            max_state_slot=len(lengths) - 1), used
 
 
+def _statement(lengths, batch, q, kc, vc, gate, H, G, d, dv, softcap=0.0, window=0, chunk=0, sink=False, score_bias=None):
+    """The attention in 64 bits, a query at a time over the keys that it sees.  vc None: values inside the key rows."""
+    page, vc, out, row = kc.shape[1], kc if vc is None else vc, [], 0
+    for i, (c, n) in enumerate(lengths):
+        pages = batch.block_tables[i, :-(-(c + n) // page)].long()
+        ks, vs = (t[pages].reshape(-1, t.shape[-1])[:c + n].double() for t in (kc, vc))
+        for t in range(n):
+            pos = c + t
+            lo = pos // chunk * chunk if chunk else max(0, pos - window + 1) if window else 0
+            for h in range(H):
+                g = h // (H // G)
+                k, v = ks[lo:pos + 1, g * d:(g + 1) * d], vs[lo:pos + 1, g * dv:(g + 1) * dv]
+                s = (k * (q[row + t, h * d:(h + 1) * d].double() * d ** -0.5)).sum(-1)
+                s = softcap * torch.tanh(s / softcap) if softcap else s
+                if score_bias is not None:
+                    w = torch.sigmoid(s + score_bias[h].double())
+                else:
+                    extra = sink[h:h + 1].double() if isinstance(sink, torch.Tensor) else s.new_zeros(1 if sink else 0)
+                    w = torch.cat([s, extra]).softmax(0)[:len(s)]
+                out.append((w[:, None] * v).sum(0))
+        row += n
+    out = torch.stack(out).view(row, H * dv)
+    return out if gate is None else out * torch.sigmoid(gate.double())
+
+
+@pytest.mark.parametrize("option", ["plain", "cap", "sigmoid", "learned sink"])
+@pytest.mark.parametrize("H,G,d", [(4, 2, 64), (3, 1, 128)])
+@pytest.mark.parametrize("lengths", [[(70, 9), (37, 40), (64, 1), (40, 1)]], ids=["prompt"])
+def test_infinities_in_the_cache(H, G, d, option, lengths):
+    """A key coordinate or value that overflowed to an infinity gives what fp32 products give: a score of -inf hides its key, a
+    capped score of inf is the cap, a value of inf stays inf.  Queries of few bits: all but the first part of theirs is zero."""
+    from splitwise_amd import _C
+    batch, pages = _step(lengths, 16)
+    g = torch.Generator(device=DEV).manual_seed(H * 100 + d)
+    rows, inf = sum(n for _, n in lengths), float("inf")
+    kc, vc = (torch.randn(pages, 16, G * d, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    q = torch.randint(1, 16, (rows, H * d), generator=g, device=DEV).float() / 8.0
+    at = lambda i, pos: (int(batch.block_tables[i, pos // 16]), pos % 16)   # noqa: E731
+    for i, (c, n) in enumerate(lengths):                     # (keys that every query of the step sees)
+        p, o = at(i, 3)
+        kc[p, o, 5::d] = -inf                                # queries are positive: a score of -inf
+        if option != "plain" and option != "learned sink":   # (a softmax over a score of inf is NaN, there as here)
+            p, o = at(i, 9)
+            kc[p, o, 7::d] = inf
+        p, o = at(i, 17)
+        vc[p, o, 2::d], vc[p, o, 11::d] = inf, -inf
+        if n == 1:                                           # the last key of all: what lies behind it is nobody's
+            p, o = at(i, c)
+            vc[p, o, 4::d] = inf
+    kw = {"cap": dict(softcap=4.0), "learned sink": dict(sink=torch.linspace(-3.0, 2.0, H, device=DEV)),
+          "sigmoid": dict(score_bias=torch.linspace(-2.0, 1.0, H, device=DEV))}.get(option, {})
+    out = torch.empty(rows, H * d, dtype=torch.bfloat16, device=DEV)
+    _C.mixer_ops.capped_attention(out, q, kc, vc, None, batch, H, G, d, d, d ** -0.5, **kw)
+    ref = _statement(lengths, batch, q, kc, vc, None, H, G, d, d, **kw)
+    assert not ref.isnan().any() and ref.isinf().any()
+    torch.testing.assert_close(out.double(), ref, atol=2e-4, rtol=2.0 ** -7)
+
+
 @pytest.mark.parametrize("H,G,d,dv,page", [(4, 4, 128, 128, 16), (8, 2, 64, 96, 16), (6, 2, 40, 24, 8), (32, 1, 16, 8, 32),
                                            (3, 1, 104, 128, 12)])
 @pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "sink", "learned sink", "sigmoid", "values in the keys"])

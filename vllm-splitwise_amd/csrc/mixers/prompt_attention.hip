@@ -5,7 +5,8 @@
 // nine times that.  Keys and values ARE bf16 numbers; queries and softmax weights are fp32 and are taken apart into three
 // bf16 numbers each by truncation, x = h + m + l with 8 + 8 + 8 significant bits: the parts are exact, a bf16 x bf16 product
 // is exact in fp32, so three bf16 products accumulated in fp32 are the fp32 product with its sums reordered -- at three
-// times the work on units nine times as fast.
+// times the work on units nine times as fast.  Except for an infinity in the cache, which a part that is zero turns into NaN: a row
+// that comes out as NaN is worked out again in fp32 (plain_row), so the result is the fp32 product's there too.
 //
 // Tile: a workgroup of 4 waves owns 4 x 32 query rows of one sequence and key/value head (row = token * R + head of the
 // group, 32 / R tokens a wave) and walks the keys it sees in stages of 32 that the waves share through LDS: global -> registers
@@ -292,6 +293,33 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attention_kernel(cons
       }
     }
     __syncthreads();
+  }
+  // ---- a row that came out as NaN again, in plain fp32 (the stages are done with: LDS is free, a part of it for each wave)
+  int odd = 0;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) odd |= o[b][r] != o[b][r];
+  const uint64_t lanes = __builtin_amdgcn_ballot_w64(row_ok && odd != 0);
+  for (uint32_t left = (uint32_t)lanes | (uint32_t)(lanes >> 32); left != 0; left &= left - 1) {      // uniform over the wave
+    const int r = __builtin_ctz(left), rt = r / R, rh = r - rt * R;
+    const int pos = wfirst + rt, low = max(a.chunk > 0 ? pos / a.chunk * a.chunk : a.window > 0 ? pos - a.window + 1 : 0, 0);
+    float* own = reinterpret_cast<float*>(pa_lds) + wave * kPlainRowLds;
+    const PlainRow row = plain_row(a, table, g, a.q + ((row0 + rt) * a.heads + g * R + rh) * (int64_t)a.dim,
+                                   sig ? a.score_bias[g * R + rh] : 0.0f, pos, low, pos - low + 1, [&](int i) { return low + i; },
+                                   own);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    own[lane] = row.o[0];
+    own[lane + 64] = row.o[1];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (qi == r) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int c = 0; c < 16; ++c) o[b][c] = own[32 * b + 8 * (c / 4) + 4 * hl + c % 4];
+      m_run = row.m * kLog2e;
+      l_part = hl == 0 ? row.l : 0.0f;
+    }
   }
   if (!row_ok) return;
 
