@@ -55,7 +55,8 @@ def _statement(lengths, batch, q, kc, vc, gate, H, G, d, dv, softcap=0.0, window
 
 @pytest.mark.parametrize("option", ["plain", "cap", "sigmoid", "learned sink"])
 @pytest.mark.parametrize("H,G,d", [(4, 2, 64), (3, 1, 128)])
-@pytest.mark.parametrize("lengths", [[(70, 9), (37, 40), (64, 1), (40, 1)]], ids=["prompt"])
+@pytest.mark.parametrize("lengths", [[(70, 9), (37, 40), (64, 1), (40, 1)], [(64, 1), (40, 2), (300, 1)], [(2100, 1), (33, 1)]],
+                         ids=["prompt", "decode", "decode, keys shared out"])
 def test_infinities_in_the_cache(H, G, d, option, lengths):
     """A key coordinate or value that overflowed to an infinity gives what fp32 products give: a score of -inf hides its key, a
     capped score of inf is the cap, a value of inf stays inf.  Queries of few bits: all but the first part of theirs is zero."""
@@ -66,7 +67,7 @@ def test_infinities_in_the_cache(H, G, d, option, lengths):
     kc, vc = (torch.randn(pages, 16, G * d, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
     q = torch.randint(1, 16, (rows, H * d), generator=g, device=DEV).float() / 8.0
     at = lambda i, pos: (int(batch.block_tables[i, pos // 16]), pos % 16)   # noqa: E731
-    for i, (c, n) in enumerate(lengths):                     # (keys that every query of the step sees)
+    for i, (c, n) in enumerate(lengths):                     # (keys that every query of the sequence sees)
         p, o = at(i, 3)
         kc[p, o, 5::d] = -inf                                # queries are positive: a score of -inf
         if option != "plain" and option != "learned sink":   # (a softmax over a score of inf is NaN, there as here)

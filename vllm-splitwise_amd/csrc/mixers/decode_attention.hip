@@ -13,6 +13,8 @@
 //   * A wave walks tiles of 32 keys by itself: 16 KB of keys and values are on their way while it works on the tile before
 //     (page numbers two tiles ahead); no barrier until the waves are joined, in a fixed order.
 // The output is referred to a new running maximum only when some lane's has grown by more than e^5.5, so a weight is below 2^8.
+// A row that comes out as NaN is worked out again in fp32 (plain_row): a part that is zero, as a fourth of the columns is, makes NaN of
+// an infinity in the cache.
 // Few sequences share each one's keys out among `parts` workgroups, joined by a second kernel.
 //
 // Measured, 61 sequences of about 2041 keys (257 MB), 16 query heads on 4 of size 128: 100 us on the vector units (8 lanes per
@@ -40,7 +42,7 @@ union DaFrag {
 };
 
 __host__ __device__ constexpr int da_vstride(int nb) { return nb * 64 + 32; }        // bytes of a staged value row
-__host__ __device__ constexpr int da_lds_bytes(int nb) { return kDaWaves * (kDaKeys * da_vstride(nb) + 8 * 2 * 4); }
+__host__ __device__ constexpr int da_lds_bytes(int nb) { return kDaWaves * (kDaKeys * da_vstride(nb) + 8 * 2 * 4 + kPlainRowLds * 4); }
 
 // part `part` of x = h + m + l (truncated to bf16 one after the other: exact), in the upper half; 0: h, 1: m, 3: l, 2: nothing.  An infinity or NaN
 // stays whole in h.  (A weight is at most 2^8: no infinity, and a NaN may spread.)
@@ -86,7 +88,7 @@ __global__ __launch_bounds__(64 * kDaWaves, 2) void decode_attention_kernel(cons
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c16 = lane & 15, g16 = lane >> 4, part = c16 >> 2, qr = c16 & 3;
   char* stage = da_lds + wave * kDaKeys * VSTRIDE;                                   // [32][VSTRIDE]; later [rows][32 NB] floats
-  float* Ml = reinterpret_cast<float*>(da_lds + kDaWaves * kDaKeys * VSTRIDE);       // [waves][8][2]
+  float* Ml = reinterpret_cast<float*>(da_lds + kDaWaves * kDaKeys * VSTRIDE);       // [waves][8][2]; then the plain rows' floats
   const int seq = blockIdx.x, g = blockIdx.y, R = a.heads / a.kv_heads;
   const int row0 = a.q_start[seq], n = a.q_start[seq + 1] - row0;
   if (n <= 0) return;                                        // the whole workgroup
@@ -285,21 +287,52 @@ __global__ __launch_bounds__(64 * kDaWaves, 2) void decode_attention_kernel(cons
     }
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < rows * a.vdim; e += 64 * kDaWaves) {
-    const int r = e / a.vdim, c = e - r * a.vdim, tt = r / R, hh = r - tt * R;
+  for (int e0 = 64 * wave; e0 < rows * a.vdim; e0 += 64 * kDaWaves) {                // uniform over the wave
+    const int e = min(e0 + lane, rows * a.vdim - 1), r = e / a.vdim, c = e - r * a.vdim, tt = r / R, hh = r - tt * R;
     float m_all = -INFINITY;
 #pragma unroll
     for (int w = 0; w < kDaWaves; ++w) m_all = fmaxf(m_all, Ml[(w * 8 + r) * 2]);
     const float sk = a.sink_logit != nullptr ? a.sink_logit[g * R + hh] : 0.0f;
-    if (partial == nullptr && a.sink) m_all = fmaxf(m_all, sk);
-    const float m_use = m_all == -INFINITY ? 0.0f : m_all;   // (a part that saw no key)
-    float num = 0.0f, den = partial == nullptr && a.sink ? da_exp(sk - m_use) : 0.0f;
+    const bool sink = partial == nullptr && a.sink;
+    float m_use = sink ? fmaxf(m_all, sk) : m_all;
+    m_use = m_use == -INFINITY ? 0.0f : m_use;               // (a part that saw no key)
+    float num = 0.0f, den = 0.0f;
 #pragma unroll
     for (int w = 0; w < kDaWaves; ++w) {
       const float f = da_exp(Ml[(w * 8 + r) * 2] - m_use);
       den += f * Ml[(w * 8 + r) * 2 + 1];
       num += f * reinterpret_cast<const float*>(da_lds + w * kDaKeys * VSTRIDE)[r * 32 * NB + c];
     }
+    for (uint64_t left = __builtin_amdgcn_ballot_w64(num != num); __builtin_expect(left != 0, 0);) {  // uniform over the wave
+      const int rr = __shfl(r, __builtin_ctzll(left), 64), rt = rr / R, rh = rr - rt * R, at = ctx + rt;
+      int hop = step;
+      asm volatile("" : "+s"(hop));                           // (or the division is made in front of the loop)
+      const int tiles = last_tile - first_tile + 1, mine = (tiles + hop - 1) / hop * kDaWaves;
+      float* own = Ml + kDaWaves * 8 * 2 + wave * kPlainRowLds;
+      const PlainRow row = plain_row(
+          a, table, g, a.q + ((int64_t)(row0 + rt) * a.heads + g * R + rh) * a.dim, sig ? a.score_bias[g * R + rh] : 0.0f, at,
+          max(low_of(at), 0), mine * kDaKeys,
+          [&](int i) {
+            const int t = i / kDaKeys;
+            return (first_tile + t / kDaWaves * hop + (int)blockIdx.z * kDaWaves + t % kDaWaves) * kDaKeys + i % kDaKeys;
+          },
+          own);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      own[lane] = row.o[0];
+      own[lane + 64] = row.o[1];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (r == rr) {
+        m_all = row.m;
+        m_use = sink ? fmaxf(m_all, sk) : m_all;
+        m_use = m_use == -INFINITY ? 0.0f : m_use;
+        const float f = da_exp(row.m - m_use);
+        den = f * row.l;
+        num = f * own[c];
+      }
+      left &= ~__builtin_amdgcn_ballot_w64(r == rr);
+    }
+    if (e0 + lane >= rows * a.vdim) continue;
+    if (sink) den += da_exp(sk - m_use);
     if (partial != nullptr) {
       const int64_t rh = (int64_t)(row0 + tt) * a.heads + g * R + hh, all = total_rows * a.heads;
       if (c == 0) {

@@ -42,18 +42,20 @@ __device__ __forceinline__ PlainRow plain_row(const PromptAttention& a, const in
                                               int pos, int low, int n, KeyOf key_of, float* own) {
   const int lane = threadIdx.x & 63;
   const bool sig = a.score_bias != nullptr;
+  int page_size = a.page_size, dim = a.dim;
+  asm volatile("" : "+s"(page_size), "+s"(dim));             // nothing of this in front of the branch to it
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  for (int c = lane; c < a.dim; c += 64) own[c] = q[c] * a.scale;
+  for (int c = lane; c < dim; c += 64) own[c] = q[c] * a.scale;
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   PlainRow row{sig ? 0.0f : -INFINITY, 0.0f, {0.0f, 0.0f}};
   for (int i0 = 0; i0 < n; i0 += 64) {
     const int key = key_of(i0 + lane);
     const bool seen = i0 + lane < n && key <= pos && key >= low;
-    const int slot = seen ? table[key / a.page_size] * a.page_size + key % a.page_size : 0;
+    const int slot = seen ? table[key / page_size] * page_size + key % page_size : 0;
     float s = 0.0f;
     if (seen) {
       const uint16_t* k = a.key_cache + (int64_t)slot * a.k_stride + (int64_t)g * a.dim;
-      for (int c = 0; c < a.dim; ++c) s += own[c] * ld<bf16_t>(k, c);
+      for (int c = 0; c < dim; ++c) s += own[c] * ld<bf16_t>(k, c);
     }
     if (a.softcap > 0.0f) s = a.softcap * fast_tanhf_(s / a.softcap);
     float p;
