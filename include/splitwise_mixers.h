@@ -270,8 +270,8 @@ int swm_head_norm_gate_act(void* out, const float* o, const void* gate, int64_t 
  * in_stride); decay_pre act_dtype [rows, heads * dim] (row stride decay_stride); decay_bias fp32 [heads * dim] (NULL:
  * none); state fp32 [slots, heads, dim, vdim]; out fp32 [rows, heads * vdim].  Key size up to 256.
  * max_query_len: the most new tokens of any sequence (0: unknown).  Steps with long runs prepare their chunks of 32
- * tokens in `workspace`, which then holds swm_gla_workspace_floats() floats (0: the step has no long run; NULL: every
- * run is walked as a decode step's is). */
+ * tokens in `workspace`, which then holds swm_gla_workspace_floats() floats (about 2 * dim + 32 a row and head; 0: the
+ * step has no long run; NULL: every run is walked as a decode step's is). */
 int64_t swm_gla_workspace_floats(int64_t rows, int num_seqs, int max_query_len, int heads, int dim, int vdim);
 int swm_gla(float* out, const void* q, const void* k, const void* v, int64_t in_stride, const void* decay_pre,
             int64_t decay_stride, const float* decay_bias, float tau, float q_scale, float* state,

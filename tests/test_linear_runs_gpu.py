@@ -1,0 +1,73 @@
+"""Linear-attention steps whose runs are cut into segments, and steps whose decoding sequences go another way than the long runs
+beside them, against the rule in 64 bits token by token.  States and outputs are fp32 sums of products whose decays are
+exponentials of sums: a relative error of about 2e-7 of their size in the 2-norm, 5e-6 of their root mean square for the worst."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _rule(q, k, v, keep, state, starts, fresh):
+    """q, k [rows, heads, dim], v [rows, heads, vdim], keep [rows, heads, dim or 1], state [sequences, heads, dim, vdim]."""
+    out, ends = torch.empty_like(v), state.clone()
+    longest = max(b - a for a, b in zip(starts, starts[1:]))
+    first, last = torch.tensor(starts[:-1], device=DEV), torch.tensor(starts[1:], device=DEV)
+    ends[fresh] = 0
+    for t in range(longest):
+        live = (first + t < last).nonzero().squeeze(1)         # every sequence's token t at once
+        at = first[live] + t
+        s = keep[at][..., None] * ends[live] + k[at][..., None] * v[at][..., None, :]
+        ends[live] = s
+        out[at] = (q[at][..., None] * s).sum(-2)
+    return out, ends
+
+
+@pytest.mark.parametrize("rule", ["gla", "lightning", "retention"])
+@pytest.mark.parametrize("heads,dim,vdim,lens", [
+    (2, 128, 40, [1100, 577, 1, 30, 576]), (1, 64, 16, [5000]), (1, 40, 17, [1024, 1025]), (2, 160, 33, [1500, 3]),
+    (3, 256, 20, [33, 2049]),                                              # segments
+    (2, 128, 128, [1] * 130 + [40] + [2] * 70 + [17, 16, 95]),              # decoding sequences beside portions
+    (4, 128, 128, [1] * 61 + [600, 1100]), (16, 64, 64, [1, 5, 0, 2] * 40 + [70])], ids=str)
+def test_segments_and_mixed_steps(rule, heads, dim, vdim, lens):
+    from splitwise_amd import _C
+    ops = _C.mixer_ops
+    rows, n = sum(lens), len(lens)
+    starts = [sum(lens[:i]) for i in range(n + 1)]
+    g = torch.Generator(device=DEV).manual_seed(rows + dim)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)               # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
+    ctx = [0 if i % 3 == 1 else 7 for i in range(n)]
+    slots = [(i * 7 + 3) % (n + 2) if (n + 2) % 7 else i + 1 for i in range(n)]
+    batch = SimpleNamespace(q_start=i32(starts), ctx_len=i32(ctx), state_slot=i32(slots), max_state_slot=n + 1, max_query_len=max(lens),
+                            token_seq=i32([i for i, m in enumerate(lens) for _ in range(m)]))
+    nk, nv = heads * dim, heads * vdim
+    proj, z, bias = rnd(rows, 2 * nk + nv + 8).bfloat16(), rnd(rows, nk).bfloat16(), 2.0 + rnd(nk)
+    decay = torch.linspace(0.3, 0.999, heads, device=DEV)
+    q, k, v = proj[:, :nk], proj[:, nk:2 * nk], proj[:, 2 * nk:2 * nk + nv]
+    state = rnd(n + 2, heads, dim, vdim) * 0.1
+    got, out = state.clone(), torch.full((rows, nv), float("nan"), device=DEV)
+    q64, k64, v64 = (t.double().view(rows, heads, -1) for t in (q, k, v))
+    keep = decay.double().view(1, heads, 1).expand(rows, heads, 1)
+    if rule == "gla":
+        ops.gla(out, q, k, v, z, bias, 16.0, dim ** -0.5, got, batch, heads, dim, vdim)
+        q64 = q64 * dim ** -0.5
+        keep = torch.exp(torch.nn.functional.logsigmoid(z.double() + bias.double()) / 16.0).view(rows, heads, dim)
+    elif rule == "lightning":
+        ops.lightning(out, q, k, v, decay, got, batch, heads, dim, vdim)
+        q64, k64, v64 = (torch.nn.functional.silu(t) for t in (q64, k64, v64))
+    else:
+        k32 = k.float() * dim ** -0.5
+        ops.retention(out, q.float(), k32, v, decay, got, batch, heads, dim, vdim)
+        k64 = k32.double().view(rows, heads, dim)
+    at = torch.tensor(slots, device=DEV)
+    ref, ends = _rule(q64, k64, v64, keep, state[at].double(), starts, torch.tensor([c == 0 for c in ctx], device=DEV))
+    some = torch.tensor([m > 0 for m in lens], device=DEV)     # a sequence without a token leaves its state alone
+    for a, b in ((out.double().view_as(ref), ref), (got[at][some].double(), ends[some])):
+        off = (a - b).abs()
+        assert a.isfinite().all()
+        assert float(off.norm() / b.norm()) < 6e-7 and float(off.max() / b.square().mean().sqrt()) < 3e-5
+    idle = [i for i in range(n + 2) if i not in slots] + [slots[i] for i in range(n) if lens[i] == 0]
+    assert torch.equal(got[idle], state[idle])

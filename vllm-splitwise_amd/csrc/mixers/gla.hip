@@ -16,16 +16,15 @@
 //    value channel join their halves of S^T q.  Exact for any decay (a product of decays that underflows is a state
 //    that has been forgotten), and the cheaper route for runs of a few tokens (a decoded token is a chunk of one).
 //
-// Runs of more than kGlaWalkFrom tokens are taken by linear_walk.hip.
+// Long runs are taken by linear_walk.hip (linear_at_most says which).
 #include "linear_walk.cuh"
+
+#include <climits>
 
 namespace swm {
 
 using f32x16 = __attribute__((ext_vector_type(16))) float;
 constexpr int kGlaChunk = 32;
-// Steps whose longest run has more tokens than this go to linear_walk.hip (us here / there, with norm and gate, the host's 30 a
-// call included: 1 x 16 heads of 128, 16 tokens 32 / 34, 31 tokens 37 / 34, 64 tokens 63 / 34, 1000 tokens 921 / 75).
-constexpr int kGlaWalkFrom = 16;
 constexpr float kSafeLog = 24.0f;      // the matrix route needs every channel's summed log-decay of a chunk above -this
 constexpr int kTokenRouteBelow = 6;    // chunks shorter than this go token by token without asking
 
@@ -38,7 +37,7 @@ __global__ __launch_bounds__(512) void gla_kernel(
     float* __restrict__ out, const void* __restrict__ q, const void* __restrict__ k, const void* __restrict__ v,
     int64_t in_stride, const void* __restrict__ decay_pre, int64_t decay_stride, const float* __restrict__ decay_bias,
     float inv_tau, float q_scale, float* __restrict__ state, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int dim, int vdim) {
+    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int dim, int vdim, int at_most) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int DS = NDB * 32 + 4;                           // row stride of the staged tiles
   constexpr int CH = NDB * 32;                               // key channels, padded
@@ -54,7 +53,7 @@ __global__ __launch_bounds__(512) void gla_kernel(
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 31, hl = lane >> 5;
   const int vb0 = blockIdx.z * nw;                           // first block of 32 value channels of the workgroup
   const int seq = blockIdx.x, n = q_start[seq + 1] - q_start[seq];
-  if (n <= 0) return;                                        // the whole workgroup
+  if (n <= 0 || n > at_most) return;                         // the whole workgroup
   const int row0 = q_start[seq];
   const int vc = (vb0 + wave) * 32 + li;                     // this lane's value channel
   const bool vc_ok = vc < vdim;
@@ -267,7 +266,7 @@ template <typename T, int NDB>
 int launch_gla(float* out, const void* q, const void* k, const void* v, int64_t in_stride, const void* decay_pre,
                int64_t decay_stride, const float* decay_bias, float tau, float q_scale, float* state,
                const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot, int num_seqs, int heads, int dim,
-               int vdim, hipStream_t stream) {
+               int vdim, int at_most, hipStream_t stream) {
   const int vblocks = (vdim + 31) / 32;
   const int waves = std::min(vblocks, 8);
   const size_t lds_bytes =
@@ -283,7 +282,7 @@ int launch_gla(float* out, const void* q, const void* k, const void* v, int64_t 
   const float inv_tau = 1.0f / tau;
   hipLaunchKernelGGL(kernel, dim3((unsigned)num_seqs, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream, out, q, k, v,
                      in_stride, decay_pre, decay_stride, decay_bias, inv_tau, q_scale, state, q_start, ctx_len, state_slot, heads,
-                     dim, vdim);
+                     dim, vdim, at_most);
   SW_CHECK_LAUNCH();
   return SW_OK;
 }
@@ -291,8 +290,7 @@ int launch_gla(float* out, const void* q, const void* k, const void* v, int64_t 
 }  // namespace swm
 
 extern "C" int64_t swm_gla_workspace_floats(int64_t rows, int num_seqs, int max_query_len, int heads, int dim, int vdim) {
-  (void)vdim;
-  return max_query_len <= swm::kGlaWalkFrom ? 0 : swm::linear_walk_floats(rows, num_seqs, heads, dim);
+  return swm::linear_walk_plan(true, rows, num_seqs, max_query_len, heads, dim, vdim).floats;
 }
 
 extern "C" int swm_gla(float* out, const void* q, const void* k, const void* v, int64_t in_stride,
@@ -307,16 +305,20 @@ extern "C" int swm_gla(float* out, const void* q, const void* k, const void* v, 
                "gla: %d heads, key size %d (at most 256), value size %d", heads, dim, vdim);
   SW_CHECK_ARG(tau > 0.0f, "gla: tau must be positive");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (workspace != nullptr && max_query_len > kGlaWalkFrom) {
+  const LinearWalkPlan plan = linear_walk_plan(true, rows, num_seqs, max_query_len, heads, dim, vdim);
+  int at_most = INT_MAX;
+  if (workspace != nullptr && plan.at_most < max_query_len) {
     const LinearStep step{out, q, k, v, in_stride, in_stride, state, q_start, ctx_len, state_slot, rows, num_seqs, heads, dim, vdim,
                           workspace};
-    return gla_walk(step, decay_pre, decay_stride, decay_bias, 1.0f / tau, q_scale, act_dtype, s);
+    const int status = gla_walk(step, plan, decay_pre, decay_stride, decay_bias, 1.0f / tau, q_scale, act_dtype, s);
+    if (status != SW_OK || plan.at_most == 0) return status;
+    at_most = plan.at_most;                                  // the others beside it
   }
 #define SWM_GLA_CASE(N)                                                                                             \
   case N:                                                                                                           \
     SWM_DISPATCH_ACT(act_dtype, return (launch_gla<T, N>(out, q, k, v, in_stride, decay_pre, decay_stride,          \
                                                          decay_bias, tau, q_scale, state, q_start, ctx_len,         \
-                                                         state_slot, num_seqs, heads, dim, vdim, s)););             \
+                                                         state_slot, num_seqs, heads, dim, vdim, at_most, s)););    \
     break;
   switch ((dim + 31) / 32) {
     SWM_GLA_CASE(1)

@@ -16,13 +16,12 @@
 // token is a chunk of one.
 #include "linear_walk.cuh"
 
+#include <climits>
+
 namespace swm {
 
 using f32x16 = __attribute__((ext_vector_type(16))) float;
 constexpr int kChunk = 32;
-// Steps whose longest run has more tokens than this go to linear_walk.hip (us here / there, with norm and gate, the host's 30 a
-// call included: 1 x 16 heads of 128, 16 tokens 33 / 33, 31 tokens 37 / 33, 64 tokens 54 / 34, 1000 tokens 665 / 76).
-constexpr int kWalkFrom = 16;
 
 // NDB: 32-coordinate blocks of the key size.  A workgroup owns (sequence, head) and up to 8 blocks of 32 value
 // channels, one wave each; the chunk's silu(q) and silu(k) are staged once in LDS for all of them.
@@ -31,7 +30,7 @@ template <typename TQ, typename T, bool SILU, int NDB>
 __global__ __launch_bounds__(512) void lightning_kernel(
     float* __restrict__ out, const void* __restrict__ q, const void* __restrict__ k, int64_t qk_stride,
     const void* __restrict__ v, int64_t v_stride, const float* __restrict__ decay, float* __restrict__ state, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int dim, int vdim) {
+    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int dim, int vdim, int at_most) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int DS = NDB * 32 + 4;                           // row stride of the staged tiles
   float* Qs = lds;                                           // [32][DS]
@@ -42,7 +41,7 @@ __global__ __launch_bounds__(512) void lightning_kernel(
   const int vb = blockIdx.z * (blockDim.x >> 6) + wave;
   // blockIdx.x is a sequence; its whole run goes from the slot's state to the slot's state
   const int seq = blockIdx.x, n = q_start[seq + 1] - q_start[seq];
-  if (n <= 0) return;                                        // the whole workgroup
+  if (n <= 0 || n > at_most) return;                         // the whole workgroup
   const int row0 = q_start[seq];
   const float lam = decay[h];
   if (threadIdx.x == 0) {
@@ -193,7 +192,7 @@ __global__ __launch_bounds__(512) void lightning_kernel(
 template <typename TQ, typename T, bool SILU, int NDB>
 int launch_lightning(float* out, const void* q, const void* k, int64_t qk_stride, const void* v, int64_t v_stride, const float* decay,
                      float* state, const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot,
-                     int num_seqs, int heads, int dim, int vdim, hipStream_t stream) {
+                     int num_seqs, int heads, int dim, int vdim, int at_most, hipStream_t stream) {
   const int vblocks = (vdim + 31) / 32;
   const int waves = std::min(vblocks, 8);
   const size_t lds_bytes = (size_t)(2 * kChunk * (NDB * 32 + 4) + kChunk + 2) * sizeof(float);
@@ -206,7 +205,7 @@ int launch_lightning(float* out, const void* q, const void* k, int64_t qk_stride
   }
   const unsigned zgroups = (unsigned)((vblocks + waves - 1) / waves);
   hipLaunchKernelGGL(kernel, dim3((unsigned)num_seqs, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream, out, q, k,
-                     qk_stride, v, v_stride, decay, state, q_start, ctx_len, state_slot, heads, dim, vdim);
+                     qk_stride, v, v_stride, decay, state, q_start, ctx_len, state_slot, heads, dim, vdim, at_most);
   SW_CHECK_LAUNCH();
   return SW_OK;
 }
@@ -215,8 +214,7 @@ int launch_lightning(float* out, const void* q, const void* k, int64_t qk_stride
 
 extern "C" int64_t swm_lightning_workspace_floats(int64_t rows, int num_seqs, int max_query_len, int heads, int dim,
                                                   int vdim) {
-  (void)vdim;
-  return max_query_len <= swm::kWalkFrom ? 0 : swm::linear_walk_floats(rows, num_seqs, heads, dim);
+  return swm::linear_walk_plan(false, rows, num_seqs, max_query_len, heads, dim, vdim).floats;
 }
 
 extern "C" int swm_lightning(float* out, const void* q, const void* k, const void* v, int64_t in_stride,
@@ -229,16 +227,20 @@ extern "C" int swm_lightning(float* out, const void* q, const void* k, const voi
   SW_CHECK_ARG(heads > 0 && heads < 65536 && dim > 0 && dim <= 256 && vdim > 0 && (vdim + 255) / 256 < 65536,
                "lightning: %d heads, key size %d (at most 256), value size %d", heads, dim, vdim);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (workspace != nullptr && max_query_len > kWalkFrom) {
+  const LinearWalkPlan plan = linear_walk_plan(false, rows, num_seqs, max_query_len, heads, dim, vdim);
+  int at_most = INT_MAX;
+  if (workspace != nullptr && plan.at_most < max_query_len) {
     const LinearStep step{out, q, k, v, in_stride, in_stride, state, q_start, ctx_len, state_slot, rows, num_seqs, heads, dim, vdim,
                           workspace};
-    return lightning_walk(step, decay, true, act_dtype, act_dtype, s);
+    const int status = lightning_walk(step, plan, decay, true, act_dtype, act_dtype, s);
+    if (status != SW_OK || plan.at_most == 0) return status;
+    at_most = plan.at_most;                                  // the others beside it
   }
 #define SWM_LIGHTNING_CASE(N)                                                                                              \
   case N:                                                                                                                  \
     SWM_DISPATCH_ACT(act_dtype, return (launch_lightning<T, T, true, N>(out, q, k, in_stride, v, in_stride, decay, state,  \
                                                                         q_start, ctx_len, state_slot, num_seqs, heads,     \
-                                                                        dim, vdim, s)););                                  \
+                                                                        dim, vdim, at_most, s)););                         \
     break;
   switch ((dim + 31) / 32) {
     SWM_LIGHTNING_CASE(1)
@@ -264,16 +266,20 @@ extern "C" int swm_retention(float* out, const float* q, const float* k, int64_t
   SW_CHECK_ARG(heads > 0 && heads < 65536 && dim > 0 && dim <= 256 && vdim > 0 && (vdim + 255) / 256 < 65536,
                "retention: %d heads, key size %d (at most 256), value size %d", heads, dim, vdim);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (workspace != nullptr && max_query_len > kWalkFrom) {
+  const LinearWalkPlan plan = linear_walk_plan(false, rows, num_seqs, max_query_len, heads, dim, vdim);
+  int at_most = INT_MAX;
+  if (workspace != nullptr && plan.at_most < max_query_len) {
     const LinearStep step{out, q, k, v, qk_stride, v_stride, state, q_start, ctx_len, state_slot, rows, num_seqs, heads, dim, vdim,
                           workspace};
-    return lightning_walk(step, decay, false, SW_F32, act_dtype, s);
+    const int status = lightning_walk(step, plan, decay, false, SW_F32, act_dtype, s);
+    if (status != SW_OK || plan.at_most == 0) return status;
+    at_most = plan.at_most;                                  // the others beside it
   }
 #define SWM_RETENTION_CASE(N)                                                                                          \
   case N:                                                                                                              \
     SWM_DISPATCH_ACT(act_dtype, return (launch_lightning<float, T, false, N>(out, q, k, qk_stride, v, v_stride, decay, \
                                                                              state, q_start, ctx_len, state_slot,      \
-                                                                             num_seqs, heads, dim, vdim, s)););        \
+                                                                             num_seqs, heads, dim, vdim, at_most, s)););\
     break;
   switch ((dim + 31) / 32) {
     SWM_RETENTION_CASE(1)

@@ -16,12 +16,17 @@
 // coordinate 32 b + 16 i + 4 (l / 16) + r), in the layout that the B operand of the next product wants.  Operands come straight
 // from memory into the A operands' registers, a chunk ahead; the waves' shares of Q~ S_0 meet in LDS behind the one barrier
 // of a chunk.  Workgroups that read the same chunks (the channels of a head) have numbers 8 apart: one XCD, one L2.
+// The chain of a long run of few heads leaves the rest of the GPU idle.  Such a run is cut into segments (linear_plan.h): a launch
+// of their own works out every segment's end from nothing, without outputs, exchange or barrier, and the walk then begins each
+// segment at the end of the one in front of it, S = D S' + local end after local end, D the segment's products of decays.
 //
 // Measured, two prompts of 4324 tokens together, 16 heads of 128, a decay per key channel: 676 + 20 us in segments of 128 tokens
 // taken twice, from nothing and from their true states, with a scan between (560 workgroups on 512 places: the second round
 // nearly empty); 52 us prologue and 139 us walk here.  Of the walk's 1.8 us a chunk the products, the exchange and its barrier
 // alone are 1.2 (38 products of 32 cycles are 0.5), the operands' way through the L1 0.5.  The prologue took 111 us with its
-// operands staged in LDS first.  Relative error of the end states against 64 bits: 1.3e-7 here, 2.2e-7 in segments.
+// operands staged in LDS first.  Relative error of the end states against 64 bits: 1.3e-7 here, 2.2e-7 in those segments.
+// One run of 16000 tokens, 4 heads of 128, decays per channel / per head: 870 / 904 us in one piece, 208 / 205 in 8 segments (415 /
+// 300 in segments of 128 tokens); of 32000 tokens, 16 heads: 2202 and 1637 in 2.
 #include "linear_walk.cuh"
 
 #include <type_traits>
@@ -34,7 +39,10 @@ constexpr int kLwChannels = 16;
 constexpr float kLwSafeLog = 12.0f;
 
 // log(sigmoid(x)) = min(x, 0) - log(1 + t), t = e^-|x|, the logarithm on the hardware's log2 with the rounding of 1 + t put back:
-// largest relative error over [-30, 30] 2.2e-7 (with log1pf 1.3e-7), root mean square 3.5e-8 (2.8e-8), a quarter of the instructions
+// largest relative error over [-30, 30] 2.2e-7 (with log1pf 1.3e-7), root mean square 3.5e-8 (2.8e-8), a quarter of the instructions.
+// The results do not show it: over runs of 40 to 3000 tokens, 4 to 16 heads of 64 to 128, tau 1 to 16, outputs are 1.5 - 2.1e-7 and
+// end states 1.0 - 1.9e-7 from 64 bits with either (2.4 - 3.4e-7 and 1.2 - 2.8e-7 before this file); with log1pf the step above
+// takes 219 us instead of 204.
 __device__ __forceinline__ float log_sigmoid(float x) {
   const float t = expf(-fabsf(x)), u = 1.0f + t;
   return fminf(x, 0.0f) - (0.69314718055994531f * __builtin_amdgcn_logf(u) + (t - (u - 1.0f)) * __builtin_amdgcn_rcpf(u));
@@ -88,7 +96,7 @@ __device__ __forceinline__ void lw_put8(float* p, const float (&x)[8]) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(kLwThreads, 3) void gla_walk_prep_kernel(const LinearStep a, const void* __restrict__ decay_pre,
+__global__ __launch_bounds__(kLwThreads, 3) void gla_walk_prep_kernel(const LinearStep a, int at_most, const void* __restrict__ decay_pre,
                                                                    int64_t decay_stride, const float* __restrict__ decay_bias,
                                                                    float inv_tau, float q_scale, int dp) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -98,8 +106,8 @@ __global__ __launch_bounds__(kLwThreads, 3) void gla_walk_prep_kernel(const Line
   float* Ko = Ks + kLwChunk * KS;                // [16][KS] the first half's keys carried to its end
   float* total = Ko + 16 * KS;                   // [2][dp] the halves' sums of log a
   int* unsafe = reinterpret_cast<int*>(total + 2 * dp);                  // [2]
-  int seq = 0, tok0 = 0;
-  const int cn = find_query_tile(a.q_start, a.num_seqs, blockIdx.x, kLwChunk, &seq, &tok0);
+  int seq = 0, tok0 = 0, before = 0;
+  const int cn = lw_find_piece(a.q_start, a.num_seqs, at_most, kLwChunk, blockIdx.x, &seq, &tok0, &before);
   if (cn <= 0) return;                           // the whole workgroup
   const int h = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int64_t row0 = a.q_start[seq] + tok0;
@@ -218,15 +226,15 @@ __global__ __launch_bounds__(kLwThreads, 3) void gla_walk_prep_kernel(const Line
 
 // vec: rows of q and k lie on 16 bytes
 template <typename TQ, bool SILU>
-__global__ __launch_bounds__(kLwThreads) void lightning_walk_prep_kernel(const LinearStep a, const float* __restrict__ decay, int dp,
+__global__ __launch_bounds__(kLwThreads) void lightning_walk_prep_kernel(const LinearStep a, int at_most, const float* __restrict__ decay, int dp,
                                                                          int vec) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int KS = dp + 4;
   float* Qs = lds;                               // [32][KS]
   float* Ks = Qs + kLwChunk * KS;                // [32][KS]
   float* pw = Ks + kLwChunk * KS;                // [33] powers of the decay, by repeated multiplication
-  int seq = 0, tok0 = 0;
-  const int cn = find_query_tile(a.q_start, a.num_seqs, blockIdx.x, kLwChunk, &seq, &tok0);
+  int seq = 0, tok0 = 0, before = 0;
+  const int cn = lw_find_piece(a.q_start, a.num_seqs, at_most, kLwChunk, blockIdx.x, &seq, &tok0, &before);
   if (cn <= 0) return;                           // the whole workgroup
   const int h = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int64_t row0 = a.q_start[seq] + tok0;
@@ -295,32 +303,153 @@ struct LwOperands {
   typename Conv<TV>::store_t v[2][4];            // tokens 16 i + 4 (l / 16) + r of this lane's channel
 };
 
+// A walk's pieces of runs: whole ones, or segments.  A segment's place in the scratch: [state: 16-channel block | 32 coordinates |
+// tile | lane], the accumulators' layout, and the products of its decays.
+struct LwPieces {
+  int at_most, segment;                          // 0: whole runs
+  int64_t items;
+  float *states, *decays;                        // [items][heads][16 vblocks dp], [items][heads][dp]
+};
+
+// The segments' own ends, side by side: a run's first segment from the true state, the others from nothing; the last one is left
+// out, and its place takes a copy of the true state, which the walk of the first segment starts from (the state's own place is
+// written by the last segment's, at a time of its own).
 template <typename TV, bool SILU, int NDB>
-__global__ __launch_bounds__(64 * NDB) void linear_walk_kernel(const LinearStep a) {
+__global__ __launch_bounds__(64 * NDB) void linear_segment_kernel(const LinearStep a, const LwPieces pc) {
+  constexpr int DP = NDB * 32;
+  const int vblocks = (a.vdim + kLwChannels - 1) / kLwChannels;
+  const int unit = (blockIdx.x >> 3) / vblocks * 8 + (blockIdx.x & 7), vb = (blockIdx.x >> 3) % vblocks;
+  const int item = unit / a.heads, h = unit - item * a.heads;
+  int seq = 0, tok0 = 0, before = 0;
+  const int n = item < pc.items ? lw_find_piece(a.q_start, a.num_seqs, pc.at_most, pc.segment, item, &seq, &tok0, &before) : 0;
+  if (n <= 0) return;                            // the whole workgroup
+  const int run = a.q_start[seq + 1] - a.q_start[seq], behind = (run - tok0 - 1) / pc.segment;      // segments behind this one
+  if (behind == 0) return;                       // (n is a whole segment otherwise)
+  const int b = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, gq = lane >> 4;
+  const int64_t row0 = (int64_t)a.q_start[seq] + tok0, chunk0 = before + tok0 / kLwChunk;
+  const int vc = vb * kLwChannels + li;
+  const bool vc_ok = vc < a.vdim;
+  auto place = [&](int64_t it) {
+    return reinterpret_cast<f32x4*>(pc.states + ((it * a.heads + h) * vblocks + vb) * (kLwChannels * DP)) + b * 128 + lane;
+  };
+  f32x4 S[2], D[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    S[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    D[i] = f32x4{1.0f, 1.0f, 1.0f, 1.0f};
+    if (tok0 == 0) {
+      const float* sp = a.state + ((int64_t)a.state_slot[seq] * a.heads + h) * (int64_t)a.dim * a.vdim;
+      const bool fresh = a.ctx_len[seq] == 0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int c = 32 * b + 16 * i + 4 * gq + r;
+        S[i][r] = (!fresh && vc_ok && c < a.dim) ? sp[(int64_t)c * a.vdim + vc] : 0.0f;
+      }
+      place(item + behind)[64 * i] = S[i];
+    }
+  }
+  const typename Conv<TV>::store_t* vsrc = static_cast<const typename Conv<TV>::store_t*>(a.v) + row0 * a.v_stride +
+                                           (int64_t)h * a.vdim + (vc_ok ? vc : a.vdim - 1);
+  struct Ops {
+    f32x4 kt[2][2], keep[2];
+    typename Conv<TV>::store_t v[2][4];
+  };
+  const int chunks = pc.segment / kLwChunk;
+  auto fetch = [&](Ops& x, int ci) {
+    const float* rec = a.workspace + ((chunk0 + ci) * a.heads + h) * lw_record(DP);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        x.kt[i][j] = *reinterpret_cast<const f32x4*>(rec + 32 * DP + (32 * b + 16 * i + li) * 32 + 16 * j + 4 * gq);
+      x.keep[i] = *reinterpret_cast<const f32x4*>(rec + 64 * DP + 32 * b + 16 * i + 4 * gq);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x.v[i][r] = vsrc[(ci * kLwChunk + 16 * i + 4 * gq + r) * a.v_stride];
+    }
+  };
+  auto chunk = [&](const Ops& x) {
+    f32x4 v[2], add[2] = {};
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float y = Conv<TV>::to_float(x.v[i][r]);
+        v[i][r] = SILU ? fast_siluf_(y) : y;
+      }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) add[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kt[i][j][r], v[j][r], add[i], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      S[i] = S[i] * x.keep[i] + add[i];
+      D[i] *= x.keep[i];
+    }
+  };
+  Ops x0, x1;
+  fetch(x0, 0);
+#pragma unroll 1
+  for (int ci = 0; ci < chunks; ci += 2) {
+    fetch(x1, min(ci + 1, chunks - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    chunk(x0);
+    if (ci + 1 >= chunks) break;
+    fetch(x0, min(ci + 2, chunks - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    chunk(x1);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    place(item)[64 * i] = S[i];
+    if (vb == 0 && li == 0)
+      *reinterpret_cast<f32x4*>(pc.decays + ((int64_t)item * a.heads + h) * DP + 32 * b + 16 * i + 4 * gq) = D[i];
+  }
+}
+
+template <typename TV, bool SILU, int NDB>
+__global__ __launch_bounds__(64 * NDB) void linear_walk_kernel(const LinearStep a, const LwPieces pc) {
   __shared__ f32x4 red[2][NDB][2][64];           // [chunk parity][wave][token tile][lane]: shares of Q~ S_0
   constexpr int DP = NDB * 32;
   const int vblocks = (a.vdim + kLwChannels - 1) / kLwChannels;
   const int unit = (blockIdx.x >> 3) / vblocks * 8 + (blockIdx.x & 7), vb = (blockIdx.x >> 3) % vblocks;
-  if (unit >= a.num_seqs * a.heads) return;      // the whole workgroup
-  const int seq = unit / a.heads, h = unit - seq * a.heads;
-  const int b = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, gq = lane >> 4;
-  const int n = a.q_start[seq + 1] - a.q_start[seq];
+  const int item = unit / a.heads, h = unit - item * a.heads;
+  int seq = 0, tok0 = 0, before = 0;
+  const int n = item < pc.items ? lw_find_piece(a.q_start, a.num_seqs, pc.at_most, pc.segment > 0 ? pc.segment : 1 << 30, item, &seq,
+                                                &tok0, &before)
+                                : 0;
   if (n <= 0) return;                            // the whole workgroup
-  const int64_t row0 = a.q_start[seq];
-  int64_t chunk0 = 0;                            // this sequence's first chunk among the step's
-  for (int s = 0; s < seq; ++s) chunk0 += (a.q_start[s + 1] - a.q_start[s] + kLwChunk - 1) / kLwChunk;
+  const int b = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, gq = lane >> 4;
+  const int64_t row0 = (int64_t)a.q_start[seq] + tok0, chunk0 = before + tok0 / kLwChunk;
+  const int run = a.q_start[seq + 1] - a.q_start[seq];
   const int vc = vb * kLwChannels + li;          // this lane's value channel
   const bool vc_ok = vc < a.vdim;
   float* sp = a.state + ((int64_t)a.state_slot[seq] * a.heads + h) * (int64_t)a.dim * a.vdim;
   f32x4 S[2];
-  const bool fresh = a.ctx_len[seq] == 0;
+  const bool fresh = a.ctx_len[seq] == 0, last = tok0 + n >= run;
+  if (pc.segment > 0 && !(tok0 == 0 && last)) {  // a segment: the true state behind the ones in front of it
+    const int index = tok0 / pc.segment, first = item - index, end = first + (run - 1) / pc.segment;
+    auto place = [&](int64_t it) {
+      return reinterpret_cast<const f32x4*>(pc.states + ((it * a.heads + h) * vblocks + vb) * (kLwChannels * DP)) + b * 128 + lane;
+    };
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) S[i] = place(index == 0 ? end : first)[64 * i];
+#pragma unroll 4
+    for (int it = first + 1; it < item; ++it) {
+      const float* d = pc.decays + ((int64_t)it * a.heads + h) * DP + 32 * b + 4 * gq;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int c = 32 * b + 16 * i + 4 * gq + r;
-      S[i][r] = (!fresh && vc_ok && c < a.dim) ? sp[(int64_t)c * a.vdim + vc] : 0.0f;
+      for (int i = 0; i < 2; ++i) S[i] = S[i] * *reinterpret_cast<const f32x4*>(d + 16 * i) + place(it)[64 * i];
     }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int c = 32 * b + 16 * i + 4 * gq + r;
+        S[i][r] = (!fresh && vc_ok && c < a.dim) ? sp[(int64_t)c * a.vdim + vc] : 0.0f;
+      }
+  }
   const typename Conv<TV>::store_t* vsrc = static_cast<const typename Conv<TV>::store_t*>(a.v) + row0 * a.v_stride +
                                            (int64_t)h * a.vdim + (vc_ok ? vc : a.vdim - 1);
   const int chunks = (n + kLwChunk - 1) / kLwChunk;
@@ -436,7 +565,7 @@ __global__ __launch_bounds__(64 * NDB) void linear_walk_kernel(const LinearStep 
   }
   collect(chunks - 1);
   finish(chunks - 1);
-  if (vc_ok) {
+  if (vc_ok && last) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -454,13 +583,22 @@ inline hipError_t lw_allow_lds(K kernel, size_t bytes) {
 }
 
 template <typename TV, bool SILU>
-int launch_walk(const LinearStep& a, hipStream_t stream) {
-  const int64_t units = ((int64_t)a.num_seqs * a.heads + 7) / 8 * 8;
-  const int64_t groups = units * ((a.vdim + kLwChannels - 1) / kLwChannels);
+int launch_walk(const LinearStep& a, const LinearWalkPlan& plan, hipStream_t stream) {
+  const int64_t dp = (a.dim + 31) / 32 * 32, vblocks = (a.vdim + kLwChannels - 1) / kLwChannels;
+  const int64_t groups = (plan.items * a.heads + 7) / 8 * 8 * vblocks;
   SW_CHECK_ARG(groups < (1ll << 31), "linear attention: too many sequences and heads");
+  LwPieces pc{plan.at_most, plan.segment, plan.items, nullptr, nullptr};
+  if (plan.segment > 0) {
+    pc.states = a.workspace + plan.chunks * a.heads * (65 * dp + 1024);
+    pc.decays = pc.states + plan.items * a.heads * kLwChannels * vblocks * dp;
+  }
 #define SWM_LW_CASE(N)                                                                                                 \
   case N:                                                                                                              \
-    hipLaunchKernelGGL((linear_walk_kernel<TV, SILU, N>), dim3((unsigned)groups), dim3(64 * N), 0, stream, a);         \
+    if (plan.segment > 0) {                                                                                            \
+      hipLaunchKernelGGL((linear_segment_kernel<TV, SILU, N>), dim3((unsigned)groups), dim3(64 * N), 0, stream, a, pc); \
+      SW_CHECK_LAUNCH();                                                                                               \
+    }                                                                                                                  \
+    hipLaunchKernelGGL((linear_walk_kernel<TV, SILU, N>), dim3((unsigned)groups), dim3(64 * N), 0, stream, a, pc);     \
     break;
   switch ((a.dim + 31) / 32) {
     SWM_LW_CASE(1)
@@ -483,33 +621,33 @@ inline bool lw_aligned(const LinearStep& a, int dtype) {
          (reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k)) % 16 == 0;
 }
 
-int gla_walk(const LinearStep& a, const void* decay_pre, int64_t decay_stride, const float* decay_bias, float inv_tau, float q_scale,
+int gla_walk(const LinearStep& a, const LinearWalkPlan& plan, const void* decay_pre, int64_t decay_stride, const float* decay_bias, float inv_tau, float q_scale,
              int act_dtype, hipStream_t stream) {
   const int dp = (a.dim + 31) / 32 * 32;
   const size_t bytes = sizeof(float) * (80 * (size_t)(dp + 4) + 2 * dp + 4);
-  const dim3 grid((unsigned)(a.rows / kLwChunk + a.num_seqs), (unsigned)a.heads);       // an upper bound of the chunks
+  const dim3 grid((unsigned)plan.chunks, (unsigned)a.heads);       // an upper bound of the chunks
   SWM_DISPATCH_ACT(act_dtype, SW_CHECK_HIP(lw_allow_lds(gla_walk_prep_kernel<T>, bytes));
-                   hipLaunchKernelGGL(gla_walk_prep_kernel<T>, grid, dim3(kLwThreads), bytes, stream, a, decay_pre, decay_stride,
+                   hipLaunchKernelGGL(gla_walk_prep_kernel<T>, grid, dim3(kLwThreads), bytes, stream, a, plan.at_most, decay_pre, decay_stride,
                                       decay_bias, inv_tau, q_scale, dp);
                    SW_CHECK_LAUNCH();
-                   return (launch_walk<T, false>(a, stream)););
+                   return (launch_walk<T, false>(a, plan, stream)););
 }
 
-int lightning_walk(const LinearStep& a, const float* decay, bool silu, int q_dtype, int v_dtype, hipStream_t stream) {
+int lightning_walk(const LinearStep& a, const LinearWalkPlan& plan, const float* decay, bool silu, int q_dtype, int v_dtype, hipStream_t stream) {
   const int dp = (a.dim + 31) / 32 * 32;
   const size_t bytes = sizeof(float) * (64 * (size_t)(dp + 4) + kLwChunk + 4);
   const int vec = lw_aligned(a, q_dtype);
-  const dim3 grid((unsigned)(a.rows / kLwChunk + a.num_seqs), (unsigned)a.heads);       // an upper bound of the chunks
+  const dim3 grid((unsigned)plan.chunks, (unsigned)a.heads);       // an upper bound of the chunks
   if (silu) {                                    // one projection: q, k and v of one type
     SWM_DISPATCH_ACT(q_dtype, SW_CHECK_HIP(lw_allow_lds(lightning_walk_prep_kernel<T, true>, bytes));
-                     hipLaunchKernelGGL((lightning_walk_prep_kernel<T, true>), grid, dim3(kLwThreads), bytes, stream, a, decay, dp, vec);
+                     hipLaunchKernelGGL((lightning_walk_prep_kernel<T, true>), grid, dim3(kLwThreads), bytes, stream, a, plan.at_most, decay, dp, vec);
                      SW_CHECK_LAUNCH();
-                     return (launch_walk<T, true>(a, stream)););
+                     return (launch_walk<T, true>(a, plan, stream)););
   }
   SW_CHECK_HIP(lw_allow_lds(lightning_walk_prep_kernel<float, false>, bytes));
-  hipLaunchKernelGGL((lightning_walk_prep_kernel<float, false>), grid, dim3(kLwThreads), bytes, stream, a, decay, dp, vec);
+  hipLaunchKernelGGL((lightning_walk_prep_kernel<float, false>), grid, dim3(kLwThreads), bytes, stream, a, plan.at_most, decay, dp, vec);
   SW_CHECK_LAUNCH();
-  SWM_DISPATCH_ACT(v_dtype, return (launch_walk<T, false>(a, stream)););
+  SWM_DISPATCH_ACT(v_dtype, return (launch_walk<T, false>(a, plan, stream)););
 }
 
 }  // namespace swm
