@@ -1,5 +1,5 @@
 """linear_plan.h, by which a linear-attention step is shared out between the decode kernels and the walk, compiled for the CPU:
-its bounds hold for every batch, and a long run of few heads is cut."""
+its bounds hold for every batch, decoding sequences do not walk beside a prompt's portion, and a long run of few heads is cut."""
 import os
 import shutil
 import subprocess
@@ -40,6 +40,16 @@ int main() {
     need(p.segment % 32 == 0, "a segment that ends inside a chunk");
     const long dp = (dim + 31) / 32 * 32, vb = (vdim + 15) / 16;
     need(p.floats >= p.chunks * heads * (65 * dp + 1024) + (p.segment ? p.items * heads * (16 * vb * dp + dp) : 0), "scratch");
+  }
+  // many short runs fill the GPU: no prologue, no walk
+  need(linear_walk_plan(true, 64 * 17, 64, 17, 16, 128, 128).floats == 0, "64 x 17 walk");
+  need(linear_walk_plan(false, 64 * 100, 64, 100, 16, 128, 128).floats == 0, "64 x 100 walk");
+  // few do not
+  need(linear_walk_plan(true, 4 * 100, 4, 100, 4, 128, 128).at_most == 0, "4 x 100 do not walk");
+  // decoding sequences beside a portion go their own way
+  for (int portion : {300, 1000, 8000}) {
+    const LinearWalkPlan p = linear_walk_plan(true, 250 + portion, 251, portion, 16, 128, 128);
+    need(p.at_most == 16, "250 decoding sequences walk");
   }
   // a long run of few heads is cut into as many pieces as the GPU has room for
   for (int n : {8000, 16000, 32000}) {

@@ -8,17 +8,37 @@ namespace swm {
 
 constexpr int kLwChunk = 32;
 
-// Sequences of at most `at_most` tokens go through the kernels of decode steps (gla.hip, lightning.hip: a workgroup takes the whole
-// run of a sequence and a head), longer ones through the walk.  -> at_most: 0: the walk takes all, max_query_len: the decode
-// kernels do.  (us here / there, with norm and gate, the host's 30 a call included: 1 x 16 heads of 128, 16 tokens 32 / 34, 31 tokens
-// 37 / 34, 64 tokens 63 / 34, 1000 tokens 921 / 75)
+// A step with long runs is shared out between two ways: sequences of at most `at_most` tokens go through the kernels of decode
+// steps (gla.hip, lightning.hip: a workgroup takes the whole run of a sequence and a head), longer ones through the walk.
+// -> at_most: 0: the walk takes all, max_query_len: the decode kernels do.
+// per_channel: decays per key channel (gla), else one per head, whose decode kernels are the cheaper ones.
+// Measured (us a call with its norm and gate; W: sequences x heads, of 128 x 128):
+//   max_query_len <= 16: as decode steps, whatever W.
+//   Sequences of about one length, decode kernels / walk.  With few the walk's chunks, side by side, win: W = 16, 100 tokens, per
+//   channel 102 / 24.  With many the decode kernels fill the GPU by themselves and are spared the prologue's trip through memory:
+//   per channel W = 256, 32 tokens 48 / 60, 64 tokens 78 / 75; W = 512, 64 tokens 106 / 118, 150 tokens 259 / 232; W = 1024, 100
+//   tokens 353 / 379, 150 tokens 512 / 471.  Per head W = 256, 64 tokens 59 / 67; W = 512, 100 tokens 136 / 178, 200 tokens
+//   253 / 277; W = 1024, 200 tokens 511 / 559.
+//   Decoding sequences beside few long ones: a token costs the decode kernels about 1 us and the walk 0.06, a decoding sequence
+//   0.04 us per W and 0.13.  16 heads, all through the decode kernels / all through the walk / each its own way: per channel 60
+//   sequences beside a portion of 100 tokens 130 / 153 / 58, 250 beside 250 419 / 998 / 180; per head 60 beside 24 tokens
+//   70 / 134 / 81, 7 beside 100 87 / 46 / 52.
 inline int linear_at_most(bool per_channel, int64_t rows, int num_seqs, int max_query_len, int heads, int dim, int vdim) {
-  return max_query_len <= 16 ? max_query_len : 0;
+  constexpr int kShort = 16;
+  if (max_query_len <= kShort) return max_query_len;
+  const int64_t w = (int64_t)num_seqs * heads;
+  if (2 * rows >= (int64_t)max_query_len * num_seqs) {
+    const int64_t most = per_channel ? w * dim / 512 - 16 : w * dim / 256 - 48, cap = per_channel ? 128 : 256;
+    return max_query_len <= (most < kShort ? kShort : most > cap ? cap : most) ? max_query_len : 0;
+  }
+  const int64_t units = w * dim / 128;
+  if (max_query_len <= (units > 160 ? 36 : units > 112 ? 24 : kShort)) return max_query_len;
+  return units <= 160 ? 0 : kShort;
 }
 
 // A walk's sizes.  Few runs leave most of the GPU idle, and a long run's chunks are then worth cutting: into segments whose own
 // ends are worked out side by side, from nothing, and joined into the states that each segment truly starts from (one run of
-// 16000 tokens, 4 heads of 128: 867 us in one piece, 8 segments: see linear_walk.hip).  As many as still leave every workgroup a
+// 16000 tokens, 4 heads of 128: 870 us in one piece, 208 in 8).  As many as still leave every workgroup a
 // compute unit, of at least 16 chunks.
 struct LinearWalkPlan {
   int at_most, segment;                 // segment: tokens of a segment; 0: runs are not cut
