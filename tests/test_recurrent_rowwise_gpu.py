@@ -109,20 +109,23 @@ def test_delta_decode_step_in_one_launch(heads, kv_heads, dim, vdim, per_channel
 
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(2, 1, 32, 16), (3, 3, 64, 17), (6, 1, 96, 40), (4, 2, 128, 128), (2, 2, 160, 33),
                                                      (1, 1, 224, 64)])
-def test_delta_chunks_agree_with_the_tokens(heads, kv_heads, dim, vdim):
-    """Runs that end at, before and behind a chunk's border, from nothing and from a state, against the rule token by token:
-    fp32 sums in another order, over states whose size the rule keeps around that of the values."""
+@pytest.mark.parametrize("lens", [[32, 31, 1, 33, 64, 95, 2], [1] * 9 + [40, 16, 17, 0, 1, 3, 70], [1] * 80 + [33], [1] * 13])
+def test_delta_chunks_agree_with_the_tokens(heads, kv_heads, dim, vdim, lens):
+    """Runs that end at, before and behind a chunk's border, from nothing and from a state, alone and beside decoding sequences
+    (which go another way in the same call), against the rule token by token: fp32 sums in another order, over states whose size
+    the rule keeps around that of the values."""
     from splitwise_amd import _C
-    lens = [32, 31, 1, 33, 64, 95, 2]
+    n = len(lens)
+    ctx, slots = [(0, 3, 9, 0, 64, 0, 1)[i % 7] for i in range(n)], [(4, 0, 8, 2, 1, 7, 3)[i % 7] + i // 7 * 9 for i in range(n)]
     starts = [sum(lens[:i]) for i in range(len(lens) + 1)]
     g = torch.Generator(device=DEV).manual_seed(dim + vdim)
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
-    batch = SimpleNamespace(q_start=i32(starts), ctx_len=i32([0, 3, 9, 0, 64, 0, 1]), max_query_len=95, max_state_slot=8,
-                            token_seq=i32([i for i, n in enumerate(lens) for _ in range(n)]), state_slot=i32([4, 0, 8, 2, 1, 7, 3]))
+    batch = SimpleNamespace(q_start=i32(starts), ctx_len=i32(ctx), max_query_len=max(lens), max_state_slot=max(slots),
+                            token_seq=i32([i for i, m in enumerate(lens) for _ in range(m)]), state_slot=i32(slots))
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)               # noqa: E731
     rows = starts[-1]
     qkv, both = rnd(rows, 2 * kv_heads * dim + heads * vdim), rnd(rows, 2 * heads).to(torch.bfloat16)
-    dt_bias, a_log, state = rnd(heads), rnd(heads) * 0.3, rnd(9, heads, dim, vdim) * 0.1
+    dt_bias, a_log, state = rnd(heads), rnd(heads) * 0.3, rnd(max(slots) + 9, heads, dim, vdim) * 0.1
     res = []
     for chunked in (True, False):
         s, out = state.clone(), torch.full((rows, heads * vdim), float("nan"), device=DEV)
@@ -131,7 +134,8 @@ def test_delta_chunks_agree_with_the_tokens(heads, kv_heads, dim, vdim):
         res.append((out, s))
     torch.testing.assert_close(res[0][0], res[1][0], atol=2e-5, rtol=1e-4)
     torch.testing.assert_close(res[0][1], res[1][1], atol=2e-5, rtol=1e-4)
-    assert torch.equal(res[0][1][[5, 6]], state[[5, 6]])
+    idle = [i for i in range(state.shape[0]) if i not in slots]
+    assert torch.equal(res[0][1][idle], state[idle])
 
 
 @pytest.mark.parametrize("rule", ["gla", "gla, strong decays", "lightning", "retention"])

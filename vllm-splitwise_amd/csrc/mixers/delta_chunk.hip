@@ -22,7 +22,10 @@
 // L is summed in 64 bits: its differences are what counts, and where decays are strong 32 bits leave the end states an error of
 // 0.5 - 1.3e-6 (1.3 - 1.5e-7 here, for the prologue's 69 us all the same).
 // Rows of a last, shorter chunk are padded with beta = 0, k = 0, g = 1: they change nothing and are not stored.
+#include "delta_step.h"
 #include "mixers_common.cuh"
+
+#include <algorithm>
 
 namespace swm {
 
@@ -30,6 +33,7 @@ using f32x4 = __attribute__((ext_vector_type(4))) float;
 using f32x16 = __attribute__((ext_vector_type(16))) float;
 constexpr int kDcChunk = 32;
 constexpr int kDcPrepThreads = 256;
+constexpr int kDcShort = 16;             // tokens of a sequence that goes the decode kernel's way in a mixed step
 constexpr int kDcChannels = 16;          // value channels of a walk's workgroup
 
 // floats of one (chunk, key head) in the workspace: K | Q ([32][dp] each) | K^T [dp][32]
@@ -46,15 +50,15 @@ template <typename T>
 __global__ __launch_bounds__(kDcPrepThreads) void delta_chunk_prep_kernel(
     float* __restrict__ keys, float* __restrict__ records, const float* __restrict__ qkv, const void* __restrict__ beta_pre,
     int64_t beta_stride, const void* __restrict__ decay_pre, int64_t decay_stride, const float* __restrict__ dt_bias,
-    const float* __restrict__ a_log, const int32_t* __restrict__ q_start, int num_seqs, int heads, int kv_heads, int dim,
-    int vdim, int dp) {
+    const float* __restrict__ a_log, const int32_t* __restrict__ q_start, int num_seqs, int at_most, int heads, int kv_heads,
+    int dim, int vdim, int dp) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int KS = dp + 4;                         // rows on 16 bytes
   float* Kn = lds;                               // [32][KS] unit keys
   float* Qn = Kn + kDcChunk * KS;                // [32][KS] unit queries times dim^-1/2
   float* red = Qn + kDcChunk * KS;               // [4 waves][2][4][64] quads: shares of K K^T and Q K^T; later A and L
-  int seq = 0, tok0 = 0;
-  const int cn = find_query_tile(q_start, num_seqs, blockIdx.x, kDcChunk, &seq, &tok0);
+  int seq = 0, tok0 = 0, before = 0;
+  const int cn = find_run_piece(q_start, num_seqs, at_most, kDcChunk, blockIdx.x, &seq, &tok0, &before);
   if (cn <= 0) return;                           // the whole workgroup
   const int g = blockIdx.y, group = heads / kv_heads;
   const int64_t row0 = q_start[seq] + tok0;
@@ -216,19 +220,17 @@ template <int NDB>
 __global__ __launch_bounds__(64 * NDB) void delta_chunk_kernel(
     float* __restrict__ out, const float* __restrict__ keys, const float* __restrict__ records, const float* __restrict__ qkv,
     float* __restrict__ state, const int32_t* __restrict__ q_start, const int32_t* __restrict__ ctx_len,
-    const int32_t* __restrict__ state_slot, int num_seqs, int heads, int kv_heads, int dim, int vdim) {
+    const int32_t* __restrict__ state_slot, int num_seqs, int at_most, int64_t runs, int heads, int kv_heads, int dim, int vdim) {
   __shared__ f32x4 red[2][2][NDB][2][64];        // [chunk parity][K S_0 | Q S_0][wave][token tile][lane]
   constexpr int DP = NDB * 32;
   const int vblocks = (vdim + kDcChannels - 1) / kDcChannels;
   const int unit = (blockIdx.x >> 3) / vblocks * 8 + (blockIdx.x & 7), vb = (blockIdx.x >> 3) % vblocks;
-  if (unit >= num_seqs * heads) return;          // the whole workgroup
-  const int seq = unit / heads, h = unit - seq * heads, g = h / (heads / kv_heads);
-  const int b = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, gq = lane >> 4;
-  const int n = q_start[seq + 1] - q_start[seq];
+  const int run = unit / heads, h = unit - run * heads, g = h / (heads / kv_heads);
+  int seq = 0, tok0 = 0, chunk0 = 0;             // chunk0: this sequence's first chunk among the step's
+  const int n = run < runs ? find_run_piece(q_start, num_seqs, at_most, 1 << 30, run, &seq, &tok0, &chunk0) : 0;
   if (n <= 0) return;                            // the whole workgroup
+  const int b = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, gq = lane >> 4;
   const int64_t row0 = q_start[seq];
-  int64_t chunk0 = 0;                            // this sequence's first chunk among the step's
-  for (int s = 0; s < seq; ++s) chunk0 += (q_start[s + 1] - q_start[s] + kDcChunk - 1) / kDcChunk;
   const int vc = vb * kDcChannels + li;          // this lane's value channel
   const bool vc_ok = vc < vdim;
   float* sp = state + ((int64_t)state_slot[seq] * heads + h) * (int64_t)dim * vdim;
@@ -245,8 +247,8 @@ __global__ __launch_bounds__(64 * NDB) void delta_chunk_kernel(
   const float* vsrc = qkv + row0 * row_w + 2 * (int64_t)kv_heads * dim + (int64_t)h * vdim + (vc_ok ? vc : vdim - 1);
   const int chunks = (n + kDcChunk - 1) / kDcChunk;
   auto fetch = [&](DcOperands& x, int ci) {
-    const float* kp = keys + ((chunk0 + ci) * kv_heads + g) * dc_keys_floats(DP);
-    const float* rec = records + ((chunk0 + ci) * heads + h) * kDcRecord;
+    const float* kp = keys + ((int64_t)(chunk0 + ci) * kv_heads + g) * dc_keys_floats(DP);
+    const float* rec = records + ((int64_t)(chunk0 + ci) * heads + h) * kDcRecord;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
 #pragma unroll
@@ -425,12 +427,12 @@ inline hipError_t dc_allow_lds(K kernel, size_t bytes) {
 
 template <int NDB>
 int launch_delta_chunk(float* out, const float* keys, const float* records, const float* qkv, float* state, const int32_t* q_start,
-                       const int32_t* ctx_len, const int32_t* state_slot, int num_seqs, int heads, int kv_heads, int dim, int vdim,
-                       hipStream_t stream) {
-  const int64_t units = ((int64_t)num_seqs * heads + 7) / 8 * 8, groups = units * ((vdim + kDcChannels - 1) / kDcChannels);
+                       const int32_t* ctx_len, const int32_t* state_slot, int num_seqs, int at_most, int64_t runs, int heads,
+                       int kv_heads, int dim, int vdim, hipStream_t stream) {
+  const int64_t units = (runs * heads + 7) / 8 * 8, groups = units * ((vdim + kDcChannels - 1) / kDcChannels);
   SW_CHECK_ARG(groups < (1ll << 31), "gated_delta_chunked: too many sequences and heads");
   hipLaunchKernelGGL(delta_chunk_kernel<NDB>, dim3((unsigned)groups), dim3(64 * NDB), 0, stream, out, keys, records, qkv, state,
-                     q_start, ctx_len, state_slot, num_seqs, heads, kv_heads, dim, vdim);
+                     q_start, ctx_len, state_slot, num_seqs, at_most, runs, heads, kv_heads, dim, vdim);
   SW_CHECK_LAUNCH();
   return SW_OK;
 }
@@ -459,20 +461,30 @@ int swm_gated_delta_chunked(float* out, const float* qkv, const void* beta_pre, 
                vdim);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int ndb = (dim + 31) / 32, dp = ndb * 32;
-  const int64_t chunks = rows / kDcChunk + num_seqs;            // an upper bound: surplus workgroups leave at once
+  // Decoding sequences beside a portion take the decode kernel: their states are read and written in whole rows there, in 64-byte
+  // pieces here, and they need no 32-row record.  Not worth the launch where most sequences are long.  (us a call, 12 heads of 96, a
+  // portion of 100 tokens beside 60 / 250 decoding sequences: 186 / 1046 all in chunks, 61 / 104 so)
+  const bool mixed = num_seqs >= 12 && rows < 128 * (int64_t)num_seqs &&
+                     delta_step(out, qkv, beta_pre, beta_stride, decay_pre, decay_stride, 1, dt_bias, a_log, state, q_start, ctx_len,
+                                state_slot, num_seqs, heads, kv_heads, dim, vdim, kDcShort, act_dtype, s);
+  SW_CHECK_LAUNCH();
+  const int at_most = mixed ? kDcShort : 0;
+  const int64_t runs = mixed ? std::min<int64_t>(num_seqs, rows / (kDcShort + 1)) : num_seqs;
+  if (runs == 0) return SW_OK;
+  const int64_t chunks = rows / kDcChunk + runs;                // an upper bound: surplus workgroups leave at once
   float* keys = workspace;
   float* records = workspace + chunks * kv_heads * dc_keys_floats(dp);
   const size_t prep_lds = sizeof(float) * (2 * (size_t)kDcChunk * (dp + 4) + 4 * 2 * 4 * 64 * 4);
   SWM_DISPATCH_ACT(act_dtype, SW_CHECK_HIP(dc_allow_lds(delta_chunk_prep_kernel<T>, prep_lds)););
   SWM_DISPATCH_ACT(act_dtype, hipLaunchKernelGGL(delta_chunk_prep_kernel<T>, dim3((unsigned)chunks, (unsigned)kv_heads),
                                                  dim3(kDcPrepThreads), prep_lds, s, keys, records, qkv, beta_pre, beta_stride,
-                                                 decay_pre, decay_stride, dt_bias, a_log, q_start, num_seqs, heads,
+                                                 decay_pre, decay_stride, dt_bias, a_log, q_start, num_seqs, at_most, heads,
                                                  kv_heads, dim, vdim, dp););
   SW_CHECK_LAUNCH();
 #define SWM_DC_CASE(N)                                                                                                       \
   case N:                                                                                                                    \
-    return launch_delta_chunk<N>(out, keys, records, qkv, state, q_start, ctx_len, state_slot, num_seqs, heads, kv_heads,     \
-                                 dim, vdim, s);
+    return launch_delta_chunk<N>(out, keys, records, qkv, state, q_start, ctx_len, state_slot, num_seqs, at_most, runs, heads, \
+                                 kv_heads, dim, vdim, s);
   switch (ndb) {
     SWM_DC_CASE(1)
     SWM_DC_CASE(2)

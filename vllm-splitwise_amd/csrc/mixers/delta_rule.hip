@@ -11,15 +11,12 @@
 // of the step (not at all when the sequence starts here) and written once after the last: a decode step moves
 // exactly the state, a prompt portion moves it once per portion.  Operands of the next 8 tokens are in flight
 // while the current 8 are worked through (see delta_recurrence_kernel).
+#include "delta_step.h"
 #include "mixers_common.cuh"
 
-namespace swm {
+#include <climits>
 
-// delta_step.hip: a decode step in one launch; false when the sizes or addresses are not for it
-bool delta_step(float* out, const float* qkv, const void* beta_pre, int64_t beta_stride, const void* decay_pre,
-                int64_t decay_stride, int decay_per_head, const float* dt_bias, const float* a_log, float* state,
-                const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot, int num_seqs, int heads, int kv_heads,
-                int dim, int vdim, int act_dtype, hipStream_t stream);
+namespace swm {
 
 constexpr int kColsPerWave = 16;
 constexpr int kPrepThreads = 256;
@@ -330,7 +327,7 @@ static int delta_with_decay(float* out, const float* qkv, const void* beta_pre, 
   hipStream_t s = static_cast<hipStream_t>(stream);
   // as many rows as sequences: a decode step (should a sequence bring none and another two, it is right all the same)
   if (rows <= num_seqs && delta_step(out, qkv, beta_pre, beta_stride, decay_pre, decay_stride, decay_per_head, dt_bias, a_log,
-                                     state, q_start, ctx_len, state_slot, num_seqs, heads, kv_heads, dim, vdim, act_dtype, s)) {
+                                     state, q_start, ctx_len, state_slot, num_seqs, heads, kv_heads, dim, vdim, INT_MAX, act_dtype, s)) {
     SW_CHECK_LAUNCH();
     return SW_OK;
   }

@@ -8,6 +8,7 @@
 // Measured, 61 sequences x 16 heads of 128 x 128 (128 MB of states read and written), convolution, norm and gate included: 100 us
 // as a prologue and a recurrence with 16 columns per wave read in pieces of 64 bytes (1.3 TB/s), 39 us here.
 // Longer runs of tokens are walked token by token with the state staying in registers.
+#include "delta_step.h"
 #include "mixers_common.cuh"
 
 #include <algorithm>
@@ -23,7 +24,7 @@ __global__ __launch_bounds__(kStepThreads) void delta_step_kernel(
     const void* __restrict__ decay_pre, int64_t decay_stride, int decay_per_head, const float* __restrict__ dt_bias,
     const float* __restrict__ a_log, float* __restrict__ state, const int32_t* __restrict__ q_start,
     const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int kv_heads, int dim, int vdim,
-    int lanes) {
+    int lanes, int at_most) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int groups = kStepThreads / lanes;                   // lanes: threads across the value channels, a power of two
   float* Q = lds;                                            // [dim] unit query times dim^-1/2
@@ -33,7 +34,7 @@ __global__ __launch_bounds__(kStepThreads) void delta_step_kernel(
   float* red = part + kStepThreads * 4;                      // [4][2]
   const int h = blockIdx.y, s = blockIdx.z;
   const int first = q_start[s], n = q_start[s + 1] - first;
-  if (n <= 0) return;                                        // the whole workgroup
+  if (n <= 0 || n > at_most) return;                         // the whole workgroup
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int piece = tid % lanes, group = tid / lanes;
   const int col = (blockIdx.x * lanes + piece) * 4;
@@ -133,14 +134,14 @@ __global__ __launch_bounds__(kStepThreads) void delta_step_kernel(
   }
 }
 
-// -> true when the step went here: value channels in pieces of 16 bytes, key sizes up to 256.  (The caller asks for decode
-// steps only: a long run of tokens meets six barriers a token here.)  Lanes across the value channels: as many as leave at most
+// Sequences of at most `at_most` tokens: a long run meets six barriers a token here.  -> true when they went here: value channels in
+// pieces of 16 bytes, key sizes up to 256.  Lanes across the value channels: as many as leave at most
 // 8 rows per thread, but a whole 128-byte line at least.
 template <typename T>
 bool try_delta_step(float* out, const float* qkv, const void* beta_pre, int64_t beta_stride, const void* decay_pre,
                     int64_t decay_stride, int decay_per_head, const float* dt_bias, const float* a_log, float* state,
                     const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot, int num_seqs, int heads,
-                    int kv_heads, int dim, int vdim, hipStream_t stream) {
+                    int kv_heads, int dim, int vdim, int at_most, hipStream_t stream) {
   const uintptr_t at = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(state);
   if (vdim % 4 != 0 || (2 * kv_heads * dim) % 4 != 0 || at % 16 != 0 || dim > kStepThreads || num_seqs > 65535 || heads > 65535)
     return false;
@@ -152,7 +153,7 @@ bool try_delta_step(float* out, const float* qkv, const void* beta_pre, int64_t 
 #define SWM_STEP(R)                                                                                                            \
   hipLaunchKernelGGL((delta_step_kernel<T, R>), grid, dim3(kStepThreads), bytes, stream, out, qkv, beta_pre, beta_stride,      \
                      decay_pre, decay_stride, decay_per_head, dt_bias, a_log, state, q_start, ctx_len, state_slot, heads,      \
-                     kv_heads, dim, vdim, lanes)
+                     kv_heads, dim, vdim, lanes, at_most)
   if (rows <= 4) SWM_STEP(4);
   else SWM_STEP(8);
 #undef SWM_STEP
@@ -162,11 +163,11 @@ bool try_delta_step(float* out, const float* qkv, const void* beta_pre, int64_t 
 bool delta_step(float* out, const float* qkv, const void* beta_pre, int64_t beta_stride, const void* decay_pre,
                 int64_t decay_stride, int decay_per_head, const float* dt_bias, const float* a_log, float* state,
                 const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot, int num_seqs, int heads, int kv_heads,
-                int dim, int vdim, int act_dtype, hipStream_t stream) {
+                int dim, int vdim, int at_most, int act_dtype, hipStream_t stream) {
   bool taken = false;
   SWM_DISPATCH_ACT(act_dtype, taken = try_delta_step<T>(out, qkv, beta_pre, beta_stride, decay_pre, decay_stride, decay_per_head,
                                                         dt_bias, a_log, state, q_start, ctx_len, state_slot, num_seqs, heads,
-                                                        kv_heads, dim, vdim, stream););
+                                                        kv_heads, dim, vdim, at_most, stream););
   return taken;
 }
 

@@ -107,7 +107,7 @@ __global__ __launch_bounds__(kLwThreads, 3) void gla_walk_prep_kernel(const Line
   float* total = Ko + 16 * KS;                   // [2][dp] the halves' sums of log a
   int* unsafe = reinterpret_cast<int*>(total + 2 * dp);                  // [2]
   int seq = 0, tok0 = 0, before = 0;
-  const int cn = lw_find_piece(a.q_start, a.num_seqs, at_most, kLwChunk, blockIdx.x, &seq, &tok0, &before);
+  const int cn = find_run_piece(a.q_start, a.num_seqs, at_most, kLwChunk, blockIdx.x, &seq, &tok0, &before);
   if (cn <= 0) return;                           // the whole workgroup
   const int h = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int64_t row0 = a.q_start[seq] + tok0;
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kLwThreads) void lightning_walk_prep_kernel(const L
   float* Ks = Qs + kLwChunk * KS;                // [32][KS]
   float* pw = Ks + kLwChunk * KS;                // [33] powers of the decay, by repeated multiplication
   int seq = 0, tok0 = 0, before = 0;
-  const int cn = lw_find_piece(a.q_start, a.num_seqs, at_most, kLwChunk, blockIdx.x, &seq, &tok0, &before);
+  const int cn = find_run_piece(a.q_start, a.num_seqs, at_most, kLwChunk, blockIdx.x, &seq, &tok0, &before);
   if (cn <= 0) return;                           // the whole workgroup
   const int h = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int64_t row0 = a.q_start[seq] + tok0;
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(64 * NDB) void linear_segment_kernel(const LinearSt
   const int unit = (blockIdx.x >> 3) / vblocks * 8 + (blockIdx.x & 7), vb = (blockIdx.x >> 3) % vblocks;
   const int item = unit / a.heads, h = unit - item * a.heads;
   int seq = 0, tok0 = 0, before = 0;
-  const int n = item < pc.items ? lw_find_piece(a.q_start, a.num_seqs, pc.at_most, pc.segment, item, &seq, &tok0, &before) : 0;
+  const int n = item < pc.items ? find_run_piece(a.q_start, a.num_seqs, pc.at_most, pc.segment, item, &seq, &tok0, &before) : 0;
   if (n <= 0) return;                            // the whole workgroup
   const int run = a.q_start[seq + 1] - a.q_start[seq], behind = (run - tok0 - 1) / pc.segment;      // segments behind this one
   if (behind == 0) return;                       // (n is a whole segment otherwise)
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(64 * NDB) void linear_walk_kernel(const LinearStep 
   const int unit = (blockIdx.x >> 3) / vblocks * 8 + (blockIdx.x & 7), vb = (blockIdx.x >> 3) % vblocks;
   const int item = unit / a.heads, h = unit - item * a.heads;
   int seq = 0, tok0 = 0, before = 0;
-  const int n = item < pc.items ? lw_find_piece(a.q_start, a.num_seqs, pc.at_most, pc.segment > 0 ? pc.segment : 1 << 30, item, &seq,
+  const int n = item < pc.items ? find_run_piece(a.q_start, a.num_seqs, pc.at_most, pc.segment > 0 ? pc.segment : 1 << 30, item, &seq,
                                                 &tok0, &before)
                                 : 0;
   if (n <= 0) return;                            // the whole workgroup
