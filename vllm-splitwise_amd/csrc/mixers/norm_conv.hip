@@ -385,7 +385,10 @@ __global__ __launch_bounds__(kRowThreads) void conv_run_kernel(
 }
 
 constexpr int kConvRun = 8;              // rows of a run; at least the most rows that read a carried input
-constexpr int kConvRunRows = 1024;       // steps of fewer rows (decode steps) take one row per workgroup
+// Steps of fewer rows than kConvRunRows take one row per workgroup, and so do steps whose runs would leave compute units without a
+// workgroup: there short sequences, one after the other in a run, cost more than the inputs read again (1100 sequences of one
+// token x 256 channels: 5.9 us a row and a channel per thread, 13.7 in runs, 5.0 a row; one of 1500 tokens 6.1, 6.2 and 5.1).
+constexpr int kConvRunRows = 1024, kConvGroups = 256;
 
 template <typename TX, typename TO>
 bool try_conv_runs(void* out, const void* x, int64_t x_stride, const float* taps, float* state, const int32_t* q_start,
@@ -394,8 +397,9 @@ bool try_conv_runs(void* out, const void* x, int64_t x_stride, const float* taps
   constexpr int V = 4;
   if (num_taps < 2 || num_taps > 4 || channels % V != 0 || x_stride % V != 0 || !on16(out) || !on16(x) || !on16(state))
     return false;
-  const int run = rows >= kConvRunRows ? kConvRun : 1;
-  const dim3 grid((unsigned)((rows + run - 1) / run), (unsigned)((channels / V + kRowThreads - 1) / kRowThreads));
+  const int64_t columns = (channels / V + kRowThreads - 1) / kRowThreads;
+  const int run = rows >= kConvRunRows && rows / kConvRun * columns >= kConvGroups ? kConvRun : 1;
+  const dim3 grid((unsigned)((rows + run - 1) / run), (unsigned)columns);
 #define SWM_CONV_RUN(NT)                                                                                                     \
   hipLaunchKernelGGL((conv_run_kernel<TX, TO, V, NT>), grid, dim3(kRowThreads), 0, stream, out, x, x_stride, taps, state,    \
                      q_start, ctx_len, token_seq, state_slot, rows, channels, silu, residual, advance, run)
