@@ -492,7 +492,7 @@ __global__ __launch_bounds__(256, 2) void expert_tile_kernel(const ExpertArgs a)
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
           const int c = n0 + wn * (BN / 2) + 32 * j + li;
-                    if (c < a.N) atomicAdd(dst + c, wt * acc[i][j][r]);
+          if (c < a.N) atomicAdd(dst + c, wt * acc[i][j][r]);
         }
       }
   }
@@ -519,14 +519,19 @@ int launch_expert_tiles(const ExpertArgs& a, int64_t pairs, hipStream_t stream) 
 //   64 experts 2048 -> 1024, four per row:  6: 114 / 115 / 120 / 149;   96: 432 / 200 / 197 / 311;   250: 994 / 365 / 308 / 640
 //   8 experts 2048 -> 1024, 250 pairs each: 148 / 64 / 70 / 108: too few tiles of 128 x 128 for 256 compute units
 constexpr int kFewPairs = 6;            // pairs per expert up to which a step's weights are streamed
+constexpr int kFewGroups = 16384;
 constexpr int kManyPairs = 96;          // pairs per expert from which tiles of 128 pairs are mostly full ...
 constexpr int kManyTiles = 384;         // ... if there are this many of them
 template <bool DOWN>
 int launch_experts(const ExpertArgs& a, int64_t pairs, hipStream_t stream) {
   if (pairs <= (int64_t)kFewPairs * a.num_experts && a.num_experts < 65536) {
-    // an expert that many more rows ask for than the average has its rows shared out among several workgroups
-    const unsigned shares = (unsigned)std::min<int64_t>(8, (pairs + 255) / 256);
-    const dim3 grid((unsigned)((a.N + kFewRows - 1) / kFewRows), (unsigned)a.num_experts, shares);
+    // an expert that many more rows ask for than the average has its rows shared out among several workgroups: one for every 64
+    // pairs where the launch stays within kFewGroups workgroups, or else for every 256 (most of them find nothing to do).  64 experts
+    // 2048 -> 1024, all of 200 rows on one: 91 us in 64 x 64 tiles, 111 with a workgroup for all, 77 with 4
+    const int64_t cols = (a.N + kFewRows - 1) / kFewRows;
+    const int64_t room = std::max<int64_t>(std::min<int64_t>(8, (pairs + 255) / 256), kFewGroups / (cols * a.num_experts));
+    const unsigned shares = (unsigned)std::min<int64_t>(room, (pairs + 63) / 64);
+    const dim3 grid((unsigned)cols, (unsigned)a.num_experts, shares);
     hipLaunchKernelGGL(expert_few_rows_kernel<DOWN>, grid, dim3(64 * kFewWaves), 0, stream, a);
     SW_CHECK_LAUNCH();
     return SW_OK;
