@@ -1,0 +1,53 @@
+"""attention_plan.h, by which a step of the paged attention finds its kernels, compiled for the CPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HEADER = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "vllm-splitwise_amd", "csrc", "mixers")
+
+PROGRAM = r"""
+#include "attention_plan.h"
+#include <cstdio>
+#include <cstdlib>
+using namespace swm;
+static void need(bool ok, const char* what) { if (!ok) { std::printf("%s\n", what); std::exit(1); } }
+int main() {
+  // one query row over few keys: the vector kernel (a page of 16 keys, a table of `width` pages)
+  auto way = [](int mql, int heads, int kv, int dim, int width, int window = 0, int chunk = 0) {
+    return attention_way(true, 4, mql, heads, kv, dim, dim, 16, width, window, chunk);
+  };
+  for (int dim : {16, 32, 40, 64, 72, 96, 104, 128}) need(way(1, 8, 8, dim, 1) == kGeneralAttention, "one row, a page of keys");
+  need(way(1, 8, 8, 128, 32) == kGeneralAttention && way(1, 8, 8, 128, 33) == kDecodeOnMatrixCores, "one row of 128");
+  need(way(1, 8, 8, 64, 16) == kGeneralAttention && way(1, 8, 8, 64, 17) == kDecodeOnMatrixCores, "one row of 64");
+  need(way(1, 8, 8, 64, 500, 200) == kGeneralAttention && way(1, 8, 8, 64, 500, 0, 256) == kGeneralAttention, "one row, masks");
+  // more rows: the matrix cores whatever the keys
+  need(way(2, 8, 8, 64, 1) == kDecodeOnMatrixCores && way(1, 8, 4, 64, 1) == kDecodeOnMatrixCores, "two rows");
+  need(way(1, 8, 1, 64, 1) == kDecodeOnMatrixCores && way(9, 8, 8, 64, 1) == kGeneralAttention, "eight and nine rows");
+  need(way(33, 8, 8, 64, 1) == kPromptOnMatrixCores && way(0, 8, 8, 64, 1) == kPromptOnMatrixCores, "a prompt");
+  for (int mql = 0; mql < 70; ++mql) need(attention_way(false, 4, mql, 8, 8, 64, 64, 16, 100, 0, 0) == kGeneralAttention, "no pieces");
+  // what the matrix kernels can read
+  need(attention_pieces(0, 128, 128, 1024, 1024) && attention_pieces(32, 8, 120, 8, 120), "pieces");
+  need(!attention_pieces(8, 128, 128, 1024, 1024) && !attention_pieces(0, 132, 128, 1024, 1024) &&
+           !attention_pieces(0, 60, 64, 1024, 1024) && !attention_pieces(0, 64, 64, 1028, 1024), "no pieces");
+  // keys are only shared out where the matrix kernel has the step
+  for (int trial = 0; trial < 100000; ++trial) {
+    const int kv = 1 + std::rand() % 8, heads = kv * (1 + std::rand() % 8), mql = std::rand() % 12, width = 1 + std::rand() % 600;
+    const int dim = 8 * (1 + std::rand() % 16), window = std::rand() % 3 ? 0 : 1 + std::rand() % 3000;
+    const int seqs = 1 + std::rand() % 20, parts = decode_attention_parts(seqs, mql, heads, kv, 16, width, window, 0);
+    need(parts >= 1 && parts <= 16, "parts");
+    if (parts > 1) need(attention_way(true, seqs, mql, heads, kv, dim, dim, 16, width, window, 0) == kDecodeOnMatrixCores, "shared keys");
+  }
+  std::printf("ok\n");
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_plan(tmp_path):
+    source = tmp_path / "plan.cpp"
+    source.write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", HEADER, str(source), "-o", str(tmp_path / "plan")], check=True)
+    done = subprocess.run([str(tmp_path / "plan")], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0 and done.stdout == "ok\n", done.stdout

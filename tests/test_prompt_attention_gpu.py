@@ -1,8 +1,12 @@
-"""Prompt steps of the mixers' attention on the bf16 matrix cores against the general kernel.
+"""Steps of the mixers' attention on the bf16 matrix cores against the attention in 64 bits and against the general kernel.
 
-The general kernel takes a call whose queries do not lie on 16 bytes, so the same step with its queries moved by one float
-is the reference.  Both keep scores, weights and sums in fp32 (an error of about 1e-5 of the largest value) and round once to
-bf16: two results are at most one unit in the last place, 2^-7 of the value at most, apart."""
+The general kernel takes a call whose queries do not lie on 16 bytes, so the same step is made with its queries moved by one
+float too.  Both keep scores, weights and sums in fp32 (an error of about 1e-5 of the largest value) and round once to bf16: two
+results are at most one unit in the last place, 2^-7 of the value at most, apart.  Which kernels a call goes to is asked of
+attention_plan.h, which the launch code goes by."""
+import ctypes
+import os
+import subprocess
 from types import SimpleNamespace
 
 import pytest
@@ -10,6 +14,35 @@ import torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+
+
+PROMPT, DECODE, GENERAL = range(3)                           # enum AttentionWay
+PLAN = r"""
+#include "attention_plan.h"
+extern "C" int way(unsigned long at, long k_stride, long v_stride, int seqs, int mql, int heads, int kv_heads, int dim, int vdim, int page,
+                   int width, int window, int chunk) {
+  return swm::attention_way(swm::attention_pieces(at, dim, vdim, k_stride, v_stride), seqs, mql, heads, kv_heads, dim, vdim, page,
+                            width, window, chunk);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def way(tmp_path_factory):
+    """-> the kernels that a call goes to."""
+    at = tmp_path_factory.mktemp("plan")
+    (at / "plan.cpp").write_text(PLAN)
+    mixers = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "vllm-splitwise_amd", "csrc", "mixers")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", mixers, str(at / "plan.cpp"), "-o", str(at / "plan.so")],
+                   check=True)
+    lib = ctypes.CDLL(str(at / "plan.so"))
+
+    def ask(q, kc, vc, batch, H, G, d, dv, window=0, chunk=0, **_):
+        vc = kc if vc is None else vc
+        at = q.data_ptr() | kc.data_ptr() | vc.data_ptr()
+        return lib.way(ctypes.c_ulong(at), ctypes.c_long(kc.shape[2]), ctypes.c_long(vc.shape[2]), batch.num_seqs, batch.max_query_len, H,
+                       G, d, dv, kc.shape[1], batch.block_tables.shape[1], window, chunk)
+    return ask
 
 
 def _step(lengths, page):
@@ -90,7 +123,7 @@ def test_infinities_in_the_cache(H, G, d, option, lengths):
 @pytest.mark.parametrize("H,G,d,dv,page", [(4, 4, 128, 128, 16), (8, 2, 64, 96, 16), (6, 2, 40, 24, 8), (32, 1, 16, 8, 32),
                                            (3, 1, 104, 128, 12)])
 @pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "sink", "learned sink", "sigmoid", "values in the keys"])
-def test_prompt_steps_agree_with_the_general_kernel(H, G, d, dv, page, option):
+def test_prompt_steps_agree_with_the_general_kernel(H, G, d, dv, page, option, way):
     from splitwise_amd import _C
     per_wg = 4 * (32 // (H // G))                            # tokens of a workgroup
     lengths = [(0, per_wg), (5, per_wg + 1), (0, 1), (31, max(1, per_wg - 1)), (0, 2 * per_wg + 33), (200, 32), (64, 1)]
@@ -119,11 +152,14 @@ def test_prompt_steps_agree_with_the_general_kernel(H, G, d, dv, page, option):
         at = torch.empty(rows * H * d + 1, device=DEV)[lead:lead + rows * H * d].view(rows, H * d)
         at.copy_(q[:rows * H * d].view(rows, H * d))
         assert at.data_ptr() % 16 == 4 * lead
+        assert way(at, kc, vc, batch, H, G, d, dv, **kw) == (GENERAL if lead else PROMPT)
         out = torch.full((rows, H * dv), float("nan"), dtype=torch.bfloat16, device=DEV)
         _C.mixer_ops.capped_attention(out, at, kc, vc, gate if option != "plain" else None, batch, H, G, d, dv, d ** -0.5,
                                       **kw)
         outs.append(out.float())
     torch.testing.assert_close(outs[0], outs[1], atol=2e-4, rtol=2.0 ** -7)
+    ref = _statement(lengths, batch, at, kc, vc, gate if option != "plain" else None, H, G, d, dv, **kw)
+    torch.testing.assert_close(outs[0].double(), ref, atol=2e-4, rtol=2.0 ** -7)
     assert outs[0].isfinite().all() and outs[0].abs().max() > 0.1
 
 
@@ -131,7 +167,7 @@ def test_prompt_steps_agree_with_the_general_kernel(H, G, d, dv, page, option):
                                            (5, 1, 104, 128, 12)])
 @pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "sink", "learned sink", "sigmoid", "values in the keys"])
 @pytest.mark.parametrize("long", [0, 1, 2])
-def test_decode_steps_agree_with_the_general_kernel(H, G, d, dv, page, option, long):
+def test_decode_steps_agree_with_the_general_kernel(H, G, d, dv, page, option, long, way):
     """Few query rows per sequence and key/value head: one or two sets of four, one or several workgroups per sequence (the
     step's longest context decides), contexts at the edges of the 32-key tiles.  Same bound as above."""
     from splitwise_amd import _C
@@ -141,6 +177,7 @@ def test_decode_steps_agree_with_the_general_kernel(H, G, d, dv, page, option, l
     batch, pages = _step(lengths, page)
     g = torch.Generator(device=DEV).manual_seed(H * 100 + d + long)
     rows = sum(n for _, n in lengths)
+    few = H == G and long == 2 and option in ("window", "chunk")             # one query row that sees few keys
     if option == "values in the keys" and G > 1:
         dv = d
     kc = torch.randn(pages, page, G * d, generator=g, device=DEV).to(torch.bfloat16)
@@ -164,10 +201,34 @@ def test_decode_steps_agree_with_the_general_kernel(H, G, d, dv, page, option, l
     for lead in (0, 1):                                      # aligned queries, then the same ones a float further on
         at = torch.empty(rows * H * d + 1, device=DEV)[lead:lead + rows * H * d].view(rows, H * d)
         at.copy_(q[:rows * H * d].view(rows, H * d))
+        assert way(at, kc, vc, batch, H, G, d, dv, **kw) == (GENERAL if lead or few else DECODE)
         out = torch.full((rows, H * dv), float("nan"), dtype=torch.bfloat16, device=DEV)
         _C.mixer_ops.capped_attention(out, at, kc, vc, gate if option != "plain" else None, batch, H, G, d, dv, d ** -0.5,
                                       **kw)
         outs.append(out.float())
     torch.testing.assert_close(outs[0], outs[1], atol=2e-4, rtol=2.0 ** -7)
+    ref = _statement(lengths, batch, at, kc, vc, gate if option != "plain" else None, H, G, d, dv, **kw)
+    torch.testing.assert_close(outs[0].double(), ref, atol=2e-4, rtol=2.0 ** -7)
     # (a mean over up to 4002 keys of values of spread 1: 4002^-1/2 = 0.016 at least, the largest of them more)
     assert outs[0].isfinite().all() and outs[0].abs().max() > 0.016
+
+
+@pytest.mark.parametrize("G,d,most", [(3, 128, 512), (8, 64, 256), (2, 96, 160), (3, 104, 512), (5, 40, 256), (1, 16, 160), (300, 32, 320)])
+@pytest.mark.parametrize("option", ["plain", "cap", "learned sink", "sigmoid"])
+def test_one_query_row_on_both_sides_of_the_rule(G, d, most, option, way):
+    """One new token per sequence, one head per key/value head: up to `most` keys the vector kernel, the matrix cores beyond."""
+    from splitwise_amd import _C
+    page = 8
+    kw = {"cap": dict(softcap=4.0), "learned sink": dict(sink=torch.linspace(-3.0, 9.0, G, device=DEV)),
+          "sigmoid": dict(score_bias=torch.linspace(-2.0, 1.0, G, device=DEV))}.get(option, {})
+    for longest, expected in ((most, GENERAL), (most + 1, DECODE)):
+        lengths = [(longest - 1, 1), (0, 1), (min(31, longest - 1), 1), (most // 2, 1)]
+        batch, pages = _step(lengths, page)
+        g = torch.Generator(device=DEV).manual_seed(G * 100 + d)
+        kc, vc = (torch.randn(pages, page, G * d, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+        q = torch.randn(len(lengths), G * d, generator=g, device=DEV) * 2
+        assert way(q, kc, vc, batch, G, G, d, d) == expected
+        out = torch.full((len(lengths), G * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+        _C.mixer_ops.capped_attention(out, q, kc, vc, None, batch, G, G, d, d, d ** -0.5, **kw)
+        ref = _statement(lengths, batch, q, kc, vc, None, G, G, d, d, **kw)
+        torch.testing.assert_close(out.double(), ref, atol=2e-4, rtol=2.0 ** -7)

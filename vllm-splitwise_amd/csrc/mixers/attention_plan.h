@@ -1,0 +1,83 @@
+// Which kernels a step of the paged attention goes to (capped_attention.hip).  Host code, no HIP headers.
+#pragma once
+
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace swm {
+
+constexpr int kAttentionTile = 32;      // query rows of a tile
+// Decode steps on the matrix cores: at most this many query rows (tokens x heads of a group) per sequence and key/value head
+constexpr int kDecodeRows = 8;
+constexpr int kDecodeGroups = 256, kDecodePartKeys = 256, kDecodeSharedKeys = 1024;
+
+enum AttentionWay {
+  kPromptOnMatrixCores,                 // prompt_attention.hip
+  kDecodeOnMatrixCores,                 // decode_attention.hip
+  kGeneralAttention                     // capped_attention.hip
+};
+
+// an upper bound of the keys that a query sees
+inline int64_t attention_most_keys(int max_query_len, int page_size, int table_width, int window, int chunk) {
+  int64_t most = (int64_t)page_size * table_width;
+  if (window > 0) most = std::min<int64_t>(most, window + max_query_len);
+  if (chunk > 0) most = std::min<int64_t>(most, chunk);
+  return most;
+}
+
+// Whether the bf16 matrix kernels can take a step: a bf16 cache whose rows can be read in 16-byte pieces, key and value sizes up
+// to 128.  Beyond 128 the three parts of a prompt's queries (96 registers at 128) no longer leave room for two waves per SIMD;
+// fp32 caches have no exact bf16 keys.  Both keep the general kernels.  addresses: those of queries, keys and values, or'ed.
+inline bool attention_pieces(uintptr_t addresses, int dim, int vdim, int64_t k_stride, int64_t v_stride) {
+  return dim <= 128 && vdim <= 128 && dim % 8 == 0 && vdim % 8 == 0 && k_stride % 8 == 0 && v_stride % 8 == 0 && addresses % 16 == 0;
+}
+
+// Steps of one query row per sequence and key/value head over few keys: the vector kernel has no parts to make, nothing to lay side
+// by side and less to join.  Up to how many keys, measured (us a step, vector / matrix; one sequence and 250, 8 heads each):
+//   128 wide:  16 keys 7.0 / 7.9 and 40 / 54, 256 keys 9.2 / 10.7 and 80 / 89, 511 keys 11.8 / 12.8 and 140 / 144, 801 keys 15.8 /
+//              15.2 and 198 / 186
+//   64 wide:   128 keys 6.0 / 6.4 and 25.1 / 27.7, 256 keys 6.8 / 7.0 and 31.9 / 35.2, 511 keys 8.7 / 8.3 and 50.5 / 48.1
+//   32 wide:   64 keys 4.9 / 5.0 and 15.1 / 18.4, 128 keys 5.4 / 5.1 and 18.0 / 20.7, 144 keys of one 5.2 / 5.5, 301 keys 6.6 / 6.0
+//              and 32.4 / 33.1
+//   96 wide (a block of 32 fewer for the matrix cores, but not for the vector kernel's lanes):  64 keys 7.4 / 7.4 and 46 / 51, 143
+//              keys 8.0 / 8.2 and 57 / 63, 256 keys 8.9 / 9.1 and 76 / 76
+// With more rows (two and more heads a group) the matrix cores win at once: 4 sequences, 8 heads on 4 of 64, 17 keys 7.2 / 6.1.
+// groups: sequences x heads.
+inline int attention_one_row_keys(int64_t groups, int dim, int vdim) {
+  const int size = std::max(dim, vdim);
+  if (size > 64) return size > 96 ? 512 : 160;
+  return groups > 1024 ? 320 : size > 32 ? 256 : 160;
+}
+
+// max_query_len 0: unknown.  pieces: attention_pieces of a bf16 cache
+inline AttentionWay attention_way(bool pieces, int num_seqs, int max_query_len, int heads, int kv_heads, int dim, int vdim,
+                                  int page_size, int table_width, int window, int chunk) {
+  const int group = heads / kv_heads;
+  if (!pieces) return kGeneralAttention;
+  if (max_query_len <= 0 || max_query_len > kAttentionTile / group) return kPromptOnMatrixCores;
+  if (max_query_len * group > kDecodeRows) return kGeneralAttention;
+  if (max_query_len * group == 1 && attention_most_keys(max_query_len, page_size, table_width, window, chunk) <=
+                                        attention_one_row_keys((int64_t)num_seqs * kv_heads, dim, vdim))
+    return kGeneralAttention;
+  return kDecodeOnMatrixCores;
+}
+
+// How many workgroups share a sequence's keys in the decode kernel on the matrix cores, given a workspace of parts x rows x heads x
+// (vdim + 2) floats.
+// One workgroup per compute unit and no more: its waves have 128 KB under way.  Two for each made 61 sequences of 2041 keys, 16
+// heads on 4, 67 us instead of 61 and 9 sequences on 8 key/value heads 28 instead of 23 (the join, and shorter runs).  A part has at
+// least a tile a wave.  Below about 1024 keys the second launch costs more than the sharing saves: 2 sequences of 700 keys 20.3 us
+// shared and 16.0 alone, 3 of 1000 20.5 and 21.2, 2 of 2500 20.5 and 22.7 (shared among a fourth as many).
+inline int decode_attention_parts(int num_seqs, int max_query_len, int heads, int kv_heads, int page_size, int table_width,
+                                  int window, int chunk) {
+  if (max_query_len <= 0 || (int64_t)max_query_len * (heads / kv_heads) > kDecodeRows) return 1;
+  const int64_t most_keys = attention_most_keys(max_query_len, page_size, table_width, window, chunk);
+  if (most_keys < kDecodeSharedKeys) return 1;
+  const int64_t groups = (int64_t)num_seqs * kv_heads;
+  int parts = 1;
+  while (parts < 16 && groups * parts * 2 <= kDecodeGroups && most_keys >= 2 * parts * kDecodePartKeys) parts <<= 1;
+  return parts;
+}
+
+}  // namespace swm

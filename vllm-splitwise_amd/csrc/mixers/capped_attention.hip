@@ -30,7 +30,7 @@ namespace swm {
 
 using f32x16 = __attribute__((ext_vector_type(16))) float;
 
-constexpr int kQT = 32;               // query rows and keys per tile
+constexpr int kQT = kAttentionTile;               // query rows and keys per tile
 constexpr int kMaxBlocks = 16;        // 32-coordinate blocks of the larger of key and value size
 
 // N consecutive elements of a cache row as they are stored (bf16 two to a register), widened where they are used:
@@ -625,9 +625,7 @@ inline int key_parts(int num_seqs, int max_query_len, int heads, int kv_heads, i
                      int chunk) {
   const int R = heads / kv_heads, tpt = kQT / R;
   if (max_query_len <= 0 || max_query_len > tpt || max_query_len * R <= 8) return 1;   // not the shared-keys loop
-  int64_t most_keys = (int64_t)page_size * table_width;
-  if (window > 0) most_keys = std::min<int64_t>(most_keys, window + max_query_len);
-  if (chunk > 0) most_keys = std::min<int64_t>(most_keys, chunk);
+  const int64_t most_keys = attention_most_keys(max_query_len, page_size, table_width, window, chunk);
   const int64_t tiles = (most_keys + kQT - 1) / kQT;
   const int64_t groups = (int64_t)num_seqs * kv_heads;
   int parts = 1;
@@ -651,7 +649,11 @@ int launch_capped_attention(void* out, int64_t out_stride, const float* q, const
   if ((page_size & (page_size - 1)) == 0)
     for (page_shift = 0; (1 << page_shift) < page_size; ++page_shift) {}
   if constexpr (std::is_same<T, bf16_t>::value && NB <= 4) {
-    if ((!split || rows_used <= kDecodeRows) && prompt_attention_fits(q, key_cache, value_cache, dim, vdim, k_stride, v_stride)) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(key_cache) |
+                         reinterpret_cast<uintptr_t>(value_cache);
+    const AttentionWay way = attention_way(attention_pieces(at, dim, vdim, k_stride, v_stride), num_seqs, max_query_len, heads,
+                                           kv_heads, dim, vdim, page_size, table_width, window, chunk);
+    if (way != kGeneralAttention) {
       PromptAttention a;
       a.out = out; a.q = q;
       a.key_cache = static_cast<const uint16_t*>(key_cache);
@@ -663,8 +665,8 @@ int launch_capped_attention(void* out, int64_t out_stride, const float* q, const
       a.table_width = table_width; a.num_seqs = num_seqs; a.heads = heads; a.kv_heads = kv_heads; a.dim = dim;
       a.vdim = vdim; a.page_size = page_size; a.page_shift = page_shift; a.window = window; a.chunk = chunk;
       a.sink = sink; a.tpt = tpt; a.scale = scale; a.softcap = softcap;
-      return split ? launch_decode_attention(a, rows, max_query_len, workspace, stream)
-                   : launch_prompt_attention(a, rows, stream);
+      return way == kDecodeOnMatrixCores ? launch_decode_attention(a, rows, max_query_len, workspace, stream)
+                                         : launch_prompt_attention(a, rows, stream);
     }
   }
   if (split) {

@@ -372,27 +372,9 @@ __global__ __launch_bounds__(128) void decode_attention_join_kernel(const Prompt
   }
 }
 
-// One workgroup per compute unit and no more: its waves have 128 KB under way.  Two for each made the step above 67 us instead
-// of 61 and 9 sequences on 8 key/value heads 28 instead of 23 (the join, and shorter runs).  A part has at least a tile a wave.
-// Below about 1024 keys the second launch costs more than the sharing saves: 2 sequences of 700 keys 20.3 us shared and 16.0
-// alone, 3 of 1000 20.5 and 21.2, 2 of 2500 20.5 and 22.7 (shared among a fourth as many).
-int decode_attention_parts(int num_seqs, int max_query_len, int heads, int kv_heads, int page_size, int table_width, int window,
-                           int chunk) {
-  if (max_query_len <= 0 || (int64_t)max_query_len * (heads / kv_heads) > kDecodeRows) return 1;
-  int64_t most_keys = (int64_t)page_size * table_width;
-  if (window > 0) most_keys = std::min<int64_t>(most_keys, window + max_query_len);
-  if (chunk > 0) most_keys = std::min<int64_t>(most_keys, chunk);
-  if (most_keys < kDecodeSharedKeys) return 1;
-  const int64_t groups = (int64_t)num_seqs * kv_heads;
-  int parts = 1;
-  while (parts < 16 && groups * parts * 2 <= kDecodeGroups && most_keys >= 2 * parts * kDecodePartKeys) parts <<= 1;
-  return parts;
-}
-
 template <int NB, int NS>
 int launch_decode_attention(const PromptAttention& a, int64_t rows, int parts, float* workspace, hipStream_t stream) {
-  static_assert(da_lds_bytes(NB) <= 80 * 1024,
-                "two workgroups per compute unit");
+  static_assert(da_lds_bytes(NB) <= 80 * 1024, "two workgroups fit a compute unit");
   static_assert(kDecodeRows * 32 * NB * 4 <= kDaKeys * da_vstride(NB), "the outputs take the place of the staged values");
   auto kernel = decode_attention_kernel<NB, NS>;
   if (da_lds_bytes(NB) > 64 * 1024)
