@@ -4,6 +4,8 @@ can go wrong: tiles' and stages' remainders, experts without rows, one expert wi
 The reference takes the products in 64 bits and rounds the hidden layer to bf16 as the kernels do.  A hidden value on the
 border between two bf16 numbers may be rounded the other way, by 2^-8 of itself; that bounds every output."""
 import math
+import os
+import re
 
 import pytest
 import torch
@@ -13,10 +15,14 @@ DEV = "cuda:0"
 
 
 def _routes(pairs, experts, n):
-    """What the rule beside the kernels says for a product of n weight rows."""
-    if pairs <= 6 * experts:
+    """What the rule beside the kernels says for a product of n weight rows, by its own numbers."""
+    source = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "vllm-splitwise_amd", "csrc", "mixers", "expert_ffn.hip")
+    with open(source) as f:
+        numbers = dict(re.findall(r"constexpr int (kFewPairs|kManyPairs|kManyTiles) = (\d+);", f.read()))
+    few, many, tiles = (int(numbers[k]) for k in ("kFewPairs", "kManyPairs", "kManyTiles"))
+    if pairs <= few * experts:
         return "few"
-    return "128" if pairs >= 96 * experts and pairs // 128 * -(-n // 128) >= 384 else "64"
+    return "128" if pairs >= many * experts and pairs // 128 * -(-n // 128) >= tiles else "64"
 
 
 @pytest.mark.parametrize("rows,width,ff,experts,top,act,skew,route", [

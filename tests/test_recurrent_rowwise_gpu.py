@@ -1,6 +1,7 @@
-"""The short convolution in runs of rows and the per-head norm in 16-byte pieces against the kernels that take one element at
-a time.  Those serve calls whose inputs do not lie on 16 bytes, so the same call with its input moved by one element is the
-reference: fp32 sums of at most 4 products, in the same order (rtol 1e-5), rounded once where the result is bf16 (2^-7)."""
+"""The short convolution in runs of rows, the per-head norm in 16-byte pieces and the delta rule's decode step in one launch, and
+the kernels that take calls whose operands do not lie on 16 bytes: every call is made both ways, aligned and with an operand moved
+by one element, and both are compared with a plain statement in 64 bits.  fp32 sums of at most 4 products, or of a head's squares
+(rtol 1e-5), rounded once where the result is bf16 (2^-7)."""
 from types import SimpleNamespace
 
 import pytest
@@ -41,7 +42,16 @@ def test_convolution_in_runs(lens, channels, taps, x_dtype, out_dtype):
     x = torch.randn(rows, channels, generator=g, device=DEV).to(x_dtype)
     w = torch.randn(channels, taps, generator=g, device=DEV)
     state = torch.randn(count + 2, taps - 1, channels, generator=g, device=DEV)
+    past = torch.zeros(count, taps - 1, channels, dtype=torch.float64, device=DEV)           # a sequence's carried inputs
+    past[1::2] = state[slots][1::2].double()
+    seen = [torch.cat([past[i], x[starts[i]:starts[i + 1]].double()]) for i in range(count)]
+    conv = torch.cat([sum(w[:, j].double() * t[j:len(t) - taps + 1 + j] for j in range(taps)) for t in seen])
+    kept = state.clone()
+    for i, t in enumerate(seen):
+        kept[slots[i]] = t[len(t) - taps + 1:].float()
     for silu, residual in ((True, False), (False, True)):
+        ref = conv + x.double() if residual else conv
+        ref = torch.nn.functional.silu(ref) if silu else ref
         res = []
         for lead in (0, 1):
             s, out = state.clone(), torch.full((rows, channels), float("nan"), dtype=out_dtype, device=DEV)
@@ -49,8 +59,9 @@ def test_convolution_in_runs(lens, channels, taps, x_dtype, out_dtype):
             assert at.data_ptr() % 16 == lead * x.element_size()
             _C.mixer_ops.causal_conv(out, at, w, s, batch, silu=silu, residual=residual)
             res.append((out, s))
+            torch.testing.assert_close(out.double(), ref, **_tol(out_dtype))
+            assert torch.equal(s, kept)                        # inputs are copied, nothing is rounded
         torch.testing.assert_close(res[0][0], res[1][0], **_tol(out_dtype))
-        assert torch.equal(res[0][1], res[1][1])               # inputs are copied, nothing is rounded
 
 
 @pytest.mark.parametrize("heads,vdim", [(3, 8), (5, 40), (16, 64), (1, 72), (2, 128), (7, 200), (3, 512), (1, 520), (2, 1024), (1, 2048),
@@ -71,7 +82,34 @@ def test_head_norm_in_pieces(heads, vdim, dtype):
                 _C.mixer_ops.head_norm_gate(out, o, _moved(gate, lead, heads * vdim + 16), weight, per_head, 1e-5, heads, vdim,
                                             gate_silu=silu)
                 res.append(out)
+                x64, g64 = o.double().view(rows, heads, vdim), gate.double()
+                ref = (x64 * (x64.square().mean(-1, keepdim=True) + 1e-5).rsqrt()).view(rows, -1)
+                if weight is not None:
+                    ref = ref * (weight if per_head else weight.repeat(heads)).double()
+                ref = ref * (torch.nn.functional.silu(g64) if silu else torch.sigmoid(g64))
+                torch.testing.assert_close(out.double(), ref, **_tol(dtype))
             torch.testing.assert_close(res[0], res[1], **_tol(dtype))
+
+
+def _delta_rule(qkv, beta, decay, dt_bias, a_log, state, batch, heads, kv_heads, dim, vdim):
+    """The rule in 64 bits, token by token -> outputs and states."""
+    rows, ends, out = qkv.shape[0], state.double(), []
+    q, k, v = qkv.double().split([kv_heads * dim, kv_heads * dim, heads * vdim], 1)
+    unit = lambda t: t * (t.square().sum(-1, keepdim=True) + 1e-6).rsqrt()  # noqa: E731
+    q, k = (unit(t.view(rows, kv_heads, dim)).repeat_interleave(heads // kv_heads, 1) for t in (q, k))
+    g = torch.nn.functional.softplus(decay.double() + dt_bias.double()).view(rows, heads, -1)
+    g, b = torch.exp(-a_log.double().exp()[:, None] * g), torch.sigmoid(beta.double())
+    owner, slots = batch.token_seq.tolist(), batch.state_slot.tolist()
+    for i, (c, lo, hi) in enumerate(zip(batch.ctx_len.tolist(), batch.q_start.tolist(), batch.q_start.tolist()[1:])):
+        if c == 0 and hi > lo:
+            ends[slots[i]] = 0
+    for t in range(rows):
+        s = g[t][..., None] * ends[slots[owner[t]]]
+        u = b[t][:, None] * (v[t].view(heads, vdim) - (s * k[t][..., None]).sum(-2))
+        s = s + k[t][..., None] * u[:, None, :]
+        ends[slots[owner[t]]] = s
+        out.append((s * q[t][..., None]).sum(-2).flatten() * dim ** -0.5)
+    return torch.stack(out), ends
 
 
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(1, 1, 4, 4), (4, 2, 24, 36), (2, 2, 64, 64), (3, 1, 100, 132), (4, 4, 128, 128),
@@ -79,8 +117,7 @@ def test_head_norm_in_pieces(heads, vdim, dtype):
 @pytest.mark.parametrize("per_channel", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_delta_decode_step_in_one_launch(heads, kv_heads, dim, vdim, per_channel, dtype):
-    """Against the prologue and recurrence, which an output off 16 bytes goes to: sums of at most 256 products of numbers
-    around 1 in fp32, in another order."""
+    """The prologue and recurrence take the output off 16 bytes.  Sums of at most 256 products of numbers around 1 in fp32."""
     from splitwise_amd import _C
     g = torch.Generator(device=DEV).manual_seed(heads * 1000 + dim + vdim)
     seqs, slots = 9, [3, 0, 11, 5, 7, 1, 8, 2, 10]
@@ -94,6 +131,7 @@ def test_delta_decode_step_in_one_launch(heads, kv_heads, dim, vdim, per_channel
     beta, dt_bias, a_log = rnd(seqs, heads + 3).to(dtype)[:, :heads], rnd(heads * (dim if per_channel else 1)), rnd(heads) * 0.3
     decay = rnd(seqs, heads * dim if per_channel else heads).to(dtype)
     state = rnd(12, heads, dim, vdim)
+    ref, ends = _delta_rule(qkv, beta, decay, dt_bias, a_log, state, batch, heads, kv_heads, dim, vdim)
     res = []
     for lead in (0, 1):
         s = state.clone()
@@ -101,6 +139,8 @@ def test_delta_decode_step_in_one_launch(heads, kv_heads, dim, vdim, per_channel
         op = _C.mixer_ops.channel_delta if per_channel else _C.mixer_ops.gated_delta
         op(out, qkv, beta, decay, dt_bias, a_log, s, batch, heads, kv_heads, dim, vdim)
         res.append((out, s))
+        torch.testing.assert_close(out.double(), ref, atol=3e-5, rtol=1e-4)
+        torch.testing.assert_close(s.double(), ends, atol=3e-5, rtol=1e-4)
     torch.testing.assert_close(res[0][0], res[1][0], atol=3e-5, rtol=1e-4)
     torch.testing.assert_close(res[0][1], res[1][1], atol=3e-5, rtol=1e-4)
     idle = [i for i in range(12) if i not in slots] + [11]     # slots of nobody, and of the sequence without a token
@@ -127,11 +167,14 @@ def test_delta_chunks_agree_with_the_tokens(heads, kv_heads, dim, vdim, lens):
     qkv, both = rnd(rows, 2 * kv_heads * dim + heads * vdim), rnd(rows, 2 * heads).to(torch.bfloat16)
     dt_bias, a_log, state = rnd(heads), rnd(heads) * 0.3, rnd(max(slots) + 9, heads, dim, vdim) * 0.1
     res = []
+    ref, ends = _delta_rule(qkv, both[:, :heads], both[:, heads:], dt_bias, a_log, state, batch, heads, kv_heads, dim, vdim)
     for chunked in (True, False):
         s, out = state.clone(), torch.full((rows, heads * vdim), float("nan"), device=DEV)
         _C.mixer_ops.gated_delta(out, qkv, both[:, :heads], both[:, heads:], dt_bias, a_log, s, batch, heads, kv_heads, dim, vdim,
                                  chunked=chunked)
         res.append((out, s))
+        torch.testing.assert_close(out.double(), ref, atol=2e-5, rtol=1e-4)
+        torch.testing.assert_close(s.double(), ends, atol=2e-5, rtol=1e-4)
     torch.testing.assert_close(res[0][0], res[1][0], atol=2e-5, rtol=1e-4)
     torch.testing.assert_close(res[0][1], res[1][1], atol=2e-5, rtol=1e-4)
     idle = [i for i in range(state.shape[0]) if i not in slots]

@@ -519,7 +519,7 @@ int launch_expert_tiles(const ExpertArgs& a, int64_t pairs, hipStream_t stream) 
 //   64 experts 2048 -> 1024, four per row:  6: 114 / 115 / 120 / 149;   96: 432 / 200 / 197 / 311;   250: 994 / 365 / 308 / 640
 //   8 experts 2048 -> 1024, 250 pairs each: 148 / 64 / 70 / 108: too few tiles of 128 x 128 for 256 compute units
 constexpr int kFewPairs = 6;            // pairs per expert up to which a step's weights are streamed
-constexpr int kFewGroups = 16384;
+constexpr int kFewGroups = 16384;      // workgroups of such a launch, of which most may find nothing to do
 constexpr int kManyPairs = 96;          // pairs per expert from which tiles of 128 pairs are mostly full ...
 constexpr int kManyTiles = 384;         // ... if there are this many of them
 template <bool DOWN>

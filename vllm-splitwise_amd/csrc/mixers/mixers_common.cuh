@@ -97,8 +97,8 @@ __device__ __forceinline__ int find_query_tile(const int32_t* __restrict__ q_sta
   return 0;
 }
 
-constexpr int kRunChunk = 32;
-// The rules that work in chunks of 32 tokens.  Piece `item` when the runs of more than `at_most` tokens are cut into pieces of `tokens`, in order: tokens in it (0: there is no
+constexpr int kRunChunk = 32;            // tokens of a chunk of the rules that work in chunks
+// Piece `item` when the runs of more than `at_most` tokens are cut into pieces of `tokens`, in order: tokens in it (0: there is no
 // such piece), its sequence, the run's tokens in front of it and the chunks of the runs before.  Every lane of a wave calls.
 __device__ __forceinline__ int find_run_piece(const int32_t* __restrict__ q_start, int num_seqs, int at_most, int tokens, int item,
                                              int* seq, int* tok0, int* chunks_before) {
