@@ -21,6 +21,10 @@ int main() {
   for (int dim : {16, 32, 40, 64, 72, 96, 104, 128}) need(way(1, 8, 8, dim, 1) == kGeneralAttention, "one row, a page of keys");
   need(way(1, 8, 8, 128, 32) == kGeneralAttention && way(1, 8, 8, 128, 33) == kDecodeOnMatrixCores, "one row of 128");
   need(way(1, 8, 8, 64, 16) == kGeneralAttention && way(1, 8, 8, 64, 17) == kDecodeOnMatrixCores, "one row of 64");
+  // up to 64 wide: 512 sequences x heads are one round of the matrix kernel's workgroups, more are two
+  auto many = [](int seqs, int width) { return attention_way(true, seqs, 1, 8, 8, 64, 64, 16, width, 0, 0); };
+  need(many(64, 17) == kDecodeOnMatrixCores && many(65, 64) == kGeneralAttention && many(96, 64) == kGeneralAttention, "512 and more");
+  need(many(97, 17) == kDecodeOnMatrixCores && many(97, 16) == kGeneralAttention && many(129, 20) == kGeneralAttention, "1024");
   need(way(1, 8, 8, 64, 500, 200) == kGeneralAttention && way(1, 8, 8, 64, 500, 0, 256) == kGeneralAttention, "one row, masks");
   // more rows: the matrix cores whatever the keys
   need(way(2, 8, 8, 64, 1) == kDecodeOnMatrixCores && way(1, 8, 4, 64, 1) == kDecodeOnMatrixCores, "two rows");

@@ -213,7 +213,7 @@ def test_decode_steps_agree_with_the_general_kernel(H, G, d, dv, page, option, l
     assert outs[0].isfinite().all() and outs[0].abs().max() > 0.016
 
 
-@pytest.mark.parametrize("G,d,most", [(3, 128, 512), (8, 64, 256), (2, 96, 160), (3, 104, 512), (5, 40, 256), (1, 16, 160), (300, 32, 320)])
+@pytest.mark.parametrize("G,d,most", [(3, 128, 512), (8, 64, 256), (2, 96, 160), (3, 104, 512), (5, 40, 256), (1, 16, 160), (300, 32, 320), (150, 64, 1024)])
 @pytest.mark.parametrize("option", ["plain", "cap", "learned sink", "sigmoid"])
 def test_one_query_row_on_both_sides_of_the_rule(G, d, most, option, way):
     """One new token per sequence, one head per key/value head: up to `most` keys the vector kernel, the matrix cores beyond."""

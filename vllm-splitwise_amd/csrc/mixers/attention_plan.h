@@ -43,10 +43,13 @@ inline bool attention_pieces(uintptr_t addresses, int dim, int vdim, int64_t k_s
 //   96 wide (a block of 32 fewer for the matrix cores, but not for the vector kernel's lanes):  64 keys 7.4 / 7.4 and 46 / 51, 143
 //              keys 8.0 / 8.2 and 57 / 63, 256 keys 8.9 / 9.1 and 76 / 76
 // With more rows (two and more heads a group) the matrix cores win at once: 4 sequences, 8 heads on 4 of 64, 17 keys 7.2 / 6.1.
-// groups: sequences x heads.
+// groups: sequences x heads.  The matrix kernel has two workgroups, of a group each, on a compute unit, 512 at once; up to 64 wide a
+// few more groups than that make a second round of it, nearly empty: 12 heads of 64, 60 sequences, 16 keys 7.5 / 10.1, 301 keys 16.8 /
+// 18.1, 801 keys 28.7 / 28.7;  10 heads of 64, 55 sequences, 1001 keys 28.5 / 31.3.
 inline int attention_one_row_keys(int64_t groups, int dim, int vdim) {
   const int size = std::max(dim, vdim);
   if (size > 64) return size > 96 ? 512 : 160;
+  if (groups > 512 && groups <= 768) return 1024;
   return groups > 1024 ? 320 : size > 32 ? 256 : 160;
 }
 
