@@ -120,6 +120,32 @@ def test_infinities_in_the_cache(H, G, d, option, lengths):
     torch.testing.assert_close(out.double(), ref, atol=2e-4, rtol=2.0 ** -7)
 
 
+@pytest.mark.parametrize("H,G,d", [(4, 2, 128), (3, 3, 96)])
+def test_an_infinity_in_shared_keys_that_one_of_two_tokens_sees(H, G, d, way):
+    """An infinite value in front of the second token's window: the channels that it spoils are worked out again, those of another
+    wave are not, and both are joined with the other workgroups' parts by one maximum."""
+    from splitwise_amd import _C
+    lengths, window = [(2100, 2), (1800, 2)], 1500
+    batch, pages = _step(lengths, 16)
+    g = torch.Generator(device=DEV).manual_seed(d)
+    kc, vc = (torch.randn(pages, 16, G * d, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(4, H * d, generator=g, device=DEV) * 2
+    for i, (c, _) in enumerate(lengths):
+        at = lambda pos: (int(batch.block_tables[i, pos // 16]), pos % 16)  # noqa: E731
+        first = c - window + 1                               # the first token's first key
+        assert first // 32 == (first + 1) // 32
+        vc[at(first)][d - 20::d] = float("inf")
+        # a score of 8 for the second token in the second tile of that tile's wave, of 4 parts of 8: its running maximum stays behind
+        own = q[2 * i + 1].view(G, H // G, d)[:, 0]
+        kc[at(first // 32 * 32 + 4 * 8 * 32 + 5)] = (8 * d ** 0.5 * own / own.square().sum(-1, keepdim=True)).flatten().bfloat16()
+    assert way(q, kc, vc, batch, H, G, d, d, window=window) == DECODE
+    out = torch.empty(4, H * d, dtype=torch.bfloat16, device=DEV)
+    _C.mixer_ops.capped_attention(out, q, kc, vc, None, batch, H, G, d, d, d ** -0.5, window=window)
+    ref = _statement(lengths, batch, q, kc, vc, None, H, G, d, d, window=window)
+    assert ref[1::2].isfinite().all() and ref[::2].isinf().any() and not ref.isnan().any()
+    torch.testing.assert_close(out.double(), ref, atol=2e-4, rtol=2.0 ** -7)
+
+
 @pytest.mark.parametrize("H,G,d,dv,page", [(4, 4, 128, 128, 16), (8, 2, 64, 96, 16), (6, 2, 40, 24, 8), (32, 1, 16, 8, 32),
                                            (3, 1, 104, 128, 12)])
 @pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "sink", "learned sink", "sigmoid", "values in the keys"])

@@ -322,7 +322,9 @@ __global__ __launch_bounds__(64 * kDaWaves, 2) void decode_attention_kernel(cons
       own[lane + 64] = row.o[1];
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       if (r == rr) {
-        m_all = row.m;
+        // Where only a value is infinite the row's other channels may be another wave's, which keeps what it has: its maximum stands,
+        // which lags behind by kDaGrowth at most.  Where scores are, every channel is worked out again.
+        if (row.m > m_all + kDaGrowth + 0.5f) m_all = row.m;
         m_use = sink ? fmaxf(m_all, sk) : m_all;
         m_use = m_use == -INFINITY ? 0.0f : m_use;
         const float f = da_exp(row.m - m_use);
