@@ -181,6 +181,40 @@ def test_delta_chunks_agree_with_the_tokens(heads, kv_heads, dim, vdim, lens):
     assert torch.equal(res[0][1][idle], state[idle])
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(3, 1, 32, 24), (2, 2, 64, 16), (5, 1, 96, 130), (6, 2, 128, 72), (2, 1, 224, 20)])
+@pytest.mark.parametrize("lead", [0, 1])
+def test_delta_chunks_through_every_turn_of_the_walk(heads, kv_heads, dim, vdim, lead):
+    """Runs of 1 to 8 chunks, whole and not, which leave the walk's loop over chunks at each of its places; one of them is NaN, and
+    stays with itself.  qkv on 16 bytes and off them.  End states within 4e-7 of 64 bits, as norms: sums of at most 256 fp32
+    products around 1, each rounded to 2^-24, over the few dozen tokens that a state remembers."""
+    from splitwise_amd import _C
+    lens = [256, 225, 191, 160, 130, 96, 64, 33]
+    starts, bad = [sum(lens[:i]) for i in range(len(lens) + 1)], 5
+    g = torch.Generator(device=DEV).manual_seed(dim + vdim)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
+    ctx, slots = [0, 3, 9, 0, 64, 0, 1, 5], [4, 0, 8, 2, 1, 7, 3, 5]
+    batch = SimpleNamespace(q_start=i32(starts), ctx_len=i32(ctx), max_query_len=max(lens), max_state_slot=8, state_slot=i32(slots),
+                            token_seq=i32([i for i, m in enumerate(lens) for _ in range(m)]))
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)               # noqa: E731
+    rows, width = starts[-1], 2 * kv_heads * dim + heads * vdim
+    qkv = torch.empty(rows * width + 1, device=DEV)[lead:lead + rows * width].view(rows, width)
+    qkv.copy_(rnd(rows, width))
+    both = rnd(rows, 2 * heads).to(torch.bfloat16)
+    dt_bias, a_log, state = rnd(heads), rnd(heads) * 0.3, rnd(9, heads, dim, vdim) * 0.1
+    ref, ends = _delta_rule(qkv, both[:, :heads], both[:, heads:], dt_bias, a_log, state, batch, heads, kv_heads, dim, vdim)
+    qkv[starts[bad]:starts[bad + 1]] = float("nan")
+    out = torch.full((rows, heads * vdim), float("nan"), device=DEV)
+    _C.mixer_ops.gated_delta(out, qkv, both[:, :heads], both[:, heads:], dt_bias, a_log, state, batch, heads, kv_heads, dim, vdim,
+                             chunked=True)
+    good = [i for i in range(len(lens)) if i != bad]
+    at = torch.cat([torch.arange(starts[i], starts[i + 1], device=DEV) for i in good])
+    assert bool(out[starts[bad]:starts[bad + 1]].isnan().all()) and bool(state[slots[bad]].isnan().all())
+    torch.testing.assert_close(out[at].double(), ref[at], atol=2e-5, rtol=1e-4)
+    for i in good:
+        err = (state[slots[i]].double() - ends[slots[i]]).norm() / ends[slots[i]].norm()
+        assert float(err) < 4e-7, (i, float(err))
+
+
 @pytest.mark.parametrize("rule", ["gla", "gla, strong decays", "lightning", "retention"])
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 32, 16), (3, 64, 17), (1, 72, 130), (2, 128, 40), (1, 160, 16), (1, 256, 33)])
 def test_linear_attention_walk_agrees_with_short_runs(rule, heads, dim, vdim):
