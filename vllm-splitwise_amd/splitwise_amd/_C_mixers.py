@@ -131,12 +131,13 @@ def _check(status: int) -> None:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 def _stream(t: torch.Tensor) -> int:
     """torch's current HIP stream on ``t``'s device (the raw handle; a step makes a hundred of these calls)."""
     if _raw_stream is not None:
-        return _raw_stream(t.device.index)
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
@@ -154,7 +155,7 @@ _SAME_DEVICE = _SameDevice()
 def _on_device_of(t: torch.Tensor):
     """Context that makes ``t``'s device current; free when it already is (an eager step makes some seventy
     of these calls, and switching devices costs more than the launch)."""
-    if t.device.index == torch.cuda.current_device():
+    if t.get_device() == _current_device():
         return _SAME_DEVICE
     return torch.cuda.device(t.device)
 
@@ -178,13 +179,16 @@ def _dev(*tensors: Optional[torch.Tensor]) -> None:
 
 
 def _f32c(t: torch.Tensor, what: str) -> None:
-    _need(t.dtype == torch.float32 and t.is_contiguous(), f"{what} must be a contiguous fp32 tensor")
+    if t.dtype != torch.float32 or not t.is_contiguous():
+        raise RuntimeError(f"{what} must be a contiguous fp32 tensor")
 
 
 def _rows(t: torch.Tensor, what: str) -> int:
     """Row stride (elements) of a 2-D view whose rows are contiguous."""
-    _need(t.dim() == 2 and t.stride(1) == 1, f"{what} must be 2-D with contiguous rows")
-    return t.stride(0)
+    stride = t.stride()
+    if len(stride) != 2 or stride[1] != 1:
+        raise RuntimeError(f"{what} must be 2-D with contiguous rows")
+    return stride[0]
 
 
 def scalar_norm_add(residual: torch.Tensor, y: torch.Tensor, gain: torch.Tensor, eps: float,
@@ -249,12 +253,13 @@ def qk_norm_cache(q_out: torch.Tensor, q: torch.Tensor, k: Optional[torch.Tensor
 
 
 def _ragged_ok(batch, rows: int) -> int:
-    n = batch.ctx_len.numel()
-    for name in ("q_start", "ctx_len", "token_seq", "state_slot"):
-        t = getattr(batch, name)
-        _need(t is not None and t.dtype == torch.int32 and t.is_contiguous() and t.is_cuda, f"ragged batch: {name}")
-    _need(batch.q_start.numel() == n + 1 and batch.token_seq.numel() == rows and batch.state_slot.numel() == n,
-          "ragged batch: lengths")
+    start, ctx, owner, slot = parts = batch.q_start, batch.ctx_len, batch.token_seq, batch.state_slot
+    for i, t in enumerate(parts):
+        if t is None or t.dtype != torch.int32 or not t.is_contiguous() or not t.is_cuda:
+            raise RuntimeError(f"ragged batch: {('q_start', 'ctx_len', 'token_seq', 'state_slot')[i]}")
+    n = ctx.numel()
+    if start.numel() != n + 1 or owner.numel() != rows or slot.numel() != n:
+        raise RuntimeError("ragged batch: lengths")
     return n
 
 

@@ -31,7 +31,8 @@ class PagedAttentionImpl:
 
     @staticmethod
     def reshape_and_cache(key, value, key_cache, value_cache, input_metadata: InputMetadata) -> None:
-        _C.cache_ops.reshape_and_cache(key, value, key_cache, value_cache, input_metadata.slot_mapping.flatten(),
+        slots = input_metadata.slot_mapping
+        _C.cache_ops.reshape_and_cache(key, value, key_cache, value_cache, slots if slots.dim() == 1 else slots.flatten(),
                                        input_metadata.kv_cache_dtype)
 
     @staticmethod
