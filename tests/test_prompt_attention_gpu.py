@@ -146,6 +146,34 @@ def test_an_infinity_in_shared_keys_that_one_of_two_tokens_sees(H, G, d, way):
     torch.testing.assert_close(out.double(), ref, atol=2e-4, rtol=2.0 ** -7)
 
 
+@pytest.mark.parametrize("H,G,d,page", [(4, 2, 128, 16), (3, 1, 96, 12), (8, 4, 24, 8)])
+@pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "learned sink", "sigmoid"])
+@pytest.mark.parametrize("lengths", [[(0, 255), (0, 40)], [(0, 257), (31, 66)], [(700, 33), (256, 1), (224, 40), (607, 2)]], ids=str)
+def test_two_groups_share_a_walk(H, G, d, page, option, lengths, way):
+    """On both sides of the number of keys from which two groups of waves share a workgroup's stages of 32; odd and even numbers of
+    stages, rows that see keys of one group's only.  In front, from the second stage on, keys that weigh next to nothing or most, and a
+    value of inf in a channel: what one group makes of it has to meet the other's sums.  (Tolerances as above.)"""
+    from splitwise_amd import _C
+    batch, pages = _step(lengths, page)
+    g = torch.Generator(device=DEV).manual_seed(d + len(lengths))
+    rows, inf = sum(n for _, n in lengths), float("inf")
+    kc, vc = (torch.randn(pages, page, G * d, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(rows, H * d, generator=g, device=DEV)
+    at = lambda i, pos: (int(batch.block_tables[i, pos // page]), pos % page)   # noqa: E731
+    for i, (c, n) in enumerate(lengths):
+        kc[at(i, min(34, c + n - 1))] *= 9.0
+        if c > 100:
+            vc[at(i, c // 32 * 32 - 20)][3::d] = inf         # the last stage but one or two that all of the sequence's rows see
+    kw = {"cap": dict(softcap=4.0), "window": dict(window=290), "chunk": dict(chunk=258), "sigmoid": dict(score_bias=torch.linspace(-2.0, 1.0, H, device=DEV)),
+          "learned sink": dict(sink=torch.linspace(-3.0, 2.0, H, device=DEV))}.get(option, {})
+    assert way(q, kc, vc, batch, H, G, d, d, **kw) == PROMPT
+    out = torch.empty(rows, H * d, dtype=torch.bfloat16, device=DEV)
+    _C.mixer_ops.capped_attention(out, q, kc, vc, None, batch, H, G, d, d, d ** -0.5, **kw)
+    ref = _statement(lengths, batch, q, kc, vc, None, H, G, d, d, **kw)
+    assert not ref.isnan().any() and (len(lengths) < 3 or ref.isinf().any())
+    torch.testing.assert_close(out.double(), ref, atol=2e-4, rtol=2.0 ** -7)
+
+
 @pytest.mark.parametrize("H,G,d,dv,page", [(4, 4, 128, 128, 16), (8, 2, 64, 96, 16), (6, 2, 40, 24, 8), (32, 1, 16, 8, 32),
                                            (3, 1, 104, 128, 12)])
 @pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "sink", "learned sink", "sigmoid", "values in the keys"])

@@ -8,10 +8,13 @@
 // times the work on units nine times as fast.  Except for an infinity in the cache, which a part that is zero turns into NaN: a row
 // that comes out as NaN is worked out again in fp32 (plain_row), so the result is the fp32 product's there too.
 //
-// Tile: a workgroup of 4 waves owns 4 x 32 query rows of one sequence and key/value head (row = token * R + head of the
-// group, 32 / R tokens a wave) and walks the keys it sees in stages of 32 that the waves share through LDS: global -> registers
-// two stages ahead, registers -> LDS one stage ahead, one barrier a stage.  (In the loop that it replaces every wave fetched
-// every key and value itself.)
+// Tile: a group of 4 waves owns 4 x 32 query rows of one sequence and key/value head (row = token * R + head of the group, 32 / R
+// tokens a wave) and walks the keys it sees in stages of 32 that the waves share through LDS: global -> registers two stages
+// ahead, registers -> LDS one stage ahead, one barrier a stage.  Where walks are long a workgroup has TWO groups for the same rows,
+// which take the stages in turn and join their sums at the end: under a causal mask the longest walk is twice the average one and the
+// rest of the GPU would wait for it.  The two are half a stage apart, one at the products while the other is at the softmax; a SIMD
+// has a wave of each.  What bounds a stage is the vector units (cap, softmax, taking weights apart: about 2300 cycles a wave), then the
+// products (1536).
 //   S^T = K Q^T : A = keys (row l % 32, 8 neighbouring coordinates per lane), B = the query parts, kept in registers;
 //                 C element r of lane l: key 8 (r / 4) + 4 (l / 32) + r % 4, query l % 32.
 //   O^T = V^T P^T: the score accumulator's layout is the B operand's, two runs of 4 keys per lane; A is read from the
@@ -21,8 +24,9 @@
 // Workgroups are numbered latest tile of a sequence first: under a causal mask those have the longest walks.
 //
 // Measured, two prompts of 4324 tokens together, 16 query heads on 4 of size 128, capped scores and a gate: 989 us with the
-// fp32 instructions (39 TFLOP/s), 169 us here (231 TFLOP/s; the matrix units do three times that).  Error against 64 bits
-// before the rounding to bf16: 1.3e-6 there, 1.2e-6 here (without a cap 6.7e-7 and 3.6e-7).
+// fp32 instructions (39 TFLOP/s), 170 us one group a workgroup, 158 us two; one prompt of 1607, 8 heads on 2, no cap: 88.5 and 74.3 us;
+// two of 1296 behind 190 others: 117 and 90.  Error against 64 bits before the rounding to bf16: 1.3e-6 with the fp32
+// instructions, 1.2e-6 here (without a cap 6.7e-7 and 3.6e-7).
 #include "prompt_attention.cuh"
 
 #include <algorithm>
@@ -31,6 +35,7 @@ namespace swm {
 
 using pa_bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
 using pa_f32x16 = __attribute__((ext_vector_type(16))) float;
+using pa_f32x4 = __attribute__((ext_vector_type(4))) float;
 using pa_u32x4 = __attribute__((ext_vector_type(4))) uint32_t;
 using pa_i16x4 = __attribute__((ext_vector_type(4))) short;
 using pa_lds_i16x4 = __attribute__((address_space(3))) pa_i16x4*;
@@ -56,18 +61,23 @@ __device__ __forceinline__ uint32_t upper_halves(uint32_t hi, uint32_t lo) { ret
 
 __host__ __device__ constexpr int pa_kstride(int nb) { return nb * 64 + 16; }                          // bytes per key row
 __host__ __device__ constexpr int pa_vstride(int nb) { return (nb * 64 + 255) / 256 * 256 + 64; }      // bytes per value row
-__host__ __device__ constexpr int pa_lds_bytes(int nb) { return 2 * kPaKeys * (pa_kstride(nb) + pa_vstride(nb)); }
+// a group's stages: two of keys, three of values
+__host__ __device__ constexpr int pa_lds_bytes(int nb) { return kPaKeys * (2 * pa_kstride(nb) + 3 * pa_vstride(nb)); }
+
+__host__ __device__ constexpr int pa_query_bytes(int nb) { return kPaWaves * 2 * 2 * nb * 1024; }         // two parts of the queries
 
 // NB: blocks of 32 coordinates of the larger of key and value size.
-template <int NB>
-__global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attention_kernel(const PromptAttention a) {
+// GROUPS: of 4 waves, which take the stages in turn, each with LDS buffers of its own; two of them have their sums meet at the end.
+template <int NB, int GROUPS>
+__global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_kernel(const PromptAttention a) {
   constexpr int KS = 2 * NB, CPR = 4 * NB, CHUNKS = kPaKeys * CPR, THREADS = 64 * kPaWaves;
   constexpr int LOADS = (CHUNKS + THREADS - 1) / THREADS;
   constexpr int KSTRIDE = pa_kstride(NB), VSTRIDE = pa_vstride(NB);
   extern __shared__ __attribute__((aligned(16))) char pa_lds[];
-  char* k_img = pa_lds;                                      // [2][32][KSTRIDE]
-  char* v_img = pa_lds + 2 * kPaKeys * KSTRIDE;              // [2][32][VSTRIDE]
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x % THREADS, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / THREADS);
+  char* k_img = pa_lds + group * pa_lds_bytes(NB);           // [2][32][KSTRIDE]
+  char* v_img = k_img + 2 * kPaKeys * KSTRIDE;               // [3][32][VSTRIDE]
   const int qi = lane & 31, hl = lane >> 5;
   const int R = a.heads / a.kv_heads, g = blockIdx.x % a.kv_heads;
 
@@ -109,7 +119,9 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attention_kernel(cons
   const float qscale = capped ? a.scale : a.scale * kLog2e;
   const float cap2 = a.softcap * kLog2e, cap_in = capped ? 2.0f * kLog2e / a.softcap : 0.0f;
   const float bias2 = sig ? a.score_bias[g * R + hh] * kLog2e : 0.0f;
-  PaFrag qh[KS], qm[KS], ql[KS];
+  // Two groups keep the leading parts in registers, the others in LDS, which both read.
+  PaFrag qh[KS], qm_own[GROUPS > 1 ? 1 : KS], ql_own[GROUPS > 1 ? 1 : KS];
+  pa_bf16x8* q_img = reinterpret_cast<pa_bf16x8*>(pa_lds + 2 * pa_lds_bytes(NB)) + wave * (2 * KS * 64) + lane;         // [part][KS][lane]
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     float x[8];
@@ -121,14 +133,24 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attention_kernel(cons
       const float4 v = ok ? *reinterpret_cast<const float4*>(p + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
       x[4 * j] = v.x * qscale; x[4 * j + 1] = v.y * qscale; x[4 * j + 2] = v.z * qscale; x[4 * j + 3] = v.w * qscale;
     }
+    PaFrag qm, ql;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       uint32_t h0, m0, l0, h1, m1, l1;
       split3(x[2 * j], h0, m0, l0);
       split3(x[2 * j + 1], h1, m1, l1);
       qh[ks].w[j] = upper_halves(h1, h0);
-      qm[ks].w[j] = upper_halves(m1, m0);
-      ql[ks].w[j] = upper_halves(l1, l0);
+      qm.w[j] = upper_halves(m1, m0);
+      ql.w[j] = upper_halves(l1, l0);
+    }
+    if constexpr (GROUPS > 1) {
+      if (group == 0) {
+        q_img[ks * 64] = qm.v;
+        q_img[(KS + ks) * 64] = ql.v;
+      }
+    } else {
+      qm_own[ks] = qm;
+      ql_own[ks] = ql;
     }
   }
 
@@ -143,29 +165,34 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attention_kernel(cons
       page_of[it] = table[a.page_shift >= 0 ? key >> a.page_shift : key / a.page_size];
     });
   };
+  // (a page's place in one 32 x 32 bit product, a key's in the page in 24 bits: 64-bit products took a seventh of the vector units' time)
+  const uint32_t krow = 2 * (uint32_t)a.k_stride, vrow = 2 * (uint32_t)a.v_stride;
+  const uint32_t kpage = krow * (uint32_t)a.page_size, vpage = vrow * (uint32_t)a.page_size;
   auto fetch = [&](int stage) {
     sw::static_for<LOADS>([&](auto IT) {
       constexpr int it = decltype(IT)::value;
       const int c = it * THREADS + tid, ch = c % CPR, key = key_of(it, stage);
-      const int64_t slot = (int64_t)page_of[it] * a.page_size + (a.page_shift >= 0 ? key & (a.page_size - 1) : key % a.page_size);
+      const uint32_t in = a.page_shift >= 0 ? key & (a.page_size - 1) : key % a.page_size, page = page_of[it];
       pa_u32x4 kv = {0u, 0u, 0u, 0u}, vv = {0u, 0u, 0u, 0u};
       if ((CHUNKS % THREADS == 0 || c < CHUNKS)) {
         if (ch * 8 < a.dim)
-          kv = *reinterpret_cast<const pa_u32x4*>(a.key_cache + slot * a.k_stride + (int64_t)g * a.dim + ch * 8);
+          kv = *reinterpret_cast<const pa_u32x4*>(reinterpret_cast<const char*>(a.key_cache + g * a.dim + ch * 8) + (uint64_t)page * kpage +
+                                                  in * krow);
         if (ch * 8 < a.vdim)
-          vv = *reinterpret_cast<const pa_u32x4*>(a.value_cache + slot * a.v_stride + (int64_t)g * a.vdim + ch * 8);
+          vv = *reinterpret_cast<const pa_u32x4*>(reinterpret_cast<const char*>(a.value_cache + g * a.vdim + ch * 8) +
+                                                  (uint64_t)page * vpage + in * vrow);
       }
       kreg[it] = kv;
       vreg[it] = vv;
     });
   };
-  auto commit = [&](int buf) {
+  auto commit = [&](int kbuf, int vbuf) {
     sw::static_for<LOADS>([&](auto IT) {
       constexpr int it = decltype(IT)::value;
       const int c = it * THREADS + tid, key = c / CPR, ch = c % CPR;
       if (CHUNKS % THREADS == 0 || c < CHUNKS) {
-        *reinterpret_cast<pa_u32x4*>(k_img + (buf * kPaKeys + key) * KSTRIDE + ch * 16) = kreg[it];
-        *reinterpret_cast<pa_u32x4*>(v_img + (buf * kPaKeys + key) * VSTRIDE + ch * 16) = vreg[it];
+        *reinterpret_cast<pa_u32x4*>(k_img + (kbuf * kPaKeys + key) * KSTRIDE + ch * 16) = kreg[it];
+        *reinterpret_cast<pa_u32x4*>(v_img + (vbuf * kPaKeys + key) * VSTRIDE + ch * 16) = vreg[it];
       }
     });
   };
@@ -186,113 +213,223 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attention_kernel(cons
   const int tr_off = (4 * (lane >> 5) + ((lane & 15) >> 2)) * VSTRIDE + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
   const int k_off = qi * KSTRIDE + hl * 16;
 
-  const int stages = s_hi - s_lo + 1;
-  tfetch(s_lo);
-  fetch(s_lo);
-  if (stages > 1) tfetch(s_lo + 1);
-  commit(0);
-  if (stages > 1) fetch(s_lo + 1);
-  if (stages > 2) tfetch(s_lo + 2);
-  __syncthreads();
-  int buf = 0;
-#pragma unroll 1
-  for (int t = 0; t < stages; ++t, buf ^= 1) {               // uniform over the workgroup: every wave meets every barrier
-    const int k0 = (s_lo + t) * kPaKeys;
-    if (t + 1 < stages) commit(buf ^ 1);
-    if (t + 2 < stages) fetch(s_lo + t + 2);
-    if (t + 3 < stages) tfetch(s_lo + t + 3);
-    if (nw > 0 && k0 <= wlast && k0 + kPaKeys > wlow) {      // wave-uniform
-      // ---- S^T = K Q^T: the leading parts in one sum, the others in a second
-      pa_f32x16 s, s2;
+  // This group's stages: first, first + GROUPS, ..  With two groups the same loads go on behind the last one, from the last key's
+  // place: the compiler counts what is in flight, and under a condition would wait for all of it.
+  const int first = s_lo + group, turns = (s_hi - s_lo + GROUPS) / GROUPS;
+  auto live = [&](int t) {                                   // this wave sees keys of the stage (wave-uniform)
+    const int k0 = (first + GROUPS * t) * kPaKeys;
+    return nw > 0 && t >= 0 && t < turns && k0 <= wlast && k0 + kPaKeys > wlow;
+  };
+  pa_f32x16 s;
+  PaFrag ph[2], pm[2], pl[2];
+  // ---- the weights of 16 keys in parts (two groups: at the end of the vector half; one: in front of their products, which takes
+  //      fewer registers)
+  auto take_apart = [&](int st) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = s2[r] = 0.0f;
-      const char* kb = k_img + buf * kPaKeys * KSTRIDE + k_off;
+    for (int j = 0; j < 4; ++j) {
+      // (no infinity to look out for: a weight is at most 2^8)
+      const float x0 = s[8 * st + 2 * j], x1 = s[8 * st + 2 * j + 1];
+      const uint32_t h0 = __float_as_uint(x0) & 0xffff0000u, h1 = __float_as_uint(x1) & 0xffff0000u;
+      const float r0 = x0 - __uint_as_float(h0), r1 = x1 - __uint_as_float(h1);
+      const uint32_t m0 = __float_as_uint(r0) & 0xffff0000u, m1 = __float_as_uint(r1) & 0xffff0000u;
+      ph[st].w[j] = upper_halves(h1, h0);
+      pm[st].w[j] = upper_halves(m1, m0);
+      pl[st].w[j] = upper_halves(__float_as_uint(r1 - __uint_as_float(m1)), __float_as_uint(r0 - __uint_as_float(m0)));
+    }
+  };
+  // ---- O^T += V^T P^T, 16 keys at a time; B element j of a lane is key 16 st + 8 (j / 4) + 4 hl + j % 4
+  auto value_products = [&](int t, int vbuf) {
+    if (!live(t)) return;
+    const char* vb = v_img + vbuf * kPaKeys * VSTRIDE + tr_off;
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      if constexpr (GROUPS == 1) take_apart(st);
+      pa_bf16x8 vf[NB];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const char* base = vb + 16 * st * VSTRIDE + b * 64;
+        union { pa_i16x4 half[2]; pa_bf16x8 f; } u;
+        u.half[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pa_lds_i16x4)(base));
+        u.half[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pa_lds_i16x4)(base + 8 * VSTRIDE));
+        vf[b] = u.f;
+      }
+#pragma unroll
+      for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[b], pl[st].v, o[b], 0, 0, 0);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[b], pm[st].v, o[b], 0, 0, 0);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[b], ph[st].v, o[b], 0, 0, 0);
+    }
+  };
+  // ---- S^T = K Q^T: the small parts of all coordinates in one sum; the leading ones on top of it, or in a second where registers
+  //      are enough (the first sum, read once, is not waited for)
+  auto key_products = [&](int t) {
+    if (!live(t)) return;
+    const char* kb = k_img + (t & 1) * kPaKeys * KSTRIDE + k_off;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+    if constexpr (GROUPS > 1) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const pa_bf16x8 kf = *reinterpret_cast<const pa_bf16x8*>(kb + 32 * ks);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, q_img[(KS + ks) * 64], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, q_img[ks * 64], s, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const pa_bf16x8*>(kb + 32 * ks), qh[ks].v, s, 0, 0, 0);
+    } else {
+      pa_f32x16 s2;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s2[r] = 0.0f;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         const pa_bf16x8 kf = *reinterpret_cast<const pa_bf16x8*>(kb + 32 * ks);
         s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qh[ks].v, s, 0, 0, 0);
-        s2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, ql[ks].v, s2, 0, 0, 0);
-        s2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qm[ks].v, s2, 0, 0, 0);
+        s2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, ql_own[ks].v, s2, 0, 0, 0);
+        s2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qm_own[ks].v, s2, 0, 0, 0);
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] += s2[r];
-      // ---- cap, mask, running softmax (this lane: query qi, keys (r, hl))
-      if (capped) {
+    }
+  };
+  // ---- the next stage into LDS, the one behind it on its way
+  auto stage_next = [&](int t, int vbuf) {
+    if (GROUPS > 1 || t + 1 < turns) commit((t + 1) & 1, vbuf == 2 ? 0 : vbuf + 1);
+    if (GROUPS > 1 || t + 2 < turns) fetch(first + GROUPS * (t + 2));
+    if (GROUPS > 1 || t + 3 < turns) tfetch(first + GROUPS * (t + 3));
+  };
+  // ---- the vector half: cap, mask, running softmax and the weights' parts (this lane: query qi, keys (r, hl))
+  auto vector_half = [&](int t) {
+    const int k0 = (first + GROUPS * t) * kPaKeys;
+    if (!live(t)) return;
+    if (capped) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r)                         // cap * tanh(s / cap) = cap (1 - 2 / (1 + e^(2 s / cap)))
-          s[r] = cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s[r] * cap_in));
-      }
-      if (k0 + kPaKeys - 1 > wfirst || k0 < wlow_last) {     // wave-uniform: something to mask
-        const int hi = pos_q - k0 - 4 * hl, lo = low_q - k0 - 4 * hl;
+      for (int r = 0; r < 16; ++r)                           // cap * tanh(s / cap) = cap (1 - 2 / (1 + e^(2 s / cap)))
+        s[r] = cap2 - 2.0f * cap2 * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s[r] * cap_in));
+    }
+    if (k0 + kPaKeys - 1 > wfirst || k0 < wlow_last) {       // wave-uniform: something to mask
+      const int hi = pos_q - k0 - 4 * hl, lo = low_q - k0 - 4 * hl;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int j = 8 * (r / 4) + r % 4;
-          s[r] = j <= hi && j >= lo ? s[r] : -INFINITY;
-        }
-      }
-      if (sig) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r)                         // a hidden key: 1 / (1 + e^inf) = 0
-          s[r] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-(s[r] + bias2)));
-      } else {
-        float tmax = s[0];
-#pragma unroll
-        for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
-        const float m_new = fmaxf(m_run, fmaxf(tmax, other_half(tmax)));
-        if (__builtin_amdgcn_ballot_w64(m_new > m_run + 8.0f) != 0) {
-          const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
-          l_part *= alpha;
-#pragma unroll
-          for (int b = 0; b < NB; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[b][r] *= alpha;
-          m_run = m_new;
-        }
-        const float m_use = m_run == -INFINITY ? 0.0f : m_run;
-        float sum0 = 0.0f, sum1 = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          s[r] = __builtin_amdgcn_exp2f(s[r] - m_use);
-          s[r + 1] = __builtin_amdgcn_exp2f(s[r + 1] - m_use);
-          sum0 += s[r];
-          sum1 += s[r + 1];
-        }
-        l_part += sum0 + sum1;
-      }
-      // ---- O^T += V^T P^T, 16 keys at a time; B element j of a lane is key 16 st + 8 (j / 4) + 4 hl + j % 4
-      const char* vb = v_img + buf * kPaKeys * VSTRIDE + tr_off;
-#pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        PaFrag ph, pm, pl;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          // (no infinity to look out for: a weight is at most 2^8)
-          const float x0 = s[8 * st + 2 * j], x1 = s[8 * st + 2 * j + 1];
-          const uint32_t h0 = __float_as_uint(x0) & 0xffff0000u, h1 = __float_as_uint(x1) & 0xffff0000u;
-          const float r0 = x0 - __uint_as_float(h0), r1 = x1 - __uint_as_float(h1);
-          const uint32_t m0 = __float_as_uint(r0) & 0xffff0000u, m1 = __float_as_uint(r1) & 0xffff0000u;
-          ph.w[j] = upper_halves(h1, h0);
-          pm.w[j] = upper_halves(m1, m0);
-          pl.w[j] = upper_halves(__float_as_uint(r1 - __uint_as_float(m1)), __float_as_uint(r0 - __uint_as_float(m0)));
-        }
-        pa_bf16x8 vf[NB];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          const char* base = vb + 16 * st * VSTRIDE + b * 64;
-          union { pa_i16x4 half[2]; pa_bf16x8 f; } u;
-          u.half[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pa_lds_i16x4)(base));
-          u.half[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((pa_lds_i16x4)(base + 8 * VSTRIDE));
-          vf[b] = u.f;
-        }
-#pragma unroll
-        for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[b], pl.v, o[b], 0, 0, 0);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[b], pm.v, o[b], 0, 0, 0);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[b], ph.v, o[b], 0, 0, 0);
+      for (int r = 0; r < 16; ++r) {
+        const int j = 8 * (r / 4) + r % 4;
+        s[r] = j <= hi && j >= lo ? s[r] : -INFINITY;
       }
     }
+    if (sig) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)                           // a hidden key: 1 / (1 + e^inf) = 0
+        s[r] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-(s[r] + bias2)));
+    } else {
+      float tmax = s[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
+      const float m_new = fmaxf(m_run, fmaxf(tmax, other_half(tmax)));
+      if (__builtin_amdgcn_ballot_w64(m_new > m_run + 8.0f) != 0) {
+        const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
+        l_part *= alpha;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[b][r] *= alpha;
+        m_run = m_new;
+      }
+      const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+      float sum0 = 0.0f, sum1 = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        s[r] = __builtin_amdgcn_exp2f(s[r] - m_use);
+        s[r + 1] = __builtin_amdgcn_exp2f(s[r + 1] - m_use);
+        sum0 += s[r];
+        sum1 += s[r + 1];
+      }
+      l_part += sum0 + sum1;
+    }
+    if constexpr (GROUPS > 1) {
+      take_apart(0);
+      take_apart(1);
+    }
+  };
+  tfetch(first);
+  fetch(first);
+  if (GROUPS > 1 || turns > 1) tfetch(first + GROUPS);
+  commit(0, 0);
+  if (GROUPS > 1 || turns > 1) fetch(first + GROUPS);
+  if (GROUPS > 1 || turns > 2) tfetch(first + 2 * GROUPS);
+  __syncthreads();
+  // A barrier a turn.  Of two groups one begins with the products, the other with the softmax of the stage before, so that a SIMD's
+  // two waves are at different units.
+  int vbuf = 0;                                              // t % 3
+  auto before = [&](int v) { return v == 0 ? 2 : v - 1; };
+  if constexpr (GROUPS == 1) {
+#pragma unroll 1
+    for (int t = 0; t < turns; ++t, vbuf = vbuf == 2 ? 0 : vbuf + 1) {
+      stage_next(t, vbuf);
+      key_products(t);
+      vector_half(t);
+      value_products(t, vbuf);
+      __syncthreads();
+    }
+  } else {
+    if (group == 0) {
+#pragma unroll 1
+      for (int t = 0; t < turns; ++t, vbuf = vbuf == 2 ? 0 : vbuf + 1) {
+        value_products(t - 1, before(vbuf));
+        key_products(t);
+        stage_next(t, vbuf);
+        vector_half(t);
+        __syncthreads();
+      }
+      value_products(turns - 1, before(vbuf));
+    } else {
+#pragma unroll 1
+      for (int t = 0; t < turns; ++t, vbuf = vbuf == 2 ? 0 : vbuf + 1) {
+        stage_next(t, vbuf);
+        vector_half(t - 1);
+        value_products(t - 1, before(vbuf));
+        key_products(t);
+        __syncthreads();
+      }
+      vector_half(turns - 1);
+      value_products(turns - 1, before(vbuf));
+    }
     __syncthreads();
+    // ---- the second group's sums, referred to the larger maximum, into the first's
+    static_assert(kPaWaves * (NB * 4096 + 512) <= 2 * pa_lds_bytes(NB), "the stages' LDS holds the sums");
+    pa_f32x4* sums = reinterpret_cast<pa_f32x4*>(pa_lds) + wave * (NB * 256 + 32) + lane;
+    float* rest = reinterpret_cast<float*>(pa_lds) + wave * (NB * 1024 + 128) + NB * 1024 + lane;
+    if (group == 1) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+          sums[(b * 4 + r4) * 64] = pa_f32x4{o[b][4 * r4], o[b][4 * r4 + 1], o[b][4 * r4 + 2], o[b][4 * r4 + 3]};
+      rest[0] = m_run;
+      rest[64] = l_part;
+    }
+    __syncthreads();
+    if (group == 0) {
+      const float m1 = rest[0], l1 = rest[64];
+      float a0 = 1.0f, a1 = 1.0f;
+      if (!sig) {
+        const float m = fmaxf(m_run, m1), m_use = m == -INFINITY ? 0.0f : m;
+        a0 = __builtin_amdgcn_exp2f(m_run - m_use);
+        a1 = __builtin_amdgcn_exp2f(m1 - m_use);
+        m_run = m;
+      }
+      l_part = l_part * a0 + l1 * a1;
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const pa_f32x4 x = sums[(b * 4 + r4) * 64];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[b][4 * r4 + r] = o[b][4 * r4 + r] * a0 + x[r] * a1;
+        }
+    }
+    __syncthreads();
+    if (group != 0) return;
   }
   // ---- a row that came out as NaN again, in plain fp32 (the stages are done with: LDS is free, a part of it for each wave)
   int odd = 0;
@@ -367,14 +504,32 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attention_kernel(cons
     }
 }
 
+template <int NB, int GROUPS>
+int launch_prompt_tiles_as(const PromptAttention& a, unsigned groups, hipStream_t stream) {
+  constexpr int lds = GROUPS * pa_lds_bytes(NB) + (GROUPS > 1 ? pa_query_bytes(NB) : 0);
+  if (lds > 64 * 1024)
+    SW_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(prompt_attention_kernel<NB, GROUPS>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  hipLaunchKernelGGL((prompt_attention_kernel<NB, GROUPS>), dim3(groups), dim3(64 * kPaWaves * GROUPS), lds, stream, a);
+  SW_CHECK_LAUNCH();
+  return SW_OK;
+}
+
+// Keys of a walk from which two groups share it (an upper bound of the longest one is known: the width of the block tables, the
+// mask).  Below that a workgroup has few stages to share, and two of one group's fit a compute unit.  One prompt of 77 tokens, 8
+// heads on 2 of 128: 18.2 us one group, 20.3 two; two of 127, 16 on 8: 15.9 and 16.4; two of 271, 12 on 4 of 64: 20.3 and 18.4; four of
+// 85 behind 209 others: 32.9 and 31.1; one of 511, 16 on 4 of 96: 30.6 and 26.0.
+constexpr int64_t kPaSharedKeys = 256;
 template <int NB>
 int launch_prompt_tiles(const PromptAttention& a, int64_t rows, hipStream_t stream) {
   const int64_t per_wg = (int64_t)kPaWaves * a.tpt;
   const int64_t groups = ((rows + per_wg - 1) / per_wg + a.num_seqs) * a.kv_heads;
   SW_CHECK_ARG(groups < (1ll << 31), "masked_attention: too many rows");
-  hipLaunchKernelGGL(prompt_attention_kernel<NB>, dim3((unsigned)groups), dim3(64 * kPaWaves), pa_lds_bytes(NB), stream, a);
-  SW_CHECK_LAUNCH();
-  return SW_OK;
+  int64_t keys = (int64_t)a.table_width * a.page_size;
+  if (a.window > 0) keys = std::min<int64_t>(keys, a.window);
+  if (a.chunk > 0) keys = std::min<int64_t>(keys, a.chunk);
+  return keys >= kPaSharedKeys ? launch_prompt_tiles_as<NB, 2>(a, (unsigned)groups, stream)
+                               : launch_prompt_tiles_as<NB, 1>(a, (unsigned)groups, stream);
 }
 
 int launch_prompt_attention(const PromptAttention& a, int64_t rows, hipStream_t stream) {
