@@ -294,7 +294,8 @@ __global__ __launch_bounds__(64 * kFewWaves) void expert_few_rows_kernel(const E
 constexpr int kTileK = 64, kTilePad = 8;
 __host__ __device__ constexpr int expert_tile_lds(int tm, int tn) { return 2 * (tm + tn) * (kTileK + kTilePad) * 2 + 2 * tm * 4; }
 
-template <bool DOWN, int BM, int BN>
+// WHOLE: K is a multiple of 64.
+template <bool DOWN, int BM, int BN, bool WHOLE>
 __global__ __launch_bounds__(256, 2) void expert_tile_kernel(const ExpertArgs a) {
   extern __shared__ __attribute__((aligned(16))) char big_lds[];
   constexpr int STRIDE = kTileK + kTilePad;
@@ -381,7 +382,7 @@ __global__ __launch_bounds__(256, 2) void expert_tile_kernel(const ExpertArgs a)
   };
   auto commit = [&](auto SET, int s, int buf) {
     constexpr int set = decltype(SET)::value;
-    if (s == stages - 1 && s * kTileK + ch >= a.K) {         // a last stage of less than 64
+    if (!WHOLE && s == stages - 1 && s * kTileK + ch >= a.K) {           // a last stage of less than 64
       sw::static_for<XL>([&](auto I) { xr[set][decltype(I)::value] = u32x4{0u, 0u, 0u, 0u}; });
       sw::static_for<WL>([&](auto I) { wr[set][decltype(I)::value] = u32x4{0u, 0u, 0u, 0u}; });
     }
@@ -405,7 +406,9 @@ __global__ __launch_bounds__(256, 2) void expert_tile_kernel(const ExpertArgs a)
   using Even = std::integral_constant<int, 0>;
   using Odd = std::integral_constant<int, 1>;
   fetch(Even{}, 0);
+  __builtin_amdgcn_sched_barrier(0);
   fetch(Odd{}, 1);
+  __builtin_amdgcn_sched_barrier(0);
   commit(Even{}, 0, 0);
   fetch(Even{}, 2);
   __syncthreads();
@@ -445,11 +448,14 @@ __global__ __launch_bounds__(256, 2) void expert_tile_kernel(const ExpertArgs a)
     __builtin_amdgcn_sched_group_barrier(0x008, PRODUCTS / 2, 0);
     __syncthreads();
   };
+  // (no condition inside the loop: what is in flight has to be the same on every way to a wait)
+  int s = 0;
 #pragma unroll 1
-  for (int s = 0; s < stages; s += 2) {
+  for (; s + 1 < stages; s += 2) {
     stage(Odd{}, s, 0);
-    if (s + 1 < stages) stage(Even{}, s + 1, 1);
+    stage(Even{}, s + 1, 1);
   }
+  if (s < stages) stage(Odd{}, s, 0);
   // C element r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32
   if constexpr (!DOWN) {
 #pragma unroll
@@ -498,17 +504,23 @@ __global__ __launch_bounds__(256, 2) void expert_tile_kernel(const ExpertArgs a)
   }
 }
 
-template <bool DOWN, int BM, int BN>
-int launch_expert_tiles(const ExpertArgs& a, int64_t pairs, hipStream_t stream) {
+template <bool DOWN, int BM, int BN, bool WHOLE>
+int launch_expert_tiles_as(const ExpertArgs& a, int64_t pairs, hipStream_t stream) {
   const int64_t tiles = ((pairs + BM - 1) / BM + a.num_experts) * ((a.N + BN - 1) / BN);           // an upper bound
   SW_CHECK_ARG(tiles < (1ll << 31) - 8, "expert_ffn: too many tiles");
   constexpr int lds = expert_tile_lds(BM, BN);
   if (lds > 64 * 1024)
-    SW_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(expert_tile_kernel<DOWN, BM, BN>),
+    SW_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(expert_tile_kernel<DOWN, BM, BN, WHOLE>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-  hipLaunchKernelGGL((expert_tile_kernel<DOWN, BM, BN>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), lds, stream, a);
+  hipLaunchKernelGGL((expert_tile_kernel<DOWN, BM, BN, WHOLE>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), lds, stream, a);
   SW_CHECK_LAUNCH();
   return SW_OK;
+}
+
+template <bool DOWN, int BM, int BN>
+int launch_expert_tiles(const ExpertArgs& a, int64_t pairs, hipStream_t stream) {
+  return a.K % kTileK == 0 ? launch_expert_tiles_as<DOWN, BM, BN, true>(a, pairs, stream)
+                           : launch_expert_tiles_as<DOWN, BM, BN, false>(a, pairs, stream);
 }
 
 // Which kernel: by the average number of pairs per expert (the host does not know the real one) and by the tiles that a
