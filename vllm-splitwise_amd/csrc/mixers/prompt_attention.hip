@@ -24,7 +24,7 @@
 // Workgroups are numbered latest tile of a sequence first: under a causal mask those have the longest walks.
 //
 // Measured, two prompts of 4324 tokens together, 16 query heads on 4 of size 128, capped scores and a gate: 989 us with the
-// fp32 instructions (39 TFLOP/s), 170 us one group a workgroup, 158 us two; one prompt of 1607, 8 heads on 2, no cap: 88.5 and 74.3 us;
+// fp32 instructions (39 TFLOP/s), 170 us one group a workgroup, 160 us two; one prompt of 1607, 8 heads on 2, no cap: 88.5 and 74.3 us;
 // two of 1296 behind 190 others: 117 and 90.  Error against 64 bits before the rounding to bf16: 1.3e-6 with the fp32
 // instructions, 1.2e-6 here (without a cap 6.7e-7 and 3.6e-7).
 #include "prompt_attention.cuh"
@@ -61,8 +61,10 @@ __device__ __forceinline__ uint32_t upper_halves(uint32_t hi, uint32_t lo) { ret
 
 __host__ __device__ constexpr int pa_kstride(int nb) { return nb * 64 + 16; }                          // bytes per key row
 __host__ __device__ constexpr int pa_vstride(int nb) { return (nb * 64 + 255) / 256 * 256 + 64; }      // bytes per value row
-// a group's stages: two of keys, three of values
-__host__ __device__ constexpr int pa_lds_bytes(int nb) { return kPaKeys * (2 * pa_kstride(nb) + 3 * pa_vstride(nb)); }
+// a group's stages: two of keys, two of values; of two groups three of values, whose products come a turn later
+__host__ __device__ constexpr int pa_lds_bytes(int nb, int groups) {
+  return kPaKeys * (2 * pa_kstride(nb) + (groups > 1 ? 3 : 2) * pa_vstride(nb));
+}
 
 __host__ __device__ constexpr int pa_query_bytes(int nb) { return kPaWaves * 2 * 2 * nb * 1024; }         // two parts of the queries
 
@@ -72,12 +74,12 @@ template <int NB, int GROUPS>
 __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_kernel(const PromptAttention a) {
   constexpr int KS = 2 * NB, CPR = 4 * NB, CHUNKS = kPaKeys * CPR, THREADS = 64 * kPaWaves;
   constexpr int LOADS = (CHUNKS + THREADS - 1) / THREADS;
-  constexpr int KSTRIDE = pa_kstride(NB), VSTRIDE = pa_vstride(NB);
+  constexpr int KSTRIDE = pa_kstride(NB), VSTRIDE = pa_vstride(NB), VBUFS = GROUPS > 1 ? 3 : 2;
   extern __shared__ __attribute__((aligned(16))) char pa_lds[];
   const int tid = threadIdx.x % THREADS, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / THREADS);
-  char* k_img = pa_lds + group * pa_lds_bytes(NB);           // [2][32][KSTRIDE]
-  char* v_img = k_img + 2 * kPaKeys * KSTRIDE;               // [3][32][VSTRIDE]
+  char* k_img = pa_lds + group * pa_lds_bytes(NB, GROUPS);           // [2][32][KSTRIDE]
+  char* v_img = k_img + 2 * kPaKeys * KSTRIDE;               // [2 or 3][32][VSTRIDE]
   const int qi = lane & 31, hl = lane >> 5;
   const int R = a.heads / a.kv_heads, g = blockIdx.x % a.kv_heads;
 
@@ -121,7 +123,7 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
   const float bias2 = sig ? a.score_bias[g * R + hh] * kLog2e : 0.0f;
   // Two groups keep the leading parts in registers, the others in LDS, which both read.
   PaFrag qh[KS], qm_own[GROUPS > 1 ? 1 : KS], ql_own[GROUPS > 1 ? 1 : KS];
-  pa_bf16x8* q_img = reinterpret_cast<pa_bf16x8*>(pa_lds + 2 * pa_lds_bytes(NB)) + wave * (2 * KS * 64) + lane;         // [part][KS][lane]
+  pa_bf16x8* q_img = reinterpret_cast<pa_bf16x8*>(pa_lds + 2 * pa_lds_bytes(NB, GROUPS)) + wave * (2 * KS * 64) + lane;         // [part][KS][lane]
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     float x[8];
@@ -238,8 +240,7 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
     }
   };
   // ---- O^T += V^T P^T, 16 keys at a time; B element j of a lane is key 16 st + 8 (j / 4) + 4 hl + j % 4
-  auto value_products = [&](int t, int vbuf) {
-    if (!live(t)) return;
+  auto value_products = [&](int vbuf) {
     const char* vb = v_img + vbuf * kPaKeys * VSTRIDE + tr_off;
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
@@ -264,7 +265,6 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
   // ---- S^T = K Q^T: the small parts of all coordinates in one sum; the leading ones on top of it, or in a second where registers
   //      are enough (the first sum, read once, is not waited for)
   auto key_products = [&](int t) {
-    if (!live(t)) return;
     const char* kb = k_img + (t & 1) * kPaKeys * KSTRIDE + k_off;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = 0.0f;
@@ -296,14 +296,13 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
   };
   // ---- the next stage into LDS, the one behind it on its way
   auto stage_next = [&](int t, int vbuf) {
-    if (GROUPS > 1 || t + 1 < turns) commit((t + 1) & 1, vbuf == 2 ? 0 : vbuf + 1);
+    if (GROUPS > 1 || t + 1 < turns) commit((t + 1) & 1, vbuf == VBUFS - 1 ? 0 : vbuf + 1);
     if (GROUPS > 1 || t + 2 < turns) fetch(first + GROUPS * (t + 2));
     if (GROUPS > 1 || t + 3 < turns) tfetch(first + GROUPS * (t + 3));
   };
   // ---- the vector half: cap, mask, running softmax and the weights' parts (this lane: query qi, keys (r, hl))
   auto vector_half = [&](int t) {
     const int k0 = (first + GROUPS * t) * kPaKeys;
-    if (!live(t)) return;
     if (capped) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)                           // cap * tanh(s / cap) = cap (1 - 2 / (1 + e^(2 s / cap)))
@@ -360,43 +359,49 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
   __syncthreads();
   // A barrier a turn.  Of two groups one begins with the products, the other with the softmax of the stage before, so that a SIMD's
   // two waves are at different units.
-  int vbuf = 0;                                              // t % 3
-  auto before = [&](int v) { return v == 0 ? 2 : v - 1; };
+  int vbuf = 0;                                              // t % VBUFS
+  auto before = [&](int v) { return v == 0 ? VBUFS - 1 : v - 1; };
   if constexpr (GROUPS == 1) {
 #pragma unroll 1
-    for (int t = 0; t < turns; ++t, vbuf = vbuf == 2 ? 0 : vbuf + 1) {
+    for (int t = 0; t < turns; ++t, vbuf = vbuf == VBUFS - 1 ? 0 : vbuf + 1) {
       stage_next(t, vbuf);
-      key_products(t);
-      vector_half(t);
-      value_products(t, vbuf);
+      if (live(t)) {
+        key_products(t);
+        vector_half(t);
+        value_products(vbuf);
+      }
       __syncthreads();
     }
   } else {
     if (group == 0) {
 #pragma unroll 1
-      for (int t = 0; t < turns; ++t, vbuf = vbuf == 2 ? 0 : vbuf + 1) {
-        value_products(t - 1, before(vbuf));
-        key_products(t);
+      for (int t = 0; t < turns; ++t, vbuf = vbuf == VBUFS - 1 ? 0 : vbuf + 1) {
+        if (live(t - 1)) value_products(before(vbuf));
+        if (live(t)) key_products(t);
         stage_next(t, vbuf);
-        vector_half(t);
+        if (live(t)) vector_half(t);
         __syncthreads();
       }
-      value_products(turns - 1, before(vbuf));
+      if (live(turns - 1)) value_products(before(vbuf));
     } else {
 #pragma unroll 1
-      for (int t = 0; t < turns; ++t, vbuf = vbuf == 2 ? 0 : vbuf + 1) {
+      for (int t = 0; t < turns; ++t, vbuf = vbuf == VBUFS - 1 ? 0 : vbuf + 1) {
         stage_next(t, vbuf);
-        vector_half(t - 1);
-        value_products(t - 1, before(vbuf));
-        key_products(t);
+        if (live(t - 1)) {
+          vector_half(t - 1);
+          value_products(before(vbuf));
+        }
+        if (live(t)) key_products(t);
         __syncthreads();
       }
-      vector_half(turns - 1);
-      value_products(turns - 1, before(vbuf));
+      if (live(turns - 1)) {
+        vector_half(turns - 1);
+        value_products(before(vbuf));
+      }
     }
     __syncthreads();
     // ---- the second group's sums, referred to the larger maximum, into the first's
-    static_assert(kPaWaves * (NB * 4096 + 512) <= 2 * pa_lds_bytes(NB), "the stages' LDS holds the sums");
+    static_assert(kPaWaves * (NB * 4096 + 512) <= 2 * pa_lds_bytes(NB, GROUPS), "the stages' LDS holds the sums");
     pa_f32x4* sums = reinterpret_cast<pa_f32x4*>(pa_lds) + wave * (NB * 256 + 32) + lane;
     float* rest = reinterpret_cast<float*>(pa_lds) + wave * (NB * 1024 + 128) + NB * 1024 + lane;
     if (group == 1) {
@@ -506,7 +511,7 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
 
 template <int NB, int GROUPS>
 int launch_prompt_tiles_as(const PromptAttention& a, unsigned groups, hipStream_t stream) {
-  constexpr int lds = GROUPS * pa_lds_bytes(NB) + (GROUPS > 1 ? pa_query_bytes(NB) : 0);
+  constexpr int lds = GROUPS * pa_lds_bytes(NB, GROUPS) + (GROUPS > 1 ? pa_query_bytes(NB) : 0);
   if (lds > 64 * 1024)
     SW_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(prompt_attention_kernel<NB, GROUPS>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds));
@@ -515,21 +520,31 @@ int launch_prompt_tiles_as(const PromptAttention& a, unsigned groups, hipStream_
   return SW_OK;
 }
 
-// Keys of a walk from which two groups share it (an upper bound of the longest one is known: the width of the block tables, the
-// mask).  Below that a workgroup has few stages to share, and two of one group's fit a compute unit.  One prompt of 77 tokens, 8
-// heads on 2 of 128: 18.2 us one group, 20.3 two; two of 127, 16 on 8: 15.9 and 16.4; two of 271, 12 on 4 of 64: 20.3 and 18.4; four of
-// 85 behind 209 others: 32.9 and 31.1; one of 511, 16 on 4 of 96: 30.6 and 26.0.
-constexpr int64_t kPaSharedKeys = 256;
+// When two groups share a walk.  They shorten the longest one, which is what a launch waits for that has few workgroups, or that has a
+// long walk beside many short ones under a causal mask; but only one such workgroup fits a compute unit, where of one group's two
+// do, and those fill one another's gaps better than two groups do.
+//   Keys (an upper bound of the longest walk: the block tables' width, the mask).  One group / two, us: one prompt of 77 tokens, 8
+//   heads on 2 of 128: 18.2 / 20.3; two of 127, 16 on 8: 15.9 / 16.4; two of 271, 12 on 4 of 64: 20.3 / 18.4; four of 85 behind 209
+//   others: 32.9 / 31.1; one of 511, 16 on 4 of 96: 30.6 / 26.0.
+//   Workgroups, few: 8 (64 tokens behind 3000) 163 / 119, 64 (300 tokens twice, 12 on 4 of 96) 22.5 / 20.6, 126 (2000 twice, 4 on 1 of
+//   128, a window of 1024) 70 / 59; 232 (200 sequences' tokens beside 1000) 70 / 73, 400 (2000 twice, 12 on 4, chunks of 512) 43 / 53.
+//   A causal mask alone, sequences of many tiles: 256 80 / 57, 400 120 / 95, 504 164 / 134, 512 81 / 61; with 488 of which most are a
+//   token each (60 sequences of 2000 keys, 8 heads of 64) 83 / 122.
+constexpr int64_t kPaSharedKeys = 256, kPaSharedFew = 200, kPaSharedCausal = 560;
+inline bool pa_two_groups(const PromptAttention& a, int64_t workgroups) {
+  const int64_t width = (int64_t)a.table_width * a.page_size;
+  const int64_t mask = a.window > 0 ? a.window : a.chunk > 0 ? a.chunk : width;
+  if (std::min(width, mask) < kPaSharedKeys) return false;
+  return workgroups <= kPaSharedFew ||
+         (mask >= width && workgroups <= kPaSharedCausal && 8 * (int64_t)a.num_seqs * a.kv_heads <= workgroups);
+}
 template <int NB>
 int launch_prompt_tiles(const PromptAttention& a, int64_t rows, hipStream_t stream) {
   const int64_t per_wg = (int64_t)kPaWaves * a.tpt;
   const int64_t groups = ((rows + per_wg - 1) / per_wg + a.num_seqs) * a.kv_heads;
   SW_CHECK_ARG(groups < (1ll << 31), "masked_attention: too many rows");
-  int64_t keys = (int64_t)a.table_width * a.page_size;
-  if (a.window > 0) keys = std::min<int64_t>(keys, a.window);
-  if (a.chunk > 0) keys = std::min<int64_t>(keys, a.chunk);
-  return keys >= kPaSharedKeys ? launch_prompt_tiles_as<NB, 2>(a, (unsigned)groups, stream)
-                               : launch_prompt_tiles_as<NB, 1>(a, (unsigned)groups, stream);
+  return pa_two_groups(a, groups) ? launch_prompt_tiles_as<NB, 2>(a, (unsigned)groups, stream)
+                                  : launch_prompt_tiles_as<NB, 1>(a, (unsigned)groups, stream);
 }
 
 int launch_prompt_attention(const PromptAttention& a, int64_t rows, hipStream_t stream) {
