@@ -72,3 +72,18 @@ def test_expert_kernels_at_their_edges(rows, width, ff, experts, top, act, skew,
     assert out.isfinite().all() and (off <= bound + 1e-5).all()
     # nearly all hidden values round the same way: in the mean the results are much closer than the bound
     assert off.norm() <= 1e-3 * ref.norm() and math.isfinite(float(ref.norm())) and float(ref.norm()) > 0
+
+
+@pytest.mark.parametrize("experts", [1, 7, 64, 65, 256])
+@pytest.mark.parametrize("pairs", [0, 1, 63, 8191, 8192, 8193, 20000])
+def test_pairs_in_groups(pairs, experts):
+    """On both sides of the pairs that one turn of the workgroup's threads takes; experts that nobody asks for; all on one."""
+    from splitwise_amd import _C
+    ops = _C.mixer_ops
+    g = torch.Generator(device=DEV).manual_seed(pairs + experts)
+    for chosen in (torch.randint(0, experts, (pairs, 1), generator=g, device=DEV), torch.full((pairs, 1), experts - 1, device=DEV)):
+        order, start = ops.group_pairs(chosen.to(torch.int32), experts)
+        count = torch.bincount(chosen.flatten(), minlength=experts)
+        assert start.tolist() == [0] + torch.cumsum(count, 0).tolist()
+        assert torch.equal(order.sort().values, torch.arange(pairs, device=DEV, dtype=torch.int32))
+        assert torch.equal(chosen.flatten()[order.long()], chosen.flatten().sort().values)
