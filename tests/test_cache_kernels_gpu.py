@@ -159,3 +159,38 @@ def test_reshape_and_cache_block_sizes(dtype, kv_cache_dtype, num_heads, head_si
     if pattern == "decode" and block_size * 96 < 42 or pattern == "padded" and block_size * 56 < 35:
         pytest.skip("the pattern needs more slots")
     test_reshape_and_cache(dtype, kv_cache_dtype, num_heads, head_size, block_size, pattern)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("kv_cache_dtype", ["auto", "fp8_e5m2"])
+@pytest.mark.parametrize("num_heads,head_size,block_size", [(3, 64, 16), (2, 80, 8), (1, 48, 32), (2, 32, 12), (1, 64, 4), (1, 32, 2)])
+@pytest.mark.parametrize("seed", range(4))
+def test_reshape_and_cache_runs_anywhere(dtype, kv_cache_dtype, num_heads, head_size, block_size, seed):
+    """Runs of slots of every length and start behind one another, so that they begin and end at any place of a tile of 16 tokens and
+    of a block: prompts behind one another, portions that go on in a block, padding and lone slots between them."""
+    C = _ops()
+    rng = random.Random(1000 * seed + block_size)
+    torch.manual_seed(seed)
+    num_blocks, slots = 160, []
+    free = list(range(num_blocks))
+    rng.shuffle(free)
+    for _ in range(12):
+        first, n = rng.choice([0, 0, rng.randrange(block_size)]), rng.choice([1, 2, rng.randint(3, 9), rng.randint(10, 18), rng.randint(19, 50)])
+        n = min(n, 8 * block_size - first)
+        blocks = [free.pop() for _ in range(-(-(first + n) // block_size))]
+        if rng.random() < 0.5:                                   # blocks that lie behind one another: the run of slots goes on
+            at = [b for b in range(num_blocks - len(blocks)) if all(b + i in free for i in range(len(blocks)))]
+            if at:
+                free += blocks
+                blocks = [at[0] + i for i in range(len(blocks))]
+                free = [b for b in free if b not in blocks]
+        slots += [blocks[(first + i) // block_size] * block_size + (first + i) % block_size for i in range(n)]
+        slots += [-1] * rng.choice([0, 0, 1, 5])
+    slot_mapping = torch.tensor(slots, dtype=torch.long)
+    qkv = torch.randn(len(slots), 3, num_heads, head_size, dtype=dtype)
+    kc, vc = make_kv_caches(num_blocks, block_size, num_heads, head_size, dtype, cache_dtype=kv_cache_dtype)
+    kc_ref, vc_ref = kc.clone(), vc.clone()
+    ocache.reshape_and_cache(qkv[:, 1], qkv[:, 2], kc_ref, vc_ref, slot_mapping, kv_cache_dtype)
+    qkv_d, kc_d, vc_d = qkv.cuda(), kc.cuda(), vc.cuda()
+    C.cache_ops.reshape_and_cache(qkv_d[:, 1], qkv_d[:, 2], kc_d, vc_d, slot_mapping.cuda(), kv_cache_dtype)
+    assert torch.equal(_bits(kc_d.cpu()), _bits(kc_ref)) and torch.equal(_bits(vc_d.cpu()), _bits(vc_ref))

@@ -48,8 +48,12 @@ __device__ __forceinline__ int lds_row_bytes(int head_size) {
 // What bounds it is memory, once the addresses are cheap: where a token goes (its slot's block and offset, a 64-bit division
 // where the block size is no power of two) is worked out once per tile by 16 lanes, and not by every thread for every piece.
 // Workgroups that run together take the heads of the same tokens: their pieces of a row lie side by side.
-// Measured, 2320 tokens x 32 heads of 128, bf16 (76 MB): 30.5 us with the divisions in every thread, 27.2 without, 24.0 with the
-// heads side by side.  61 tokens x 8 heads into an fp8 cache: 8.7 and 5.9 us.  251 tokens x 32 heads into slots of their own
+// Vectors of V are VT neighbouring slots from a multiple of VT on.  Prompts of any length lie behind one another in a step, so a
+// tile's tokens seldom begin at such a slot: a tile's V is moved on to the next one where the run of slots goes on (its first
+// tokens are then the tile's before it), and only what is left over at a run's ends goes element by element.
+// Measured, 2320 tokens x 32 heads of 128, bf16 (76 MB): 30.5 us with the divisions in every thread, 27.2 without, 16.2 with the
+// heads side by side as one prompt; as prompts of 699, 938 and 790 tokens 26.0 with V vectors only where a tile's own eighths
+// are aligned, 18.3 here.  61 tokens x 8 heads into an fp8 cache: 8.7 us with the divisions, 5.1 here.  251 tokens x 32 heads into slots of their own
 // take 19 us before and after: every element of V is a 2-byte write into a 32-byte sector (36 MB for 4).
 template <typename act_t, bool FP8, int VT>
 __global__ void __launch_bounds__(kRcThreads)
@@ -63,9 +67,10 @@ reshape_and_cache_tile_kernel(const char* __restrict__ key, const char* __restri
   constexpr int CS = FP8 ? 1 : ES;              // cache element bytes
   constexpr int X = 16 / CS;                    // cache elements per 16 bytes
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  __shared__ int64_t bases[kTileTokens];        // byte offset of the token's [block, head] tile, -1: no slot
-  __shared__ int offsets[kTileTokens];          // the token's place in its block
-  __shared__ uint32_t runs;                     // bit t: token t follows its group's first one, which begins a vector
+  constexpr int GROUP = VT > 0 ? VT : 8, PARTS = kTileTokens / GROUP, kSeen = kTileTokens + GROUP;
+  __shared__ int64_t bases[kSeen];              // byte offset of the token's [block, head] tile, -1: no slot
+  __shared__ int offsets[kSeen];                // the token's place in its block
+  __shared__ int heads[PARTS], loose[kSeen];    // tokens that begin a vector of V, tokens that no vector takes
 
   const int t0 = blockIdx.x / num_heads * kTileTokens;
   const int head = blockIdx.x % num_heads;
@@ -76,37 +81,58 @@ reshape_and_cache_tile_kernel(const char* __restrict__ key, const char* __restri
   const int64_t head_bytes = (int64_t)head_size * block_size * CS;
   const int64_t block_bytes = head_bytes * num_heads;
 
+  // ---- every wave looks at the tile's slots, the one in front of them and those up to a vector's length behind: lane l is token
+  //      t0 + l - 1
+  const int lane = tid & 63, j = lane - 1;
   int64_t slot = -1;
-  if (tid < kTileTokens && t0 + tid < num_tokens) slot = slot_mapping[t0 + tid];
+  if (t0 + j >= 0 && t0 + j < num_tokens && j < kSeen) slot = slot_mapping[t0 + j];
 
   // ---- stage K and V rows of this head: 16-byte pieces, token-major (coalesced), 16 lanes a row
-  {
-    const int tok = tid / 16, chunks = head_size * ES / 16;
-    if (t0 + tok < num_tokens) {
-      const int64_t off = (int64_t)head * head_size * ES;
-      const char* kr = key + (t0 + tok) * key_stride_bytes + off;
-      const char* vr = value + (t0 + tok) * value_stride_bytes + off;
-      for (int ch = tid % 16; ch < chunks; ch += 16) {
-        const uint4 kv = *reinterpret_cast<const uint4*>(kr + ch * 16);
-        const uint4 vv = *reinterpret_cast<const uint4*>(vr + ch * 16);
-        *reinterpret_cast<uint4*>(k_tile + tok * row_bytes + ch * 16) = kv;
-        *reinterpret_cast<uint4*>(v_tile + tok * row_bytes + ch * 16) = vv;
-      }
+  const int tok16 = tid / 16, chunks = head_size * ES / 16;
+  const int64_t head_off = (int64_t)head * head_size * ES;
+  if (t0 + tok16 < num_tokens) {
+    const char* kr = key + (t0 + tok16) * key_stride_bytes + head_off;
+    const char* vr = value + (t0 + tok16) * value_stride_bytes + head_off;
+    for (int ch = tid % 16; ch < chunks; ch += 16) {
+      const uint4 kv = *reinterpret_cast<const uint4*>(kr + ch * 16);
+      const uint4 vv = *reinterpret_cast<const uint4*>(vr + ch * 16);
+      *reinterpret_cast<uint4*>(k_tile + tok16 * row_bytes + ch * 16) = kv;
+      *reinterpret_cast<uint4*>(v_tile + tok16 * row_bytes + ch * 16) = vv;
     }
   }
+  // ---- V's tokens [v0, v1) of this tile, which of them begin a vector and which go alone
+  const int64_t prev = __shfl_up(slot, 1, 64);
+  const uint64_t follows = __ballot(lane > 0 && slot >= 0 && prev >= 0 && slot == prev + 1);
+  auto moved = [&](int first) {                 // tokens from `first` on that belong to a vector begun in front of it
+    if constexpr (VT == 0) return 0;
+    const int64_t s = __shfl(slot, first + 1, 64);
+    const int n = s < 0 ? 0 : (int)((GROUP - s % GROUP) % GROUP);
+    const uint64_t need = ((1ull << n) - 1) << (first + 1);
+    return (follows & need) == need ? n : 0;
+  };
+  const int v0 = moved(0), v1 = min(kTileTokens + moved(kTileTokens), num_tokens - t0);
+  uint64_t begins = 0;
+  if constexpr (VT > 0) {
+    const uint64_t rest = ((1ull << (GROUP - 1)) - 1) << (lane + 1);
+    begins = __ballot(j >= v0 && j + GROUP <= v1 && slot >= 0 && slot % GROUP == 0 && (follows & rest) == rest);
+  }
+  const bool taken = ((begins << (GROUP - 1)) >> lane & ((1ull << GROUP) - 1)) != 0;
+  const uint64_t alone = __ballot(j >= v0 && j < v1 && slot >= 0 && !taken);
+  const int num_heads_v = __popcll(begins), num_loose = __popcll(alone);
   if (tid < 64) {                               // one wave
-    bool follows = false;
-    if constexpr (VT > 0) {
-      const int64_t first = __shfl(slot, tid & ~(VT - 1), 64);
-      follows = first >= 0 && first % VT == 0 && slot == first + (tid & (VT - 1));
-    }
-    const uint64_t mask = __ballot(follows);
-    if (tid < kTileTokens) {
+    const uint64_t below = (1ull << lane) - 1;
+    if (begins >> lane & 1) heads[__popcll(begins & below)] = j;
+    if (alone >> lane & 1) loose[__popcll(alone & below)] = j;
+    if (j >= 0 && j < kSeen) {
       const int64_t blk = block_shift >= 0 ? slot >> block_shift : slot / block_size;
-      bases[tid] = slot < 0 ? -1 : blk * block_bytes + head * head_bytes;
-      offsets[tid] = slot < 0 ? 0 : (int)(slot - blk * block_size);
-      if (tid == 0) runs = (uint32_t)mask;
+      bases[j] = slot < 0 ? -1 : blk * block_bytes + head * head_bytes;
+      offsets[j] = slot < 0 ? 0 : (int)(slot - blk * block_size);
     }
+  }
+  if (kTileTokens + tok16 < v1) {               // (fewer than a vector's tokens)
+    const char* vr = value + (t0 + kTileTokens + tok16) * value_stride_bytes + head_off;
+    for (int ch = tid % 16; ch < chunks; ch += 16)
+      *reinterpret_cast<uint4*>(v_tile + (kTileTokens + tok16) * row_bytes + ch * 16) = *reinterpret_cast<const uint4*>(vr + ch * 16);
   }
   __syncthreads();
 
@@ -137,28 +163,25 @@ reshape_and_cache_tile_kernel(const char* __restrict__ key, const char* __restri
     }
   }
 
-  // ---- V: cache row d holds block_size tokens.  A group of tokens takes the vector path when its slots are consecutive and
-  // start at a multiple of VT (block_size is one: they share a cache row segment); otherwise one element per lane.
-  constexpr int GROUP = VT > 0 ? VT : 8, PARTS = kTileTokens / GROUP;
+  // ---- V: cache row d holds block_size tokens.  A vector takes VT tokens of it (block_size is a multiple: they share a row segment),
+  // what no vector takes goes one element per lane.
   const int part = tid % PARTS;
-  constexpr uint32_t all = (uint32_t)((1ull << GROUP) - 1);
-  const bool fast = VT > 0 && ((runs >> (part * GROUP)) & all) == all;
-  const int64_t base0 = bases[part * GROUP];
-  const int boff0 = offsets[part * GROUP];
-  for (int d = tid / PARTS; d < head_size; d += kRcThreads / PARTS) {
-    const char* src = v_tile + part * GROUP * row_bytes + d * ES;
-    if (fast) {
-      char* dst = value_cache + base0 + ((int64_t)d * block_size + boff0) * CS;
+  if (part < num_heads_v) {
+    const int first = heads[part];
+    char* const dst0 = value_cache + bases[first] + (int64_t)offsets[first] * CS;
+    for (int d = tid / PARTS; d < head_size; d += kRcThreads / PARTS) {
+      const char* src = v_tile + first * row_bytes + d * ES;
+      char* dst = dst0 + (int64_t)d * block_size * CS;
       uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
-      for (int j = 0; j < GROUP; ++j) {
-        const S e = *reinterpret_cast<const S*>(src + j * row_bytes);
+      for (int q = 0; q < GROUP; ++q) {
+        const S e = *reinterpret_cast<const S*>(src + q * row_bytes);
         if constexpr (FP8) {
-          w[j >> 2] |= (uint32_t)Conv<act_t>::to_e5m2(e) << (8 * (j & 3));
+          w[q >> 2] |= (uint32_t)Conv<act_t>::to_e5m2(e) << (8 * (q & 3));
         } else if constexpr (ES == 2) {
-          w[j >> 1] |= (uint32_t)e << (16 * (j & 1));
+          w[q >> 1] |= (uint32_t)e << (16 * (q & 1));
         } else {
-          w[j & 3] = __float_as_uint(e);
+          w[q & 3] = __float_as_uint(e);
         }
       }
       if constexpr (GROUP * CS >= 16) {
@@ -166,18 +189,19 @@ reshape_and_cache_tile_kernel(const char* __restrict__ key, const char* __restri
       } else {
         *reinterpret_cast<uint2*>(dst) = make_uint2(w[0], w[1]);
       }
-    } else {
-#pragma unroll
-      for (int j = 0; j < GROUP; ++j) {
-        const int64_t base = bases[part * GROUP + j];
-        if (base < 0) continue;
-        char* dst = value_cache + base + ((int64_t)d * block_size + offsets[part * GROUP + j]) * CS;
-        const S e = *reinterpret_cast<const S*>(src + j * row_bytes);
-        if constexpr (FP8) {
-          *reinterpret_cast<uint8_t*>(dst) = Conv<act_t>::to_e5m2(e);
-        } else {
-          *reinterpret_cast<S*>(dst) = e;
-        }
+    }
+  }
+#pragma unroll 4
+  for (int k = tid / 64; k < num_loose; k += kRcThreads / 64) {          // a wave per token
+    const int tok = __builtin_amdgcn_readfirstlane(loose[k]);
+    char* const dst0 = value_cache + bases[tok] + (int64_t)offsets[tok] * CS;
+    for (int d = lane; d < head_size; d += 64) {
+      char* dst = dst0 + (int64_t)d * block_size * CS;
+      const S e = *reinterpret_cast<const S*>(v_tile + tok * row_bytes + d * ES);
+      if constexpr (FP8) {
+        *reinterpret_cast<uint8_t*>(dst) = Conv<act_t>::to_e5m2(e);
+      } else {
+        *reinterpret_cast<S*>(dst) = e;
       }
     }
   }
@@ -262,7 +286,6 @@ int launch_reshape_and_cache(const void* key, const void* value, void* key_cache
   using S = typename Conv<act_t>::store_t;
   const int es = sizeof(S);
   const int row_bytes = head_size * es + 16;
-  const size_t smem = 2 * kTileTokens * row_bytes;
   const unsigned grid = (unsigned)((num_tokens + kTileTokens - 1) / kTileTokens * num_heads);
   int block_shift = -1;
   if ((block_size & (block_size - 1)) == 0)
@@ -272,6 +295,8 @@ int launch_reshape_and_cache(const void* key, const void* value, void* key_cache
   auto kernel = block_size % VT == 0         ? reshape_and_cache_tile_kernel<act_t, FP8, VT>
                 : block_size % (VT / 2) == 0 ? reshape_and_cache_tile_kernel<act_t, FP8, VT / 2>
                                              : reshape_and_cache_tile_kernel<act_t, FP8, 0>;
+  // a tile's rows of K, and of V up to a vector's length less one more
+  const size_t smem = (2 * kTileTokens + (block_size % VT == 0 ? VT : block_size % (VT / 2) == 0 ? VT / 2 : 0)) * (size_t)row_bytes;
   kernel<<<grid, kRcThreads, smem, stream>>>(
       static_cast<const char*>(key), static_cast<const char*>(value), static_cast<char*>(key_cache),
       static_cast<char*>(value_cache), slot_mapping, num_tokens, num_heads, head_size, block_size, block_shift,
