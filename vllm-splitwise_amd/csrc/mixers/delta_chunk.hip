@@ -34,7 +34,6 @@
 namespace swm {
 
 using f32x4 = __attribute__((ext_vector_type(4))) float;
-using f32x2 = __attribute__((ext_vector_type(2))) float;
 constexpr int kDcChunk = 32;
 constexpr int kDcPrepThreads = 256;
 constexpr int kDcPrepHeads = 2;          // value heads of a prologue's workgroup
@@ -615,6 +614,8 @@ int launch_delta_chunk(const DcStep& a, hipStream_t stream) {
   const int64_t units = (a.runs * a.heads + 7) / 8 * 8, groups = units * vblocks;
   const int group = a.heads / a.kv_heads, parts = (group + kDcPrepHeads - 1) / kDcPrepHeads;
   SW_CHECK_ARG(groups < (1ll << 31), "gated_delta_chunked: too many sequences and heads");
+  SW_CHECK_ARG(2 * (int64_t)a.kv_heads * a.dim + (int64_t)a.heads * a.vdim < (1ll << 25),
+               "gated_delta_chunked: a row of 128 MiB (a chunk of them has its offsets in 32 bits)");
   float* records = a.workspace;
   float* keys = a.workspace + a.chunks * a.heads * dc_record_floats(DP);
   const int vec = a.dim % 4 == 0 && (2 * (int64_t)a.kv_heads * a.dim + (int64_t)a.heads * a.vdim) % 4 == 0 &&
