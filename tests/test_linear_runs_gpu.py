@@ -71,3 +71,61 @@ def test_segments_and_mixed_steps(rule, heads, dim, vdim, lens):
         assert float(off.norm() / b.norm()) < 6e-7 and float(off.max() / b.square().mean().sqrt()) < 3e-5
     idle = [i for i in range(n + 2) if i not in slots] + [slots[i] for i in range(n) if lens[i] == 0]
     assert torch.equal(got[idle], state[idle])
+
+
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 40), (1, 160, 16), (3, 64, 17)])
+@pytest.mark.parametrize("lens", [[70, 33, 130], [1600]], ids=["runs", "segments"])
+def test_gates_that_overflowed(heads, dim, vdim, lens):
+    """A gate of +inf keeps a channel as it is, one of -inf or -3e38 forgets it: in single tokens of a long run, in both halves of a
+    chunk and next to one another, against the rule in 64 bits and against the same tokens in portions of 13, which take the decode
+    kernel.  A gate that is NaN makes its channel NaN, and with it the outputs from there on, and nothing else."""
+    from splitwise_amd import _C
+    n, inf = len(lens), float("inf")
+    starts, rows = [sum(lens[:i]) for i in range(n + 1)], sum(lens)
+    g = torch.Generator(device=DEV).manual_seed(rows + dim)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)               # noqa: E731
+    nk, nv = heads * dim, heads * vdim
+    proj, z, bias = rnd(rows, 2 * nk + nv).bfloat16(), rnd(rows, nk).bfloat16(), 2.0 + rnd(nk)
+    for first, m in zip(starts, lens):
+        for at, channel, gate in ((3, 0, -inf), (5, 1, inf), (17, 2, -inf), (20, 2, -inf), (6, 3, -3e38), (7, 3, inf), (22, 4, 1e38),
+                                  (0, 5, -inf), (m - 1, 6, -inf), (31, 7, -1e38), (32, 7, -inf)):
+            z[first + at, channel::dim] = gate
+    q, k, v = proj[:, :nk], proj[:, nk:2 * nk], proj[:, 2 * nk:]
+    state, slots, ctx = rnd(n, heads, dim, vdim) * 0.1, list(range(n)), [7, 0, 9][:n]
+
+    def step(parts, out, s):
+        """parts: (sequence, tokens before it, tokens)."""
+        pick = torch.cat([torch.arange(starts[i] + lo, starts[i] + lo + m, device=DEV) for i, lo, m in parts])
+        i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)      # noqa: E731
+        batch = SimpleNamespace(q_start=i32([sum(m for _, _, m in parts[:i]) for i in range(len(parts) + 1)]),
+                                ctx_len=i32([ctx[i] + lo for i, lo, _ in parts]), state_slot=i32([slots[i] for i, _, _ in parts]),
+                                max_state_slot=n - 1, max_query_len=max(m for _, _, m in parts),
+                                token_seq=i32([j for j, (_, _, m) in enumerate(parts) for _ in range(m)]))
+        p, o = proj[pick], torch.empty(len(pick), nv, device=DEV)
+        _C.mixer_ops.gla(o, p[:, :nk], p[:, nk:2 * nk], p[:, 2 * nk:], z[pick].contiguous(), bias, 16.0, dim ** -0.5, s, batch, heads,
+                         dim, vdim)
+        out[pick] = o
+
+    whole = [(i, 0, m) for i, m in enumerate(lens)]
+    keep = torch.exp(torch.nn.functional.logsigmoid(z.double() + bias.double()) / 16.0).view(rows, heads, dim)
+    q64, k64, v64 = (t.double().view(rows, heads, -1) for t in (q, k, v))
+    ref, ends = _rule(q64 * dim ** -0.5, k64, v64, keep, state.double(), starts, torch.tensor([c == 0 for c in ctx], device=DEV))
+    got, out = state.clone(), torch.full((rows, nv), float("nan"), device=DEV)
+    step(whole, out, got)
+    short, pieces = state.clone(), torch.full((rows, nv), float("nan"), device=DEV)
+    for lo in range(0, max(lens), 13):
+        step([(i, lo, min(13, m - lo)) for i, m in enumerate(lens) if m > lo], pieces, short)
+    for a, b in ((out.double().view_as(ref), ref), (got.double(), ends), (pieces.double().view_as(ref), ref), (short.double(), ends)):
+        off = (a - b).abs()
+        assert a.isfinite().all()
+        assert float(off.norm() / b.norm()) < 6e-7 and float(off.max() / b.square().mean().sqrt()) < 3e-5
+    z[starts[-2] + 40, 9] = float("nan")                       # the first head of the last sequence
+    bad, res = state.clone(), out.clone()
+    step(whole, res, bad)
+    spoilt = torch.zeros_like(bad, dtype=torch.bool)
+    spoilt[n - 1, 0, 9] = True
+    assert torch.equal(bad.isnan(), spoilt) and torch.equal(bad[~spoilt], got[~spoilt])
+    late = slice(starts[-2] + 40, None)
+    assert res[late, :vdim].isnan().all() and torch.equal(res[late, vdim:], out[late, vdim:])
+    before = starts[-2] + 40 // 32 * 32                        # (its chunk's outputs are sums over the whole channel)
+    assert torch.equal(res[:before], out[:before])

@@ -42,11 +42,12 @@ constexpr int kLwChannels = 16;
 constexpr float kLwSafeLog = 12.0f;
 
 // e^x, x <= 0: the hardware's 2^x, which is good to its last place, with the rounding of x log2(e) put back; half of expf's
-// instructions, which allow for overflow and results below 2^-126 (0 here)
+// instructions, which allow for overflow and results below 2^-126 (0 here).  The rounding is below 2^-16 wherever 2^x is not 0.  It is
+// bounded because a gate that overflowed is a log decay of -inf, of which it would be inf - inf: 0 as expf's, and NaN stays NaN.
 __device__ __forceinline__ float exp_of_sum(float x) {
   const float y = x * 1.44269504f, rest = fmaf(x, 1.44269504f, -y) + x * 1.92596299e-8f;
   const float e = __builtin_amdgcn_exp2f(y);
-  return fmaf(e, rest * 0.69314718f, e);
+  return fmaf(e, __builtin_amdgcn_fmed3f(rest, -1.0f, 1.0f) * 0.69314718f, e);
 }
 // 1 / p, e^-kLwSafeLog <= p <= 1
 __device__ __forceinline__ float reciprocal_of(float p) {
