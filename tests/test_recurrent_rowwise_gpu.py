@@ -215,6 +215,35 @@ def test_delta_chunks_through_every_turn_of_the_walk(heads, kv_heads, dim, vdim,
         assert float(err) < 4e-7, (i, float(err))
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(4, 2, 64, 24), (2, 1, 128, 40)])
+def test_decays_that_overflowed(heads, kv_heads, dim, vdim):
+    """A decay gate of +inf, or one large enough for a decay of 0 in fp32, makes a head forget what was in front of the token, one of
+    -inf keeps it: single tokens of long runs, next to one another and at a chunk's ends, in chunks and token by token.  (Bounds as
+    for the chunks above.)"""
+    from splitwise_amd import _C
+    lens, inf = [70, 33, 130], float("inf")
+    starts, ctx, slots = [sum(lens[:i]) for i in range(4)], [3, 0, 9], [1, 2, 0]
+    g = torch.Generator(device=DEV).manual_seed(dim)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
+    batch = SimpleNamespace(q_start=i32(starts), ctx_len=i32(ctx), max_query_len=max(lens), max_state_slot=2, state_slot=i32(slots),
+                            token_seq=i32([i for i, m in enumerate(lens) for _ in range(m)]))
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)               # noqa: E731
+    rows = starts[-1]
+    qkv, both = rnd(rows, 2 * kv_heads * dim + heads * vdim), rnd(rows, 2 * heads).to(torch.bfloat16)
+    for first, m in zip(starts, lens):
+        for at, head, gate in ((9, 0, inf), (12, 0, inf), (13, 0, -inf), (20, 1, 1e30), (21, 1, 3e38), (0, 1, inf), (31, 0, 500.0),
+                               (32, 0, 1e9), (m - 1, 1, inf)):
+            both[first + at, heads + head] = gate
+    dt_bias, a_log, state = rnd(heads), rnd(heads) * 0.3, rnd(3, heads, dim, vdim) * 0.1
+    ref, ends = _delta_rule(qkv, both[:, :heads], both[:, heads:], dt_bias, a_log, state, batch, heads, kv_heads, dim, vdim)
+    for chunked in (True, False):
+        s, out = state.clone(), torch.full((rows, heads * vdim), float("nan"), device=DEV)
+        _C.mixer_ops.gated_delta(out, qkv, both[:, :heads], both[:, heads:], dt_bias, a_log, s, batch, heads, kv_heads, dim, vdim,
+                                 chunked=chunked)
+        torch.testing.assert_close(out.double(), ref, atol=2e-5, rtol=1e-4)
+        torch.testing.assert_close(s.double(), ends, atol=2e-5, rtol=1e-4)
+
+
 @pytest.mark.parametrize("rule", ["gla", "gla, strong decays", "lightning", "retention"])
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 32, 16), (3, 64, 17), (1, 72, 130), (2, 128, 40), (1, 160, 16), (1, 256, 33)])
 def test_linear_attention_walk_agrees_with_short_runs(rule, heads, dim, vdim):

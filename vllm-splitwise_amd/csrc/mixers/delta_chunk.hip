@@ -176,7 +176,8 @@ __global__ __launch_bounds__(kDcPrepThreads, NDB <= 4 ? 4 : 2) void delta_chunk_
     double L = 0.0;                              // of token l32, in both halves
     if (l32 < cn) {
       beta = sigmoidf_(beta_raw);
-      L = -expf(alog) * softplusf_(decay_raw + bias);
+      const float g = -expf(alog) * softplusf_(decay_raw + bias);
+      L = g < -200.0f ? -200.0f : g;             // a decay of 0; differences of sums with -inf or -1e30 in them would be of nothing
     }
 #pragma unroll
     for (int step = 1; step < 32; step <<= 1) {
