@@ -194,3 +194,24 @@ def test_reshape_and_cache_runs_anywhere(dtype, kv_cache_dtype, num_heads, head_
     qkv_d, kc_d, vc_d = qkv.cuda(), kc.cuda(), vc.cuda()
     C.cache_ops.reshape_and_cache(qkv_d[:, 1], qkv_d[:, 2], kc_d, vc_d, slot_mapping.cuda(), kv_cache_dtype)
     assert torch.equal(_bits(kc_d.cpu()), _bits(kc_ref)) and torch.equal(_bits(vc_d.cpu()), _bits(vc_ref))
+
+
+@pytest.mark.parametrize("dtype,kv_cache_dtype,head_size", [(torch.float32, "fp8_e5m2", 848), (torch.float32, "fp8_e5m2", 864),
+                                                            (torch.float32, "fp8_e5m2", 1024), (torch.float32, "fp8_e5m2", 1264),
+                                                            (torch.float32, "auto", 1132), (torch.float32, "auto", 1272),
+                                                            (torch.bfloat16, "auto", 2040), (torch.bfloat16, "auto", 2272),
+                                                            (torch.bfloat16, "auto", 2544), (torch.float16, "fp8_e5m2", 1712),
+                                                            (torch.float16, "fp8_e5m2", 2544)])
+def test_reshape_and_cache_of_the_largest_heads(dtype, kv_cache_dtype, head_size):
+    """Up to 160 KB of LDS: vectors of V as long as the block allows, half as long, none."""
+    test_reshape_and_cache(dtype, kv_cache_dtype, 2, head_size, 16, "prompt")
+
+
+@pytest.mark.parametrize("dtype,kv_cache_dtype,head_size", [(torch.float32, "auto", 1276), (torch.float32, "fp8_e5m2", 1280),
+                                                            (torch.bfloat16, "auto", 2552), (torch.float16, "fp8_e5m2", 2560)])
+def test_reshape_and_cache_refuses_larger_ones(dtype, kv_cache_dtype, head_size):
+    C = _ops()
+    qkv = torch.zeros(17, 3, 1, head_size, dtype=dtype).cuda()
+    kc, vc = (t.cuda() for t in make_kv_caches(2, 16, 1, head_size, dtype, cache_dtype=kv_cache_dtype))
+    with pytest.raises(RuntimeError, match="too much LDS"):
+        C.cache_ops.reshape_and_cache(qkv[:, 1], qkv[:, 2], kc, vc, torch.arange(17).cuda(), kv_cache_dtype)

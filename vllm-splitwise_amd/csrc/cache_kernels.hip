@@ -35,6 +35,11 @@ void set_error(const char* fmt, ...) {
 
 constexpr int kTileTokens = 16;
 constexpr int kRcThreads = 256;
+constexpr size_t kRcLds = 160 * 1024;
+// Tokens that the kernel looks at: a tile's, and a vector's behind it.  Its own arrays in LDS: 16 bytes for each, 4 per vector of a tile.
+constexpr int rc_group(int vt) { return vt > 0 ? vt : 8; }
+constexpr int rc_seen(int vt) { return kTileTokens + rc_group(vt); }
+constexpr size_t rc_arrays(int vt) { return (size_t)(16 * rc_seen(vt) + 4 * (kTileTokens / rc_group(vt)) + 15) / 16 * 16; }
 
 // LDS row = head_size activations + 16 bytes of padding (keeps 16-byte row reads
 // of consecutive tokens on different bank groups).
@@ -67,10 +72,11 @@ reshape_and_cache_tile_kernel(const char* __restrict__ key, const char* __restri
   constexpr int CS = FP8 ? 1 : ES;              // cache element bytes
   constexpr int X = 16 / CS;                    // cache elements per 16 bytes
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr int GROUP = VT > 0 ? VT : 8, PARTS = kTileTokens / GROUP, kSeen = kTileTokens + GROUP;
+  constexpr int GROUP = rc_group(VT), PARTS = kTileTokens / GROUP, kSeen = rc_seen(VT);
   __shared__ int64_t bases[kSeen];              // byte offset of the token's [block, head] tile, -1: no slot
   __shared__ int offsets[kSeen];                // the token's place in its block
   __shared__ int heads[PARTS], loose[kSeen];    // tokens that begin a vector of V, tokens that no vector takes
+  static_assert(sizeof(bases) + sizeof(offsets) + sizeof(heads) + sizeof(loose) <= rc_arrays(VT), "the launch counts on them");
 
   const int t0 = blockIdx.x / num_heads * kTileTokens;
   const int head = blockIdx.x % num_heads;
@@ -292,12 +298,18 @@ int launch_reshape_and_cache(const void* key, const void* value, void* key_cache
     for (block_shift = 0; (1 << block_shift) < block_size; ++block_shift) {}
   // 16 bytes of tokens per store where a block holds a whole number of them, 8 for the small blocks, else single elements
   constexpr int VT = FP8 ? 16 : 16 / (int)sizeof(S);
-  auto kernel = block_size % VT == 0         ? reshape_and_cache_tile_kernel<act_t, FP8, VT>
-                : block_size % (VT / 2) == 0 ? reshape_and_cache_tile_kernel<act_t, FP8, VT / 2>
-                                             : reshape_and_cache_tile_kernel<act_t, FP8, 0>;
-  // a tile's rows of K, and of V up to a vector's length less one more
-  const size_t smem = (2 * kTileTokens + (block_size % VT == 0 ? VT : block_size % (VT / 2) == 0 ? VT / 2 : 0)) * (size_t)row_bytes;
-  kernel<<<grid, kRcThreads, smem, stream>>>(
+  int vt = block_size % VT == 0 ? VT : block_size % (VT / 2) == 0 ? VT / 2 : 0;
+  // LDS: a tile's rows of K, and of V up to a vector's length less one more (40 rows of 16-bit activations, 48 into an fp8 cache).
+  // The largest heads (from 848 on fp32 into fp8, from 2040 on 16 bits) leave room for shorter vectors, or for none.  Without the check
+  // a launch that passes 160 KB only with the kernel's own arrays would not be refused but end its queue.
+  auto smem = [&](int v) { return (size_t)(2 * kTileTokens + v) * row_bytes; };
+  auto fits = [&](int v) { return smem(v) + rc_arrays(v) <= kRcLds; };
+  while (vt > 0 && !fits(vt)) vt = vt == VT ? VT / 2 : 0;
+  SW_CHECK_ARG(fits(vt), "reshape_and_cache: heads of %d elements need too much LDS", head_size);
+  auto kernel = vt == VT  ? reshape_and_cache_tile_kernel<act_t, FP8, VT>
+                : vt > 0 ? reshape_and_cache_tile_kernel<act_t, FP8, VT / 2>
+                         : reshape_and_cache_tile_kernel<act_t, FP8, 0>;
+  kernel<<<grid, kRcThreads, smem(vt), stream>>>(
       static_cast<const char*>(key), static_cast<const char*>(value), static_cast<char*>(key_cache),
       static_cast<char*>(value_cache), slot_mapping, num_tokens, num_heads, head_size, block_size, block_shift,
       key_stride * es, value_stride * es);
