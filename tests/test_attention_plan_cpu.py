@@ -31,6 +31,13 @@ int main() {
   need(way(1, 8, 1, 64, 1) == kDecodeOnMatrixCores && way(9, 8, 8, 64, 1) == kGeneralAttention, "eight and nine rows");
   need(way(33, 8, 8, 64, 1) == kPromptOnMatrixCores && way(0, 8, 8, 64, 1) == kPromptOnMatrixCores, "a prompt");
   for (int mql = 0; mql < 70; ++mql) need(attention_way(false, 4, mql, 8, 8, 64, 64, 16, 100, 0, 0) == kGeneralAttention, "no pieces");
+  // the prompt kernel's places in a page have 32 bits
+  auto paged = [](int mql, int page, int64_t k, int64_t v) {
+    return attention_way(true, 4, mql, 8, 8, 64, 64, page, 4, 0, 0, attention_page_bytes(page, k, v));
+  };
+  need(paged(40, 1 << 20, 2040, 512) == kPromptOnMatrixCores && paged(40, 1 << 20, 2048, 512) == kGeneralAttention &&
+           paged(40, 1 << 20, 512, 2048) == kGeneralAttention && paged(0, 16, 1ll << 32, 512) == kGeneralAttention &&
+           paged(40, 16, 1024, 1024) == kPromptOnMatrixCores && paged(2, 1 << 20, 2048, 512) == kDecodeOnMatrixCores, "pages of 4 GiB");
   // what the matrix kernels can read
   need(attention_pieces(0, 128, 128, 1024, 1024) && attention_pieces(32, 8, 120, 8, 120), "pieces");
   need(!attention_pieces(8, 128, 128, 1024, 1024) && !attention_pieces(0, 132, 128, 1024, 1024) &&

@@ -174,6 +174,26 @@ def test_two_groups_share_a_walk(H, G, d, page, option, lengths, way):
     torch.testing.assert_close(out.double(), ref, atol=2e-4, rtol=2.0 ** -7)
 
 
+def test_a_page_of_4_gib():
+    """The second page of a cache begins 2^32 bytes behind the first."""
+    from splitwise_amd import _C
+    H = G = 16
+    d, page = 128, 1 << 20
+    lengths = [(0, 40)]
+    batch, _ = _step(lengths, page)
+    batch.block_tables.fill_(1)
+    batch.max_page_id = 1
+    g = torch.Generator(device=DEV).manual_seed(3)
+    kc = torch.zeros(2, page, G * d, dtype=torch.bfloat16, device=DEV)       # values are the keys
+    kc[1, :40] = torch.randn(40, G * d, generator=g, device=DEV).to(torch.bfloat16)
+    q = torch.randn(40, H * d, generator=g, device=DEV)
+    out = torch.empty(40, H * d, dtype=torch.bfloat16, device=DEV)
+    _C.mixer_ops.capped_attention(out, q, kc, None, None, batch, H, G, d, d, d ** -0.5)
+    near = SimpleNamespace(block_tables=torch.zeros_like(batch.block_tables))
+    ref = _statement(lengths, near, q, kc[1:, :64], None, None, H, G, d, d)
+    torch.testing.assert_close(out.double(), ref, atol=2e-4, rtol=2.0 ** -7)
+
+
 @pytest.mark.parametrize("H,G,d,dv,page", [(4, 4, 128, 128, 16), (8, 2, 64, 96, 16), (6, 2, 40, 24, 8), (32, 1, 16, 8, 32),
                                            (3, 1, 104, 128, 12)])
 @pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "sink", "learned sink", "sigmoid", "values in the keys"])

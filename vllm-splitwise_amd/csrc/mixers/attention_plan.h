@@ -53,12 +53,19 @@ inline int attention_one_row_keys(int64_t groups, int dim, int vdim) {
   return groups > 1024 ? 320 : size > 32 ? 256 : 160;
 }
 
-// max_query_len 0: unknown.  pieces: attention_pieces of a bf16 cache
+// The larger of a page's bytes of keys and of values (bf16), from one slot to the next of the same place.
+inline int64_t attention_page_bytes(int page_size, int64_t k_stride, int64_t v_stride) {
+  return 2 * (int64_t)page_size * std::max(k_stride, v_stride);
+}
+
+// max_query_len 0: unknown.  pieces: attention_pieces of a bf16 cache.  page_bytes: the prompt kernel has a key's place in its page in
+// 32 bits (64-bit products took a seventh of its vector units' time); a page of 4 GiB and more goes to the general kernel.
 inline AttentionWay attention_way(bool pieces, int num_seqs, int max_query_len, int heads, int kv_heads, int dim, int vdim,
-                                  int page_size, int table_width, int window, int chunk) {
+                                  int page_size, int table_width, int window, int chunk, int64_t page_bytes = 0) {
   const int group = heads / kv_heads;
   if (!pieces) return kGeneralAttention;
-  if (max_query_len <= 0 || max_query_len > kAttentionTile / group) return kPromptOnMatrixCores;
+  if (max_query_len <= 0 || max_query_len > kAttentionTile / group)
+    return page_bytes < (int64_t)1 << 32 ? kPromptOnMatrixCores : kGeneralAttention;
   if (max_query_len * group > kDecodeRows) return kGeneralAttention;
   if (max_query_len * group == 1 && attention_most_keys(max_query_len, page_size, table_width, window, chunk) <=
                                         attention_one_row_keys((int64_t)num_seqs * kv_heads, dim, vdim))

@@ -652,7 +652,8 @@ int launch_capped_attention(void* out, int64_t out_stride, const float* q, const
     const uintptr_t at = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(key_cache) |
                          reinterpret_cast<uintptr_t>(value_cache);
     const AttentionWay way = attention_way(attention_pieces(at, dim, vdim, k_stride, v_stride), num_seqs, max_query_len, heads,
-                                           kv_heads, dim, vdim, page_size, table_width, window, chunk);
+                                           kv_heads, dim, vdim, page_size, table_width, window, chunk,
+                                           attention_page_bytes(page_size, k_stride, v_stride));
     if (way != kGeneralAttention) {
       PromptAttention a;
       a.out = out; a.q = q;

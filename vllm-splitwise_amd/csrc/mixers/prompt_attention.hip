@@ -167,7 +167,8 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
       page_of[it] = table[a.page_shift >= 0 ? key >> a.page_shift : key / a.page_size];
     });
   };
-  // (a page's place in one 32 x 32 bit product, a key's in the page in 24 bits: 64-bit products took a seventh of the vector units' time)
+  // (a page's place in one product of 32 by 32 bits, a key's in the page in 32, which attention_way sees to: 64-bit products took a
+  // seventh of the vector units' time)
   const uint32_t krow = 2 * (uint32_t)a.k_stride, vrow = 2 * (uint32_t)a.v_stride;
   const uint32_t kpage = krow * (uint32_t)a.page_size, vpage = vrow * (uint32_t)a.page_size;
   auto fetch = [&](int stage) {
