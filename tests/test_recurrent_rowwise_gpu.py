@@ -215,6 +215,23 @@ def test_delta_chunks_through_every_turn_of_the_walk(heads, kv_heads, dim, vdim,
         assert float(err) < 4e-7, (i, float(err))
 
 
+def test_delta_chunks_of_the_widest_rows():
+    """Rows of 128 MiB: a chunk of them passes 32-bit places.  Sums of 4 products in fp32."""
+    from splitwise_amd import _C
+    dim, vdim, lens = 4, 1 << 25, [2, 1]
+    g = torch.Generator(device=DEV).manual_seed(1)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
+    batch = SimpleNamespace(q_start=i32([0, 2, 3]), ctx_len=i32([0, 5]), max_query_len=2, max_state_slot=1, state_slot=i32([1, 0]),
+                            token_seq=i32([0, 0, 1]))
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)               # noqa: E731
+    qkv, both, dt_bias, a_log = rnd(sum(lens), 2 * dim + vdim), rnd(sum(lens), 2).bfloat16(), rnd(1), rnd(1) * 0.3
+    state, out = rnd(2, 1, dim, vdim), torch.full((sum(lens), vdim), float("nan"), device=DEV)
+    ref, ends = _delta_rule(qkv, both[:, :1], both[:, 1:], dt_bias, a_log, state, batch, 1, 1, dim, vdim)
+    _C.mixer_ops.gated_delta(out, qkv, both[:, :1], both[:, 1:], dt_bias, a_log, state, batch, 1, 1, dim, vdim, chunked=True)
+    for a, b in ((out, ref), (state, ends)):
+        assert float((a.double() - b).abs().max()) < 2e-5
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(4, 2, 64, 24), (2, 1, 128, 40)])
 def test_decays_that_overflowed(heads, kv_heads, dim, vdim):
     """A decay gate of +inf, or one large enough for a decay of 0 in fp32, makes a head forget what was in front of the token, one of

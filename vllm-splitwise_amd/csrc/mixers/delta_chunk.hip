@@ -615,8 +615,6 @@ int launch_delta_chunk(const DcStep& a, hipStream_t stream) {
   const int64_t units = (a.runs * a.heads + 7) / 8 * 8, groups = units * vblocks;
   const int group = a.heads / a.kv_heads, parts = (group + kDcPrepHeads - 1) / kDcPrepHeads;
   SW_CHECK_ARG(groups < (1ll << 31), "gated_delta_chunked: too many sequences and heads");
-  SW_CHECK_ARG(2 * (int64_t)a.kv_heads * a.dim + (int64_t)a.heads * a.vdim < (1ll << 25),
-               "gated_delta_chunked: a row of 128 MiB (a chunk of them has its offsets in 32 bits)");
   float* records = a.workspace;
   float* keys = a.workspace + a.chunks * a.heads * dc_record_floats(DP);
   const int vec = a.dim % 4 == 0 && (2 * (int64_t)a.kv_heads * a.dim + (int64_t)a.heads * a.vdim) % 4 == 0 &&
@@ -657,6 +655,10 @@ int swm_gated_delta_chunked(float* out, const float* qkv, const void* beta_pre, 
                "gated_delta_chunked: heads %d, kv heads %d, key size %d (up to 224), value size %d", heads, kv_heads, dim,
                vdim);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // The walk has a chunk's places in 32 bits: rows of 128 MiB and more go token by token (whose workspace is the smaller one).
+  if (2 * (int64_t)kv_heads * dim + (int64_t)heads * vdim >= 1ll << 25)
+    return swm_gated_delta(out, qkv, beta_pre, beta_stride, decay_pre, decay_stride, dt_bias, a_log, state, q_start, ctx_len, state_slot,
+                           rows, num_seqs, heads, kv_heads, dim, vdim, workspace, act_dtype, stream);
   // Decoding sequences beside a portion take the decode kernel: their states are read and written in whole rows there, in 64-byte
   // pieces here, and they need no 32-row record.  Not worth the launch where most sequences are long.  (us a call, 12 heads of 96, a
   // portion of 100 tokens beside 60 / 250 decoding sequences: 186 / 1046 all in chunks, 61 / 104 so)
