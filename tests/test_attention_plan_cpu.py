@@ -38,6 +38,21 @@ int main() {
   need(paged(40, 1 << 20, 2040, 512) == kPromptOnMatrixCores && paged(40, 1 << 20, 2048, 512) == kGeneralAttention &&
            paged(40, 1 << 20, 512, 2048) == kGeneralAttention && paged(0, 16, 1ll << 32, 512) == kGeneralAttention &&
            paged(40, 16, 1024, 1024) == kPromptOnMatrixCores && paged(2, 1 << 20, 2048, 512) == kDecodeOnMatrixCores, "pages of 4 GiB");
+  // two groups of waves a walk: 16 query heads on 4, 32 tokens a workgroup
+  auto groups = [](int64_t rows, int seqs, int mql, int width, int window = 0, int chunk = 0) {
+    return prompt_attention_groups(rows, seqs, mql, 16, 4, 16, width, window, chunk);
+  };
+  need(prompt_attention_workgroups(65, 2, 16, 4) == 20 && prompt_attention_workgroups(64, 2, 16, 4) == 16, "workgroups");
+  need(groups(240, 1, 240, 15) == 1 && groups(240, 1, 240, 16) == 2 && groups(240, 1, 240, 99, 255) == 1 && groups(240, 1, 240, 99, 256) == 2 &&
+           groups(240, 1, 240, 99, 0, 255) == 1 && groups(240, 1, 240, 99, 0, 256) == 2, "keys");
+  need(groups(63 * 32, 1, 2016, 126) == 2 && groups(62 * 32, 2, 1000, 126, 300) == 2 && groups(62 * 32 + 1, 2, 1000, 126, 300) == 1 &&
+           groups(62 * 32 + 1, 2, 1000, 126, 0, 300) == 1, "a compute unit each");
+  need(groups(62 * 32 + 1, 2, 1100, 70) == 2 && groups(98 * 32, 2, 50 * 32, 100) == 2 && groups(98 * 32, 2, 49 * 32, 100) == 1, "half of the workgroups");
+  need(groups(3000, 5, 2900, 182) == 2 && groups(3000, 7, 2900, 182) == 1, "sequences beside");
+  need(groups(127 * 32, 1, 4064, 254) == 2 && groups(127 * 32, 1, 4064, 900) == 2 && groups(128 * 32, 1, 4096, 900) == 1 &&
+           groups(128 * 32, 1, 4096, 321) == 2 && groups(128 * 32, 1, 4096, 322) == 1, "keys in front of the prompt");
+  need(groups(139 * 32, 1, 139 * 32, 278) == 2 && groups(139 * 32 + 1, 1, 139 * 32 + 1, 279) == 1, "the last line");
+  need(groups(3000, 1, 0, 188) == 1 && groups(2000, 1, 0, 125) == 2, "longest unknown");
   // what the matrix kernels can read
   need(attention_pieces(0, 128, 128, 1024, 1024) && attention_pieces(32, 8, 120, 8, 120), "pieces");
   need(!attention_pieces(8, 128, 128, 1024, 1024) && !attention_pieces(0, 132, 128, 1024, 1024) &&

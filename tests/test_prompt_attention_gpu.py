@@ -24,6 +24,9 @@ extern "C" int way(unsigned long at, long k_stride, long v_stride, int seqs, int
   return swm::attention_way(swm::attention_pieces(at, dim, vdim, k_stride, v_stride), seqs, mql, heads, kv_heads, dim, vdim, page,
                             width, window, chunk);
 }
+extern "C" int groups(long rows, int seqs, int mql, int heads, int kv_heads, int page, int width, int window, int chunk) {
+  return swm::prompt_attention_groups(rows, seqs, mql, heads, kv_heads, page, width, window, chunk);
+}
 """
 
 
@@ -42,6 +45,12 @@ def way(tmp_path_factory):
         at = q.data_ptr() | kc.data_ptr() | vc.data_ptr()
         return lib.way(ctypes.c_ulong(at), ctypes.c_long(kc.shape[2]), ctypes.c_long(vc.shape[2]), batch.num_seqs, batch.max_query_len, H,
                        G, d, dv, kc.shape[1], batch.block_tables.shape[1], window, chunk)
+
+    def groups(batch, H, G, page, window=0, chunk=0, **_):
+        """-> how many groups of waves share a workgroup's walk in the prompt kernel."""
+        return lib.groups(ctypes.c_long(batch.token_seq.numel()), batch.num_seqs, batch.max_query_len, H, G, page,
+                          batch.block_tables.shape[1], window, chunk)
+    ask.groups = groups
     return ask
 
 
@@ -148,11 +157,14 @@ def test_an_infinity_in_shared_keys_that_one_of_two_tokens_sees(H, G, d, way):
 
 @pytest.mark.parametrize("H,G,d,page", [(4, 2, 128, 16), (3, 1, 96, 12), (8, 4, 24, 8)])
 @pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "learned sink", "sigmoid"])
-@pytest.mark.parametrize("lengths", [[(0, 255), (0, 40)], [(0, 257), (31, 66)], [(700, 33), (256, 1), (224, 40), (607, 2)]], ids=str)
+@pytest.mark.parametrize("lengths", [[(0, 240), (0, 40)], [(0, 255), (0, 40)], [(0, 257), (31, 66)], [(700, 33), (256, 1), (224, 40), (607, 2)],
+                                     [(700, 33), (256, 1), (224, 40), (607, 2)] + [(i * 37 % 700, 1) for i in range(256)]],
+                         ids=lambda v: str(v[:4]) + " and 256 more" * (len(v) > 4))
 def test_two_groups_share_a_walk(H, G, d, page, option, lengths, way):
-    """On both sides of the number of keys from which two groups of waves share a workgroup's stages of 32; odd and even numbers of
-    stages, rows that see keys of one group's only.  In front, from the second stage on, keys that weigh next to nothing or most, and a
-    value of inf in a channel: what one group makes of it has to meet the other's sums.  (Tolerances as above.)"""
+    """On both sides of the number of keys from which two groups of waves share a workgroup's stages of 32, and of the number of
+    workgroups beyond which long walks go to one group; odd and even numbers of stages, rows that see keys of one group's only.  In
+    front, from the second stage on, keys that weigh next to nothing or most, and a value of inf in a channel: what one group makes of
+    it has to meet the other's sums.  (Tolerances as above.)"""
     from splitwise_amd import _C
     batch, pages = _step(lengths, page)
     g = torch.Generator(device=DEV).manual_seed(d + len(lengths))
@@ -167,6 +179,7 @@ def test_two_groups_share_a_walk(H, G, d, page, option, lengths, way):
     kw = {"cap": dict(softcap=4.0), "window": dict(window=290), "chunk": dict(chunk=258), "sigmoid": dict(score_bias=torch.linspace(-2.0, 1.0, H, device=DEV)),
           "learned sink": dict(sink=torch.linspace(-3.0, 2.0, H, device=DEV))}.get(option, {})
     assert way(q, kc, vc, batch, H, G, d, d, **kw) == PROMPT
+    assert way.groups(batch, H, G, page, **kw) == (1 if len(lengths) > 4 or lengths[0] == (0, 240) else 2)
     out = torch.empty(rows, H * d, dtype=torch.bfloat16, device=DEV)
     _C.mixer_ops.capped_attention(out, q, kc, vc, None, batch, H, G, d, d, d ** -0.5, **kw)
     ref = _statement(lengths, batch, q, kc, vc, None, H, G, d, d, **kw)

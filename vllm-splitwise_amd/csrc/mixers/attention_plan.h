@@ -8,6 +8,7 @@
 namespace swm {
 
 constexpr int kAttentionTile = 32;      // query rows of a tile
+constexpr int kPromptWaves = 4;         // tiles of a workgroup of the prompt kernel
 // Decode steps on the matrix cores: at most this many query rows (tokens x heads of a group) per sequence and key/value head
 constexpr int kDecodeRows = 8;
 constexpr int kDecodeGroups = 256, kDecodePartKeys = 256, kDecodeSharedKeys = 1024;
@@ -71,6 +72,44 @@ inline AttentionWay attention_way(bool pieces, int num_seqs, int max_query_len, 
                                         attention_one_row_keys((int64_t)num_seqs * kv_heads, dim, vdim))
     return kGeneralAttention;
   return kDecodeOnMatrixCores;
+}
+
+// The prompt kernel's workgroups, an upper bound: tiles of every sequence's tokens for every key/value head.
+inline int prompt_tokens(int heads, int kv_heads) { return kPromptWaves * (kAttentionTile / (heads / kv_heads)); }
+inline int64_t prompt_attention_workgroups(int64_t rows, int num_seqs, int heads, int kv_heads) {
+  const int tokens = prompt_tokens(heads, kv_heads);
+  return ((rows + tokens - 1) / tokens + num_seqs) * kv_heads;
+}
+
+// How many groups of waves share a workgroup's walk in the prompt kernel, 1 or 2.  Two shorten the longest walk, which is what a launch
+// waits for that leaves it a compute unit of its own; but only one such workgroup fits a compute unit, where of one group's two do, and
+// those fill one another's gaps better than two groups do (by 5 to 12 % where a launch has many rounds of them).
+// Measured in 1435 steps (us, one group / two; W: workgroups, as counted above; 16 query heads on 4 of 128 unless stated):
+//   Keys, an upper bound of the longest walk (the block tables' width, the mask): below 256 the two cost more than they save (80 steps,
+//   0.96 on average): one prompt of 77 tokens, 8 heads on 2: 18.2 / 20.3; from there on they gain, 271 twice, 12 on 4 of 64: 20.3 / 18.4.
+//   W up to 256, a compute unit for each: 1.19 on average whatever the mask, the lengths and the decoding sequences beside: 64 tokens
+//   behind 1406, window 256 25.4 / 23.7, 1766 tokens 110.7 / 92.2, 723 tokens six times, 8 on 2, window 256 (W 238) 26.8 / 27.3; about a
+//   hundred decoding sequences over 500 keys each lose up to 5 % (W 135, 8 on 1 of 64, 35.9 / 37.8).
+//   Beyond, a second round begins where the first one's short walks end: the causal mask's, of tiles at the front of a sequence.  That
+//   pays where the longest sequence has at least half of the workgroups and there are few of one token: 3446 tokens (W 436) 201.8 /
+//   154.1, 1419 and 1903 (W 424) 129.5 / 94.9; not with 950 at most of five sequences (W 464) 63.8 / 73.4, with ten decoding sequences
+//   beside 3520 tokens (W 488) 202 / 258, 371 tokens six times, 32 on 8 (W 512), 35.1 / 46.1, and not
+//   under a window or chunks of fewer keys (20 steps, 0.75 to 1.26).
+//   With keys in front of the prompt walks are less uneven: up to W 512 1.01 to 1.33, beyond 0.84 to 1.05 (2271 behind 1047, 32 on 8,
+//   W 576: 242 / 288).  Without, 1.25 to 1.33 on average up to W 512, 1.12 (1.01 to 1.30) from 544 to 560, 1.08 (0.94 to 1.23) to 576,
+//   1.01 (0.86 to 1.14) from 592 to 608, 0.98 from 640 on.
+constexpr int64_t kSharedWalkKeys = 256, kSharedWalksAlone = 256, kSharedWalksBehind = 512, kSharedWalks = 560;
+inline int prompt_attention_groups(int64_t rows, int num_seqs, int max_query_len, int heads, int kv_heads, int page_size, int table_width,
+                                   int window, int chunk) {
+  const int64_t keys = (int64_t)table_width * page_size, mask = window > 0 ? window : chunk > 0 ? chunk : keys;
+  const int64_t all = prompt_attention_workgroups(rows, num_seqs, heads, kv_heads);
+  if (std::min(keys, mask) < kSharedWalkKeys) return 1;
+  if (all <= kSharedWalksAlone) return 2;
+  const int tokens = prompt_tokens(heads, kv_heads);
+  const int64_t longest = (int64_t)((max_query_len + tokens - 1) / tokens) * kv_heads;
+  const bool whole = keys - page_size <= (int64_t)max_query_len * 5 / 4;       // next to nothing in front of the longest prompt
+  return mask >= keys && 2 * longest >= all && 16 * (int64_t)num_seqs * kv_heads <= all && all <= (whole ? kSharedWalks : kSharedWalksBehind)
+             ? 2 : 1;
 }
 
 // How many workgroups share a sequence's keys in the decode kernel on the matrix cores, given a workspace of parts x rows x heads x

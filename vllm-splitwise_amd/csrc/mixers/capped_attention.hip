@@ -667,7 +667,7 @@ int launch_capped_attention(void* out, int64_t out_stride, const float* q, const
       a.vdim = vdim; a.page_size = page_size; a.page_shift = page_shift; a.window = window; a.chunk = chunk;
       a.sink = sink; a.tpt = tpt; a.scale = scale; a.softcap = softcap;
       return way == kDecodeOnMatrixCores ? launch_decode_attention(a, rows, max_query_len, workspace, stream)
-                                         : launch_prompt_attention(a, rows, stream);
+                                         : launch_prompt_attention(a, rows, max_query_len, stream);
     }
   }
   if (split) {

@@ -77,7 +77,7 @@ __device__ __forceinline__ PlainRow plain_row(const PromptAttention& a, const in
   return row;
 }
 
-int launch_prompt_attention(const PromptAttention& a, int64_t rows, hipStream_t stream);
+int launch_prompt_attention(const PromptAttention& a, int64_t rows, int max_query_len, hipStream_t stream);
 
 int launch_decode_attention(const PromptAttention& a, int64_t rows, int max_query_len, float* workspace, hipStream_t stream);
 

@@ -40,7 +40,7 @@ using pa_u32x4 = __attribute__((ext_vector_type(4))) uint32_t;
 using pa_i16x4 = __attribute__((ext_vector_type(4))) short;
 using pa_lds_i16x4 = __attribute__((address_space(3))) pa_i16x4*;
 
-constexpr int kPaKeys = 32, kPaWaves = 4;
+constexpr int kPaKeys = 32, kPaWaves = kPromptWaves;
 constexpr float kLog2e = 1.4426950408889634f;
 
 // one 16-byte fragment: 8 neighbouring bf16 numbers
@@ -521,39 +521,21 @@ int launch_prompt_tiles_as(const PromptAttention& a, unsigned groups, hipStream_
   return SW_OK;
 }
 
-// When two groups share a walk.  They shorten the longest one, which is what a launch waits for that has few workgroups, or that has a
-// long walk beside many short ones under a causal mask; but only one such workgroup fits a compute unit, where of one group's two
-// do, and those fill one another's gaps better than two groups do.
-//   Keys (an upper bound of the longest walk: the block tables' width, the mask).  One group / two, us: one prompt of 77 tokens, 8
-//   heads on 2 of 128: 18.2 / 20.3; two of 127, 16 on 8: 15.9 / 16.4; two of 271, 12 on 4 of 64: 20.3 / 18.4; four of 85 behind 209
-//   others: 32.9 / 31.1; one of 511, 16 on 4 of 96: 30.6 / 26.0.
-//   Workgroups, few: 8 (64 tokens behind 3000) 163 / 119, 64 (300 tokens twice, 12 on 4 of 96) 22.5 / 20.6, 126 (2000 twice, 4 on 1 of
-//   128, a window of 1024) 70 / 59; 232 (200 sequences' tokens beside 1000) 70 / 73, 400 (2000 twice, 12 on 4, chunks of 512) 43 / 53.
-//   A causal mask alone, sequences of many tiles: 256 80 / 57, 400 120 / 95, 504 164 / 134, 512 81 / 61; with 488 of which most are a
-//   token each (60 sequences of 2000 keys, 8 heads of 64) 83 / 122.
-constexpr int64_t kPaSharedKeys = 256, kPaSharedFew = 200, kPaSharedCausal = 560;
-inline bool pa_two_groups(const PromptAttention& a, int64_t workgroups) {
-  const int64_t width = (int64_t)a.table_width * a.page_size;
-  const int64_t mask = a.window > 0 ? a.window : a.chunk > 0 ? a.chunk : width;
-  if (std::min(width, mask) < kPaSharedKeys) return false;
-  return workgroups <= kPaSharedFew ||
-         (mask >= width && workgroups <= kPaSharedCausal && 8 * (int64_t)a.num_seqs * a.kv_heads <= workgroups);
-}
 template <int NB>
-int launch_prompt_tiles(const PromptAttention& a, int64_t rows, hipStream_t stream) {
-  const int64_t per_wg = (int64_t)kPaWaves * a.tpt;
-  const int64_t groups = ((rows + per_wg - 1) / per_wg + a.num_seqs) * a.kv_heads;
+int launch_prompt_tiles(const PromptAttention& a, int64_t rows, int max_query_len, hipStream_t stream) {
+  const int64_t groups = prompt_attention_workgroups(rows, a.num_seqs, a.heads, a.kv_heads);
   SW_CHECK_ARG(groups < (1ll << 31), "masked_attention: too many rows");
-  return pa_two_groups(a, groups) ? launch_prompt_tiles_as<NB, 2>(a, (unsigned)groups, stream)
-                                  : launch_prompt_tiles_as<NB, 1>(a, (unsigned)groups, stream);
+  return prompt_attention_groups(rows, a.num_seqs, max_query_len, a.heads, a.kv_heads, a.page_size, a.table_width, a.window, a.chunk) > 1
+             ? launch_prompt_tiles_as<NB, 2>(a, (unsigned)groups, stream)
+             : launch_prompt_tiles_as<NB, 1>(a, (unsigned)groups, stream);
 }
 
-int launch_prompt_attention(const PromptAttention& a, int64_t rows, hipStream_t stream) {
+int launch_prompt_attention(const PromptAttention& a, int64_t rows, int max_query_len, hipStream_t stream) {
   switch ((std::max(a.dim, a.vdim) + 31) / 32) {
-    case 1: return launch_prompt_tiles<1>(a, rows, stream);
-    case 2: return launch_prompt_tiles<2>(a, rows, stream);
-    case 3: return launch_prompt_tiles<3>(a, rows, stream);
-    default: return launch_prompt_tiles<4>(a, rows, stream);
+    case 1: return launch_prompt_tiles<1>(a, rows, max_query_len, stream);
+    case 2: return launch_prompt_tiles<2>(a, rows, max_query_len, stream);
+    case 3: return launch_prompt_tiles<3>(a, rows, max_query_len, stream);
+    default: return launch_prompt_tiles<4>(a, rows, max_query_len, stream);
   }
 }
 
