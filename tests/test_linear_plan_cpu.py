@@ -38,6 +38,9 @@ int main() {
       }
     need(runs <= p.runs && chunks <= p.chunks && items <= p.items, "a bound that does not hold");
     need(p.segment % 32 == 0, "a segment that ends inside a chunk");
+    const int64_t groups = linear_walk_groups(p, heads, vdim), walkers = linear_walkers(p, heads, dim, vdim), width = (vdim + 15) / 16;
+    need(groups >= p.items * heads * width && walkers > 0 && walkers <= groups && walkers % (8 * width) == 0, "whole eights of workgroups");
+    need(walkers == groups || (p.at_most > 0 && walkers >= 496), "workgroups that go on");
     const long dp = (dim + 31) / 32 * 32, vb = (vdim + 15) / 16;
     need(p.floats >= p.chunks * heads * (65 * dp + 1024) + (p.segment ? p.items * heads * (16 * vb * dp + dp) : 0), "scratch");
   }
@@ -51,6 +54,9 @@ int main() {
     const LinearWalkPlan p = linear_walk_plan(true, 250 + portion, 251, portion, 16, 128, 128);
     need(p.at_most == 16, "250 decoding sequences walk");
   }
+  // ... and leave no queue of workgroups that find no piece: 251 sequences, 1250 rows may be 73 runs, 9344 workgroups, and are one run
+  const LinearWalkPlan mixed = linear_walk_plan(true, 1250, 251, 1000, 16, 128, 128);
+  need(linear_walk_groups(mixed, 16, 128) == 9344 && linear_walkers(mixed, 16, 128, 128) == 512, "250 decoding sequences' workgroups");
   // a long run of few heads is cut into as many pieces as the GPU has room for
   for (int n : {8000, 16000, 32000}) {
     const LinearWalkPlan p = linear_walk_plan(false, n, 1, n, 4, 128, 128);

@@ -30,7 +30,10 @@ def _rule(q, k, v, keep, state, starts, fresh):
     (2, 128, 40, [1100, 577, 1, 30, 576]), (1, 64, 16, [5000]), (1, 40, 17, [1024, 1025]), (2, 160, 33, [1500, 3]),
     (3, 256, 20, [33, 2049]),                                              # segments
     (2, 128, 128, [1] * 130 + [40] + [2] * 70 + [17, 16, 95]),              # decoding sequences beside portions
-    (4, 128, 128, [1] * 61 + [600, 1100]), (16, 64, 64, [1, 5, 0, 2] * 40 + [70])], ids=str)
+    (4, 128, 128, [1] * 61 + [600, 1100]), (16, 64, 64, [1, 5, 0, 2] * 40 + [70]),
+    # workgroups that go on to further pieces: several of them, of a run's segments, a few at most, narrow ones
+    (2, 128, 128, [n for i in range(60) for n in (1, 17 + i % 17)] + [200, 64] + [30] * 20), (4, 128, 128, [1] * 100 + [2100] + [40] * 3),
+    (32, 256, 33, [1] * 150 + [300, 0, 21, 50]), (32, 32, 40, [1, 18] * 130 + [97])], ids=str)
 def test_segments_and_mixed_steps(rule, heads, dim, vdim, lens):
     from splitwise_amd import _C
     ops = _C.mixer_ops

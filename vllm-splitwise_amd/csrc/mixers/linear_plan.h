@@ -71,4 +71,22 @@ inline LinearWalkPlan linear_walk_plan(bool per_channel, int64_t rows, int num_s
   return p;
 }
 
+// The walk's workgroups: one for each piece, head and 16 value channels, in eights of pieces and heads.
+inline int64_t linear_walk_groups(const LinearWalkPlan& p, int heads, int vdim) {
+  return (p.items * heads + 7) / 8 * 8 * ((vdim + 15) / 16);
+}
+// ... and how many of them are launched.  Beside decoding sequences the pieces are a far upper bound (a run for every 17 rows), and a
+// workgroup that finds no piece still takes its turn in a compute unit that holds one of 8 waves at a time.  From 6 rounds of
+// workgroups on two rounds of them go on to the next pieces instead, which costs a launch 1 - 2 us (their loop keeps more registers).
+// us, one workgroup a piece / so; gla, heads of 128 unless stated.  5.8 rounds: 2 heads, 82 decoding sequences beside 10 portions,
+// 49.1 / 48.7;  6.2: lightning, 16 of 64, 113 beside 10 67.0 / 65.8;  9: 32 heads, 61 beside 92 tokens 83.8 / 79.1;  29: 16 heads, 250
+// beside 1000 tokens 237.6 / 177.7;  35: 32 heads, 96 beside 10 portions 202 / 172;  53: 8 of 256, 102 beside 4 550 / 458.
+// One round: 79.1 -> 77.6 there, but lightning, 16 of 96, 21 beside 10 portions 85.5 -> 103.8: what a workgroup takes is settled then.
+inline int64_t linear_walkers(const LinearWalkPlan& p, int heads, int dim, int vdim) {
+  const int64_t groups = linear_walk_groups(p, heads, vdim), vblocks = (vdim + 15) / 16;
+  const int64_t round = 256 * (dim <= 32 ? 4 : dim <= 96 ? 2 : 1);             // as many as the GPU holds at once, by their registers
+  if (p.at_most == 0 || groups <= 6 * round) return groups;
+  return (2 * round / vblocks + 7) / 8 * 8 * vblocks;
+}
+
 }  // namespace swm

@@ -466,22 +466,22 @@ __global__ __launch_bounds__(64 * NDB) void linear_segment_kernel(const LinearSt
   }
 }
 
+// Piece unit / heads of head unit % heads, 16 value channels of it; false when there is no such piece (and none behind it).
+// (No barrier is needed between two calls: what the readers of the last chunk may still read is written behind the next call's first.)
 template <typename TV, bool SILU, int NDB>
-__global__ __launch_bounds__(128 * NDB, 2) void linear_walk_kernel(const LinearStep a, const LwPieces pc) {
+__device__ __forceinline__ bool linear_walk_piece(const LinearStep& a, const LwPieces& pc, int unit, int vb, int vblocks, int tid) {
   __shared__ f32x4 states[2][NDB][2][64];        // [chunk parity][32 coordinates][16 coordinates][lane]: S_0
   __shared__ f32x4 queried[2][NDB][2][64];       // [chunk parity][wave][token tile][lane]: shares of Q~ S_0
   __shared__ f32x4 values[2][2][64];             // [chunk parity][token tile][lane]: V
   constexpr int DP = NDB * 32, kAhead = NDB <= 4 ? 2 : 1;
-  const int vblocks = (a.vdim + kLwChannels - 1) / kLwChannels;
-  const int unit = (blockIdx.x >> 3) / vblocks * 8 + (blockIdx.x & 7), vb = (blockIdx.x >> 3) % vblocks;
   const int item = unit / a.heads, h = unit - item * a.heads;
   int seq = 0, tok0 = 0, before = 0;
   const int n = item < pc.items ? find_run_piece(a.q_start, a.num_seqs, pc.at_most, pc.segment > 0 ? pc.segment : 1 << 30, item, &seq,
                                                 &tok0, &before)
                                 : 0;
-  if (n <= 0) return;                            // the whole workgroup
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = wave % NDB;
-  const int lane = threadIdx.x & 63, li = lane & 15, gq = lane >> 4;
+  if (n <= 0) return false;                      // the whole workgroup
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), b = wave % NDB;
+  const int lane = tid & 63, li = lane & 15, gq = lane >> 4;
   const int64_t row0 = (int64_t)a.q_start[seq] + tok0, chunk0 = before + tok0 / kLwChunk;
   // This lane's value channel; lanes beyond the last one do its work over again, which spares the stores a condition.
   const int vc = min(vb * kLwChannels + li, a.vdim - 1);
@@ -576,7 +576,7 @@ __global__ __launch_bounds__(128 * NDB, 2) void linear_walk_kernel(const LinearS
           if (c < a.dim) sp[(int64_t)c * a.vdim + vc] = S[i][r];
         }
     }
-    return;
+    return true;
   }
   // ------------------------------------------------------------------------------------------------------------ the outputs
   // O = A V + Q~ S_0: the shares of Q~ S_0 meet behind the next chunk's barrier.  The values are widened a chunk ahead of the state.
@@ -716,6 +716,24 @@ __global__ __launch_bounds__(128 * NDB, 2) void linear_walk_kernel(const LinearS
       }
     }
   }
+  return true;
+}
+
+// MANY: a workgroup goes on to further pieces, as far as there are any (linear_plan.h says when).
+template <typename TV, bool SILU, int NDB, bool MANY>
+__global__ __launch_bounds__(128 * NDB, 2) void linear_walk_kernel(const LinearStep a, const LwPieces pc) {
+  const int vblocks = (a.vdim + kLwChannels - 1) / kLwChannels;
+  const int first = (blockIdx.x >> 3) / vblocks * 8 + (blockIdx.x & 7), vb = (blockIdx.x >> 3) % vblocks;
+  if constexpr (!MANY) {
+    linear_walk_piece<TV, SILU, NDB>(a, pc, first, vb, vblocks, threadIdx.x);
+  } else {
+#pragma unroll 1
+    for (int unit = first;; unit += gridDim.x / vblocks) {
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));              // nothing of a piece's is worked out in front of the loop, and kept
+      if (!linear_walk_piece<TV, SILU, NDB>(a, pc, unit, vb, vblocks, tid)) return;
+    }
+  }
 }
 
 template <typename K>
@@ -727,7 +745,7 @@ inline hipError_t lw_allow_lds(K kernel, size_t bytes) {
 template <typename TV, bool SILU>
 int launch_walk(const LinearStep& a, const LinearWalkPlan& plan, hipStream_t stream) {
   const int64_t dp = (a.dim + 31) / 32 * 32, vblocks = (a.vdim + kLwChannels - 1) / kLwChannels;
-  const int64_t groups = (plan.items * a.heads + 7) / 8 * 8 * vblocks;
+  const int64_t groups = linear_walk_groups(plan, a.heads, a.vdim), walkers = linear_walkers(plan, a.heads, a.dim, a.vdim);
   SW_CHECK_ARG(groups < (1ll << 31), "linear attention: too many sequences and heads");
   LwPieces pc{plan.at_most, plan.segment, plan.items, nullptr, nullptr};
   if (plan.segment > 0) {
@@ -740,7 +758,10 @@ int launch_walk(const LinearStep& a, const LinearWalkPlan& plan, hipStream_t str
       hipLaunchKernelGGL((linear_segment_kernel<TV, SILU, N>), dim3((unsigned)groups), dim3(64 * N), 0, stream, a, pc); \
       SW_CHECK_LAUNCH();                                                                                               \
     }                                                                                                                  \
-    hipLaunchKernelGGL((linear_walk_kernel<TV, SILU, N>), dim3((unsigned)groups), dim3(128 * N), 0, stream, a, pc);    \
+    if (walkers < groups)                                                                                              \
+      hipLaunchKernelGGL((linear_walk_kernel<TV, SILU, N, true>), dim3((unsigned)walkers), dim3(128 * N), 0, stream, a, pc); \
+    else                                                                                                               \
+      hipLaunchKernelGGL((linear_walk_kernel<TV, SILU, N, false>), dim3((unsigned)groups), dim3(128 * N), 0, stream, a, pc); \
     break;
   switch ((a.dim + 31) / 32) {
     SWM_LW_CASE(1)
