@@ -661,7 +661,8 @@ int swm_gated_delta_chunked(float* out, const float* qkv, const void* beta_pre, 
                            rows, num_seqs, heads, kv_heads, dim, vdim, workspace, act_dtype, stream);
   // Decoding sequences beside a portion take the decode kernel: their states are read and written in whole rows there, in 64-byte
   // pieces here, and they need no 32-row record.  Not worth the launch where most sequences are long.  (us a call, 12 heads of 96, a
-  // portion of 100 tokens beside 60 / 250 decoding sequences: 186 / 1046 all in chunks, 61 / 104 so)
+  // portion of 100 tokens beside 11 / 20 / 60 / 250 decoding sequences: 29 / 44 / 87 / 360 all in chunks, 25 / 26 / 35 / 76 so; beside 6
+  // 24.1 and 24.7; 2000 tokens beside 11 105.4 and 106.7)
   const bool mixed = num_seqs >= 12 && rows < 128 * (int64_t)num_seqs &&
                      delta_step(out, qkv, beta_pre, beta_stride, decay_pre, decay_stride, 1, dt_bias, a_log, state, q_start, ctx_len,
                                 state_slot, num_seqs, heads, kv_heads, dim, vdim, kDcShort, act_dtype, s);

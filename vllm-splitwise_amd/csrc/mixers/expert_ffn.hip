@@ -289,8 +289,8 @@ __global__ __launch_bounds__(64 * kFewWaves) void expert_few_rows_kernel(const E
 // that follow one another there.
 // Measured, 3989 rows of width 2048, 32 gated experts of 1024, two per row (7978 pairs), up / down: 287 / 188 us in the 64 x 64
 // tiles with a load, a barrier and a product in turn that these replace; 168 / 119 us with 128 x 128 tiles whose loads were
-// one stage ahead; 127 / 105 us as it is (530 / 318 TFLOP/s).  Of the down-projection 18 us are its additions into the fp32
-// output (plain stores instead: 87 us).
+// one stage ahead; 134 / 109 us as it is (498 / 308 TFLOP/s; one by one under a profiler, 5 % less in a stream of calls).  Of the
+// down-projection 26 us are its additions into the fp32 output (plain stores instead: 82 us).
 constexpr int kTileK = 64, kTilePad = 8;
 __host__ __device__ constexpr int expert_tile_lds(int tm, int tn) { return 2 * (tm + tn) * (kTileK + kTilePad) * 2 + 2 * tm * 4; }
 

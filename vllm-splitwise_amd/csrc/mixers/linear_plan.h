@@ -12,17 +12,18 @@ constexpr int kLwChunk = 32;
 // steps (gla.hip, lightning.hip: a workgroup takes the whole run of a sequence and a head), longer ones through the walk.
 // -> at_most: 0: the walk takes all, max_query_len: the decode kernels do.
 // per_channel: decays per key channel (gla), else one per head, whose decode kernels are the cheaper ones.
-// Measured (us a call with its norm and gate; W: sequences x heads, of 128 x 128):
+// Measured (us a call of the rule alone; W: sequences x heads, of 128 x 128):
 //   max_query_len <= 16: as decode steps, whatever W.
 //   Sequences of about one length, decode kernels / walk.  With few the walk's chunks, side by side, win: W = 16, 100 tokens, per
-//   channel 102 / 24.  With many the decode kernels fill the GPU by themselves and are spared the prologue's trip through memory:
-//   per channel W = 256, 32 tokens 48 / 60, 64 tokens 78 / 75; W = 512, 64 tokens 106 / 118, 150 tokens 259 / 232; W = 1024, 100
-//   tokens 353 / 379, 150 tokens 512 / 471.  Per head W = 256, 64 tokens 59 / 67; W = 512, 100 tokens 136 / 178, 200 tokens
-//   253 / 277; W = 1024, 200 tokens 511 / 559.
+//   channel 94 / 17.  With many the decode kernels fill the GPU by themselves and are spared the prologue's trip through memory:
+//   per channel W = 256, 32 tokens 38 / 45, 64 tokens 75 / 55; W = 512, 64 tokens 95 / 95, 100 143 / 128, 150 218 / 159; W = 1024, 48
+//   tokens 165 / 172, 100 282 / 278, 150 460 / 344.  Per head W = 256, 32 tokens 34 / 41, 64 58 / 51; W = 512, 64 tokens 76 / 86, 100
+//   119 / 119, 200 202 / 176; W = 1024, 100 tokens 237 / 266, 150 308 / 328, 200 462 / 395.  (The lines were drawn for a walk of half
+//   the speed: between them and the crossings above, at W = 512 and 1024 per head from 120 and 170 tokens on, calls take the slower way.)
 //   Decoding sequences beside few long ones: a token costs the decode kernels about 1 us and the walk 0.06, a decoding sequence
-//   0.04 us per W and 0.13.  16 heads, all through the decode kernels / all through the walk / each its own way: per channel 60
-//   sequences beside a portion of 100 tokens 130 / 153 / 58, 250 beside 250 419 / 998 / 180; per head 60 beside 24 tokens
-//   70 / 134 / 81, 7 beside 100 87 / 46 / 52.
+//   0.03 us per W and 0.13.  16 heads, all through the decode kernels / all through the walk / each its own way: per channel 60
+//   sequences beside a portion of 24 tokens 55 / 126 / 46, of 100 128 / 128 / 50, 250 beside 24 141 / 635 / 140, beside 250
+//   392 / 645 / 148; per head 60 beside 24 tokens 74 / 118 / 79, 250 beside 24 264 / 612 / 279, 7 beside 100 81 / 29 / 42.
 inline int linear_at_most(bool per_channel, int64_t rows, int num_seqs, int max_query_len, int heads, int dim, int vdim) {
   constexpr int kShort = 16;
   if (max_query_len <= kShort) return max_query_len;
@@ -38,8 +39,8 @@ inline int linear_at_most(bool per_channel, int64_t rows, int num_seqs, int max_
 
 // A walk's sizes.  Few runs leave most of the GPU idle, and a long run's chunks are then worth cutting: into segments whose own
 // ends are worked out side by side, from nothing, and joined into the states that each segment truly starts from (one run of
-// 16000 tokens, 4 heads of 128: 870 us in one piece, 208 in 8).  As many as still leave every workgroup a
-// compute unit, of at least 16 chunks.
+// 16000 tokens, 4 heads of 128: 448 us in one piece, 381 in 2, 218 in 4, 138 in 8; of 2000 tokens 71, 64, and 51 in 3).  As many as
+// still leave every workgroup a compute unit, of at least 16 chunks.
 struct LinearWalkPlan {
   int at_most, segment;                 // segment: tokens of a segment; 0: runs are not cut
   int64_t runs, chunks, items;          // upper bounds: runs that walk, their chunks, their segments

@@ -28,8 +28,8 @@
 // under a condition; 45 and 78 here.  Of the walk's 1.0 us a chunk the products are 0.5 (38 of 32 cycles), the rest the exchange and
 // its barrier, and 37 KB of operands through the L1.  The prologue's time is the exponentials' (52 us with expf and divisions).
 // Relative error of the end states against 64 bits: 1.3e-7 here, 2.2e-7 in segments taken twice.
-// One run of 16000 tokens, 4 heads of 128, decays per channel / per head: 870 / 904 us in one piece, 208 / 205 in 8 segments (415 /
-// 300 in segments of 128 tokens); of 32000 tokens, 16 heads: 2202 and 1637 in 2.
+// One run of 16000 tokens, 4 heads of 128, decays per channel / per head: 448 / 468 us in one piece, 138 / 140 in 8 segments (415 /
+// 300 in segments of 128 tokens); of 32000 tokens, 16 heads: 1120 and 1015 in 2.
 #include "linear_walk.cuh"
 
 #include <type_traits>
@@ -56,10 +56,10 @@ __device__ __forceinline__ float reciprocal_of(float p) {
 }
 
 // log(sigmoid(x)) = min(x, 0) - log(1 + t), t = e^-|x|, the logarithm on the hardware's log2 with the rounding of 1 + t put back:
-// largest relative error over [-30, 30] 2.2e-7 (with log1pf 1.3e-7), root mean square 3.5e-8 (2.8e-8), a quarter of the instructions.
+// largest relative error over [-30, 30] 2.7e-7 (with log1pf 1.3e-7), root mean square 3.8e-8 (2.6e-8), a quarter of the instructions.
 // The results do not show it: over runs of 40 to 3000 tokens, 4 to 16 heads of 64 to 128, tau 1 to 16, outputs are 1.5 - 2.1e-7 and
-// end states 1.0 - 1.9e-7 from 64 bits with either (2.4 - 3.4e-7 and 1.2 - 2.8e-7 before this file); with log1pf the step above
-// takes 219 us instead of 204.
+// end states 1.0 - 1.9e-7 from 64 bits with either (2.4 - 3.4e-7 and 1.2 - 2.8e-7 before this file); with log1pf prologue and walk
+// of the step above take 128 us together instead of 111.
 __device__ __forceinline__ float log_sigmoid(float x) {
   const float t = exp_of_sum(-fabsf(x)), u = 1.0f + t;
   return fminf(x, 0.0f) - (0.69314718055994531f * __builtin_amdgcn_logf(u) + (t - (u - 1.0f)) * __builtin_amdgcn_rcpf(u));

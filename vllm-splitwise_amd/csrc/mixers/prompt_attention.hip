@@ -24,8 +24,8 @@
 // Workgroups are numbered latest tile of a sequence first: under a causal mask those have the longest walks.
 //
 // Measured, two prompts of 4324 tokens together, 16 query heads on 4 of size 128, capped scores and a gate: 989 us with the
-// fp32 instructions (39 TFLOP/s), 170 us one group a workgroup, 160 us two; one prompt of 1607, 8 heads on 2, no cap: 88.5 and 74.3 us;
-// two of 1296 behind 190 others: 117 and 90.  Error against 64 bits before the rounding to bf16: 1.3e-6 with the fp32
+// fp32 instructions (39 TFLOP/s), 177 us one group a workgroup, 162 us two; one prompt of 1607, 8 heads on 2, no cap: 88.7 and 69.2 us;
+// two of 1296 behind 190 tokens each, 16 on 4: 95.7 and 74.8.  Error against 64 bits before the rounding to bf16: 1.3e-6 with the fp32
 // instructions, 1.2e-6 here (without a cap 1.5 - 1.6e-7; 1.7 - 2.0e-7 with the small parts in a sum of their own).
 #include "prompt_attention.cuh"
 
