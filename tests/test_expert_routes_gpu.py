@@ -75,7 +75,7 @@ def test_expert_kernels_at_their_edges(rows, width, ff, experts, top, act, skew,
 
 
 @pytest.mark.parametrize("experts", [1, 7, 64, 65, 256])
-@pytest.mark.parametrize("pairs", [0, 1, 63, 8191, 8192, 8193, 20000])
+@pytest.mark.parametrize("pairs", [0, 1, 63, 1024, 1025, 2048, 2049, 8191, 8192, 8193, 20000])
 def test_pairs_in_groups(pairs, experts):
     """On both sides of the pairs that one turn of the workgroup's threads takes; experts that nobody asks for; all on one."""
     from splitwise_amd import _C

@@ -388,21 +388,24 @@ __global__ __launch_bounds__(256) void group_router_kernel(
 // inside an expert is whatever the LDS counters hand out: the experts' rows are independent, so it does not matter.
 // What bounds it is latency: a thread's choices are asked for together, and up to 8 a thread what the histogram's counters
 // returned is the pair's place in its expert, without a second round of counters.  7978 pairs, 32 experts: 8.5 us with a load and a
-// counter in turn, twice, and a sum in one thread; 7.4 us here, most of them the counters.
-constexpr int kPairThreads = 1024, kPairsOwn = 8;
+// counter in turn, twice, and a sum in one thread; 7.4 us here, most of them the counters.  Few pairs take a kernel of one or two
+// a thread: 244 pairs, 32 experts 2.95 us, 3.28 with eight (3.0 in turn); 32 experts' 2 pairs 2.9 and 3.3.
+constexpr int kPairThreads = 1024;
 
+// OWN: pairs of a thread at a time.
+template <int OWN>
 __global__ __launch_bounds__(kPairThreads) void group_pairs_kernel(int32_t* __restrict__ order,
                                                                    int32_t* __restrict__ expert_start,
                                                                    const int32_t* __restrict__ chosen, int64_t pairs,
                                                                    int experts) {
   __shared__ int count[kMaxRouterExperts];
   __shared__ int cursor[kMaxRouterExperts];
-  constexpr int64_t kBatch = (int64_t)kPairThreads * kPairsOwn;
+  constexpr int64_t kBatch = (int64_t)kPairThreads * OWN;
   const int tid = threadIdx.x;
-  int e[kPairsOwn], place[kPairsOwn];
+  int e[OWN], place[OWN];
   auto fetch = [&](int64_t base) {
 #pragma unroll
-    for (int i = 0; i < kPairsOwn; ++i) {
+    for (int i = 0; i < OWN; ++i) {
       const int64_t p = base + i * kPairThreads + tid;
       e[i] = p < pairs ? chosen[p] : -1;
     }
@@ -413,7 +416,7 @@ __global__ __launch_bounds__(kPairThreads) void group_pairs_kernel(int32_t* __re
   for (int64_t base = 0; base < pairs; base += kBatch) {
     if (base > 0) fetch(base);
 #pragma unroll
-    for (int i = 0; i < kPairsOwn; ++i)
+    for (int i = 0; i < OWN; ++i)
       if (e[i] >= 0) place[i] = atomicAdd(&count[e[i]], 1);
   }
   __syncthreads();
@@ -435,14 +438,14 @@ __global__ __launch_bounds__(kPairThreads) void group_pairs_kernel(int32_t* __re
   __syncthreads();
   if (pairs <= kBatch) {
 #pragma unroll
-    for (int i = 0; i < kPairsOwn; ++i)
+    for (int i = 0; i < OWN; ++i)
       if (e[i] >= 0) order[cursor[e[i]] + place[i]] = i * kPairThreads + tid;
     return;
   }
   for (int64_t base = 0; base < pairs; base += kBatch) {
     fetch(base);
 #pragma unroll
-    for (int i = 0; i < kPairsOwn; ++i)
+    for (int i = 0; i < OWN; ++i)
       if (e[i] >= 0) order[atomicAdd(&cursor[e[i]], 1)] = (int32_t)(base + i * kPairThreads + tid);
   }
 }
@@ -596,8 +599,9 @@ int swm_group_pairs(int32_t* order, int32_t* expert_start, const int32_t* chosen
   using namespace swm;
   SW_CHECK_ARG(experts > 0 && experts <= kMaxRouterExperts && pairs >= 0 && pairs < (1ll << 31),
                "group_pairs: %d experts (1..%d supported)", experts, kMaxRouterExperts);
-  hipLaunchKernelGGL(group_pairs_kernel, dim3(1), dim3(kPairThreads), 0, static_cast<hipStream_t>(stream), order,
-                     expert_start, chosen, pairs, experts);
+  auto kernel = pairs <= kPairThreads ? group_pairs_kernel<1> : pairs <= 2 * kPairThreads ? group_pairs_kernel<2> : group_pairs_kernel<8>;
+  hipLaunchKernelGGL(kernel, dim3(1), dim3(kPairThreads), 0,
+                     static_cast<hipStream_t>(stream), order, expert_start, chosen, pairs, experts);
   SW_CHECK_LAUNCH();
   return SW_OK;
 }
