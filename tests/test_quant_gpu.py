@@ -114,6 +114,32 @@ def test_gptq_gemm_64_row_tiles_in_chunks_of_512(m, k, n, group):
     test_gptq_gemm_shuffled(m, k, n, group)
 
 
+@pytest.mark.parametrize("m,k,n,group", [
+    # 32 x 128: as many stages as are asked for ahead; splits, a ragged last column tile
+    (24, 512, 93760, 128), (31, 5120, 9400, 32),
+    # 64 x 64: one stage; a split for each stage; splits that are not alike
+    (33, 256, 8, 32), (64, 768, 72, 64), (61, 2816, 328, 128), (100, 4096, 1000, 4096),
+    # 64 x 128: fewer stages than are asked for ahead, one more; splits
+    (33, 256, 16392, 32), (64, 512, 16520, 64), (128, 6912, 5128, 128), (193, 2560, 5064, 32),
+    # 128 x 128: the same
+    (65, 256, 16520, 32), (200, 768, 11008, 128), (250, 5376, 5128, 128), (129, 512, 16392, 32)])
+def test_gptq_gemm_streamed_tiles(m, k, n, group):
+    test_gptq_gemm_shuffled(m, k, n, group)
+
+
+@pytest.mark.parametrize("m", [20, 40, 100, 140])
+def test_gptq_gemm_takes_an_input_on_any_element(m):
+    from splitwise_amd import _C
+    k, n = 512, 136
+    qweight, qzeros, scales, _ = _gptq_case(k, n, 64, m)
+    a = np.random.default_rng(m).standard_normal((m, k)).astype(np.float16)
+    w = quant.gptq_shuffle(qweight)
+    off = torch.empty(m * k + 1, dtype=torch.float16, device="cuda")[1:].view(m, k)
+    off.copy_(_dev(a))
+    got = _C.ops.gptq_gemm(off, _dev(w), _dev(qzeros), _dev(scales), torch.empty((1, 1), device="meta"), True, 4)
+    _close(got, quant.gptq_gemm(a, w, qzeros, scales, None, True))
+
+
 def test_gptq_gemm_tile_kernel_on_seeded_random_shapes():
     """Shapes drawn at random inside the 128-row tile kernel's domain (rows 129..256, k in multiples of 256,
     columns in multiples of 8, groups of 64 / 128 / 256 / all of k), against the CPU restatement."""

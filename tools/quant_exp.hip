@@ -25,7 +25,7 @@ void set_error(const char* fmt, ...) {
     if (e_ != hipSuccess) { printf("HIP error %s at %d\n", hipGetErrorString(e_), __LINE__); exit(1); } \
   } while (0)
 
-struct Variant { const char* name; const char* waves; const char* tmt; const char* chunk; const char* ks; const char* t128 = "0"; };
+struct Variant { const char* name; const char* waves; const char* tmt; const char* chunk; const char* ks; const char* tile = "0"; };
 
 int main(int argc, char** argv) {
   const int M = argc > 1 ? atoi(argv[1]) : 256, N = argc > 2 ? atoi(argv[2]) : 13824, K = argc > 3 ? atoi(argv[3]) : 5120;
@@ -52,30 +52,31 @@ int main(int argc, char** argv) {
   hipEvent_t e0, e1; CK(hipEventCreate(&e0)); CK(hipEventCreate(&e1));
   std::vector<Variant> vars = {
       {"w8 mt2 c256 (shipped)", "8", "2", "256", nullptr},
-      {"t128 kq2 auto", "8", "2", "256", nullptr, "2"},
-      {"t128 kq2 ks1", "8", "2", "256", "1", "2"},
-      {"t128 kq2 ks2", "8", "2", "256", "2", "2"},
-      {"t128 kq2 ks3", "8", "2", "256", "3", "2"},
-      {"t128 kq2 ks4", "8", "2", "256", "4", "2"},
-      {"t128 kq4 auto", "8", "2", "256", nullptr, "4"},
-      {"t128 kq4 ks1", "8", "2", "256", "1", "4"},
-      {"t128 kq8 auto", "8", "2", "256", nullptr, "8"},
-      {"t128 kq8 ks1", "8", "2", "256", "1", "8"},
-      {"t64 kq8 auto", "8", "2", "256", nullptr, "68"},
-      {"t64 kq8 ks1", "8", "2", "256", "1", "68"},
-      {"t32 kq8 auto", "8", "2", "256", nullptr, "38"},
-      {"t32 kq8 ks1", "8", "2", "256", "1", "38"},
-      {"t32 kq8 ks2", "8", "2", "256", "2", "38"},
-      {"t256 kq2 auto", "8", "2", "256", nullptr, "82"},
-      {"t256 kq2 ks1", "8", "2", "256", "1", "82"},
-      {"t256 kq4cg1 ks1", "8", "2", "256", "1", "84"},
-      {"t256 kq4cg1 ks2", "8", "2", "256", "2", "84"},
-      {"t256 kq2 ks2", "8", "2", "256", "2", "82"},
-      {"t256 kq2 ks3", "8", "2", "256", "3", "82"},
-      {"t256 kq2 ks4", "8", "2", "256", "4", "82"},
-      {"t128 kq4 ks2", "8", "2", "256", "2", "4"},
-      {"t128 kq4 ks3", "8", "2", "256", "3", "4"},
-      {"t128 kq4 ks4", "8", "2", "256", "4", "4"},
+      {"32x128 auto", "8", "2", "256", nullptr, "1"},
+      {"32x128 ks1", "8", "2", "256", "1", "1"},
+      {"32x128 ks2", "8", "2", "256", "2", "1"},
+      {"32x128 ks3", "8", "2", "256", "3", "1"},
+      {"32x128 ks4", "8", "2", "256", "4", "1"},
+      {"64x64 auto", "8", "2", "256", nullptr, "2"},
+      {"64x64 ks1", "8", "2", "256", "1", "2"},
+      {"64x64 ks2", "8", "2", "256", "2", "2"},
+      {"64x64 ks3", "8", "2", "256", "3", "2"},
+      {"64x64 ks4", "8", "2", "256", "4", "2"},
+      {"64x128 auto", "8", "2", "256", nullptr, "3"},
+      {"64x128 ks1", "8", "2", "256", "1", "3"},
+      {"64x128 ks2", "8", "2", "256", "2", "3"},
+      {"64x128 ks3", "8", "2", "256", "3", "3"},
+      {"64x128 ks4", "8", "2", "256", "4", "3"},
+      {"128x128 auto", "8", "2", "256", nullptr, "4"},
+      {"128x128 ks1", "8", "2", "256", "1", "4"},
+      {"128x128 ks2", "8", "2", "256", "2", "4"},
+      {"128x128 ks3", "8", "2", "256", "3", "4"},
+      {"128x128 ks4", "8", "2", "256", "4", "4"},
+      {"128x256 auto", "8", "2", "256", nullptr, "5"},
+      {"128x256 ks1", "8", "2", "256", "1", "5"},
+      {"128x256 ks2", "8", "2", "256", "2", "5"},
+      {"128x256 ks3", "8", "2", "256", "3", "5"},
+      {"128x256 ks4", "8", "2", "256", "4", "5"},
       {"w8 mt2 ks1", "8", "2", "256", "1"},
       {"shipped path ks2", "8", "2", "256", "2"},
       {"shipped path ks3", "8", "2", "256", "3"},
@@ -87,7 +88,7 @@ int main(int argc, char** argv) {
     if (only && v != 0 && !strstr(vars[v].name, only)) continue;
     setenv("SW_QUANT_WAVES", vars[v].waves, 1); setenv("SW_QUANT_TMT", vars[v].tmt, 1);
     setenv("SW_QUANT_CHUNK", vars[v].chunk, 1);
-    setenv("SW_QUANT_T128", vars[v].t128, 1);
+    setenv("SW_QUANT_TILE", vars[v].tile, 1);
     if (vars[v].ks) setenv("SW_QUANT_KSPLIT", vars[v].ks, 1); else unsetenv("SW_QUANT_KSPLIT");
     CK(hipMemsetAsync(dc, 0, (size_t)M * N * 2, st));
     CK(hipMemsetAsync(ws, 0, 16384, st));

@@ -29,6 +29,7 @@
 //     launch, no atomics on data, bitwise reproducible results.
 #include "common.cuh"
 #include <stdlib.h>
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -73,9 +74,9 @@ struct GptqCol {
 
 __device__ __forceinline__ GptqCol gptq_col(uint32_t zero, uint16_t scale_bits) {
   GptqCol c;
-  const uint32_t zb = 0xe400u | zero;               // -(1024 + zero) for zero <= 16
+  const uint32_t zb = 0xe400u | zero, z16 = 0xd400u | (zero << 4);   // -(1024 + zero), -(64 + zero) for zero <= 16
   c.z1 = as_h2(zb | (zb << 16));
-  c.z16 = splat((_Float16)(-64 - (int)zero));
+  c.z16 = as_h2(z16 | (z16 << 16));
   c.s = as_h2((uint32_t)scale_bits | ((uint32_t)scale_bits << 16));
   return c;
 }
@@ -551,42 +552,34 @@ gptq_gemm_tiled_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ a,
                                  row_tile * col_tiles + col_tile, split, &s_last);
 }
 
-// Variant "128-row tiles" (rows of A in blocks of 128, groups that are multiples of the wave's k part): a workgroup
-// owns 128 rows x (8 / KQ) * 64 columns over its k range.  Its 8 waves are 8 / KQ column groups of 64 columns x KQ
-// k parts: in every chunk of KQ * SPW * 16 k of A (three buffers in LDS, one barrier per chunk) a wave multiplies its
-// SPW steps of 16 k, so one unpacked weight word feeds four matrix instructions, and the k parts meet once, through
-// LDS, at the end (the wave of k part q ends up with row blocks q * 4 / KQ ..).  The A pieces of chunk n+2 are
+// Variant "128 x 256 tiles" (groups that are multiples of 64): a workgroup owns 128 rows x 256 columns over its k range.  Its 8
+// waves are 4 column groups of 64 columns x 2 k parts: in every chunk of 128 k of A (three buffers in LDS, one barrier per
+// chunk) a wave multiplies its 4 steps of 16 k, so one unpacked weight word feeds four matrix instructions, and the k parts
+// meet once, through LDS, at the end (the wave of k part q ends up with row blocks 2 q and 2 q + 1).  The A pieces of chunk n+2 are
 // requested while chunk n is multiplied and written to LDS a whole chunk later; the weights run 8 steps ahead.  The
 // loop over a chunk has no branch in it: prefetches past the end of the k range re-read the last chunk instead.
 constexpr int kT128ARowPad = 16;                     // the pad keeps 16 rows on distinct bank groups
-template <int KQ, int SPW> constexpr int t128_chunk() { return KQ * SPW * 16; }
-template <int MT, int KQ, int SPW, int NBUF> constexpr int t128_lds() {
-  return NBUF * 32 * MT * (t128_chunk<KQ, SPW>() * 2 + kT128ARowPad);
-}
+constexpr int kT128Chunk = 128, kT128Lds = 3 * 128 * (kT128Chunk * 2 + kT128ARowPad);
 
-template <int MT, int KQ, int CG, int SPW, int NBUF>
-__global__ void __launch_bounds__(KQ * CG * 64)
+__global__ void __launch_bounds__(512)
 gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ a, const uint32_t* __restrict__ qweight,
                          const uint32_t* __restrict__ qzeros, const uint16_t* __restrict__ scales, int M, int N, int K,
                          int group_size, int ksplit, int col_tiles, int row_tiles, int zoff,
                          float* __restrict__ partials, int32_t* __restrict__ counters) {
+  constexpr int MT = 4, KQ = 2, CG = 4, SPW = 4;      // row blocks of 32; k parts, column groups; steps of a wave and chunk
   constexpr int CP = 2;                               // columns per lane
   constexpr int NT = KQ * CG * 64;                    // threads
   constexpr int BM = 32 * MT;                         // rows of A per workgroup
   constexpr int BPO = MT / KQ;                        // row blocks a wave keeps at the end
   constexpr int RD = 8 / SPW;                         // chunks of weights in flight (8 steps)
-  constexpr int CHUNK = t128_chunk<KQ, SPW>();
+  constexpr int CHUNK = kT128Chunk;
   constexpr int AROW = CHUNK * 2 + kT128ARowPad;      // LDS bytes per A row
   constexpr int ABUF = BM * AROW;
   constexpr int SEGS = CHUNK / 8;                     // 16-byte pieces per A row
   constexpr int PPT = BM * SEGS / NT;                 // pieces per thread and chunk
   constexpr int PH = PPT / 2;                         // moved in two halves, at the top and in the middle of a chunk
-  constexpr bool kAllK = KQ > MT;                     // more k parts than row blocks: the parts meet as in the k-waves kernel
-  static_assert(PPT % 2 == 0 && (BPO >= 1 || (kAllK && CG == 1 && KQ == 8)), "tile shape");
-  static_assert(kAllK || KQ * CG * 32 * 64 * 4 <= NBUF * ABUF,
+  static_assert(KQ * SPW * 16 == CHUNK && KQ * CG * 32 * 64 * 4 <= kT128Lds,
                 "the A buffers must hold one 32-register block per wave at the end");
-  static_assert(!kAllK || 8 * MT * CP * 8 * 64 * 4 <= NBUF * ABUF,
-                "the A buffers must hold 8 accumulator rows of every wave at the end");
   extern __shared__ __attribute__((aligned(16))) char a_lds[];
   __shared__ int s_last;
   const int tid = threadIdx.x;
@@ -619,8 +612,7 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
   const DequantRegs dq = dequant_regs();
 
   // ---- A staging: 128 rows x SEGS pieces of 16 bytes per chunk, PPT per thread in two halves
-  constexpr int SETS = NBUF == 3 ? 2 : 1;             // register sets for pieces in flight
-  u32x4 a_stage[SETS][PH];
+  u32x4 a_stage[2][PH];
   auto a_fetch = [&](auto HALF, int chunk) {
     constexpr int hf = decltype(HALF)::value;
     const int ch = min(chunk, c_end - 1);
@@ -628,7 +620,7 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
       constexpr int qi = decltype(Q)::value;
       const int p = tid + (hf * PH + qi) * NT;
       const int row = p / SEGS, seg = p % SEGS;
-      a_stage[hf % SETS][qi] =
+      a_stage[hf][qi] =
           *reinterpret_cast<const u32x4*>(a + (size_t)min(m0 + row, M - 1) * K + ch * CHUNK + seg * 8);
     });
   };
@@ -638,7 +630,7 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
       constexpr int qi = decltype(Q)::value;
       const int p = tid + (hf * PH + qi) * NT;
       const int row = p / SEGS, seg = p % SEGS;
-      *reinterpret_cast<u32x4*>(a_lds + buf_off + row * AROW + seg * 16) = a_stage[hf % SETS][qi];
+      *reinterpret_cast<u32x4*>(a_lds + buf_off + row * AROW + seg * 16) = a_stage[hf][qi];
     });
   };
 
@@ -665,19 +657,11 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
   // of half step h, so the matrix pipe never waits for the vector pipe inside a chunk.
   auto body = [&](auto SLOT, int chunk, int buf_cur, int buf_next) {
     constexpr int slot = decltype(SLOT)::value;
-    // Three buffers: the pieces of chunk + 2 are requested while those of chunk + 1, requested a chunk ago, go into
-    // buf_next (nobody reads it any more after this barrier).  Two buffers: a thread holds one half of a chunk at a
-    // time, so a half is written half a chunk after it was requested.
-    if constexpr (MT > 4) {                              // 256 accumulator registers: keep them in the AGPR half
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int cc = 0; cc < CP; ++cc) asm volatile("" : "+a"(acc[t][cc]));
-    }
-    if constexpr (NBUF == 2) a_commit(H1{}, buf_cur * ABUF);
+    // The pieces of chunk + 2 are requested while those of chunk + 1, requested a chunk ago, go into buf_next (nobody
+    // reads it any more after this barrier).
     __syncthreads();
-    if constexpr (NBUF == 3) a_commit(H0{}, buf_next * ABUF);
-    a_fetch(H0{}, chunk + (NBUF == 3 ? 2 : 1));
+    a_commit(H0{}, buf_next * ABUF);
+    a_fetch(H0{}, chunk + 2);
     const uint32_t z = zq[slot] >> zshift;
     GptqCol col[CP];
     col[0] = gptq_col((z & 0xfu) + zoff, (uint16_t)(sq[slot] & 0xffffu));
@@ -706,7 +690,7 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
       for (int t = 0; t < MT; ++t)
         acc[t][cc] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i & 1][t], b_cur, acc[t][cc], 0, 0, 0);
       // 0x8 matrix, 0x2 vector ALU, 0x100 LDS read, 0x20 memory read
-      constexpr int VPM = MT >= 8 ? 2 : 4;              // vector instructions placed after each matrix instruction
+      constexpr int VPM = 4;              // vector instructions placed after each matrix instruction
       if constexpr (cc == 0) {
         static_for<MT>([&](auto) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -722,9 +706,8 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
       }
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (h == SPW - 1) {                     // mid chunk: the second half of chunk + 1 goes in, the second
-        if constexpr (NBUF == 3) a_commit(H1{}, buf_next * ABUF);
-        else a_commit(H0{}, buf_next * ABUF);
-        a_fetch(H1{}, chunk + (NBUF == 3 ? 2 : 1));
+        a_commit(H1{}, buf_next * ABUF);
+        a_fetch(H1{}, chunk + 2);
         __builtin_amdgcn_sched_barrier(0);
       }
     });
@@ -735,24 +718,18 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
       static_for<SPW>([&](auto STEP) { w_load(SLOT, STEP, c_begin + decltype(SLOT)::value); });
       g_load(SLOT, c_begin + decltype(SLOT)::value);
     });
-    if constexpr (NBUF == 3) {
-      a_fetch(H0{}, c_begin);
-      a_fetch(H1{}, c_begin);
-      a_commit(H0{}, 0);
-      a_commit(H1{}, 0);
-      a_fetch(H0{}, c_begin + 1);
-      a_fetch(H1{}, c_begin + 1);
-    } else {
-      a_fetch(H0{}, c_begin);
-      a_commit(H0{}, 0);
-      a_fetch(H1{}, c_begin);
-    }
+    a_fetch(H0{}, c_begin);
+    a_fetch(H1{}, c_begin);
+    a_commit(H0{}, 0);
+    a_commit(H1{}, 0);
+    a_fetch(H0{}, c_begin + 1);
+    a_fetch(H1{}, c_begin + 1);
     int buf = 0;
     for (int chunk = c_begin; chunk < c_end; chunk += RD) {
       static_for<RD>([&](auto SLOT) {
         constexpr int u = decltype(SLOT)::value;
         if (u == 0 || chunk + u < c_end) {
-          const int nxt = buf == NBUF - 1 ? 0 : buf + 1;
+          const int nxt = buf == 2 ? 0 : buf + 1;
           body(SLOT, chunk + u, buf, nxt);
           buf = nxt;
         }
@@ -760,40 +737,6 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
     }
   }
 
-  if constexpr (kAllK) {
-    // ---- 8 k parts, one column group: the parts meet as in the k-waves kernel -- two passes of 8 accumulator rows
-    // through LDS, after which wave w owns accumulator row 8 * pass + w of every row block.
-    float* red = reinterpret_cast<float*>(a_lds);
-    float vals[2 * MT][CP];
-#pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-      __syncthreads();
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int cc = 0; cc < CP; ++cc)
-#pragma unroll
-          for (int r8 = 0; r8 < 8; ++r8)
-            red[(((wave * MT + t) * CP + cc) * 8 + r8) * 64 + lane] = acc[t][cc][8 * pass + r8];
-      __syncthreads();
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int cc = 0; cc < CP; ++cc) {
-          float v = 0.f;
-#pragma unroll
-          for (int w = 0; w < 8; ++w) v += red[(((w * MT + t) * CP + cc) * 8 + wave) * 64 + lane];
-          vals[pass * MT + t][cc] = v;
-        }
-    }
-    auto row_of = [&](int i) {                            // i = pass * MT + t, accumulator row r = 8 * pass + wave
-      const int pass = i / MT, t = i % MT;
-      return m0 + 32 * t + 16 * pass + 8 * (wave >> 2) + 4 * half + (wave & 3);
-    };
-    auto val_of = [&](int i, int cc) { return vals[i][cc]; };
-    combine_and_store<CP, 2 * MT>(val_of, row_of, col_ok, ncol, c, M, N, ksplit, partials, counters,
-                                  row_tile * col_tiles + col_tile, split, &s_last);
-  } else {
   // ---- the k parts meet: the wave of k part q keeps row blocks q * BPO .. + BPO - 1 and is sent the other parts'
   // sums of them through LDS, one block per pass.
   // (selects between VALUES of fixed accumulator elements: a branch or a conditional expression between two
@@ -837,8 +780,227 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
     return v;
   };
   combine_and_store<CP, 16 * BPO>(val_of, row_of, col_ok, ncol, c, M, N, ksplit, partials, counters,
-                                  row_tile * col_tiles + col_tile, split, &s_last);
+                                 row_tile * col_tiles + col_tile, split, &s_last);
+}
+
+// Variant "streamed" (k in multiples of 256): a workgroup owns 32 * MT rows x 64 * CG columns over its k range; its 8 waves are CG
+// column groups of 64 x 8 / CG k parts.  A stage is 32 k of every part.  Its A goes straight from memory to LDS, its weights, scales
+// and zeros into the waves' registers, all of it R stages ahead: what is left between two stages is one wait for the wave's OWN
+// loads (counted, so that the newer ones stay in flight) and one barrier.  What bounds it: at 61 rows a stage of 64 x 64 x 256 takes
+// 0.95 us of which the vector units work a third (unpacking) and the matrix cores a quarter; A is read from the L2 once per column
+// tile.  Against tiles whose A went through registers and was written to LDS a chunk later (61 rows, both matrices of 5120 rows
+// and both of 5120 columns of a 13B layer): 24.4 -> 20.1 us, 14.1 -> 13.1, 43.7 -> 28.0, 23.3 -> 20.3.
+//
+// The waits count this wave's loads, so nothing may move past them: the pointers are not __restrict__ (a load of memory that nothing
+// else writes could be moved behind a wait, which then would not wait for the A before it), the loop has no way around it,
+// and sched_barriers keep the order inside a block.
+template <int CG> constexpr int stage_k() { return 256 / CG; }              // 32 k for each of the 8 / CG k parts
+template <int MT, int CG, int R> constexpr int stream_lds() {
+  constexpr int ring = R * MT * 64 * stage_k<CG>(), red = (MT > 2 || CG == 1 ? 2 : 1) * 65536;
+  return ring > red ? ring : red;
+}
+template <int N> __device__ __forceinline__ void wait_loads() {     // all but the N newest
+  static_assert(N < 64, "vmcnt has 6 bits");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0x7fffffff, 0x00020000);
+}
+// from memory to LDS, past the registers: lane l's 16 bytes go to `to` + 16 l
+__device__ __forceinline__ void lds_fetch16(__amdgpu_buffer_rsrc_t from, uint32_t offset, char* to) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)to, 16, offset, 0, 0, 0);
+}
+
+template <int MT, int CG, int R, int PER_SIMD>
+__global__ void __launch_bounds__(512, PER_SIMD)
+gptq_gemm_stream_kernel(uint16_t* c, const uint16_t* a, const uint32_t* qweight,
+                        const uint32_t* qzeros, const uint16_t* scales, int M, int N, int K, int group_size, int ksplit,
+                        int col_tiles, int row_tiles, int zoff, float* partials, int32_t* counters) {
+  constexpr int SK = stage_k<CG>(), ROW = 2 * SK;      // k of a stage; its bytes of a row of A
+  constexpr int KP = 8 / CG, KD = SK / 32 / KP;       // k parts; pairs of 16-k steps of a part in a stage
+  constexpr int AQ = MT * SK / 128, STAGE = 32 * MT * ROW, LOADS = AQ + 2 * KD + 2;        // of a wave and stage: A, weights, scales and zeros
+  extern __shared__ __attribute__((aligned(16))) char ring[];
+  __shared__ int s_last;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cg = wave % CG, kp = wave / CG;
+  const int j = lane & 31, half = lane >> 5;
+  // workgroup order as in the tiled kernel: the k splits and row tiles of a column tile share an XCD
+  const int total = col_tiles * row_tiles * ksplit;
+  const int per_xcd = (total + 7) / 8;
+  const int work = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (work >= total) return;
+  const int split = work % ksplit;
+  const int row_tile = (work / ksplit) % row_tiles;
+  const int col_tile = work / (ksplit * row_tiles);
+  const int n0 = col_tile * 64 * CG, ncol = n0 + 64 * cg + 2 * j;
+  const bool col_ok = ncol < N;
+  const int m0 = row_tile * 32 * MT;
+  const int stages = K / SK;
+  const int s_begin = stages * split / ksplit, n = stages * (split + 1) / ksplit - s_begin;
+
+  f32x16 acc[MT][2];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[t][cc][r] = 0.f;
+  const DequantRegs dq = dequant_regs();
+
+  // ---- this wave's loads of a stage.  A: 4 rows x 256 bytes a load, the 16-byte pieces of a row in the order piece ^ (row % 16): the
+  // fragments (one piece of 32 rows) come from distinct banks.
+  uint32_t a_off[AQ];
+#pragma unroll
+  for (int q = 0; q < AQ; ++q) {
+    const int at = (wave * AQ + q) * 1024 + lane * 16, row = at / ROW;
+    a_off[q] = (uint32_t)(min(row, M - 1 - m0) * K + 8 * ((at % ROW / 16) ^ (row & 15))) * 2u;
   }
+  const int ncl = min(ncol, N - 2);
+  uint32_t w_off[2];                                  // word row 2 half + i of a pair of steps, this lane's two columns
+#pragma unroll
+  for (int i = 0; i < 2; ++i) w_off[i] = (uint32_t)((4 * KD * kp + 2 * half + i) * N + ncl - n0) * 4u;
+  const uint16_t* a_at = a + (size_t)m0 * K + (size_t)s_begin * SK;
+  const uint32_t* w_at = qweight + (size_t)s_begin * (SK / 8) * N + n0;
+  const uint32_t s_off = (uint32_t)(ncl)*2u, z_off = (uint32_t)(ncl / 8) * 4u;
+  int ahead = 0;                                      // stages asked for
+  // Behind the last stage the loads are still asked for, of one address: what is in flight is the same number everywhere.
+  auto issue_a = [&](auto SLOT) {
+    const auto r = buffer_of(ahead < n ? a_at : a);
+    const uint32_t there = ahead < n ? ~0u : 0u;
+#pragma unroll
+    for (int q = 0; q < AQ; ++q)
+      lds_fetch16(r, a_off[q] & there, ring + decltype(SLOT)::value * STAGE + (wave * AQ + q) * 1024);
+    a_at += SK;
+  };
+  u32x2 w[R][2 * KD];
+  uint32_t z[R], sc[R];
+  auto issue_w = [&](auto SLOT) {
+    constexpr int slot = decltype(SLOT)::value;
+    const auto r = buffer_of(ahead < n ? w_at : qweight);
+    const uint32_t there = ahead < n ? ~0u : 0u;
+#pragma unroll
+    for (int x = 0; x < 2 * KD; ++x)
+      w[slot][x] = __builtin_amdgcn_raw_buffer_load_b64(r, w_off[x % 2] & there, ((x / 2) * 16 * N) & there, 0);
+    const uint32_t g = (uint32_t)((s_begin + min(ahead, n - 1)) * SK + kp * (32 * KD)) / (uint32_t)group_size;
+    z[slot] = __builtin_amdgcn_raw_buffer_load_b32(buffer_of(qzeros + (size_t)g * (N / 8)), z_off, 0, 0);
+    sc[slot] = __builtin_amdgcn_raw_buffer_load_b32(buffer_of(scales + (size_t)g * N), s_off, 0, 0);
+    w_at += (size_t)(SK / 8) * N;
+    ++ahead;
+  };
+  int a_piece[2 * KD];                                // this lane's fragments of a stage: row j, piece 4 (KD kp + d) + 2 half + i
+#pragma unroll
+  for (int x = 0; x < 2 * KD; ++x) a_piece[x] = j * ROW + ((4 * (KD * kp + x / 2) + 2 * half + x % 2) ^ (j & 15)) * 16;
+  // A stage is multiplied in two halves of KD steps of 16 k.  Between them the wave has read out the stage's A, waits for the next one's
+  // and meets the others, whereupon the place takes the loads of a later stage, and the next stage's first half is read while the
+  // matrix cores work on the second half of this one.
+  struct Half { f16x8 a[KD][MT]; };
+  auto read = [&](Half& h, auto SLOT, auto SECOND) {
+    constexpr int x0 = decltype(SECOND)::value * KD;
+#pragma unroll
+    for (int y = 0; y < KD; ++y)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        h.a[y][t] = *reinterpret_cast<const f16x8*>(ring + decltype(SLOT)::value * STAGE + t * 32 * ROW + a_piece[x0 + y]);
+  };
+  // a product's weights are unpacked while the one before is on the matrix cores
+  auto multiply = [&](const Half& h, const u32x2* w, const GptqCol (&col)[2]) {
+    f16x8 next = gptq_dequant8(w[0].x, col[0], dq);
+#pragma unroll
+    for (int x = 0; x < 2 * KD; ++x) {
+      const f16x8 b = next;
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[t][x % 2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(h.a[x / 2][t], b, acc[t][x % 2], 0, 0, 0);
+      if (x + 1 < 2 * KD) next = gptq_dequant8((x + 1) % 2 ? w[(x + 1) / 2].y : w[(x + 1) / 2].x, col[(x + 1) % 2], dq);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  using First = std::integral_constant<int, 0>;
+  using Second = std::integral_constant<int, 1>;
+  auto arrived = [&]() {                              // the next stage's A is in LDS, for all waves
+    wait_loads<(R - 1) * LOADS - AQ>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  Half first, second;
+  const int zshift = 4 * (ncl & 7);
+  // (what has been asked for is counted: the order of the loads stays as written)
+  static_for<R - 1>([&](auto SLOT) {
+    issue_a(SLOT);
+    __builtin_amdgcn_sched_barrier(0);
+    issue_w(SLOT);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  issue_a(std::integral_constant<int, R - 1>{});
+  wait_loads<(R - 1) * LOADS>();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  issue_w(std::integral_constant<int, R - 1>{});
+  __builtin_amdgcn_sched_barrier(0);
+  read(first, std::integral_constant<int, 0>{}, First{});
+  int s = 0;
+#pragma unroll 1
+  do {                                                // (n >= 1)
+    static_for<R>([&](auto SLOT) {
+      constexpr int slot = decltype(SLOT)::value;
+      const bool more = slot == 0 || s + slot < n;    // (a stage behind the last is gone through without its products)
+      read(second, SLOT, Second{});
+      GptqCol col[2];
+      col[0] = gptq_col(((z[slot] >> zshift) & 0xfu) + zoff, (uint16_t)(sc[slot] & 0xffffu));
+      col[1] = gptq_col(((z[slot] >> (zshift + 4)) & 0xfu) + zoff, (uint16_t)(sc[slot] >> 16));
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) multiply(first, w[slot], col);
+      arrived();
+      issue_a(SLOT);
+      read(first, std::integral_constant<int, (slot + 1) % R>{}, First{});
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) multiply(second, w[slot] + KD, col);
+      issue_w(SLOT);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    s += R;
+  } while (s < n);
+  wait_loads<0>();
+
+  // ---- the k parts meet in LDS, two row blocks at a time: of the pairs of quads (block t, rows 8 q + 4 half .. + 3, both columns)
+  // part kp adds up those with (4 t + q) % KP == kp, in the order of the parts
+  constexpr int TP = MT > 2 || CG == 1 ? 2 : 1, OWN = 4 * TP / KP;           // row blocks of a pass; pairs of quads of a wave
+  using f32x4v = __attribute__((ext_vector_type(4))) float;
+  f32x4v* red = reinterpret_cast<f32x4v*>(ring);
+  f32x4v vals[MT / TP][OWN][2];
+#pragma unroll
+  for (int pass = 0; pass < MT / TP; ++pass) {
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < TP; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc) {
+          const f32x16& v = acc[pass * TP + t][cc];
+          red[((wave * TP + t) * 8 + q * 2 + cc) * 64 + lane] = f32x4v{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+        }
+    __syncthreads();
+#pragma unroll
+    for (int o = 0; o < OWN; ++o)
+#pragma unroll
+      for (int cc = 0; cc < 2; ++cc) {
+        f32x4v v = red[(cg * TP * 8 + (o * KP + kp) * 2 + cc) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < KP; ++w) v += red[((w * CG + cg) * TP * 8 + (o * KP + kp) * 2 + cc) * 64 + lane];
+        vals[pass][o][cc] = v;
+      }
+  }
+  auto row_of = [&](int i) {
+    const int p = (i / 4 % OWN) * KP + kp;
+    return m0 + 32 * (i / 4 / OWN * TP) + 8 * p + 4 * half + i % 4;            // (a pass's quads are 8 rows apart)
+  };
+  auto val_of = [&](int i, int cc) { return vals[i / 4 / OWN][i / 4 % OWN][cc][i % 4]; };
+  combine_and_store<2, 4 * OWN * (MT / TP)>(val_of, row_of, col_ok, ncol, c, M, N, ksplit, partials, counters,
+                                            row_tile * col_tiles + col_tile, split, &s_last);
 }
 
 // ------------------------------------------------------------------ GPTQ, plain (unshuffled) weights + g_idx
@@ -1289,6 +1451,44 @@ int pick_ksplit(int tiles, int units, int min_units, int M, int N, int64_t works
   return ks < 1 ? 1 : ks;
 }
 
+// Which tiles the streamed kernel takes, rows x columns.  A launch is one round of at most 256 workgroups where the tiles allow it; k
+// is split as often as that leaves room for.  Measured in microseconds at the matrices of 7B and 13B layers, whole and halved:
+enum class StreamTile { kNone, k32x128, k64x64, k64x128, k128x128 };
+StreamTile stream_tile(int64_t M, int64_t N, int64_t K) {
+  auto tiles = [&](int rows, int cols) { return ((M + rows - 1) / rows) * ((N + cols - 1) / cols); };
+  if (M <= 32) {
+    // k across waves reads A from memory: the more rows and weights, the sooner the streamed tile is ahead (32 rows: 13824 k x 5120
+    // 20.5 with k across waves / 18.8 streamed, 12288 x 4096 16.0 / 14.2, 5120 x 5120 12.1 / 12.4; 24 rows: 18.2 / 18.4,
+    // 14.3 / 14.2; 17 rows: 15360 x 5120 17.0 / 16.8, 12288 x 4096 13.3 / 14.1; 12 rows: 22016 x 4096 21.6 / 19.8, 15360 x 5120
+    // 16.2 / 16.8; 8 rows: 27648 x 5120 25.2 / 24.9)
+    const int64_t from = M >= 24 ? 48000000 : M > 16 ? 78000000 : M > 8 ? 90000000 : INT64_MAX;
+    return N * K >= from ? StreamTile::k32x128 : StreamTile::kNone;
+  }
+  if (tiles(64, 64) <= 256) {
+    // up to 64 rows always (128 columns instead: 13.1 -> 14.7 at 5120 x 5120, 20.3 -> 21.3 at 13824 x 5120); with more rows where the
+    // splits fill the chip or k is short (100 rows: 7680 x 5120 18.6, 64 x 128 19.8; 6912 k x 5120 21.0 / 19.0)
+    const int64_t t = tiles(64, 64), filled = 256 / t * t;
+    if (M <= 64 || K <= 5120 || filled >= 224) return StreamTile::k64x64;
+  }
+  if (M <= 64) return StreamTile::k64x128;            // 27648 x 5120 28.9, 64 x 64 in two rounds 36.3
+  const int64_t t128 = tiles(128, 128);
+  // 27648 columns 42.2, 64 x 128 50.3; 15360 columns 30.0 / 30.6; 12288 24.2 / 24.0
+  if (M <= 128) return t128 > 128 ? StreamTile::k128x128 : StreamTile::k64x128;
+  if (t128 > 256) return StreamTile::kNone;
+  // 192 rows: 11008 k x 4096 32.4 (96 tiles, 2 splits), 128 x 128 35.1; 256 rows: 13824 k x 5120 65.5 (160 tiles) / 45.5, but 2560 k 16.2 / 21.7
+  const int64_t t = tiles(64, 128), filled = t <= 256 ? 256 / t * t : 0;
+  return t <= 256 && (K <= 4096 || filled >= 180) ? StreamTile::k64x128 : StreamTile::k128x128;
+}
+int stream_splits(int64_t tiles, int stages, int M, int N, int64_t workspace_bytes, int forced) {
+  if (tiles > kCounterInts) return 1;
+  int64_t ks = forced > 0 ? forced : 256 / tiles;
+  if (ks > stages) ks = stages;
+  const int64_t per_split = (int64_t)M * N * 4;
+  ks = std::min(ks, (workspace_bytes - kCounterBytes) / per_split);
+  ks = std::min(ks, ((int64_t)1 << 31) / per_split);  // 32-bit buffer offsets
+  return ks < 1 ? 1 : (int)ks;
+}
+
 }  // namespace
 }  // namespace sw
 
@@ -1416,34 +1616,18 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
     ap = a_perm;
   }
   float* partials = reinterpret_cast<float*>(ws + kCounterBytes);
-  // Kernel choice, from measurements on the 13B / TP2 matrices (tools/quant_exp.hip):
-  //   * up to 32 rows: one row tile per workgroup, k split across its waves, A straight from memory;
-  //   * tile kernels (A through LDS; they need k in multiples of 256 and groups in multiples of 64):
-  //       33..64 rows    64 x 64 tiles, the 8 waves are 8 k parts of every chunk; chunks of 512 k where k is a multiple of
-  //                      that and can be split as often (half the barriers: 61 rows x 5120 x 15360 25.3 -> 23.1 us,
-  //                      x 27648 44.0 -> 40.4, 13824 x 5120 25.2 -> 23.4; 5120 x 5120, in 2 splits instead of 3, 15.1 -> 15.4);
-  //       65..128 rows   128 x 64 tiles of the same form -- a 13824-column matrix is 216 of them, so k is not split
-  //                      across workgroups and no fp32 partial tile goes through memory; with a short k (<= 3072) and
-  //                      few columns two 64-row tiles per column tile, k unsplit, are faster than 128-row tiles whose
-  //                      k is split three ways;
-  //       129.. rows     128 x 128 tiles (2 column groups x 4 k parts), 128 x 256 when that keeps the launch to one
-  //                      round of workgroups (the 27648-column matrix of an unsharded 13B model at 256 rows);
-  //   * shapes the tile kernels do not take: k across waves up to 128 rows, the 64-row tiled kernel above.
+  // Kernel choice: streamed tiles where stream_tile() names one (k in multiples of 256, A on 16 bytes); above 128 rows and past
+  // 256 tiles of 128 x 128, tiles of 128 x 256, which are one round of workgroups (27648 columns at 256 rows: 79 us against 87);
+  // up to 32 rows otherwise one row tile per workgroup, k split across its waves, A straight from memory; every other shape k
+  // across waves up to 128 rows, the 64-row tiled kernel above.
   int cp = 2, mt = M > 64 ? 4 : M > 32 ? 2 : 1;
   bool tiled = M > 128 && K % kChunkK == 0 && group_size % 16 == 0;
   int waves = 8, chunk = kChunkK, tiled_mt = 2, force_ks = 0;
-  int t_variant = 0;
-  if (K % 256 == 0 && group_size % 64 == 0) {
-    if (M > 128) {
-      t_variant = (int64_t)((M + 127) / 128) * ((N + 127) / 128) > 256 ? 2 : 4;
-      // a short k and few columns (13B / TP2 o_proj: 22.5 -> 19.5 us at 256 rows): 128 x 64 tiles, k unsplit
-      if (K <= 3072 && (int64_t)((M + 127) / 128) * ((N + 63) / 64) <= 256) { t_variant = 8; force_ks = 1; }
-    } else if (M > 64) {
-      t_variant = 8;
-      if (K <= 3072 && 2 * ((N + 63) / 64) <= 256) { t_variant = 68; force_ks = 1; }
-    } else if (M > 32) {
-      t_variant = 68;
-    }
+  StreamTile stream_to = StreamTile::kNone;
+  bool wide = false;                                  // 128 x 256 tiles
+  if (K % 256 == 0 && reinterpret_cast<uintptr_t>(ap) % 16 == 0) {
+    stream_to = stream_tile(M, N, K);
+    wide = stream_to == StreamTile::kNone && M > 128 && group_size % 64 == 0;
   }
 #ifdef SW_QUANT_EXPERIMENT                                     // tuning builds only: never in the shipped library
   if (const char* env = getenv("SW_QUANT_CP")) cp = atoi(env) == 4 ? 4 : 2;
@@ -1453,52 +1637,46 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
   if (const char* env = getenv("SW_QUANT_CHUNK")) chunk = atoi(env) == 128 ? 128 : 256;
   if (const char* env = getenv("SW_QUANT_TMT")) tiled_mt = atoi(env);
   if (const char* env = getenv("SW_QUANT_KSPLIT")) force_ks = atoi(env);
-  // 0: off; 2, 4, 8: 128 rows x 8 waves with 2 / 4 / 8 k parts; 68: 64 rows, 8 k parts; 82, 84: 256 rows x 4 waves
-  if (const char* env = getenv("SW_QUANT_T128")) t_variant = atoi(env);
+  // 0: off; 1..4: the StreamTile; 5: 128 x 256
+  if (const char* env = getenv("SW_QUANT_TILE")) {
+    const int t = atoi(env);
+    stream_to = t >= 1 && t <= 4 && K % 256 == 0 ? static_cast<StreamTile>(t) : StreamTile::kNone;
+    wide = t == 5 && K % 256 == 0 && group_size % 64 == 0;
+  }
 #endif
   if (mt == 3 || mt > 4) mt = 4;
   if (tiled) mt = tiled_mt;
-  if (t_variant != 0) {
-    // variant -> rows per tile, k parts, column groups of 64, k per chunk
-    int t_rows = 128, t_kq = 4, t_cg = 2, chunk_k = 256;
-    switch (t_variant) {
-      case 4: break;
-      case 2: t_kq = 2; t_cg = 4; chunk_k = 128; break;
-      case 8: t_kq = 8; t_cg = 1; break;
-      case 68:
-      case 70: t_rows = 64; t_kq = 8; t_cg = 1; break;
-      case 38: t_rows = 32; t_kq = 8; t_cg = 1; break;
-      case 82: t_rows = 256; t_kq = 2; t_cg = 2; chunk_k = 128; break;
-      case 84: t_rows = 256; t_kq = 4; t_cg = 1; chunk_k = 128; break;
-      default: SW_CHECK_ARG(false, "gptq_gemm: no 128-row tile variant %d", t_variant);
-    }
-    SW_CHECK_ARG(K % 256 == 0 && group_size % 64 == 0,
-                 "gptq_gemm: no 128-row tile variant %d for K=%d, group size %d", t_variant, K, group_size);
-    const int rt = (M + t_rows - 1) / t_rows, ct = (N + 64 * t_cg - 1) / (64 * t_cg);
-    int ks = pick_ksplit(ct * rt, K / chunk_k, 4, M, N, avail, 1, 256);
-    if (t_variant == 68 && M <= 64 && K % 512 == 0 && pick_ksplit(ct * rt, K / 512, 4, M, N, avail, 1, 256) == ks) t_variant = 70;
-    if (force_ks > 0 && force_ks <= K / chunk_k) ks = force_ks;
-#define SW_GPTQ_T128(MT_, KQ_, CG_, SPW_, NB_)                                                                 \
+  if (stream_to != StreamTile::kNone) {
+#define SW_GPTQ_STREAM(MT_, CG_, R_, PER_SIMD_)                                                                  \
   do {                                                                                                           \
-    auto kern = gptq_gemm_tile128_kernel<MT_, KQ_, CG_, SPW_, NB_>;                                              \
-    constexpr int lds_bytes = t128_lds<MT_, KQ_, SPW_, NB_>();                                                   \
+    auto kern = gptq_gemm_stream_kernel<MT_, CG_, R_, PER_SIMD_>;                                                \
+    constexpr int lds_bytes = stream_lds<MT_, CG_, R_>();                                                        \
     SW_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, \
                                      lds_bytes));                                                                \
-    hipLaunchKernelGGL(kern, dim3((ct * rt * ks + 7) / 8 * 8), dim3(KQ_ * CG_ * 64), lds_bytes, st, out, ap,     \
-                       qweight, qzeros, sp, M, N, K, group_size, ks, ct, rt, zoff, partials, counters);          \
+    const int rt = (M + 32 * MT_ - 1) / (32 * MT_), ct = (N + 64 * CG_ - 1) / (64 * CG_);                        \
+    const int ks = stream_splits((int64_t)rt * ct, K / stage_k<CG_>(), M, N, avail, force_ks);                   \
+    hipLaunchKernelGGL(kern, dim3((ct * rt * ks + 7) / 8 * 8), dim3(512), lds_bytes, st, out, ap, qweight,       \
+                       qzeros, sp, M, N, K, group_size, ks, ct, rt, zoff, partials, counters);                   \
   } while (0)
-    if (t_variant == 4) SW_GPTQ_T128(4, 4, 2, 4, 2);
-    else if (t_variant == 2) SW_GPTQ_T128(4, 2, 4, 4, 3);
-    else if (t_variant == 8) SW_GPTQ_T128(4, 8, 1, 2, 2);
-    else if (t_variant == 68) SW_GPTQ_T128(2, 8, 1, 2, 2);
-    else if (t_variant == 70) SW_GPTQ_T128(2, 8, 1, 4, 2);
-#ifdef SW_QUANT_EXPERIMENT
-    else if (t_variant == 38) SW_GPTQ_T128(1, 8, 1, 2, 2);    // 32-row tiles: behind the k-across-waves kernel at every shape
-    else if (t_variant == 82) SW_GPTQ_T128(8, 2, 2, 4, 2);
-    else if (t_variant == 84) SW_GPTQ_T128(8, 4, 1, 2, 2);
-#endif
-    else SW_CHECK_ARG(false, "gptq_gemm: no 128-row tile variant %d", t_variant);
-#undef SW_GPTQ_T128
+    switch (stream_to) {
+      case StreamTile::k32x128: SW_GPTQ_STREAM(1, 2, 4, 4); break;
+      case StreamTile::k64x64: SW_GPTQ_STREAM(2, 1, 3, 2); break;
+      case StreamTile::k64x128: SW_GPTQ_STREAM(2, 2, 3, 4); break;
+      default: SW_GPTQ_STREAM(4, 2, 3, 2); break;
+    }
+#undef SW_GPTQ_STREAM
+    SW_CHECK_LAUNCH();
+    return SW_OK;
+  }
+  if (wide) {
+    auto kern = gptq_gemm_tile128_kernel;
+    SW_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     kT128Lds));
+    const int rt = (M + 127) / 128, ct = (N + 255) / 256;
+    int ks = pick_ksplit(ct * rt, K / kT128Chunk, 4, M, N, avail, 1, 256);
+    if (force_ks > 0 && force_ks < ks) ks = force_ks;
+    hipLaunchKernelGGL(kern, dim3((ct * rt * ks + 7) / 8 * 8), dim3(512), kT128Lds, st, out, ap, qweight, qzeros, sp, M, N,
+                       K, group_size, ks, ct, rt, zoff, partials, counters);
     SW_CHECK_LAUNCH();
     return SW_OK;
   }
