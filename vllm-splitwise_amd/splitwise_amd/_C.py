@@ -20,6 +20,8 @@ from typing import Dict, List, Optional
 
 import torch
 
+from ._native import bind_library, step_ops as _native
+
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libsplitwise_hip.so")
 
 SW_F32, SW_F16, SW_BF16, SW_FP8_E5M2 = 0, 1, 2, 3
@@ -129,6 +131,7 @@ def load_library() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = _RESTYPES.get(name, _c_int)
+    bind_library(lib, list(_SIGNATURES), ABI_VERSION, "SW_ABI_VERSION")
     _lib = lib
     return lib
 
@@ -200,6 +203,9 @@ def reshape_and_cache(key: torch.Tensor, value: torch.Tensor, key_cache: torch.T
                       value_cache: torch.Tensor, slot_mapping: torch.Tensor,
                       kv_cache_dtype: str) -> None:
     """``cache_ops.reshape_and_cache`` (csrc/cache_kernels.cu:228-268)."""
+    status = _native.reshape_and_cache(key, value, key_cache, value_cache, slot_mapping, kv_cache_dtype)
+    if status is not None:
+        return _check(status)
     _require_cuda(key, value, key_cache, value_cache, slot_mapping)
     act = _act_dtype(key)
     cache = _cache_dtype(kv_cache_dtype, act)
@@ -314,6 +320,10 @@ def paged_attention_v1(out: torch.Tensor, query: torch.Tensor, key_cache: torch.
                        max_context_len: int, alibi_slopes: Optional[torch.Tensor],
                        kv_cache_dtype: str) -> None:
     """``ops.paged_attention_v1`` (csrc/attention/attention_kernels.cu:711-747)."""
+    status = _native.paged_attention_v1(out, query, key_cache, value_cache, num_kv_heads, scale, block_tables,
+                                        context_lens, block_size, max_context_len, alibi_slopes, kv_cache_dtype)
+    if status is not None:
+        return _check(status)
     alibi_slopes = _pa_common(query, key_cache, value_cache, block_tables, context_lens, alibi_slopes)
     act = _act_dtype(query)
     cache = _cache_dtype(kv_cache_dtype, act)
@@ -375,6 +385,10 @@ def prefill_attention(out: torch.Tensor, query: torch.Tensor, key: torch.Tensor,
                       alibi_slopes: Optional[torch.Tensor] = None, sliding_window: Optional[int] = None) -> None:
     """Causal prompt attention over (start, length) sequences; stands where the reference calls
     xformers / flash-attn (backends/xformers.py:155-164).  query [T, H, D], key/value [T, KVH, D]."""
+    status = _native.prefill_attention(out, query, key, value, seq_starts, seq_lens,
+                                       max_seq_len, scale, alibi_slopes, sliding_window)
+    if status is not None:
+        return _check(status)
     _require_cuda(out, query, key, value, seq_starts, seq_lens)
     if seq_starts.dtype != torch.int32 or seq_lens.dtype != torch.int32:
         raise RuntimeError("prefill_attention: seq_starts and seq_lens must be int32")

@@ -16,6 +16,8 @@ from typing import Optional, Union
 
 import torch
 
+from ._native import bind_library, step_ops as _native
+
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_PKG_DIR, "libsplitwise_mixers.so")
 ABI_VERSION = 7
@@ -120,6 +122,9 @@ def load_library() -> ctypes.CDLL:
     for name, argtypes in _SIGNATURES.items():
         fn = getattr(lib, name)
         fn.argtypes, fn.restype = argtypes, _i
+    bind_library(lib, list(_SIGNATURES) + [f"swm_{op}_workspace_floats" for op in ("lightning", "masked_attention", "gla",
+                                                                                   "gated_delta_chunked")],
+                 ABI_VERSION, "SWM_ABI_VERSION")
     _lib = lib
     return lib
 
@@ -327,6 +332,9 @@ def causal_conv(out: torch.Tensor, x: torch.Tensor, taps: torch.Tensor, state: t
     """out [rows, channels] (any activation dtype) = act(conv(x) + x) (``residual``) or act(conv(x)), act = silu or
     none; x: a 2-D view, fp32 or bf16; the state [slots, taps - 1, channels] (fp32: the sequence's last inputs) is read
     and moved past the step's tokens in the same launch."""
+    status = _native.causal_conv(out, x, taps, state, batch, silu, residual)
+    if status is not None:
+        return _check(status)
     _dev(out, x, taps, state)
     _f32c(taps, "taps")
     _f32c(state, "state")
@@ -351,6 +359,10 @@ def gated_delta(out: torch.Tensor, qkv: torch.Tensor, beta_pre: torch.Tensor, de
     dt_bias, a_log fp32 [heads]; qkv fp32 [rows, 2 * kv_heads * dim + heads * vdim] from the short convolution;
     state fp32 [slots, heads, dim, vdim]; out fp32 [rows, heads * vdim].  ``chunked``: chunks of 32 tokens on the matrix
     cores instead of token by token (default: when some sequence brings at least 32 tokens; key sizes up to 224)."""
+    status = _native.gated_delta(out, qkv, beta_pre, decay_pre, dt_bias, a_log, state,
+                                 batch, heads, kv_heads, dim, vdim, chunked)
+    if status is not None:
+        return _check(status)
     _dev(out, qkv, beta_pre, decay_pre, dt_bias, a_log, state)
     for t, what in ((out, "out"), (qkv, "qkv"), (dt_bias, "dt_bias"), (a_log, "a_log"), (state, "state")):
         _f32c(t, what)
@@ -433,6 +445,9 @@ def head_norm_gate(out: torch.Tensor, o: torch.Tensor, gate: torch.Tensor, weigh
                    per_head_weight: bool, eps: float, heads: int, vdim: int, gate_silu: bool = False) -> None:
     """``per_head_weight``: weight is [heads * vdim]; otherwise [vdim], shared by the heads (None: no weight).
     ``gate_silu``: the normed output is multiplied by gate * sigmoid(gate) instead of sigmoid(gate)."""
+    status = _native.head_norm_gate(out, o, gate, weight, per_head_weight, eps, heads, vdim, gate_silu)
+    if status is not None:
+        return _check(status)
     _dev(out, o, gate, weight)
     _f32c(o, "o")
     if weight is not None:
@@ -460,6 +475,9 @@ def expert_ffn(out: torch.Tensor, x: torch.Tensor, up: torch.Tensor, down: torch
     g sigmoid(alpha g) (u + shift) with g = min(gate x, limit), u = clamp(up x, -limit, limit), worked out in the
     up-projection's epilogue -- ``up`` then holds gate and up rows in runs of 16 (``glu_rows``).  ``weigh_input``: the pair's
     weight multiplies what the expert reads instead of what it returns."""
+    status = _native.expert_ffn(out, x, up, down, order, expert_start, top, weight, activation, pair_weight, glu, weigh_input)
+    if status is not None:
+        return _check(status)
     _dev(out, x, up, down, order, expert_start, pair_weight)
     _f32c(out, "out")
     rows, width = x.shape
@@ -669,6 +687,9 @@ def group_router(logits: torch.Tensor, correction: Optional[torch.Tensor], top: 
 def group_pairs(chosen: torch.Tensor, experts: int):
     """chosen int32 [rows, top] -> (order int32 [rows * top]: pair indices row * top + choice grouped by expert,
     expert_start int32 [experts + 1]); one launch, nothing travels to the host."""
+    done = _native.group_pairs(chosen, experts)
+    if done is not None:
+        return done if type(done) is tuple else _check(done)
     _dev(chosen)
     _need(chosen.dtype == torch.int32 and chosen.is_contiguous(), "group_pairs: chosen must be contiguous int32")
     pairs = chosen.numel()
@@ -690,6 +711,10 @@ def capped_attention(out: torch.Tensor, q: torch.Tensor, key_cache: torch.Tensor
     denominator, exp(0), or exp(sink[head]) when it is a tensor (fp32 [heads]).  ``value_cache`` None: a token's values are the first kv_heads * vdim elements of its
     key row (attention over a shared latent).  ``score_bias`` (fp32 [heads]): no softmax -- a seen key weighs
     sigmoid(score + score_bias[head]) and the weights are not normalised (window mask only)."""
+    status = _native.capped_attention(out, q, key_cache, value_cache, gate, batch, heads, kv_heads, dim,
+                                      vdim, scale, softcap, window, chunk, sink, score_bias)
+    if status is not None:
+        return _check(status)
     learned = sink if isinstance(sink, torch.Tensor) else None
     _dev(out, q, key_cache, value_cache, gate, score_bias, learned)
     if learned is not None:
@@ -996,6 +1021,9 @@ def gla(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, de
         dim: int, vdim: int) -> None:
     """out fp32 [rows, heads * vdim]; q, k, v: column ranges of one projection output; decay_pre [rows, heads * dim]
     in the same dtype; decay_bias fp32 [heads * dim]; state fp32 [slots, heads, dim, vdim]."""
+    status = _native.gla(out, q, k, v, decay_pre, decay_bias, tau, q_scale, state, batch, heads, dim, vdim)
+    if status is not None:
+        return _check(status)
     _dev(out, q, k, v, decay_pre, decay_bias, state)
     for t, what in ((out, "out"), (state, "state")):
         _f32c(t, what)
@@ -1024,6 +1052,9 @@ def lightning(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tens
               state: torch.Tensor, batch, heads: int, dim: int, vdim: int) -> None:
     """out fp32 [rows, heads * vdim]; q, k, v: column ranges of one projection output (before their silu);
     decay fp32 [heads]; state fp32 [slots, heads, dim, vdim]."""
+    status = _native.lightning(out, q, k, v, decay, state, batch, heads, dim, vdim)
+    if status is not None:
+        return _check(status)
     _dev(out, q, k, v, decay, state)
     for t, what in ((out, "out"), (decay, "decay"), (state, "state")):
         _f32c(t, what)
@@ -1050,6 +1081,9 @@ def retention(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tens
     """S <- decay[h] S + k v^T;  o = S^T q.  out fp32 [rows, heads * vdim]; q, k fp32 [rows, heads * dim] (the caller's
     rotation and scale are in them); v: a 2-D view in an activation dtype; decay fp32 [heads]; state fp32 [slots, heads,
     dim, vdim]."""
+    status = _native.retention(out, q, k, v, decay, state, batch, heads, dim, vdim)
+    if status is not None:
+        return _check(status)
     _dev(out, q, k, v, decay, state)
     for t, what in ((out, "out"), (q, "q"), (k, "k"), (decay, "decay"), (state, "state")):
         _f32c(t, what)
