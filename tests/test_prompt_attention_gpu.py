@@ -250,6 +250,35 @@ def test_prompt_steps_agree_with_the_general_kernel(H, G, d, dv, page, option, w
     assert outs[0].isfinite().all() and outs[0].abs().max() > 0.1
 
 
+@pytest.mark.parametrize("H,G,d,dv", [(4, 1, 32, 32), (8, 2, 64, 56), (6, 2, 96, 96), (16, 4, 128, 128), (5, 1, 128, 104)])
+def test_finished_rows_go_out_alike_whatever_the_alignment(H, G, d, dv, way):
+    """Gates and results on 16 bytes and off them, gates at sigmoid's ends: the same bits four times, those of the 64-bit statement
+    within the bound above."""
+    from splitwise_amd import _C
+    lengths = [(0, 40), (5, 3), (0, 33), (17, 1)]
+    batch, pages = _step(lengths, 16)
+    g = torch.Generator(device=DEV).manual_seed(H * dv)
+    rows = sum(n for _, n in lengths)
+    kc, vc = (torch.randn(pages, 16, G * n, generator=g, device=DEV).to(torch.bfloat16) for n in (d, dv))
+    q = torch.randn(rows, H * d, generator=g, device=DEV)
+    gate = torch.randn(rows, H * dv, generator=g, device=DEV).to(torch.bfloat16) * 4
+    gate[1, :8] = torch.tensor([float("inf"), -float("inf"), 80.0, -80.0, 88.5, -88.5, 3e38, -3e38])
+    assert way(q, kc, vc, batch, H, G, d, dv) == PROMPT
+    outs = []
+    for gate_at, out_at in ((0, 0), (0, 3), (1, 0), (1, 3)):
+        wide = torch.full((rows, H * dv + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+        out = wide[:, out_at:out_at + H * dv]
+        at = torch.empty(rows, H * dv + 8, dtype=torch.bfloat16, device=DEV)[:, gate_at:gate_at + H * dv]
+        at.copy_(gate)
+        _C.mixer_ops.capped_attention(out, q, kc, vc, at, batch, H, G, d, dv, d ** -0.5)
+        assert (wide[:, :out_at] == 7).all() and (wide[:, out_at + H * dv:] == 7).all()
+        outs.append(out.float())
+    for other in outs[1:]:
+        assert torch.equal(outs[0], other)
+    ref = _statement(lengths, batch, q, kc, vc, gate, H, G, d, dv)
+    torch.testing.assert_close(outs[0].double(), ref, atol=2e-4, rtol=2.0 ** -7)
+
+
 @pytest.mark.parametrize("H,G,d,dv,page", [(4, 4, 128, 128, 16), (8, 2, 64, 96, 16), (6, 2, 40, 24, 8), (8, 1, 16, 8, 32),
                                            (5, 1, 104, 128, 12)])
 @pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "sink", "learned sink", "sigmoid", "values in the keys"])

@@ -24,7 +24,7 @@
 // Workgroups are numbered latest tile of a sequence first: under a causal mask those have the longest walks.
 //
 // Measured, two prompts of 4324 tokens together, 16 query heads on 4 of size 128, capped scores and a gate: 989 us with the
-// fp32 instructions (39 TFLOP/s), 177 us one group a workgroup, 162 us two; one prompt of 1607, 8 heads on 2, no cap: 88.7 and 69.2 us;
+// fp32 instructions (39 TFLOP/s), 177 us one group a workgroup, 159 us two; one prompt of 1607, 8 heads on 2, no cap: 88.7 and 69.2 us;
 // two of 1296 behind 190 tokens each, 16 on 4: 95.7 and 74.8.  Error against 64 bits before the rounding to bf16: 1.3e-6 with the fp32
 // instructions, 1.2e-6 here (without a cap 1.5 - 1.6e-7; 1.7 - 2.0e-7 with the small parts in a sum of their own).
 #include "prompt_attention.cuh"
@@ -67,6 +67,20 @@ __host__ __device__ constexpr int pa_lds_bytes(int nb, int groups) {
 }
 
 __host__ __device__ constexpr int pa_query_bytes(int nb) { return kPaWaves * 2 * 2 * nb * 1024; }         // two parts of the queries
+
+// 1 / (1 + e^-x) in a third of the instructions of expf and a division, to 2^-22: 2^t with t = -x log2 e and the product's rounding
+// error put right (beyond 2^120 it is no matter)
+__device__ __forceinline__ float short_sigmoid(float x) {
+  const float t = -kLog2e * x;
+  const float lost = fmaf(-kLog2e, x, -t) - 1.92596299e-8f * x;          // log2 e = kLog2e + 1.926e-8
+  const float e = __builtin_amdgcn_exp2f(t);
+  return __builtin_amdgcn_rcpf(1.0f + (fabsf(t) < 120.0f ? fmaf(e, 0.69314718f * lost, e) : e));
+}
+
+// a wave's finished rows, or the row that it works out again
+__host__ __device__ constexpr int pa_rows_bytes(int nb) {
+  return 4 * (32 * (nb * 32 + 4) > kPlainRowLds ? 32 * (nb * 32 + 4) : kPlainRowLds);
+}
 
 // NB: blocks of 32 coordinates of the larger of key and value size.
 // GROUPS: of 4 waves, which take the stages in turn, each with LDS buffers of its own; two of them have their sums meet at the end.
@@ -351,6 +365,40 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
       take_apart(1);
     }
   };
+  // ---- the finished rows go out 8 neighbouring channels a lane: piece 64 u + lane of 32 rows x 4 NB pieces (sizes are multiples of 8);
+  //      rows without a token: the last one's again
+  const bool gated = a.gate != nullptr && nw > 0;
+  uint4 gates[2 * NB];
+  auto place = [&](int u, int& row, int& c, int64_t& at_row, int& col) {
+    const int i = 64 * u + lane;
+    row = i / (4 * NB);
+    c = i % (4 * NB) * 8;
+    const int t = row / R;
+    at_row = row0 + min(t, nw - 1);
+    col = (g * R + row - t * R) * a.vdim + min(c, a.vdim - 8);
+    return t < nw && c < a.vdim;
+  };
+  auto fetch_gates = [&]() {                                 // all of them, when the walk is through
+    if (!gated) return;
+    if (a.gate_stride % 8 == 0 && reinterpret_cast<uintptr_t>(a.gate) % 16 == 0) {
+#pragma unroll
+      for (int u = 0; u < 2 * NB; ++u) {
+        int row, c, col;
+        int64_t at_row;
+        place(u, row, c, at_row, col);
+        gates[u] = *reinterpret_cast<const uint4*>(a.gate + at_row * a.gate_stride + col);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 2 * NB; ++u) {
+        int row, c, col;
+        int64_t at_row;
+        place(u, row, c, at_row, col);
+        const uint16_t* p = a.gate + at_row * a.gate_stride + col;
+        gates[u] = make_uint4(p[0] | p[1] << 16, p[2] | p[3] << 16, p[4] | p[5] << 16, p[6] | p[7] << 16);
+      }
+    }
+  };
   tfetch(first);
   fetch(first);
   if (GROUPS > 1 || turns > 1) tfetch(first + GROUPS);
@@ -373,6 +421,7 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
       }
       __syncthreads();
     }
+    fetch_gates();
   } else {
     if (group == 0) {
 #pragma unroll 1
@@ -383,6 +432,7 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
         if (live(t)) vector_half(t);
         __syncthreads();
       }
+      fetch_gates();
       if (live(turns - 1)) value_products(before(vbuf));
     } else {
 #pragma unroll 1
@@ -447,7 +497,7 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
   for (uint32_t left = (uint32_t)lanes | (uint32_t)(lanes >> 32); left != 0; left &= left - 1) {      // uniform over the wave
     const int r = __builtin_ctz(left), rt = r / R, rh = r - rt * R;
     const int pos = wfirst + rt, low = max(a.chunk > 0 ? pos / a.chunk * a.chunk : a.window > 0 ? pos - a.window + 1 : 0, 0);
-    float* own = reinterpret_cast<float*>(pa_lds) + wave * kPlainRowLds;
+    float* own = reinterpret_cast<float*>(pa_lds + wave * pa_rows_bytes(NB));
     const PlainRow row = plain_row(a, table, g, a.q + ((row0 + rt) * a.heads + g * R + rh) * (int64_t)a.dim,
                                    sig ? a.score_bias[g * R + rh] : 0.0f, pos, low, pos - low + 1, [&](int i) { return low + i; },
                                    own);
@@ -464,9 +514,12 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
       l_part = hl == 0 ? row.l : 0.0f;
     }
   }
-  if (!row_ok) return;
+  if (nw == 0) return;                                       // the whole wave
 
-  // ---- normalise, gate, store: this lane holds query qi, channels 32 b + 8 (r / 4) + 4 hl + r % 4
+  // ---- normalise, gate, store: this lane holds query qi, channels 32 b + 8 (r / 4) + 4 hl + r % 4.  Through LDS, so that a lane
+  //      stores 8 neighbouring channels and a short loop does it: from the accumulators' places it was 18 KB of instructions, gone
+  //      through once, with a wait for a gate in front of every store, 8 us of a launch (one prompt of 40 tokens, 16 heads on 4 of
+  //      128: 16.6 -> 12.3 us, two of 200: 27.0 -> 23.2, one of 700: 44.3 -> 40.7, four of 1000: 92 -> 88)
   const float l_run = l_part + other_half(l_part);
   float inv = 1.0f;
   if (!sig) {
@@ -476,43 +529,49 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
     const float fin = a.sink ? __builtin_amdgcn_exp2f(m_run - m_fin) : 1.0f;
     inv = fin / (l_run * fin + (a.sink ? __builtin_amdgcn_exp2f(sk - m_fin) : 0.0f));
   }
-  const int64_t col0 = (int64_t)(g * R + hh) * a.vdim;
-  uint16_t* op = static_cast<uint16_t*>(a.out) + (row0 + tt) * a.out_stride + col0;
-  const uint16_t* gp = a.gate != nullptr ? a.gate + (row0 + tt) * a.gate_stride + col0 : nullptr;
-  const bool quads = a.out_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.out) % 8 == 0;
-  const bool gquads = a.gate_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.gate) % 8 == 0;
+  constexpr int OROW = NB * 32 + 4;                          // floats: 8 rows' quads on distinct banks
+  float* rows_lds = reinterpret_cast<float*>(pa_lds + wave * pa_rows_bytes(NB));
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int r4 = 0; r4 < 4; ++r4) {
-      const int c = 32 * b + 8 * r4 + 4 * hl;
-      if (c >= a.vdim) continue;
-      float v[4];
+    for (int r4 = 0; r4 < 4; ++r4)
+      *reinterpret_cast<pa_f32x4*>(rows_lds + qi * OROW + 32 * b + 8 * r4 + 4 * hl) =
+          pa_f32x4{o[b][4 * r4] * inv, o[b][4 * r4 + 1] * inv, o[b][4 * r4 + 2] * inv, o[b][4 * r4 + 3] * inv};
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  const bool whole = a.out_stride % 8 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0;
+#pragma unroll 1
+  for (int half = 0; half < 2; ++half)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = o[b][4 * r4 + j] * inv;
-      if (gp != nullptr) {
-        float gv[4];
-        if (gquads) {
-          ld_vec<bf16_t, 4>(gv, gp, c);
-        } else {
+    for (int u = 0; u < NB; ++u) {
+      int row, c, col;
+      int64_t at_row;
+      const bool mine = place(half * NB + u, row, c, at_row, col);
+      const pa_f32x4 x0 = *reinterpret_cast<const pa_f32x4*>(rows_lds + row * OROW + c);
+      const pa_f32x4 x1 = *reinterpret_cast<const pa_f32x4*>(rows_lds + row * OROW + c + 4);
+      float v[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+      if (gated) {
+        const uint4 gw = half ? gates[NB + u] : gates[u];
+        const uint32_t w[4] = {gw.x, gw.y, gw.z, gw.w};
 #pragma unroll
-          for (int j = 0; j < 4; ++j) gv[j] = ld<bf16_t>(gp, c + j);
+        for (int j = 0; j < 4; ++j) {
+          v[2 * j] *= short_sigmoid(__uint_as_float(w[j] << 16));
+          v[2 * j + 1] *= short_sigmoid(__uint_as_float(w[j] & 0xffff0000u));
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] *= sigmoidf_(gv[j]);
       }
-      if (quads) {
-        st_vec<bf16_t, 4>(op, c, v);
+      if (!mine) continue;
+      uint16_t* op = static_cast<uint16_t*>(a.out) + at_row * a.out_stride + col;
+      if (whole) {
+        st_vec<bf16_t, 8>(op, 0, v);
       } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) st<bf16_t>(op, c + j, v[j]);
+        for (int j = 0; j < 8; ++j) st<bf16_t>(op, j, v[j]);
       }
     }
 }
 
 template <int NB, int GROUPS>
 int launch_prompt_tiles_as(const PromptAttention& a, unsigned groups, hipStream_t stream) {
-  constexpr int lds = GROUPS * pa_lds_bytes(NB, GROUPS) + (GROUPS > 1 ? pa_query_bytes(NB) : 0);
+  constexpr int lds = std::max(GROUPS * pa_lds_bytes(NB, GROUPS) + (GROUPS > 1 ? pa_query_bytes(NB) : 0), kPaWaves * pa_rows_bytes(NB));
   if (lds > 64 * 1024)
     SW_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(prompt_attention_kernel<NB, GROUPS>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds));
