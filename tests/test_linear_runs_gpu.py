@@ -76,6 +76,38 @@ def test_segments_and_mixed_steps(rule, heads, dim, vdim, lens):
     assert torch.equal(got[idle], state[idle])
 
 
+@pytest.mark.parametrize("rule", ["gla", "lightning", "retention"])
+@pytest.mark.parametrize("heads,dim,vdim", [(16, 128, 128), (2, 256, 260), (64, 8, 4), (16, 40, 12), (2, 96, 132), (1, 200, 1024), (2, 33, 64),
+                                            (2, 64, 17)])
+@pytest.mark.parametrize("lens", [[1] * 7, [5, 1, 0, 3, 5], [1] * 9 + [40, 6, 16, 2]], ids=str)
+def test_few_tokens(rule, heads, dim, vdim, lens):
+    """Token by token with the state in whole rows, alone and with longer runs left to the chunks' kernels: key sizes that fill the threads' rows or not, value sizes of one piece of 16
+    bytes, of part of a workgroup's, of several workgroups (and one that has no such pieces and goes by chunks).  (Some hundred outputs: one of a
+    few may be a small difference of its terms.)"""
+    test_segments_and_mixed_steps(rule, heads, dim, vdim, lens)
+
+
+@pytest.mark.parametrize("said", [0, 1, 3])
+def test_a_run_longer_than_the_batch_says(said):
+    """The longest run is a hint: a sequence that brings more is worked out all the same."""
+    from splitwise_amd import _C
+    heads, dim, lens = 2, 64, [1, 9, 40, 2]
+    rows, n = sum(lens), len(lens)
+    g = torch.Generator(device=DEV).manual_seed(said)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
+    batch = SimpleNamespace(q_start=i32([sum(lens[:i]) for i in range(n + 1)]), ctx_len=i32([3] * n), state_slot=i32(list(range(n))),
+                            max_state_slot=n - 1, max_query_len=said, token_seq=i32([i for i, m in enumerate(lens) for _ in range(m)]))
+    q, k, v = (torch.randn(rows, heads * dim, generator=g, device=DEV) for _ in range(3))
+    decay, state = torch.linspace(0.3, 0.99, heads, device=DEV), torch.randn(n, heads, dim, dim, generator=g, device=DEV)
+    got, out = state.clone(), torch.full_like(v, float("nan"))
+    _C.mixer_ops.retention(out, q, k, v, decay, got, batch, heads, dim, dim)
+    q64, k64, v64 = (t.double().view(rows, heads, dim) for t in (q, k, v))
+    ref, ends = _rule(q64, k64, v64, decay.double().view(1, heads, 1).expand(rows, heads, 1), state.double(),
+                      batch.q_start.tolist(), torch.zeros(n, dtype=torch.bool, device=DEV))
+    for a, b in ((out.double().view_as(ref), ref), (got.double(), ends)):
+        assert float((a - b).norm() / b.norm()) < 6e-7
+
+
 @pytest.mark.parametrize("heads,dim,vdim", [(2, 128, 40), (1, 160, 16), (3, 64, 17)])
 @pytest.mark.parametrize("lens", [[70, 33, 130], [1600]], ids=["runs", "segments"])
 def test_gates_that_overflowed(heads, dim, vdim, lens):

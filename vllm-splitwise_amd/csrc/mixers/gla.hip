@@ -16,7 +16,7 @@
 //    value channel join their halves of S^T q.  Exact for any decay (a product of decays that underflows is a state
 //    that has been forgotten), and the cheaper route for runs of a few tokens (a decoded token is a chunk of one).
 //
-// Long runs are taken by linear_walk.hip (linear_at_most says which).
+// Long runs are taken by linear_walk.hip (linear_at_most says which), a few tokens by linear_step.hip (linear_step_tokens).
 #include "linear_walk.cuh"
 
 #include <climits>
@@ -28,16 +28,13 @@ constexpr int kGlaChunk = 32;
 constexpr float kSafeLog = 24.0f;      // the matrix route needs every channel's summed log-decay of a chunk above -this
 constexpr int kTokenRouteBelow = 6;    // chunks shorter than this go token by token without asking
 
-// log(sigmoid(x)) = min(x, 0) - log1p(exp(-|x|))
-__device__ __forceinline__ float logsigmoidf_(float x) { return fminf(x, 0.0f) - log1pf(expf(-fabsf(x))); }
-
 // blockIdx.x is a sequence; its whole run goes from the slot's state to the slot's state.
 template <typename T, int NDB>
 __global__ __launch_bounds__(512) void gla_kernel(
     float* __restrict__ out, const void* __restrict__ q, const void* __restrict__ k, const void* __restrict__ v,
     int64_t in_stride, const void* __restrict__ decay_pre, int64_t decay_stride, const float* __restrict__ decay_bias,
     float inv_tau, float q_scale, float* __restrict__ state, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int dim, int vdim, int at_most) {
+    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int dim, int vdim, int above, int at_most) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int DS = NDB * 32 + 4;                           // row stride of the staged tiles
   constexpr int CH = NDB * 32;                               // key channels, padded
@@ -53,7 +50,7 @@ __global__ __launch_bounds__(512) void gla_kernel(
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 31, hl = lane >> 5;
   const int vb0 = blockIdx.z * nw;                           // first block of 32 value channels of the workgroup
   const int seq = blockIdx.x, n = q_start[seq + 1] - q_start[seq];
-  if (n <= 0 || n > at_most) return;                         // the whole workgroup
+  if (n <= above || n > at_most) return;                     // the whole workgroup
   const int row0 = q_start[seq];
   const int vc = (vb0 + wave) * 32 + li;                     // this lane's value channel
   const bool vc_ok = vc < vdim;
@@ -266,7 +263,7 @@ template <typename T, int NDB>
 int launch_gla(float* out, const void* q, const void* k, const void* v, int64_t in_stride, const void* decay_pre,
                int64_t decay_stride, const float* decay_bias, float tau, float q_scale, float* state,
                const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot, int num_seqs, int heads, int dim,
-               int vdim, int at_most, hipStream_t stream) {
+               int vdim, int above, int at_most, hipStream_t stream) {
   const int vblocks = (vdim + 31) / 32;
   const int waves = std::min(vblocks, 8);
   const size_t lds_bytes =
@@ -282,7 +279,7 @@ int launch_gla(float* out, const void* q, const void* k, const void* v, int64_t 
   const float inv_tau = 1.0f / tau;
   hipLaunchKernelGGL(kernel, dim3((unsigned)num_seqs, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream, out, q, k, v,
                      in_stride, decay_pre, decay_stride, decay_bias, inv_tau, q_scale, state, q_start, ctx_len, state_slot, heads,
-                     dim, vdim, at_most);
+                     dim, vdim, above, at_most);
   SW_CHECK_LAUNCH();
   return SW_OK;
 }
@@ -314,11 +311,22 @@ extern "C" int swm_gla(float* out, const void* q, const void* k, const void* v, 
     if (status != SW_OK || plan.at_most == 0) return status;
     at_most = plan.at_most;                                  // the others beside it
   }
+  int above = 0;                                             // sequences of this many tokens have been seen to
+  if (const int few = linear_step_tokens(at_most, rows, num_seqs, max_query_len)) {
+    const LinearStep step{out, q, k, v, in_stride, in_stride, state, q_start, ctx_len, state_slot, rows, num_seqs, heads, dim, vdim,
+                          nullptr};
+    const bool all = few >= std::min(at_most, max_query_len);
+    if (gla_step(step, decay_pre, decay_stride, decay_bias, 1.0f / tau, q_scale, all ? at_most : few, act_dtype, s)) {
+      SW_CHECK_LAUNCH();
+      if (all) return SW_OK;
+      above = few;
+    }
+  }
 #define SWM_GLA_CASE(N)                                                                                             \
   case N:                                                                                                           \
     SWM_DISPATCH_ACT(act_dtype, return (launch_gla<T, N>(out, q, k, v, in_stride, decay_pre, decay_stride,          \
                                                          decay_bias, tau, q_scale, state, q_start, ctx_len,         \
-                                                         state_slot, num_seqs, heads, dim, vdim, at_most, s)););    \
+                                                         state_slot, num_seqs, heads, dim, vdim, above, at_most, s)););    \
     break;
   switch ((dim + 31) / 32) {
     SWM_GLA_CASE(1)

@@ -12,8 +12,8 @@
 // One wave owns (sequence, head, 32 value channels) and keeps its slice of the state in registers across the
 // whole run (the waves of a workgroup share the chunk's queries and keys, staged once in LDS), in the matrix cores' accumulator layout (lane l: value channel l % 32; element r of block b:
 // key coordinate 32 b + 8 (r / 4) + 4 (l / 32) + r % 4).  That layout is also what the A operand of S^T q needs
-// when q is read in the same order of coordinates, so the state never moves between registers.  A decoded
-// token is a chunk of one.
+// when q is read in the same order of coordinates, so the state never moves between registers.  Long
+// runs are taken by linear_walk.hip (linear_at_most says which), a few tokens by linear_step.hip (linear_step_tokens).
 #include "linear_walk.cuh"
 
 #include <climits>
@@ -30,7 +30,7 @@ template <typename TQ, typename T, bool SILU, int NDB>
 __global__ __launch_bounds__(512) void lightning_kernel(
     float* __restrict__ out, const void* __restrict__ q, const void* __restrict__ k, int64_t qk_stride,
     const void* __restrict__ v, int64_t v_stride, const float* __restrict__ decay, float* __restrict__ state, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int dim, int vdim, int at_most) {
+    const int32_t* __restrict__ ctx_len, const int32_t* __restrict__ state_slot, int heads, int dim, int vdim, int above, int at_most) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int DS = NDB * 32 + 4;                           // row stride of the staged tiles
   float* Qs = lds;                                           // [32][DS]
@@ -41,7 +41,7 @@ __global__ __launch_bounds__(512) void lightning_kernel(
   const int vb = blockIdx.z * (blockDim.x >> 6) + wave;
   // blockIdx.x is a sequence; its whole run goes from the slot's state to the slot's state
   const int seq = blockIdx.x, n = q_start[seq + 1] - q_start[seq];
-  if (n <= 0 || n > at_most) return;                         // the whole workgroup
+  if (n <= above || n > at_most) return;                     // the whole workgroup
   const int row0 = q_start[seq];
   const float lam = decay[h];
   if (threadIdx.x == 0) {
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(512) void lightning_kernel(
 template <typename TQ, typename T, bool SILU, int NDB>
 int launch_lightning(float* out, const void* q, const void* k, int64_t qk_stride, const void* v, int64_t v_stride, const float* decay,
                      float* state, const int32_t* q_start, const int32_t* ctx_len, const int32_t* state_slot,
-                     int num_seqs, int heads, int dim, int vdim, int at_most, hipStream_t stream) {
+                     int num_seqs, int heads, int dim, int vdim, int above, int at_most, hipStream_t stream) {
   const int vblocks = (vdim + 31) / 32;
   const int waves = std::min(vblocks, 8);
   const size_t lds_bytes = (size_t)(2 * kChunk * (NDB * 32 + 4) + kChunk + 2) * sizeof(float);
@@ -205,7 +205,7 @@ int launch_lightning(float* out, const void* q, const void* k, int64_t qk_stride
   }
   const unsigned zgroups = (unsigned)((vblocks + waves - 1) / waves);
   hipLaunchKernelGGL(kernel, dim3((unsigned)num_seqs, (unsigned)heads, zgroups), dim3(64 * waves), lds_bytes, stream, out, q, k,
-                     qk_stride, v, v_stride, decay, state, q_start, ctx_len, state_slot, heads, dim, vdim, at_most);
+                     qk_stride, v, v_stride, decay, state, q_start, ctx_len, state_slot, heads, dim, vdim, above, at_most);
   SW_CHECK_LAUNCH();
   return SW_OK;
 }
@@ -236,11 +236,22 @@ extern "C" int swm_lightning(float* out, const void* q, const void* k, const voi
     if (status != SW_OK || plan.at_most == 0) return status;
     at_most = plan.at_most;                                  // the others beside it
   }
+  int above = 0;                                             // sequences of this many tokens have been seen to
+  if (const int few = linear_step_tokens(at_most, rows, num_seqs, max_query_len)) {
+    const LinearStep step{out, q, k, v, in_stride, in_stride, state, q_start, ctx_len, state_slot, rows, num_seqs, heads, dim, vdim,
+                          nullptr};
+    const bool all = few >= std::min(at_most, max_query_len);
+    if (lightning_step(step, decay, true, all ? at_most : few, act_dtype, s)) {
+      SW_CHECK_LAUNCH();
+      if (all) return SW_OK;
+      above = few;
+    }
+  }
 #define SWM_LIGHTNING_CASE(N)                                                                                              \
   case N:                                                                                                                  \
     SWM_DISPATCH_ACT(act_dtype, return (launch_lightning<T, T, true, N>(out, q, k, in_stride, v, in_stride, decay, state,  \
                                                                         q_start, ctx_len, state_slot, num_seqs, heads,     \
-                                                                        dim, vdim, at_most, s)););                         \
+                                                                        dim, vdim, above, at_most, s)););                         \
     break;
   switch ((dim + 31) / 32) {
     SWM_LIGHTNING_CASE(1)
@@ -275,11 +286,22 @@ extern "C" int swm_retention(float* out, const float* q, const float* k, int64_t
     if (status != SW_OK || plan.at_most == 0) return status;
     at_most = plan.at_most;                                  // the others beside it
   }
+  int above = 0;                                             // sequences of this many tokens have been seen to
+  if (const int few = linear_step_tokens(at_most, rows, num_seqs, max_query_len)) {
+    const LinearStep step{out, q, k, v, qk_stride, v_stride, state, q_start, ctx_len, state_slot, rows, num_seqs, heads, dim, vdim,
+                          nullptr};
+    const bool all = few >= std::min(at_most, max_query_len);
+    if (lightning_step(step, decay, false, all ? at_most : few, act_dtype, s)) {
+      SW_CHECK_LAUNCH();
+      if (all) return SW_OK;
+      above = few;
+    }
+  }
 #define SWM_RETENTION_CASE(N)                                                                                          \
   case N:                                                                                                              \
     SWM_DISPATCH_ACT(act_dtype, return (launch_lightning<float, T, false, N>(out, q, k, qk_stride, v, v_stride, decay, \
                                                                              state, q_start, ctx_len, state_slot,      \
-                                                                             num_seqs, heads, dim, vdim, at_most, s)););\
+                                                                             num_seqs, heads, dim, vdim, above, at_most, s)););\
     break;
   switch ((dim + 31) / 32) {
     SWM_RETENTION_CASE(1)

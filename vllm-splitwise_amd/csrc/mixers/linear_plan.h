@@ -20,10 +20,9 @@ constexpr int kLwChunk = 32;
 //   tokens 165 / 172, 100 282 / 278, 150 460 / 344.  Per head W = 256, 32 tokens 34 / 41, 64 58 / 51; W = 512, 64 tokens 76 / 86, 100
 //   119 / 119, 200 202 / 176; W = 1024, 100 tokens 237 / 266, 150 308 / 328, 200 462 / 395.  (The lines were drawn for a walk of half
 //   the speed: between them and the crossings above, at W = 512 and 1024 per head from 120 and 170 tokens on, calls take the slower way.)
-//   Decoding sequences beside few long ones: a token costs the decode kernels about 1 us and the walk 0.06, a decoding sequence
-//   0.03 us per W and 0.13.  16 heads, all through the decode kernels / all through the walk / each its own way: per channel 60
-//   sequences beside a portion of 24 tokens 55 / 126 / 46, of 100 128 / 128 / 50, 250 beside 24 141 / 635 / 140, beside 250
-//   392 / 645 / 148; per head 60 beside 24 tokens 74 / 118 / 79, 250 beside 24 264 / 612 / 279, 7 beside 100 81 / 29 / 42.
+//   Decoding sequences beside few long ones: all through the walk they are the dearest, 0.13 us a sequence and W; each its own way is the
+//   cheapest from W = 160 on (us, all through the decode kernels / each its own way, 16 heads: per channel 60 sequences beside a portion of
+//   24 tokens 55 / 42, 250 beside 24 154 / 129, per head 76 / 37, 268 / 123).
 inline int linear_at_most(bool per_channel, int64_t rows, int num_seqs, int max_query_len, int heads, int dim, int vdim) {
   constexpr int kShort = 16;
   if (max_query_len <= kShort) return max_query_len;
@@ -33,8 +32,26 @@ inline int linear_at_most(bool per_channel, int64_t rows, int num_seqs, int max_
     return max_query_len <= (most < kShort ? kShort : most > cap ? cap : most) ? max_query_len : 0;
   }
   const int64_t units = w * dim / 128;
-  if (max_query_len <= (units > 160 ? 36 : units > 112 ? 24 : kShort)) return max_query_len;
-  return units <= 160 ? 0 : kShort;
+  if (units > 160) return kShort;
+  return max_query_len <= (units > 112 ? 24 : kShort) ? max_query_len : 0;
+}
+
+// Up to how many tokens a sequence that does not walk goes token by token with the state in whole rows (linear_step.hip; 0: none does)
+// and not by chunks, whose kernels hold a state's columns (gla.hip, lightning.hip); max_query_len 0: not known.  Up to 5, where the
+// per-channel rule's chunks go token by token too: from there on a chunk rounds its state less often (1600 tokens in portions of 13: an
+// error of 9.4e-7 token by token, below 6e-7 by chunks).  Measured, norm and gate included (us, by chunks / token by token), 16 heads of
+// 128 x 128:
+//   1 token each, 1 sequence: gla 13.1 / 8.0, lightning 29.0 / 9.7, retention 25.8 / 6.6; 61: 35.3 / 28.4, 74.1 / 30.4, 68.3 / 25.7;
+//   4 tokens: 15.8 / 11.2, 29.2 / 12.3, 25.5 / 8.7; 61: 37.0 / 29.6, 70.1 / 29.2, 63.4 / 23.1.
+// 8 heads of 256 x 256, 61 sequences, 1 token: 197 / 64, 186 / 65, 179 / 62.
+// Where the rest of a step walks, runs of 6 tokens and more that do not are left to the chunks' kernels in a launch of their own, unless
+// what is not a multiple of the longest run looks like most of them (20 of 12 tokens beside 300: 71 us without that launch, 74 with it).
+inline int linear_step_tokens(int at_most, int64_t rows, int num_seqs, int max_query_len) {
+  constexpr int kSteps = 5;
+  if (max_query_len <= 0) return 0;
+  const int longest = at_most < max_query_len ? at_most : max_query_len;
+  if (longest <= kSteps) return longest;
+  return at_most < max_query_len && rows % max_query_len <= kSteps * (int64_t)num_seqs ? kSteps : 0;
 }
 
 // A walk's sizes.  Few runs leave most of the GPU idle, and a long run's chunks are then worth cutting: into segments whose own

@@ -46,6 +46,8 @@ __device__ __forceinline__ float softplusf_(float x) { return fmaxf(x, 0.0f) + l
 // exp, sigmoid-weighted unit and tanh on the hardware's exp2 and reciprocal (a few ulp; for the inner loops of kernels
 // whose arithmetic is otherwise bound by these functions)
 __device__ __forceinline__ float fast_expf_(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
+// log(sigmoid(x)) = min(x, 0) - log1p(exp(-|x|))
+__device__ __forceinline__ float logsigmoidf_(float x) { return fminf(x, 0.0f) - log1pf(expf(-fabsf(x))); }
 __device__ __forceinline__ float fast_siluf_(float x) { return x * __builtin_amdgcn_rcpf(1.0f + fast_expf_(-x)); }
 // tanh(x) = 1 - 2 / (1 + e^(2x)); e^(2x) -> inf gives 1, -> 0 gives -1
 __device__ __forceinline__ float fast_tanhf_(float x) {
