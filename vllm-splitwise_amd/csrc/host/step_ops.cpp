@@ -1,15 +1,15 @@
-// The operators that small steps consist of, called without a Python frame per argument: the checks of the functions of the same
-// names in _C.py / _C_mixers.py, their scratch allocation and the library call, in C++.
+// The operators that small steps consist of, called without a Python frame per argument: the checks of the functions of the
+// same names in _C.py / _C_mixers.py, their scratch allocation and the library call, in C++.
 //
-// Why: a launch costs the host 3 us; a call through the Python functions cost 7 to 11 us, of which ctypes takes 1 and the checks,
-// data pointers and the device guard the rest, so that a decode step of two conversations waited for the host (21 us a layer, 12.6 on
-// the GPU).  Measured, us a pass of calls, before / now: cache write + attention of a decode step 20.9 / 16.6, of a prompt of
-// 40 tokens 21.0 / 15.7; the delta rule with its convolution and norm 34.9 / 23.4; experts 27.4 / 21.9; gated linear attention 28.7 / 21.3;
-// the mixers' attention 15.3 / 8.3.
+// Why: a launch costs the host 3 us; a call through the Python functions cost 7 to 11 us, of which ctypes takes 1 and the
+// checks, data pointers and the device guard the rest, so that a decode step of two conversations waited for the host (21 us
+// a layer, 12.6 on the GPU).  Measured, us a pass of calls, before / now: cache write + attention of a decode step 20.9 /
+// 16.6, of a prompt of 40 tokens 21.0 / 15.7; the delta rule with its convolution and norm 34.9 / 23.4; experts 27.4 / 21.9;
+// gated linear attention 28.7 / 21.3; the mixers' attention 15.3 / 8.3.
 //
-// A function takes a call only if every argument is of the plain kind (exact tensors on the current device, Python numbers) and passes
-// every check; otherwise it returns None before anything happened and the Python function goes on, which knows the other
-// forms and words the refusals.  It returns the library's status otherwise.
+// A function takes a call only if every argument is of the plain kind (exact tensors on the current device, Python numbers)
+// and passes every check; otherwise it returns None before anything happened and the Python function goes on, which knows
+// the other forms and words the refusals.  It returns the library's status otherwise.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -194,6 +194,7 @@ template <typename F> PyObject* call(F body) {
   try {
     return body();
   } catch (...) {                                  // also what torch throws: the Python function meets it again
+    PyErr_Clear();
     Py_RETURN_NONE;
   }
 }
