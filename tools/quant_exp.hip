@@ -3,8 +3,8 @@
 // first one run on the same inputs.
 //   hipcc -O3 -std=c++17 --offload-arch=gfx950 -Xclang -target-feature -Xclang -packed-fp32-ops \
 //         -DSW_QUANT_EXPERIMENT -I include -I vllm-splitwise_amd/csrc \
-//         tools/quant_exp.hip -o gpurun_out/quant_exp
-//   SW_QUANT_WAVES=4 SW_QUANT_TMT=4 gpurun_out/quant_exp 256 13824 5120
+//         tools/quant_exp.hip -o build/quant_exp
+//   SW_QUANT_WAVES=4 SW_QUANT_TMT=4 build/quant_exp 256 13824 5120
 #include "../vllm-splitwise_amd/csrc/quant_gemm.hip"
 #include <cmath>
 #include <cstdio>
