@@ -1,9 +1,13 @@
 """What `make` builds: both HIP libraries with hipcc alone; the native host side of small steps beside them where its headers are."""
+import importlib
 import os
 import shutil
 import stat
 import subprocess
 import sys
+import sysconfig
+import types
+import warnings
 
 import pytest
 
@@ -33,7 +37,7 @@ def tree(tmp_path):
         env = {k: v for k, v in os.environ.items() if not k.startswith("MAKE")}
         return subprocess.run(["make", "-C", str(pkg), f"HIPCC={compiler}", f"CXX={cxx}", f"PYTHON={python}", *args],
                               capture_output=True, text=True, env=env, timeout=60)
-    make.broken = broken
+    make.broken, make.compiler, make.directory = broken, compiler, str(pkg)
     make.built = lambda: sorted(p.name for p in (pkg / "splitwise_amd").glob("*.so"))
     return make
 
@@ -56,3 +60,66 @@ def test_with_its_headers_everything_is_built(tree):
     done = tree("-j4")
     assert done.returncode == 0, done.stderr
     assert len(tree.built()) == 3 and any(n.startswith("_step_ops") for n in tree.built())
+
+
+def _loaded(monkeypatch, extension):
+    """The module that chooses the extension, imported anew where `import _step_ops` gives `extension` -> what it took, its warnings."""
+    import splitwise_amd
+    kept = importlib.import_module("splitwise_amd._native")
+    monkeypatch.setitem(sys.modules, "splitwise_amd._step_ops", extension)
+    monkeypatch.setattr(splitwise_amd, "_native", kept)                     # (put back what the import below sets)
+    monkeypatch.delitem(sys.modules, "splitwise_amd._native")
+    with warnings.catch_warnings(record=True) as said:
+        warnings.simplefilter("always")
+        taken = importlib.import_module("splitwise_amd._native").step_ops
+    return taken, [str(w.message) for w in said]
+
+
+@pytest.mark.parametrize("torch_was", [None, "0.0.0 other", "same version, another commit"])
+def test_an_extension_of_another_torch_is_not_used(monkeypatch, torch_was):
+    import torch
+    if torch_was is not None and "commit" in torch_was:
+        torch_was = torch.__version__ + " 0000"
+    stale = types.SimpleNamespace(__file__="stale.so", SW_ABI_VERSION=7, SWM_ABI_VERSION=7, gla=lambda *a: 0)
+    if torch_was is not None:
+        stale.TORCH = torch_was
+    taken, said = _loaded(monkeypatch, stale)
+    assert taken is not stale and taken.gla(1, 2) is None
+    assert len(said) == 1 and "not used" in said[0]
+
+
+def test_the_extension_that_was_built_here_is_used(monkeypatch):
+    kept = importlib.import_module("splitwise_amd._native")
+    try:
+        ours = importlib.import_module("splitwise_amd._step_ops")
+    except ImportError:
+        pytest.skip("built without the extension")
+    assert kept.step_ops is ours
+    taken, said = _loaded(monkeypatch, ours)
+    assert taken is ours and said == []
+
+
+def test_an_extension_that_does_not_load_is_named(monkeypatch, tmp_path):
+    """None in sys.modules makes the import fail as an undefined symbol does."""
+    kept = importlib.import_module("splitwise_amd._native")
+    monkeypatch.setattr(kept.glob, "glob", lambda pattern: [pattern])
+    taken, said = _loaded(monkeypatch, None)
+    assert taken.gla(1, 2) is None and len(said) == 1 and "does not load" in said[0]
+    monkeypatch.setattr(kept.glob, "glob", lambda pattern: [])
+    assert _loaded(monkeypatch, None)[1] == []                              # it is optional
+
+
+def test_the_extension_follows_torch(tree, tmp_path):
+    """Built again when another torch is there, not otherwise, under the name of this Python's extensions."""
+    fake = tmp_path / "site" / "torch"
+    (fake / "include" / "ATen").mkdir(parents=True)
+    (fake / "include" / "ATen" / "ATen.h").write_text("")
+    (fake / "__init__.py").write_text("")
+    env = dict(os.environ, PYTHONPATH=str(tmp_path / "site"))
+    for version, anew in (("1.0", True), ("1.0", False), ("2.0", True), ("2.0", False)):
+        (fake / "version.py").write_text(f"__version__, git_version = {version!r}, 'abc'\n")
+        done = subprocess.run(["make", "-C", tree.directory, "step-ops", f"CXX={tree.compiler}", f"PYTHON={sys.executable}"],
+                              capture_output=True, text=True, env=env, timeout=60)
+        assert done.returncode == 0, done.stderr
+        assert (f"-DSTEP_OPS_TORCH='\"{version} abc\"'" in done.stdout) == anew
+    assert tree.built() == ["_step_ops" + sysconfig.get_config_var("EXT_SUFFIX")]

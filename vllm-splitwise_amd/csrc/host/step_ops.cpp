@@ -587,6 +587,7 @@ PyMODINIT_FUNC PyInit__step_ops() {
 #undef NAME
   PyObject* m = PyModule_Create(&kModule);
   if (m == nullptr) return nullptr;
+  PyModule_AddStringConstant(m, "TORCH", STEP_OPS_TORCH);      // _native.py uses no other torch's
   PyModule_AddIntConstant(m, "SW_ABI_VERSION", SW_ABI_VERSION);
   PyModule_AddIntConstant(m, "SWM_ABI_VERSION", SWM_ABI_VERSION);
   return m;
