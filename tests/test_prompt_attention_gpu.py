@@ -279,6 +279,33 @@ def test_finished_rows_go_out_alike_whatever_the_alignment(H, G, d, dv, way):
     torch.testing.assert_close(outs[0].double(), ref, atol=2e-4, rtol=2.0 ** -7)
 
 
+def test_every_gate_weighs_as_in_the_general_kernel(way):
+    """A first token sees its own value alone, so that its result is value times sigmoid(gate) rounded once: the general kernel's bits
+    for every bf16 gate there is, and with large values those whose sigmoid is no normal number any more (2^-126 is reached at -87.3)."""
+    from splitwise_amd import _C
+    H, G, d, lengths = 16, 4, 128, [(0, 33)] * 32
+    batch, pages = _step(lengths, 16)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    rows, first = 32 * 33, torch.arange(0, 32 * 33, 33, device=DEV)
+    kc = torch.randn(pages, 16, G * d, generator=g, device=DEV).to(torch.bfloat16)
+    vc = (torch.randn(pages, 16, G * d, generator=g, device=DEV) * 2.0 ** 40).to(torch.bfloat16)
+    q = torch.randn(rows * H * d + 1, generator=g, device=DEV)
+    gate = torch.zeros(rows, H * d, dtype=torch.bfloat16, device=DEV)
+    gate[first] = torch.arange(-32768, 32768, device=DEV).to(torch.int16).view(torch.bfloat16).view(32, H * d)
+    outs = []
+    for lead in (0, 1):
+        at = q[lead:lead + rows * H * d].view(rows, H * d)
+        assert way(at, kc, vc, batch, H, G, d, d) == (GENERAL if lead else PROMPT)
+        out = torch.empty(rows, H * d, dtype=torch.bfloat16, device=DEV)
+        _C.mixer_ops.capped_attention(out, at, kc, vc, gate, batch, H, G, d, d, d ** -0.5)
+        outs.append(out[first].float())
+    torch.testing.assert_close(outs[0], outs[1], atol=0, rtol=0, equal_nan=True)
+    value = vc[batch.block_tables[:, 0].long(), 0].double().view(32, G, 1, d).expand(32, G, H // G, d).reshape(32, H * d)
+    ref = value * torch.sigmoid(gate[first].double())
+    seen = (gate[first].double() > -88.5) & ref.abs().isfinite()             # (from -88.7 on e^-gate overflows in fp32)
+    assert float(((outs[0].double() - ref).abs() / ref.abs())[seen].max()) < 2.0 ** -8 * 1.001
+
+
 @pytest.mark.parametrize("H,G,d,dv,page", [(4, 4, 128, 128, 16), (8, 2, 64, 96, 16), (6, 2, 40, 24, 8), (8, 1, 16, 8, 32),
                                            (5, 1, 104, 128, 12)])
 @pytest.mark.parametrize("option", ["plain", "cap", "window", "chunk", "sink", "learned sink", "sigmoid", "values in the keys"])

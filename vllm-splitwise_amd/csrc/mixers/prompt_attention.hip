@@ -68,15 +68,6 @@ __host__ __device__ constexpr int pa_lds_bytes(int nb, int groups) {
 
 __host__ __device__ constexpr int pa_query_bytes(int nb) { return kPaWaves * 2 * 2 * nb * 1024; }         // two parts of the queries
 
-// 1 / (1 + e^-x) in a third of the instructions of expf and a division, to 2^-22: 2^t with t = -x log2 e and the product's rounding
-// error put right (beyond 2^120 it is no matter)
-__device__ __forceinline__ float short_sigmoid(float x) {
-  const float t = -kLog2e * x;
-  const float lost = fmaf(-kLog2e, x, -t) - 1.92596299e-8f * x;          // log2 e = kLog2e + 1.926e-8
-  const float e = __builtin_amdgcn_exp2f(t);
-  return __builtin_amdgcn_rcpf(1.0f + (fabsf(t) < 120.0f ? fmaf(e, 0.69314718f * lost, e) : e));
-}
-
 // a wave's finished rows, or the row that it works out again
 __host__ __device__ constexpr int pa_rows_bytes(int nb) {
   return 4 * (32 * (nb * 32 + 4) > kPlainRowLds ? 32 * (nb * 32 + 4) : kPlainRowLds);
@@ -554,8 +545,8 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
         const uint32_t w[4] = {gw.x, gw.y, gw.z, gw.w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          v[2 * j] *= short_sigmoid(__uint_as_float(w[j] << 16));
-          v[2 * j + 1] *= short_sigmoid(__uint_as_float(w[j] & 0xffff0000u));
+          v[2 * j] *= sigmoidf_(__uint_as_float(w[j] << 16));
+          v[2 * j + 1] *= sigmoidf_(__uint_as_float(w[j] & 0xffff0000u));
         }
       }
       if (!mine) continue;
