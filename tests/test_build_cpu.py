@@ -123,3 +123,28 @@ def test_the_extension_follows_torch(tree, tmp_path):
         assert done.returncode == 0, done.stderr
         assert (f"-DSTEP_OPS_TORCH='\"{version} abc\"'" in done.stdout) == anew
     assert tree.built() == ["_step_ops" + sysconfig.get_config_var("EXT_SUFFIX")]
+
+
+def test_calls_that_the_extension_does_not_take_are_not_offered(monkeypatch):
+    """Slopes, sigmoid weights and values inside the key rows are common forms that it leaves to Python, by a throw."""
+    import torch
+    from splitwise_amd import _C, _C_mixers
+    offered = []
+    spy = types.SimpleNamespace(**{name: (lambda *args, name=name: offered.append(name))
+                                   for name in ("paged_attention_v1", "prefill_attention", "capped_attention")})
+    monkeypatch.setattr(_C, "_native", spy)
+    monkeypatch.setattr(_C_mixers, "_native", spy)
+    t = torch.zeros(1)
+    calls = {"paged_attention_v1": (lambda slopes: _C.ops.paged_attention_v1(t, t, t, t, 1, 1.0, t, t, 16, 1, slopes, "auto"), [None], [t]),
+             "prefill_attention": (lambda slopes: _C.ops.prefill_attention(t, t, t, t, t, t, 1, 1.0, slopes), [None], [t]),
+             "capped_attention": (lambda v, bias: _C_mixers.capped_attention(t, t, t, v, None, None, 1, 1, 8, 8, 1.0, score_bias=bias),
+                                  [t, None], [None, None, t, t])}
+    for name, (call, plain, others) in calls.items():
+        for i in range(0, len(others), len(plain)):
+            with pytest.raises(RuntimeError, match="need tensors on a HIP device"):
+                call(*others[i:i + len(plain)])
+        assert offered == []
+        with pytest.raises(RuntimeError, match="need tensors on a HIP device"):
+            call(*plain)
+        assert offered == [name]
+        offered.clear()

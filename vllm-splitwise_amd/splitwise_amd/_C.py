@@ -320,10 +320,11 @@ def paged_attention_v1(out: torch.Tensor, query: torch.Tensor, key_cache: torch.
                        max_context_len: int, alibi_slopes: Optional[torch.Tensor],
                        kv_cache_dtype: str) -> None:
     """``ops.paged_attention_v1`` (csrc/attention/attention_kernels.cu:711-747)."""
-    status = _native.paged_attention_v1(out, query, key_cache, value_cache, num_kv_heads, scale, block_tables,
-                                        context_lens, block_size, max_context_len, alibi_slopes, kv_cache_dtype)
-    if status is not None:
-        return _check(status)
+    if alibi_slopes is None:                       # (a call that the native function does not take costs 2 us there)
+        status = _native.paged_attention_v1(out, query, key_cache, value_cache, num_kv_heads, scale, block_tables,
+                                            context_lens, block_size, max_context_len, alibi_slopes, kv_cache_dtype)
+        if status is not None:
+            return _check(status)
     alibi_slopes = _pa_common(query, key_cache, value_cache, block_tables, context_lens, alibi_slopes)
     act = _act_dtype(query)
     cache = _cache_dtype(kv_cache_dtype, act)
@@ -385,10 +386,11 @@ def prefill_attention(out: torch.Tensor, query: torch.Tensor, key: torch.Tensor,
                       alibi_slopes: Optional[torch.Tensor] = None, sliding_window: Optional[int] = None) -> None:
     """Causal prompt attention over (start, length) sequences; stands where the reference calls
     xformers / flash-attn (backends/xformers.py:155-164).  query [T, H, D], key/value [T, KVH, D]."""
-    status = _native.prefill_attention(out, query, key, value, seq_starts, seq_lens,
-                                       max_seq_len, scale, alibi_slopes, sliding_window)
-    if status is not None:
-        return _check(status)
+    if alibi_slopes is None:
+        status = _native.prefill_attention(out, query, key, value, seq_starts, seq_lens,
+                                           max_seq_len, scale, alibi_slopes, sliding_window)
+        if status is not None:
+            return _check(status)
     _require_cuda(out, query, key, value, seq_starts, seq_lens)
     if seq_starts.dtype != torch.int32 or seq_lens.dtype != torch.int32:
         raise RuntimeError("prefill_attention: seq_starts and seq_lens must be int32")

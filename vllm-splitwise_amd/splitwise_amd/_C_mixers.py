@@ -711,10 +711,11 @@ def capped_attention(out: torch.Tensor, q: torch.Tensor, key_cache: torch.Tensor
     denominator, exp(0), or exp(sink[head]) when it is a tensor (fp32 [heads]).  ``value_cache`` None: a token's values are the first kv_heads * vdim elements of its
     key row (attention over a shared latent).  ``score_bias`` (fp32 [heads]): no softmax -- a seen key weighs
     sigmoid(score + score_bias[head]) and the weights are not normalised (window mask only)."""
-    status = _native.capped_attention(out, q, key_cache, value_cache, gate, batch, heads, kv_heads, dim,
-                                      vdim, scale, softcap, window, chunk, sink, score_bias)
-    if status is not None:
-        return _check(status)
+    if value_cache is not None and score_bias is None:      # (a call that the native function does not take costs 2 us there)
+        status = _native.capped_attention(out, q, key_cache, value_cache, gate, batch, heads, kv_heads, dim,
+                                          vdim, scale, softcap, window, chunk, sink, score_bias)
+        if status is not None:
+            return _check(status)
     learned = sink if isinstance(sink, torch.Tensor) else None
     _dev(out, q, key_cache, value_cache, gate, score_bias, learned)
     if learned is not None:
