@@ -140,6 +140,33 @@ def test_gptq_gemm_takes_an_input_on_any_element(m):
     _close(got, quant.gptq_gemm(a, w, qzeros, scales, None, True))
 
 
+@pytest.mark.parametrize("m,k,n", [(33, 1536, 136), (61, 2816, 328), (100, 1024, 1000), (128, 2560, 520), (160, 1024, 264),
+                                   (250, 1280, 520), (200, 512, 16648)])
+def test_gptq_gemm_an_input_off_16_bytes_takes_the_same_tiles(m, k, n):
+    """... copied in front of them (or as it is, where they take it): the same bits.  In a workspace without room for the copy, or
+    whose end is on no boundary, the result stays right, and nothing is written behind that end."""
+    from splitwise_amd import _C
+    qweight, qzeros, scales, _ = _gptq_case(k, n, 128, m)
+    a = np.random.default_rng(m).standard_normal((m, k)).astype(np.float16)
+    w, z, sc = _dev(quant.gptq_shuffle(qweight)), _dev(qzeros), _dev(scales)
+    off = torch.empty(m * k + 1, dtype=torch.float16, device="cuda")[1:].view(m, k)
+    off.copy_(_dev(a))
+    got = _C.ops.gptq_gemm(off, w, z, sc, None, True, 4)
+    assert torch.equal(got, _C.ops.gptq_gemm(_dev(a), w, z, sc, None, True, 4))
+    ref = quant.gptq_gemm(a, w.cpu().numpy(), qzeros, scales, None, True)
+    _close(got, ref)
+    for room in (0, -(-m * k * 2 // 256) * 256 + 6):
+        size = (16 << 10) + room
+        ws = torch.zeros(size + 64, dtype=torch.uint8, device="cuda")
+        ws[size:] = 77
+        c = torch.full((m, n), float("nan"), dtype=torch.float16, device="cuda")
+        lib = _C.load_library()
+        assert lib.sw_gptq_gemm(c.data_ptr(), off.data_ptr(), w.data_ptr(), z.data_ptr(), sc.data_ptr(), None, m, n, k, k // 128, 1, 4,
+                                ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream) == 0
+        _close(c, ref)
+        assert (ws[size:] == 77).all() and (ws[:16 << 10] == 0).all()
+
+
 def test_gptq_gemm_tile_kernel_on_seeded_random_shapes():
     """Shapes drawn at random inside the 128-row tile kernel's domain (rows 129..256, k in multiples of 256,
     columns in multiples of 8, groups of 64 / 128 / 256 / all of k), against the CPU restatement."""

@@ -1072,6 +1072,16 @@ __global__ void permute_columns_kernel(uint16_t* __restrict__ dst, const uint16_
   dst[idx] = src[(size_t)m * K + perm[k]];
 }
 
+// eights of fp16 from any element to 16 bytes
+__global__ void copy_halves_kernel(uint16_t* __restrict__ dst, const uint16_t* __restrict__ src, int64_t eights) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= eights) return;
+  uint32_t w[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) w[j] = src[8 * i + 2 * j] | (uint32_t)src[8 * i + 2 * j + 1] << 16;
+  *reinterpret_cast<uint4*>(dst + 8 * i) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+
 // one thread: one word row x 4 columns -> 8 rows x 4 fp16
 __global__ void gptq_dequant_kernel(uint16_t* __restrict__ out, const uint32_t* __restrict__ qweight,
                                     const uint32_t* __restrict__ qzeros, const uint16_t* __restrict__ scales,
@@ -1604,31 +1614,36 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
   int32_t* counters = static_cast<int32_t*>(workspace);
   char* ws = static_cast<char*>(workspace);
   int64_t avail = workspace_bytes;
-  if (g_idx) {                                        // act-order: A's columns follow the shuffled row order
-    const int64_t abytes = ((int64_t)M * K * 2 + 255) / 256 * 256;
+  StreamTile stream_to = K % 256 == 0 ? stream_tile(M, N, K) : StreamTile::kNone;
+  // Streamed tiles take A on 16 bytes.  An input of more than 32 rows that lies elsewhere is copied in front of them; the kernels that
+  // take it as it is are 1.4 to 5 times slower (us, as it is / copied: 4096 k x 12288, 33 rows 44 / 20, 61 rows 61 / 20.5, 128 rows
+  // 120 / 27; 5120 x 5120, 61 rows 30 / 16, 250 rows 39 / 29).
+  const int64_t abytes = ((int64_t)M * K * 2 + 255) / 256 * 256;
+  const bool moved = !g_idx && stream_to != StreamTile::kNone && M > 32 && reinterpret_cast<uintptr_t>(ap) % 16 != 0 &&
+                     workspace_bytes >= kCounterBytes + abytes;
+  if (g_idx || moved) {                               // act-order: A's columns follow the shuffled row order
     SW_CHECK_ARG(workspace_bytes >= kCounterBytes + abytes, "gptq_gemm: workspace too small for the permuted input");
-    avail -= abytes;
-    uint16_t* a_perm = reinterpret_cast<uint16_t*>(ws + avail);
+    avail = (workspace_bytes - abytes) / 256 * 256;
+    uint16_t* at_end = reinterpret_cast<uint16_t*>(ws + avail);
     const int64_t total = (int64_t)M * K;
-    hipLaunchKernelGGL(permute_columns_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, a_perm, ap,
-                       g_idx, M, K);
+    if (g_idx)
+      hipLaunchKernelGGL(permute_columns_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, at_end, ap,
+                         g_idx, M, K);
+    else                                              // (k is a multiple of 256: so are the elements)
+      hipLaunchKernelGGL(copy_halves_kernel, dim3((unsigned)((total / 8 + 255) / 256)), dim3(256), 0, st, at_end, ap, total / 8);
     SW_CHECK_LAUNCH();
-    ap = a_perm;
+    ap = at_end;
   }
   float* partials = reinterpret_cast<float*>(ws + kCounterBytes);
-  // Kernel choice: streamed tiles where stream_tile() names one (k in multiples of 256, A on 16 bytes); above 128 rows and past
-  // 256 tiles of 128 x 128, tiles of 128 x 256, which are one round of workgroups (27648 columns at 256 rows: 79 us against 87);
+  // Kernel choice: streamed tiles where stream_tile() names one (k in multiples of 256, A on 16 bytes); otherwise above 128 rows
+  // tiles of 128 x 256, which are one round of workgroups where 128 x 128 are more (27648 columns at 256 rows: 79 us against 87);
   // up to 32 rows otherwise one row tile per workgroup, k split across its waves, A straight from memory; every other shape k
   // across waves up to 128 rows, the 64-row tiled kernel above.
   int cp = 2, mt = M > 64 ? 4 : M > 32 ? 2 : 1;
   bool tiled = M > 128 && K % kChunkK == 0 && group_size % 16 == 0;
   int waves = 8, chunk = kChunkK, tiled_mt = 2, force_ks = 0;
-  StreamTile stream_to = StreamTile::kNone;
-  bool wide = false;                                  // 128 x 256 tiles
-  if (K % 256 == 0 && reinterpret_cast<uintptr_t>(ap) % 16 == 0) {
-    stream_to = stream_tile(M, N, K);
-    wide = stream_to == StreamTile::kNone && M > 128 && group_size % 64 == 0;
-  }
+  if (reinterpret_cast<uintptr_t>(ap) % 16 != 0) stream_to = StreamTile::kNone;
+  bool wide = stream_to == StreamTile::kNone && M > 128 && K % 256 == 0 && group_size % 64 == 0;      // 128 x 256 tiles
 #ifdef SW_QUANT_EXPERIMENT                                     // tuning builds only: never in the shipped library
   if (const char* env = getenv("SW_QUANT_CP")) cp = atoi(env) == 4 ? 4 : 2;
   if (const char* env = getenv("SW_QUANT_MT")) mt = atoi(env);
