@@ -114,15 +114,23 @@ def test_gptq_gemm_64_row_tiles_in_chunks_of_512(m, k, n, group):
     test_gptq_gemm_shuffled(m, k, n, group)
 
 
-@pytest.mark.parametrize("m,k,n,group", [
-    # 32 x 128: as many stages as are asked for ahead; splits, a ragged last column tile
-    (24, 512, 93760, 128), (31, 5120, 9400, 32),
-    # 64 x 64: one stage; a split for each stage; splits that are not alike
-    (33, 256, 8, 32), (64, 768, 72, 64), (61, 2816, 328, 128), (100, 4096, 1000, 4096),
-    # 64 x 128: fewer stages than are asked for ahead, one more; splits
-    (33, 256, 16392, 32), (64, 512, 16520, 64), (128, 6912, 5128, 128), (193, 2560, 5064, 32),
-    # 128 x 128: the same
-    (65, 256, 16520, 32), (200, 768, 11008, 128), (250, 5376, 5128, 128), (129, 512, 16392, 32)])
+# by the kernel that they go to (test_quant_plan_cpu.py asks the rule)
+ROUTES = {
+    # as many stages as are asked for ahead; splits, a ragged last column tile; few splits and many
+    "k32x128": [(28, 512, 93760, 128), (31, 5120, 9400, 32), (17, 5120, 11272, 128), (32, 28672, 2056, 128)],
+    # one stage; a split for each stage; splits that are not alike
+    "k64x64": [(33, 256, 8, 32), (64, 768, 72, 64), (61, 2816, 328, 128), (100, 4096, 1000, 4096)],
+    # fewer stages than are asked for ahead, one more; splits
+    "k64x128": [(33, 256, 16392, 32), (64, 512, 16520, 64), (128, 6912, 5128, 128), (193, 2560, 5064, 32)],
+    # the same; long walks
+    "k128x128": [(65, 256, 33288, 32), (200, 768, 11008, 128), (250, 5376, 5128, 128), (129, 512, 16384, 32), (70, 19456, 8200, 128)],
+    "k128x256": [(200, 256, 16648, 128)],
+    "kAcrossWaves": [(24, 512, 93760, 128), (8, 5120, 9400, 128)],
+    "k64Rows": [(140, 256, 33032, 32), (129, 512, 16392, 32)],
+}
+
+
+@pytest.mark.parametrize("m,k,n,group", [shape for shapes in ROUTES.values() for shape in shapes] + [(65, 256, 16520, 32)])
 def test_gptq_gemm_streamed_tiles(m, k, n, group):
     test_gptq_gemm_shuffled(m, k, n, group)
 

@@ -28,6 +28,7 @@
 //     arrive at a tile (counted with one atomic) adds the partials in a fixed order: one
 //     launch, no atomics on data, bitwise reproducible results.
 #include "common.cuh"
+#include "quant_plan.h"
 #include <stdlib.h>
 #include <algorithm>
 #include <type_traits>
@@ -1461,34 +1462,6 @@ int pick_ksplit(int tiles, int units, int min_units, int M, int N, int64_t works
   return ks < 1 ? 1 : ks;
 }
 
-// Which tiles the streamed kernel takes, rows x columns.  A launch is one round of at most 256 workgroups where the tiles allow it; k
-// is split as often as that leaves room for.  Measured in microseconds at the matrices of 7B and 13B layers, whole and halved:
-enum class StreamTile { kNone, k32x128, k64x64, k64x128, k128x128 };
-StreamTile stream_tile(int64_t M, int64_t N, int64_t K) {
-  auto tiles = [&](int rows, int cols) { return ((M + rows - 1) / rows) * ((N + cols - 1) / cols); };
-  if (M <= 32) {
-    // k across waves reads A from memory: the more rows and weights, the sooner the streamed tile is ahead (32 rows: 13824 k x 5120
-    // 20.5 with k across waves / 18.8 streamed, 12288 x 4096 16.0 / 14.2, 5120 x 5120 12.1 / 12.4; 24 rows: 18.2 / 18.4,
-    // 14.3 / 14.2; 17 rows: 15360 x 5120 17.0 / 16.8, 12288 x 4096 13.3 / 14.1; 12 rows: 22016 x 4096 21.6 / 19.8, 15360 x 5120
-    // 16.2 / 16.8; 8 rows: 27648 x 5120 25.2 / 24.9)
-    const int64_t from = M >= 24 ? 48000000 : M > 16 ? 78000000 : M > 8 ? 90000000 : INT64_MAX;
-    return N * K >= from ? StreamTile::k32x128 : StreamTile::kNone;
-  }
-  if (tiles(64, 64) <= 256) {
-    // up to 64 rows always (128 columns instead: 13.1 -> 14.7 at 5120 x 5120, 20.3 -> 21.3 at 13824 x 5120); with more rows where the
-    // splits fill the chip or k is short (100 rows: 7680 x 5120 18.6, 64 x 128 19.8; 6912 k x 5120 21.0 / 19.0)
-    const int64_t t = tiles(64, 64), filled = 256 / t * t;
-    if (M <= 64 || K <= 5120 || filled >= 224) return StreamTile::k64x64;
-  }
-  if (M <= 64) return StreamTile::k64x128;            // 27648 x 5120 28.9, 64 x 64 in two rounds 36.3
-  const int64_t t128 = tiles(128, 128);
-  // 27648 columns 42.2, 64 x 128 50.3; 15360 columns 30.0 / 30.6; 12288 24.2 / 24.0
-  if (M <= 128) return t128 > 128 ? StreamTile::k128x128 : StreamTile::k64x128;
-  if (t128 > 256) return StreamTile::kNone;
-  // 192 rows: 11008 k x 4096 32.4 (96 tiles, 2 splits), 128 x 128 35.1; 256 rows: 13824 k x 5120 65.5 (160 tiles) / 45.5, but 2560 k 16.2 / 21.7
-  const int64_t t = tiles(64, 128), filled = t <= 256 ? 256 / t * t : 0;
-  return t <= 256 && (K <= 4096 || filled >= 180) ? StreamTile::k64x128 : StreamTile::k128x128;
-}
 int stream_splits(int64_t tiles, int stages, int M, int N, int64_t workspace_bytes, int forced) {
   if (tiles > kCounterInts) return 1;
   int64_t ks = forced > 0 ? forced : 256 / tiles;
@@ -1614,13 +1587,13 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
   int32_t* counters = static_cast<int32_t*>(workspace);
   char* ws = static_cast<char*>(workspace);
   int64_t avail = workspace_bytes;
-  StreamTile stream_to = K % 256 == 0 ? stream_tile(M, N, K) : StreamTile::kNone;
   // Streamed tiles take A on 16 bytes.  An input of more than 32 rows that lies elsewhere is copied in front of them; the kernels that
   // take it as it is are 1.4 to 5 times slower (us, as it is / copied: 4096 k x 12288, 33 rows 44 / 20, 61 rows 61 / 20.5, 128 rows
   // 120 / 27; 5120 x 5120, 61 rows 30 / 16, 250 rows 39 / 29).
   const int64_t abytes = ((int64_t)M * K * 2 + 255) / 256 * 256;
-  const bool moved = !g_idx && stream_to != StreamTile::kNone && M > 32 && reinterpret_cast<uintptr_t>(ap) % 16 != 0 &&
-                     workspace_bytes >= kCounterBytes + abytes;
+  const bool ws16 = reinterpret_cast<uintptr_t>(ws) % 16 == 0, a16 = reinterpret_cast<uintptr_t>(ap) % 16 == 0;
+  Int4Way way = int4_way(M, N, K, group_size, g_idx ? ws16 : a16, ws16 && workspace_bytes >= kCounterBytes + abytes);
+  const bool moved = !g_idx && !a16 && int4_streamed(way);
   if (g_idx || moved) {                               // act-order: A's columns follow the shuffled row order
     SW_CHECK_ARG(workspace_bytes >= kCounterBytes + abytes, "gptq_gemm: workspace too small for the permuted input");
     avail = (workspace_bytes - abytes) / 256 * 256;
@@ -1635,15 +1608,9 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
     ap = at_end;
   }
   float* partials = reinterpret_cast<float*>(ws + kCounterBytes);
-  // Kernel choice: streamed tiles where stream_tile() names one (k in multiples of 256, A on 16 bytes); otherwise above 128 rows
-  // tiles of 128 x 256, which are one round of workgroups where 128 x 128 are more (27648 columns at 256 rows: 79 us against 87);
-  // up to 32 rows otherwise one row tile per workgroup, k split across its waves, A straight from memory; every other shape k
-  // across waves up to 128 rows, the 64-row tiled kernel above.
   int cp = 2, mt = M > 64 ? 4 : M > 32 ? 2 : 1;
-  bool tiled = M > 128 && K % kChunkK == 0 && group_size % 16 == 0;
+  bool tiled = way == Int4Way::k64Rows;
   int waves = 8, chunk = kChunkK, tiled_mt = 2, force_ks = 0;
-  if (reinterpret_cast<uintptr_t>(ap) % 16 != 0) stream_to = StreamTile::kNone;
-  bool wide = stream_to == StreamTile::kNone && M > 128 && K % 256 == 0 && group_size % 64 == 0;      // 128 x 256 tiles
 #ifdef SW_QUANT_EXPERIMENT                                     // tuning builds only: never in the shipped library
   if (const char* env = getenv("SW_QUANT_CP")) cp = atoi(env) == 4 ? 4 : 2;
   if (const char* env = getenv("SW_QUANT_MT")) mt = atoi(env);
@@ -1652,16 +1619,16 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
   if (const char* env = getenv("SW_QUANT_CHUNK")) chunk = atoi(env) == 128 ? 128 : 256;
   if (const char* env = getenv("SW_QUANT_TMT")) tiled_mt = atoi(env);
   if (const char* env = getenv("SW_QUANT_KSPLIT")) force_ks = atoi(env);
-  // 0: off; 1..4: the StreamTile; 5: 128 x 256
+  // 0: none; 1..5: streamed tiles as in Int4Way, 128 x 256
   if (const char* env = getenv("SW_QUANT_TILE")) {
     const int t = atoi(env);
-    stream_to = t >= 1 && t <= 4 && K % 256 == 0 ? static_cast<StreamTile>(t) : StreamTile::kNone;
-    wide = t == 5 && K % 256 == 0 && group_size % 64 == 0;
+    if (t >= 1 && t <= 5 && K % 256 == 0 && (t < 5 || group_size % 64 == 0)) way = static_cast<Int4Way>(t);
+    else way = Int4Way::kAcrossWaves;
   }
 #endif
   if (mt == 3 || mt > 4) mt = 4;
   if (tiled) mt = tiled_mt;
-  if (stream_to != StreamTile::kNone) {
+  if (int4_streamed(way)) {
 #define SW_GPTQ_STREAM(MT_, CG_, R_, PER_SIMD_)                                                                  \
   do {                                                                                                           \
     auto kern = gptq_gemm_stream_kernel<MT_, CG_, R_, PER_SIMD_>;                                                \
@@ -1673,17 +1640,17 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
     hipLaunchKernelGGL(kern, dim3((ct * rt * ks + 7) / 8 * 8), dim3(512), lds_bytes, st, out, ap, qweight,       \
                        qzeros, sp, M, N, K, group_size, ks, ct, rt, zoff, partials, counters);                   \
   } while (0)
-    switch (stream_to) {
-      case StreamTile::k32x128: SW_GPTQ_STREAM(1, 2, 4, 4); break;
-      case StreamTile::k64x64: SW_GPTQ_STREAM(2, 1, 3, 2); break;
-      case StreamTile::k64x128: SW_GPTQ_STREAM(2, 2, 3, 4); break;
+    switch (way) {
+      case Int4Way::k32x128: SW_GPTQ_STREAM(1, 2, 4, 4); break;
+      case Int4Way::k64x64: SW_GPTQ_STREAM(2, 1, 3, 2); break;
+      case Int4Way::k64x128: SW_GPTQ_STREAM(2, 2, 3, 4); break;
       default: SW_GPTQ_STREAM(4, 2, 3, 2); break;
     }
 #undef SW_GPTQ_STREAM
     SW_CHECK_LAUNCH();
     return SW_OK;
   }
-  if (wide) {
+  if (way == Int4Way::k128x256) {
     auto kern = gptq_gemm_tile128_kernel;
     SW_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                      kT128Lds));
