@@ -794,7 +794,8 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
 //
 // The waits count this wave's loads, so nothing may move past them: the pointers are not __restrict__ (a load of memory that nothing
 // else writes could be moved behind a wait, which then would not wait for the A before it), the loop has no way around it,
-// and sched_barriers keep the order inside a block.
+// and sched_barriers keep the order inside a block.  tests/test_quant_waits_cpu.py follows every path of the built kernels: a register
+// spilled or a load added, split or moved would make a wait too short.
 template <int CG> constexpr int stage_k() { return 256 / CG; }              // 32 k for each of the 8 / CG k parts
 template <int MT, int CG, int R> constexpr int stream_lds() {
   constexpr int ring = R * MT * 64 * stage_k<CG>(), red = (MT > 2 || CG == 1 ? 2 : 1) * 65536;
