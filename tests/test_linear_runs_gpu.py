@@ -1,6 +1,9 @@
 """Linear-attention steps whose runs are cut into segments, and steps whose decoding sequences go another way than the long runs
 beside them, against the rule in 64 bits token by token.  States and outputs are fp32 sums of products whose decays are
 exponentials of sums: a relative error of about 2e-7 of their size in the 2-norm, 5e-6 of their root mean square for the worst."""
+import ctypes
+import os
+import subprocess
 from types import SimpleNamespace
 
 import pytest
@@ -81,10 +84,70 @@ def test_segments_and_mixed_steps(rule, heads, dim, vdim, lens):
                                             (2, 64, 17)])
 @pytest.mark.parametrize("lens", [[1] * 7, [5, 1, 0, 3, 5], [1] * 9 + [40, 6, 16, 2]], ids=str)
 def test_few_tokens(rule, heads, dim, vdim, lens):
-    """Token by token with the state in whole rows, alone and with longer runs left to the chunks' kernels: key sizes that fill the threads' rows or not, value sizes of one piece of 16
-    bytes, of part of a workgroup's, of several workgroups (and one that has no such pieces and goes by chunks).  (Some hundred outputs: one of a
-    few may be a small difference of its terms.)"""
+    """Token by token with the state in whole rows, alone and in steps of few sequences of which one walks: key sizes that fill the
+    threads' rows or not, value sizes of one piece of 16 bytes, of part of a workgroup's, of several workgroups (and one that has no
+    such pieces and goes by chunks).  (Some hundred outputs: one of a few may be a small difference of its terms.)"""
     test_segments_and_mixed_steps(rule, heads, dim, vdim, lens)
+
+
+@pytest.fixture(scope="module")
+def shares(tmp_path_factory):
+    """-> up to how many tokens a sequence of the step goes token by token and up to how many it does not walk, by linear_plan.h."""
+    at = tmp_path_factory.mktemp("plan")
+    (at / "plan.cpp").write_text(r"""
+#include "linear_plan.h"
+extern "C" void shares(int per_channel, long rows, int seqs, int longest, int heads, int dim, int vdim, int* out) {
+  out[1] = swm::linear_at_most(per_channel, rows, seqs, longest, heads, dim, vdim);
+  out[0] = swm::linear_step_tokens(out[1], rows, seqs, longest);
+}
+""")
+    mixers = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "vllm-splitwise_amd", "csrc", "mixers")
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I", mixers, str(at / "plan.cpp"), "-o", str(at / "plan.so")], check=True)
+    lib = ctypes.CDLL(str(at / "plan.so"))
+
+    def ask(per_channel, lens, heads, dim, vdim):
+        out = (ctypes.c_int * 2)()
+        lib.shares(per_channel, ctypes.c_long(sum(lens)), len(lens), max(lens), heads, dim, vdim, out)
+        return tuple(out)
+    return ask
+
+
+@pytest.mark.parametrize("rule", ["gla", "lightning", "retention"])
+@pytest.mark.parametrize("heads,dim,vdim", [(16, 128, 128), (2, 256, 260), (64, 8, 4), (16, 40, 12), (2, 96, 132), (1, 200, 1024), (2, 33, 64),
+                                            (2, 64, 17)])
+def test_few_tokens_beside_runs_by_chunks_and_runs_that_walk(rule, heads, dim, vdim, shares):
+    """The three ways in one step, for the same sizes."""
+    lens = ([1] * 9 + [5, 0, 3, 2]) * -(-180 * 128 // (heads * dim * 13)) + [97, 16, 6, 60]
+    assert shares(rule == "gla", lens, heads, dim, vdim) == (5, 16)
+    test_segments_and_mixed_steps(rule, heads, dim, vdim, lens)
+
+
+@pytest.mark.parametrize("rule", ["lightning", "retention"])
+@pytest.mark.parametrize("portion", [1, 2, 3, 5])
+def test_portions_of_few_tokens_add_up(rule, portion):
+    """1600 tokens in portions of as many as go token by token, one decay per head.  A token rounds the state about once, by 2^-24 of
+    an element at most and half of that typically; those of the last 1 / (1 - decay^2) tokens (500 at the slowest of the decays) are still
+    in it: 22 x 3e-8, measured 7e-7.  (A chunk's power of the decay would be rounded alike in every portion: 3e-6 to 8e-6.)"""
+    from splitwise_amd import _C
+    heads, dim, seqs, total = 4, 64, 2, 1600
+    g = torch.Generator(device=DEV).manual_seed(portion)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)          # noqa: E731
+    q, k, v = (torch.randn(total, seqs, heads * dim, generator=g, device=DEV) for _ in range(3))
+    decay, state = torch.linspace(0.3, 0.999, heads, device=DEV), torch.zeros(seqs, heads, dim, dim, device=DEV)
+    q64, k64, v64 = (t.double().view(total, seqs, heads, dim) for t in (q, k, v))
+    if rule == "lightning":
+        q64, k64, v64 = (torch.nn.functional.silu(t) for t in (q64, k64, v64))
+    end = state.double()
+    for t in range(total):
+        end = decay.double().view(1, heads, 1, 1) * end + k64[t][..., None] * v64[t][..., None, :]
+    for first in range(0, total, portion):
+        m = min(portion, total - first)
+        batch = SimpleNamespace(q_start=i32([0, m, 2 * m]), ctx_len=i32([first] * seqs), state_slot=i32([0, 1]), max_state_slot=1,
+                                max_query_len=m, token_seq=i32([0] * m + [1] * m))
+        part = [t[first:first + m].transpose(0, 1).reshape(seqs * m, -1).contiguous() for t in (q, k, v)]
+        out = torch.empty(seqs * m, heads * dim, device=DEV)
+        getattr(_C.mixer_ops, rule)(out, *part, decay, state, batch, heads, dim, dim)
+    assert float((state.double() - end).norm() / end.norm()) < 1.2e-6
 
 
 @pytest.mark.parametrize("said", [0, 1, 3])

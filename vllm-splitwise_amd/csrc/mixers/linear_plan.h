@@ -38,14 +38,17 @@ inline int linear_at_most(bool per_channel, int64_t rows, int num_seqs, int max_
 
 // Up to how many tokens a sequence that does not walk goes token by token with the state in whole rows (linear_step.hip; 0: none does)
 // and not by chunks, whose kernels hold a state's columns (gla.hip, lightning.hip); max_query_len 0: not known.  Up to 5, where the
-// per-channel rule's chunks go token by token too: from there on a chunk rounds its state less often (1600 tokens in portions of 13: an
-// error of 9.4e-7 token by token, below 6e-7 by chunks).  Measured, norm and gate included (us, by chunks / token by token), 16 heads of
-// 128 x 128:
+// per-channel rule's chunks go token by token too; beyond, its chunks round the state less often.  The state's error after 1600 tokens in
+// portions, 4 heads of 128 x 128, token by token / by chunks: per channel 1.2e-6 / 1.2e-6 up to 5 tokens, chunks of 6 3.3e-7, of 13 3.0e-7; per
+// head 7e-7 / 7e-7 for 1 token, 7e-7 / 4e-6 for 2, 8e-6 for 3, 3e-6 for 5 (every portion multiplies by the same rounded power of the decay).
+// Measured, norm and gate included (us, by chunks / token by token), 16 heads of 128 x 128:
 //   1 token each, 1 sequence: gla 13.1 / 8.0, lightning 29.0 / 9.7, retention 25.8 / 6.6; 61: 35.3 / 28.4, 74.1 / 30.4, 68.3 / 25.7;
 //   4 tokens: 15.8 / 11.2, 29.2 / 12.3, 25.5 / 8.7; 61: 37.0 / 29.6, 70.1 / 29.2, 63.4 / 23.1.
 // 8 heads of 256 x 256, 61 sequences, 1 token: 197 / 64, 186 / 65, 179 / 62.
 // Where the rest of a step walks, runs of 6 tokens and more that do not are left to the chunks' kernels in a launch of their own, unless
 // what is not a multiple of the longest run looks like most of them (20 of 12 tokens beside 300: 71 us without that launch, 74 with it).
+// That looks at one long run: beside two of different length (512 and 400 tokens) decoding sequences go by chunks, as in steps whose
+// longest run has 6 to 16 tokens.
 inline int linear_step_tokens(int at_most, int64_t rows, int num_seqs, int max_query_len) {
   constexpr int kSteps = 5;
   if (max_query_len <= 0) return 0;
