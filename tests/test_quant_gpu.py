@@ -85,13 +85,11 @@ GEMM_SHAPES = [          # (M, K, N, group)
     (1, 128, 128, 128), (1, 2560, 5120, 128), (3, 256, 136, 32), (7, 1024, 520, 64), (8, 5120, 7680, 128),
     (16, 512, 384, 512), (32, 6912, 1024, 128), (33, 512, 256, 128), (50, 1024, 384, 64), (64, 2048, 1000, 128),
     (100, 512, 264, 32), (200, 1024, 512, 128), (5, 96, 64, 32), (40, 160, 72, 32), (130, 384, 200, 64),
-    # the 128-row tile kernel: ragged rows and columns, one and two row tiles, groups of 64 / 128 / 256 / all of k,
-    # k split across workgroups (few column tiles) and not (many), and the wide-matrix case from 97 rows on
+    # above 128 rows: ragged rows and columns, one and two row tiles, groups of 64 / 128 / 256 / all of k,
+    # k split across workgroups (few column tiles) and not (many); a wide matrix
     (129, 512, 136, 64), (256, 1024, 264, 128), (255, 768, 1024, 256), (192, 2560, 320, 64), (250, 1280, 72, 1280),
     (160, 256, 3200, 128), (100, 256, 7680, 128), (200, 256, 16648, 128),
-    # 33..128 rows: tiles of 64 columns whose 8 waves are 8 k parts -- 64-row tiles up to 64 rows (and, with a short
-    # k and few columns, two of them up to 128 rows), 128-row tiles otherwise; k split across workgroups (few
-    # columns, long k) and not
+    # 33..128 rows: tiles of 64 and 128 columns; k split across workgroups (few columns, long k) and not
     (40, 4096, 72, 128), (64, 256, 520, 64), (65, 3328, 72, 128), (100, 4096, 1000, 128), (128, 5120, 520, 64),
     (96, 512, 16648, 128), (128, 512, 264, 64), (70, 1024, 136, 128), (127, 3072, 8192, 256),
 ]
@@ -109,8 +107,8 @@ def test_gptq_gemm_shuffled(m, k, n, group):
 
 
 @pytest.mark.parametrize("m,k,n,group", [(33, 512, 72, 64), (64, 1536, 16648, 128), (61, 6144, 5120, 128), (47, 6656, 5128, 512)])
-def test_gptq_gemm_64_row_tiles_in_chunks_of_512(m, k, n, group):
-    """33..64 rows with k a multiple of 512: one chunk, several, and k split across workgroups (evenly and not)."""
+def test_gptq_gemm_k_in_multiples_of_512(m, k, n, group):
+    """33..64 rows with k a multiple of 512: not split, and split across workgroups (evenly and not)."""
     test_gptq_gemm_shuffled(m, k, n, group)
 
 
@@ -124,7 +122,8 @@ ROUTES = {
     "k64x128": [(33, 256, 16392, 32), (64, 512, 16520, 64), (128, 6912, 5128, 128), (193, 2560, 5064, 32)],
     # the same; long walks
     "k128x128": [(65, 256, 33288, 32), (200, 768, 11008, 128), (250, 5376, 5128, 128), (129, 512, 16384, 32), (70, 19456, 8200, 128)],
-    "k128x256": [(200, 256, 16648, 128)],
+    # chunks of 128 k: two, ten and forty of them, through three buffers two at a time; ragged rows and columns, two groups a chunk
+    "k128x256": [(200, 256, 16648, 128), (129, 1280, 16520, 64), (250, 5120, 16648, 128), (256, 2816, 16392, 2816)],
     "kAcrossWaves": [(24, 512, 93760, 128), (8, 5120, 9400, 128)],
     "k64Rows": [(140, 256, 33032, 32), (129, 512, 16392, 32)],
 }
@@ -175,9 +174,30 @@ def test_gptq_gemm_an_input_off_16_bytes_takes_the_same_tiles(m, k, n):
         assert (ws[size:] == 77).all() and (ws[:16 << 10] == 0).all()
 
 
-def test_gptq_gemm_tile_kernel_on_seeded_random_shapes():
-    """Shapes drawn at random inside the 128-row tile kernel's domain (rows 129..256, k in multiples of 256,
-    columns in multiples of 8, groups of 64 / 128 / 256 / all of k), against the CPU restatement."""
+@pytest.mark.parametrize("m,k,n,group,splits", [(160, 1280, 264, 128, 2), (250, 2816, 520, 64, 2), (129, 2304, 264, 2304, 3)])
+def test_gptq_gemm_wide_tiles_over_an_odd_number_of_chunks(m, k, n, group, splits):
+    """An input off 16 bytes without room for its copy: 128 x 256 tiles at any number of columns, k split as often as the workspace has
+    room for partial tiles; chunks of 128 k by split 5 and 5, 11 and 11, 6 each."""
+    from splitwise_amd import _C
+    qweight, qzeros, scales, _ = _gptq_case(k, n, group, m)
+    a = np.random.default_rng(m).standard_normal((m, k)).astype(np.float16)
+    w, z, sc = _dev(quant.gptq_shuffle(qweight)), _dev(qzeros), _dev(scales)
+    off = torch.empty(m * k + 1, dtype=torch.float16, device="cuda")[1:].view(m, k)
+    off.copy_(_dev(a))
+    room = splits * m * n * 4
+    assert room < m * k * 2
+    ws = torch.zeros((16 << 10) + room, dtype=torch.uint8, device="cuda")
+    lib = _C.load_library()
+    for _ in range(2):                                       # (the counters are left as they were)
+        c = torch.full((m, n), float("nan"), dtype=torch.float16, device="cuda")
+        assert lib.sw_gptq_gemm(c.data_ptr(), off.data_ptr(), w.data_ptr(), z.data_ptr(), sc.data_ptr(), None, m, n, k, k // group, 1, 4,
+                                ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream) == 0
+        _close(c, quant.gptq_gemm(a, w.cpu().numpy(), qzeros, scales, None, True))
+
+
+def test_gptq_gemm_above_128_rows_on_seeded_random_shapes():
+    """Shapes drawn at random (rows 129..256, k in multiples of 256, columns in multiples of 8, groups of 64 / 128 / 256 / all of k),
+    against the CPU restatement."""
     from splitwise_amd import _C
     rng = np.random.default_rng(2024)
     for case in range(10):
@@ -192,8 +212,8 @@ def test_gptq_gemm_tile_kernel_on_seeded_random_shapes():
         _close(got, quant.gptq_gemm(a, w, qzeros, scales, None, True))
 
 
-def test_gptq_gemm_64_column_tiles_on_seeded_random_shapes():
-    """Shapes drawn at random inside the domain of the 64-column tile kernels (rows 33..128, k in multiples of 256,
+def test_gptq_gemm_up_to_128_rows_on_seeded_random_shapes():
+    """Shapes drawn at random (rows 33..128, k in multiples of 256,
     columns in multiples of 8, groups of 64 / 128 / 256 / all of k), against the CPU restatement; every launch
     twice, bit for bit the same (the k parts and the k splits are summed in a fixed order)."""
     from splitwise_amd import _C
