@@ -109,6 +109,21 @@ def test_an_extension_that_does_not_load_is_named(monkeypatch, tmp_path):
     assert _loaded(monkeypatch, None)[1] == []                              # it is optional
 
 
+@pytest.mark.parametrize("theirs,bound", [(7, True), (6, False)])
+def test_an_extension_of_another_interface_is_named(monkeypatch, theirs, bound):
+    import ctypes
+    native = importlib.import_module("splitwise_amd._native")
+    seen = []
+    monkeypatch.setattr(native, "step_ops", types.SimpleNamespace(__file__="stale.so", SW_ABI_VERSION=theirs, bind=seen.append))
+    with warnings.catch_warnings(record=True) as said:
+        warnings.simplefilter("always")
+        native.bind_library(ctypes.CDLL(None), ["malloc"], 7, "SW_ABI_VERSION")
+        assert len(seen) == bound and len(said) == (not bound)
+        monkeypatch.setattr(native, "step_ops", native._NotBuilt())          # none there: nothing to name
+        native.bind_library(ctypes.CDLL(None), ["malloc"], 7, "SW_ABI_VERSION")
+    assert len(seen) == bound and len(said) == (not bound)
+
+
 def test_the_extension_follows_torch(tree, tmp_path):
     """Built again when another torch is there, not otherwise, under the name of this Python's extensions."""
     fake = tmp_path / "site" / "torch"

@@ -9,7 +9,8 @@
 //
 // A function takes a call only if every argument is of the plain kind (exact tensors on the current device, Python numbers)
 // and passes every check; otherwise it returns None before anything happened and the Python function goes on, which knows
-// the other forms and words the refusals.  It returns the library's status otherwise.
+// the other forms and words the refusals.  It returns the library's status otherwise.  Leaving a call is a throw, 2 us: common forms that
+// it does not take (slopes, sigmoid weights, values inside the key rows) are not offered to it.
 #include <Python.h>
 
 #include <ATen/ATen.h>

@@ -17,7 +17,7 @@ _TORCH = f"{torch.__version__} {torch.version.git_version}"
 
 class _NotBuilt:
     def __getattr__(self, name):
-        if name.startswith("__"):
+        if name.startswith("__") or name.isupper():
             raise AttributeError(name)
         return lambda *args: None
 
@@ -42,5 +42,8 @@ step_ops = _load()
 
 def bind_library(lib: ctypes.CDLL, names, version: int, constant: str) -> None:
     """Tells the extension where ``lib``'s entry points are."""
-    if getattr(step_ops, constant, None) == version:
+    if getattr(step_ops, constant, version) != version:
+        warnings.warn(f"{step_ops.__file__} was built for another interface of the libraries and is not used, rebuild it "
+                      "(`make step-ops`)")
+    elif not isinstance(step_ops, _NotBuilt):
         step_ops.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in names})
