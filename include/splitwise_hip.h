@@ -234,7 +234,9 @@ int sw_kv_wait(const int32_t* flags, int slot, int32_t epoch, int64_t max_spins,
  * Workspace: the fused GEMMs split k across workgroups and combine fp32 partial tiles in
  * device memory.  `workspace` must hold at least 16 KiB, whose first 16 KiB are ZERO the first
  * time it is passed and are left zero by every call; a larger workspace allows more splits
- * (sw_quant_gemm_workspace_bytes gives a size that never limits them).  Calls that share a
+ * (sw_quant_gemm_workspace_bytes gives a size that never limits them).  From 33 rows on an
+ * input that does not lie on 16 bytes is copied to its end where there is room (slower tiles
+ * take it where there is none).  Calls that share a
  * workspace must be ordered on one stream.                                              */
 int64_t sw_quant_gemm_workspace_bytes(int M, int N, int K);
 

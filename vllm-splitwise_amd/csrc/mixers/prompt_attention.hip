@@ -509,8 +509,9 @@ __global__ __launch_bounds__(64 * kPaWaves * GROUPS, 2) void prompt_attention_ke
 
   // ---- normalise, gate, store: this lane holds query qi, channels 32 b + 8 (r / 4) + 4 hl + r % 4.  Through LDS, so that a lane
   //      stores 8 neighbouring channels and a short loop does it: from the accumulators' places it was 18 KB of instructions, gone
-  //      through once, with a wait for a gate in front of every store, 8 us of a launch (one prompt of 40 tokens, 16 heads on 4 of
-  //      128: 16.6 -> 12.3 us, two of 200: 27.0 -> 23.2, one of 700: 44.3 -> 40.7, four of 1000: 92 -> 88)
+  //      through once, with a wait for a gate in front of every store (one prompt of 40 tokens, 16 heads on 4 of 128: 17.0 -> 14.4 us,
+  //      two of 200: 25.4 -> 23.0, one of 700: 44.4 -> 42.1, four of 1000: 93.8 -> 91.4).  2 us of what is left are the gates' sigmoids;
+  //      by the hardware's 2^x and reciprocal they would be 2^-18 off at gates near -84 and 0 from -87.4 on
   const float l_run = l_part + other_half(l_part);
   float inv = 1.0f;
   if (!sig) {

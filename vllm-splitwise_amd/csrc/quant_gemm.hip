@@ -789,8 +789,9 @@ gptq_gemm_tile128_kernel(uint16_t* __restrict__ c, const uint16_t* __restrict__ 
 // and zeros into the waves' registers, all of it R stages ahead: what is left between two stages is one wait for the wave's OWN
 // loads (counted, so that the newer ones stay in flight) and one barrier.  What bounds it: at 61 rows a stage of 64 x 64 x 256 takes
 // 0.95 us of which the vector units work a third (unpacking) and the matrix cores a quarter; A is read from the L2 once per column
-// tile.  Against tiles whose A went through registers and was written to LDS a chunk later (61 rows, both matrices of 5120 rows
-// and both of 5120 columns of a 13B layer): 24.4 -> 20.1 us, 14.1 -> 13.1, 43.7 -> 28.0, 23.3 -> 20.3.
+// tile.  Against tiles whose A went through registers and was written to LDS a chunk later (61 rows, the four matrices of a 13B layer,
+// each in a replayed graph): 5120 k x 15360 22.2 -> 20.7 us, x 5120 14.7 -> 14.3, x 27648 45.0 -> 30.5, 13824 x 5120 23.0 -> 21.7, a layer's
+// four in turn 105.6 -> 85.8; of a 7B layer 84.7 -> 68.4.  quant_plan.h says which tiles a size takes.
 //
 // The waits count this wave's loads, so nothing may move past them: the pointers are not __restrict__ (a load of memory that nothing
 // else writes could be moved behind a wait, which then would not wait for the A before it), the loop has no way around it,

@@ -23,24 +23,24 @@ inline Int4Way int4_tile(int64_t M, int64_t N, int64_t K) {
   };
   if (M <= 32) {
     // k across waves reads A from memory, once per 64 columns, and has nothing to set up: the streamed tile is ahead where a workgroup
-    // has enough to go through, and the sooner the more rows (across waves / streamed: 5120 x 5120, 7 stages, 28 rows 11.3 / 11.9, 32
-    // rows 12.3 / 12.0; 8192 x 10240, 22 stages, 12 rows 22.0 / 18.1, 16 rows 24.2 / 18.8).  Over 414 sizes 1.5 % slower on average than the
+    // has enough to go through, and the sooner the more rows (across waves / streamed: 5120 x 5120, 7 stages, 28 rows 11.3 / 12.1, 32
+    // rows 12.0 / 12.1; 8192 x 10240, 22 stages, 12 rows 22.0 / 18.1, 16 rows 23.4 / 18.2).  Over 414 sizes 1.5 % slower on average than the
     // better of the two, at most 10 % slower than k across waves (20480 x 4096, 17 rows 17.7 / 19.4).
     return M > 8 && stages(32, 128) * M >= 320 ? Int4Way::k32x128 : Int4Way::kAcrossWaves;
   }
   auto named = [&]() {
     if (tiles(64, 64) <= 256) {
-      // up to 64 rows always (128 columns instead: 13.1 -> 14.7 at 5120 x 5120, 20.3 -> 21.3 at 13824 x 5120); with more rows where the
-      // splits fill the chip or k is short (100 rows: 7680 x 5120 18.6, 64 x 128 19.8; 6912 k x 5120 21.0 / 19.0)
+      // up to 64 rows always (128 columns instead: 13.2 -> 14.5 at 5120 x 5120, level at 13824 x 5120); with more rows where the
+      // splits fill the chip or k is short (96 rows: 5120 k x 7680 18.2, 64 x 128 19.1; 6912 k x 5120 20.6 / 18.3)
       const int64_t t = tiles(64, 64), filled = 256 / t * t;
       if (M <= 64 || K <= 5120 || filled >= 224) return Int4Way::k64x64;
     }
-    if (M <= 64) return Int4Way::k64x128;             // 27648 x 5120 28.9, 64 x 64 in two rounds 36.3
+    if (M <= 64) return Int4Way::k64x128;             // 5120 k x 27648 28.6, 64 x 64 in two rounds 38.0
     const int64_t t128 = tiles(128, 128);
-    // 27648 columns 42.2, 64 x 128 50.3; 15360 columns 30.0 / 30.6; 12288 24.2 / 24.0
+    // 128 rows: 5120 k x 27648 43.0, 64 x 128 49.5; 5120 k x 15360 30.1 / 28.9, 4096 k x 12288 24.2 / 22.0
     if (M <= 128) return t128 > 128 ? Int4Way::k128x128 : Int4Way::k64x128;
     if (t128 > 256) return Int4Way::k128x256;
-    // 192 rows: 11008 k x 4096 32.4 (96 tiles, 2 splits), 128 x 128 35.1; 256 rows: 13824 k x 5120 65.5 (160 tiles) / 45.5, but 2560 k 16.2 / 21.7
+    // 192 rows: 6144 k x 8192 30.6 (192 tiles), 128 x 128 32.3; 13824 k x 5120 38.8 (120 tiles, 2 splits) / 44.2; 256 rows 60.9 (160 tiles) / 45.6
     const int64_t t = tiles(64, 128), filled = t <= 256 ? 256 / t * t : 0;
     return t <= 256 && (K <= 4096 || filled >= 180) ? Int4Way::k64x128 : Int4Way::k128x128;
   };
