@@ -1610,6 +1610,14 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
     ap = at_end;
   }
   float* partials = reinterpret_cast<float*>(ws + kCounterBytes);
+#ifdef SW_QUANT_EXPERIMENT                                     // tuning builds only: never in the shipped library
+  // 1..5: streamed tiles as in Int4Way, 128 x 256; 0: what is left
+  if (const char* env = getenv("SW_QUANT_TILE")) {
+    const int t = atoi(env);
+    if (t >= 1 && t <= 5 && K % 256 == 0 && (t < 5 || group_size % 64 == 0)) way = static_cast<Int4Way>(t);
+    else way = M > 128 && K % kChunkK == 0 ? Int4Way::k64Rows : Int4Way::kAcrossWaves;
+  }
+#endif
   int cp = 2, mt = M > 64 ? 4 : M > 32 ? 2 : 1;
   bool tiled = way == Int4Way::k64Rows;
   int waves = 8, chunk = kChunkK, tiled_mt = 2, force_ks = 0;
@@ -1621,12 +1629,6 @@ static int kmajor_gemm(void* c, const void* a, const uint32_t* qweight, const ui
   if (const char* env = getenv("SW_QUANT_CHUNK")) chunk = atoi(env) == 128 ? 128 : 256;
   if (const char* env = getenv("SW_QUANT_TMT")) tiled_mt = atoi(env);
   if (const char* env = getenv("SW_QUANT_KSPLIT")) force_ks = atoi(env);
-  // 0: none; 1..5: streamed tiles as in Int4Way, 128 x 256
-  if (const char* env = getenv("SW_QUANT_TILE")) {
-    const int t = atoi(env);
-    if (t >= 1 && t <= 5 && K % 256 == 0 && (t < 5 || group_size % 64 == 0)) way = static_cast<Int4Way>(t);
-    else way = Int4Way::kAcrossWaves;
-  }
 #endif
   if (mt == 3 || mt > 4) mt = 4;
   if (tiled) mt = tiled_mt;
