@@ -174,6 +174,27 @@ def test_gptq_gemm_an_input_off_16_bytes_takes_the_same_tiles(m, k, n):
         assert (ws[size:] == 77).all() and (ws[:16 << 10] == 0).all()
 
 
+@torch.inference_mode()                                      # (as the workers capture theirs)
+def test_gptq_gemm_an_input_off_16_bytes_in_a_graph():
+    """The copy is a part of the graph: replays follow the input, with other calls in between."""
+    from splitwise_amd import _C
+    m, k, n = 61, 1536, 328
+    qweight, qzeros, scales, _ = _gptq_case(k, n, 128, m)
+    weights = (_dev(quant.gptq_shuffle(qweight)), _dev(qzeros), _dev(scales), None, True, 4)
+    off = torch.zeros(m * k + 1, dtype=torch.float16, device="cuda")[1:].view(m, k)
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        _C.ops.gptq_gemm(off, *weights)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        got = _C.ops.gptq_gemm(off, *weights)
+    for i in range(3):
+        off.copy_(_dev(np.random.default_rng(i).standard_normal((m, k)).astype(np.float16)))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, _C.ops.gptq_gemm(off.clone(), *weights)) and got.any()
+
+
 @pytest.mark.parametrize("m,k,n,group,splits", [(160, 1280, 264, 128, 2), (250, 2816, 520, 64, 2), (129, 2304, 264, 2304, 3)])
 def test_gptq_gemm_wide_tiles_over_an_odd_number_of_chunks(m, k, n, group, splits):
     """An input off 16 bytes without room for its copy: 128 x 256 tiles at any number of columns, k split as often as the workspace has
