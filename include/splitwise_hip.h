@@ -52,7 +52,7 @@ const char* sw_last_error(void);
  * 6: sw_kv_push_mapped added.
  * 7: sw_context_attention_split, sw_context_attention_split_parts, sw_context_attention_split_workspace_bytes
  *    added. */
-#define SW_ABI_VERSION 7
+#define SW_ABI_VERSION 8
 int sw_abi_version(void);
 
 /* csrc/cuda_utils_kernels.cu:16-35 get_max_shared_memory_per_block_device_attribute:
@@ -178,6 +178,18 @@ int sw_prefill_attention(void* out, const void* query, const void* key,
                          float scale, const float* alibi_slopes, int64_t q_stride,
                          int64_t k_stride, int64_t v_stride, int64_t out_stride,
                          int sliding_window, int act_dtype, void* stream);
+
+/* sw_prefill_attention and sw_reshape_and_cache (of the same keys and values, [num_tokens] rows of them) in one launch: what the
+ * attention leaves idle of the GPU writes the cache.  Takes f16 / bf16, caches whose blocks hold a whole number of 16 bytes of
+ * tokens (8 of them; 16 of fp8), and calls in which both have something to do; refuses others before anything is launched. */
+int sw_prefill_attention_and_cache(void* out, const void* query, const void* key, const void* value,
+                                   const int32_t* seq_starts, const int32_t* seq_lens, int num_seqs,
+                                   int max_seq_len, int num_heads, int num_kv_heads, int head_size, float scale,
+                                   const float* alibi_slopes, int64_t q_stride, int64_t k_stride, int64_t v_stride,
+                                   int64_t out_stride, int sliding_window, int act_dtype, void* key_cache,
+                                   void* value_cache, const int64_t* slot_mapping, int num_tokens, int block_size,
+                                   int x, int cache_dtype, void* stream);
+
 
 /* --------------------------------------------------------------- KV transport
  * Replaces the reference's MSCCL++ proxy-channel kernels (csrc/kv_comm_kernels.cu:3-29) and

@@ -12,7 +12,7 @@
 //     arbitrary slots (decode) every token is still placed individually.
 //   * copy_blocks moves 16 bytes per lane with the pointer tables resident on
 //     the device (no per-call pointer upload).
-#include "common.cuh"
+#include "cache_tile.cuh"
 
 #include <algorithm>
 #include <string>
@@ -33,184 +33,10 @@ void set_error(const char* fmt, ...) {
   g_last_error = buf;
 }
 
-constexpr int kTileTokens = 16;
-constexpr int kRcThreads = 256;
-constexpr size_t kRcLds = 160 * 1024;
-// Tokens that the kernel looks at: a tile's, and a vector's behind it.  Its own arrays in LDS: 16 bytes for each, 4 per vector of a tile.
-constexpr int rc_group(int vt) { return vt > 0 ? vt : 8; }
-constexpr int rc_seen(int vt) { return kTileTokens + rc_group(vt); }
-constexpr size_t rc_arrays(int vt) { return (size_t)(16 * rc_seen(vt) + 4 * (kTileTokens / rc_group(vt)) + 15) / 16 * 16; }
-
-// LDS row = head_size activations + 16 bytes of padding (keeps 16-byte row reads
-// of consecutive tokens on different bank groups).
-template <typename act_t>
-__device__ __forceinline__ int lds_row_bytes(int head_size) {
-  return head_size * (int)sizeof(typename Conv<act_t>::store_t) + 16;
-}
-
-// act_t: float / f16_t / bf16_t.  FP8: cache holds e5m2 bytes, else the same bits as the activations.  VT: tokens per vector
-// store of a value cache row (0: element by element).
-// What bounds it is memory, once the addresses are cheap: where a token goes (its slot's block and offset, a 64-bit division
-// where the block size is no power of two) is worked out once per tile by 16 lanes, and not by every thread for every piece.
-// Workgroups that run together take the heads of the same tokens: their pieces of a row lie side by side.
-// Vectors of V are VT neighbouring slots from a multiple of VT on.  Prompts of any length lie behind one another in a step, so a
-// tile's tokens seldom begin at such a slot: a tile's V is moved on to the next one where the run of slots goes on (its first
-// tokens are then the tile's before it), and only what is left over at a run's ends goes element by element.
-// Measured, 2320 tokens x 32 heads of 128, bf16 (76 MB): 30.5 us with the divisions in every thread, 27.2 without, 16.2 with the
-// heads side by side as one prompt; as prompts of 699, 938 and 790 tokens 26.0 with V vectors only where a tile's own eighths
-// are aligned, 18.3 here.  61 tokens x 8 heads into an fp8 cache: 8.7 us with the divisions, 5.1 here.  251 tokens x 32 heads into slots of their own
-// take 19 us before and after: every element of V is a 2-byte write into a 32-byte sector (36 MB for 4).
 template <typename act_t, bool FP8, int VT>
-__global__ void __launch_bounds__(kRcThreads)
-reshape_and_cache_tile_kernel(const char* __restrict__ key, const char* __restrict__ value,
-                              char* __restrict__ key_cache, char* __restrict__ value_cache,
-                              const int64_t* __restrict__ slot_mapping, int num_tokens,
-                              int num_heads, int head_size, int block_size, int block_shift,
-                              int64_t key_stride_bytes, int64_t value_stride_bytes) {
-  using S = typename Conv<act_t>::store_t;
-  constexpr int ES = sizeof(S);                 // activation element bytes
-  constexpr int CS = FP8 ? 1 : ES;              // cache element bytes
-  constexpr int X = 16 / CS;                    // cache elements per 16 bytes
+__global__ void __launch_bounds__(kRcThreads) reshape_and_cache_tile_kernel(const CacheWrite w) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr int GROUP = rc_group(VT), PARTS = kTileTokens / GROUP, kSeen = rc_seen(VT);
-  __shared__ int64_t bases[kSeen];              // byte offset of the token's [block, head] tile, -1: no slot
-  __shared__ int offsets[kSeen];                // the token's place in its block
-  __shared__ int heads[PARTS], loose[kSeen];    // tokens that begin a vector of V, tokens that no vector takes
-  static_assert(sizeof(bases) + sizeof(offsets) + sizeof(heads) + sizeof(loose) <= rc_arrays(VT), "the launch counts on them");
-
-  const int t0 = blockIdx.x / num_heads * kTileTokens;
-  const int head = blockIdx.x % num_heads;
-  const int tid = threadIdx.x;
-  const int row_bytes = lds_row_bytes<act_t>(head_size);
-  char* k_tile = smem;
-  char* v_tile = smem + kTileTokens * row_bytes;
-  const int64_t head_bytes = (int64_t)head_size * block_size * CS;
-  const int64_t block_bytes = head_bytes * num_heads;
-
-  // ---- every wave looks at the tile's slots, the one in front of them and those up to a vector's length behind: lane l is token
-  //      t0 + l - 1
-  const int lane = tid & 63, j = lane - 1;
-  int64_t slot = -1;
-  if (t0 + j >= 0 && t0 + j < num_tokens && j < kSeen) slot = slot_mapping[t0 + j];
-
-  // ---- stage K and V rows of this head: 16-byte pieces, token-major (coalesced), 16 lanes a row
-  const int tok16 = tid / 16, chunks = head_size * ES / 16;
-  const int64_t head_off = (int64_t)head * head_size * ES;
-  if (t0 + tok16 < num_tokens) {
-    const char* kr = key + (t0 + tok16) * key_stride_bytes + head_off;
-    const char* vr = value + (t0 + tok16) * value_stride_bytes + head_off;
-    for (int ch = tid % 16; ch < chunks; ch += 16) {
-      const uint4 kv = *reinterpret_cast<const uint4*>(kr + ch * 16);
-      const uint4 vv = *reinterpret_cast<const uint4*>(vr + ch * 16);
-      *reinterpret_cast<uint4*>(k_tile + tok16 * row_bytes + ch * 16) = kv;
-      *reinterpret_cast<uint4*>(v_tile + tok16 * row_bytes + ch * 16) = vv;
-    }
-  }
-  // ---- V's tokens [v0, v1) of this tile, which of them begin a vector and which go alone
-  const int64_t prev = __shfl_up(slot, 1, 64);
-  const uint64_t follows = __ballot(lane > 0 && slot >= 0 && prev >= 0 && slot == prev + 1);
-  auto moved = [&](int first) {                 // tokens from `first` on that belong to a vector begun in front of it
-    if constexpr (VT == 0) return 0;
-    const int64_t s = __shfl(slot, first + 1, 64);
-    const int n = s < 0 ? 0 : (int)((GROUP - s % GROUP) % GROUP);
-    const uint64_t need = ((1ull << n) - 1) << (first + 1);
-    return (follows & need) == need ? n : 0;
-  };
-  const int v0 = moved(0), v1 = min(kTileTokens + moved(kTileTokens), num_tokens - t0);
-  uint64_t begins = 0;
-  if constexpr (VT > 0) {
-    const uint64_t rest = ((1ull << (GROUP - 1)) - 1) << (lane + 1);
-    begins = __ballot(j >= v0 && j + GROUP <= v1 && slot >= 0 && slot % GROUP == 0 && (follows & rest) == rest);
-  }
-  const bool taken = ((begins << (GROUP - 1)) >> lane & ((1ull << GROUP) - 1)) != 0;
-  const uint64_t alone = __ballot(j >= v0 && j < v1 && slot >= 0 && !taken);
-  const int num_heads_v = __popcll(begins), num_loose = __popcll(alone);
-  if (tid < 64) {                               // one wave
-    const uint64_t below = (1ull << lane) - 1;
-    if (begins >> lane & 1) heads[__popcll(begins & below)] = j;
-    if (alone >> lane & 1) loose[__popcll(alone & below)] = j;
-    if (j >= 0 && j < kSeen) {
-      const int64_t blk = block_shift >= 0 ? slot >> block_shift : slot / block_size;
-      bases[j] = slot < 0 ? -1 : blk * block_bytes + head * head_bytes;
-      offsets[j] = slot < 0 ? 0 : (int)(slot - blk * block_size);
-    }
-  }
-  if (kTileTokens + tok16 < v1) {               // (fewer than a vector's tokens)
-    const char* vr = value + (t0 + kTileTokens + tok16) * value_stride_bytes + head_off;
-    for (int ch = tid % 16; ch < chunks; ch += 16)
-      *reinterpret_cast<uint4*>(v_tile + (kTileTokens + tok16) * row_bytes + ch * 16) = *reinterpret_cast<const uint4*>(vr + ch * 16);
-  }
-  __syncthreads();
-
-  // ---- K: one 16-byte cache vector (X elements of one token) per lane, token-fastest
-  {
-    const int tok = tid % kTileTokens;
-    const int64_t base = bases[tok];
-    const int boff = offsets[tok];
-    for (int c = tid / kTileTokens; base >= 0 && c < head_size / X; c += kRcThreads / kTileTokens) {
-      char* dst = key_cache + base + ((int64_t)c * block_size + boff) * 16;
-      const char* src = k_tile + tok * row_bytes + c * X * ES;
-      if constexpr (!FP8) {
-        *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(src);
-      } else {
-        uint32_t w[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          uint32_t acc = 0;
-#pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            const S e = *reinterpret_cast<const S*>(src + (q * 4 + b) * ES);
-            acc |= (uint32_t)Conv<act_t>::to_e5m2(e) << (8 * b);
-          }
-          w[q] = acc;
-        }
-        *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
-      }
-    }
-  }
-
-  // ---- V: cache row d holds block_size tokens.  A vector takes VT tokens of it (block_size is a multiple: they share a row segment),
-  // what no vector takes goes one element per lane.
-  const int part = tid % PARTS;
-  if (part < num_heads_v) {
-    const int first = heads[part];
-    char* const dst0 = value_cache + bases[first] + (int64_t)offsets[first] * CS;
-    for (int d = tid / PARTS; d < head_size; d += kRcThreads / PARTS) {
-      const char* src = v_tile + first * row_bytes + d * ES;
-      char* dst = dst0 + (int64_t)d * block_size * CS;
-      uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int q = 0; q < GROUP; ++q) {
-        const S e = *reinterpret_cast<const S*>(src + q * row_bytes);
-        if constexpr (FP8) {
-          w[q >> 2] |= (uint32_t)Conv<act_t>::to_e5m2(e) << (8 * (q & 3));
-        } else if constexpr (ES == 2) {
-          w[q >> 1] |= (uint32_t)e << (16 * (q & 1));
-        } else {
-          w[q & 3] = __float_as_uint(e);
-        }
-      }
-      if constexpr (GROUP * CS >= 16) {
-        *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
-      } else {
-        *reinterpret_cast<uint2*>(dst) = make_uint2(w[0], w[1]);
-      }
-    }
-  }
-#pragma unroll 4
-  for (int k = tid / 64; k < num_loose; k += kRcThreads / 64) {          // a wave per token
-    const int tok = __builtin_amdgcn_readfirstlane(loose[k]);
-    char* const dst0 = value_cache + bases[tok] + (int64_t)offsets[tok] * CS;
-    for (int d = lane; d < head_size; d += 64) {
-      char* dst = dst0 + (int64_t)d * block_size * CS;
-      const S e = *reinterpret_cast<const S*>(v_tile + tok * row_bytes + d * ES);
-      if constexpr (FP8) {
-        *reinterpret_cast<uint8_t*>(dst) = Conv<act_t>::to_e5m2(e);
-      } else {
-        *reinterpret_cast<S*>(dst) = e;
-      }
-    }
-  }
+  cache_tile<act_t, FP8, VT>(w, blockIdx.x, threadIdx.x, smem);
 }
 
 // Grid: (2 * num_pairs, num_layers, splits).  blockIdx.x even = K, odd = V.
@@ -289,30 +115,21 @@ int launch_reshape_and_cache(const void* key, const void* value, void* key_cache
                              const int64_t* slot_mapping, int num_tokens, int num_heads,
                              int head_size, int block_size, int64_t key_stride, int64_t value_stride,
                              hipStream_t stream) {
-  using S = typename Conv<act_t>::store_t;
-  const int es = sizeof(S);
-  const int row_bytes = head_size * es + 16;
-  const unsigned grid = (unsigned)((num_tokens + kTileTokens - 1) / kTileTokens * num_heads);
-  int block_shift = -1;
-  if ((block_size & (block_size - 1)) == 0)
-    for (block_shift = 0; (1 << block_shift) < block_size; ++block_shift) {}
+  constexpr int ES = sizeof(typename Conv<act_t>::store_t);
+  CacheWrite w = cache_write(key, value, key_cache, value_cache, slot_mapping, num_tokens, num_heads, head_size, block_size, key_stride,
+                             value_stride, ES);
   // 16 bytes of tokens per store where a block holds a whole number of them, 8 for the small blocks, else single elements
-  constexpr int VT = FP8 ? 16 : 16 / (int)sizeof(S);
+  constexpr int VT = FP8 ? 16 : 16 / ES;
   int vt = block_size % VT == 0 ? VT : block_size % (VT / 2) == 0 ? VT / 2 : 0;
-  // LDS: a tile's rows of K, and of V up to a vector's length less one more (40 rows of 16-bit activations, 48 into an fp8 cache).
   // The largest heads (from 848 on fp32 into fp8, from 2040 on 16 bits) leave room for shorter vectors, or for none.  Without the check
-  // a launch that passes 160 KB only with the kernel's own arrays would not be refused but end its queue.
-  auto smem = [&](int v) { return (size_t)(2 * kTileTokens + v) * row_bytes; };
-  auto fits = [&](int v) { return smem(v) + rc_arrays(v) <= kRcLds; };
+  // a launch that passes 160 KB would not be refused but end its queue.
+  auto fits = [&](int v) { return rc_lds(v, head_size, ES) <= kRcLds; };
   while (vt > 0 && !fits(vt)) vt = vt == VT ? VT / 2 : 0;
   SW_CHECK_ARG(fits(vt), "reshape_and_cache: heads of %d elements need too much LDS", head_size);
   auto kernel = vt == VT  ? reshape_and_cache_tile_kernel<act_t, FP8, VT>
                 : vt > 0 ? reshape_and_cache_tile_kernel<act_t, FP8, VT / 2>
                          : reshape_and_cache_tile_kernel<act_t, FP8, 0>;
-  kernel<<<grid, kRcThreads, smem(vt), stream>>>(
-      static_cast<const char*>(key), static_cast<const char*>(value), static_cast<char*>(key_cache),
-      static_cast<char*>(value_cache), slot_mapping, num_tokens, num_heads, head_size, block_size, block_shift,
-      key_stride * es, value_stride * es);
+  kernel<<<(unsigned)w.tiles(), kRcThreads, rc_lds(vt, w.head_size, ES), stream>>>(w);
   SW_CHECK_LAUNCH();
   return SW_OK;
 }
@@ -323,7 +140,7 @@ extern "C" {
 
 const char* sw_last_error(void) { return sw::g_last_error.c_str(); }
 
-int sw_abi_version(void) { return 7; }       // SW_ABI_VERSION of the header; tests/test_abi.py compares the two
+int sw_abi_version(void) { return 8; }       // SW_ABI_VERSION of the header; tests/test_abi.py compares the two
 
 int sw_get_max_shared_memory_per_block(int device, int* out_bytes) {
   SW_CHECK_ARG(out_bytes != nullptr, "out_bytes is NULL");

@@ -23,7 +23,7 @@
 namespace {
 
 #define STEP_OPS(X)                                                                                                     \
-  X(sw_reshape_and_cache) X(sw_paged_attention_v1) X(sw_prefill_attention) X(swm_causal_conv) X(swm_gated_delta)        \
+  X(sw_reshape_and_cache) X(sw_paged_attention_v1) X(sw_prefill_attention) X(sw_prefill_attention_and_cache) X(swm_causal_conv) X(swm_gated_delta)        \
   X(swm_gated_delta_chunked) X(swm_gated_delta_chunked_workspace_floats) X(swm_head_norm_gate_act) X(swm_group_pairs)   \
   X(swm_expert_up_weighted) X(swm_expert_down_weighted) X(swm_masked_attention) X(swm_sink_attention)                   \
   X(swm_masked_attention_workspace_floats) X(swm_gla) X(swm_gla_workspace_floats) X(swm_lightning) X(swm_retention)     \
@@ -265,6 +265,29 @@ STEP_OP(prefill_attention) {
                                      ptr<int32_t>(lens), (int)lens.numel(), longest, (int)q.size(1), (int)k.size(1),
                                      (int)q.size(2), scale, nullptr, q.stride(0), k.stride(0), v.stride(0), out.stride(0), window,
                                      act, stream);
+    }));
+  });
+}
+
+STEP_OP(prefill_attention_and_cache) {
+  return call([&] {
+    const Args c(args, nargs, 14);
+    take(sw_prefill_attention_and_cache_at != nullptr && args[8] == Py_None);
+    const Tensor &out = c.tensor(0), &q = c.tensor(1), &k = c.tensor(2), &v = c.tensor(3), &starts = c.tensor(4),
+                 &lens = c.tensor(5), &kc = c.tensor(10), &vc = c.tensor(11), &slots = c.tensor(12);
+    const int longest = c.i32(6), window = args[9] == Py_None ? 0 : c.i32(9);
+    const float scale = c.f32(7);
+    take(starts.scalar_type() == at::kInt && lens.scalar_type() == at::kInt && slots.scalar_type() == at::kLong && kc.dim() == 5);
+    for (const Tensor* t : {&out, &q, &k, &v}) take(t->dim() == 3 && t->stride(2) == 1 && t->stride(1) == t->size(2));
+    const int act = hip_act(q), cache = cache_dtype(args[13], act);
+    take(k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type() && out.scalar_type() == q.scalar_type()
+         && v.sizes() == k.sizes() && k.size(2) == q.size(2));
+    void* stream = c.stream();
+    return PyLong_FromLong(unlocked([&] {
+      return sw_prefill_attention_and_cache_at(
+          ptr<void>(out), ptr<void>(q), ptr<void>(k), ptr<void>(v), ptr<int32_t>(starts), ptr<int32_t>(lens), (int)lens.numel(), longest,
+          (int)q.size(1), (int)k.size(1), (int)q.size(2), scale, nullptr, q.stride(0), k.stride(0), v.stride(0), out.stride(0), window,
+          act, ptr<void>(kc), ptr<void>(vc), ptr<int64_t>(slots), (int)k.size(0), (int)kc.size(3), (int)kc.size(4), cache, stream);
     }));
   });
 }
@@ -569,6 +592,7 @@ PyObject* bind(PyObject*, PyObject* table) {
 #define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr},
 PyMethodDef kMethods[] = {
     METHOD(reshape_and_cache) METHOD(paged_attention_v1) METHOD(prefill_attention) METHOD(causal_conv) METHOD(gated_delta)
+    METHOD(prefill_attention_and_cache)
     METHOD(head_norm_gate) METHOD(gla) METHOD(lightning) METHOD(retention) METHOD(group_pairs) METHOD(expert_ffn)
     METHOD(capped_attention) {"bind", bind, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -33,7 +33,7 @@
 //   * launches of less than one workgroup per CU (KSW = 2): the workgroup's waves are pairs that share 32 query rows
 //     and take one score tile of every stage each, then join their (maximum, sum, output) through LDS: half as many
 //     query rows per workgroup, so twice the workgroups, each wave with half the matrix work of its key loop.
-#include "common.cuh"
+#include "cache_tile.cuh"
 #include <float.h>
 #include <stdlib.h>
 #include <algorithm>
@@ -101,6 +101,20 @@ struct PfContext {
   int64_t total_rows;
 };
 
+// Workgroups from `first` on write the step's keys and values into the paged cache, 256 threads a tile (cache_tile.cuh), and have nothing
+// to do with the attention, which reads them where they are.
+// Why in one launch: the attention waits for its longest walks, beside which many of the GPU's places for workgroups stand empty, and the
+// write waits for memory; and a launch is spared.  They come last, when all of the attention's have begun: in front of them they keep the
+// longest walks waiting (3 x 773 tokens, 32 heads of 128: 50 us, 54 with the write first).
+// Measured, a layer's prompt step in a stream of calls, two launches / one (us): 1 x 40 tokens, 32 heads of 128 14.1 / 11.3, 1 x 773
+// 24.5 / 19.6, 3 x 773 54.3 / 48.7, 2 x 2000 with 40 heads 166.9 / 164.7; 64 heads on 8, 2 x 300 21.9 / 18.7; 12 of 64 into an fp8 cache,
+// 4 x 700 29.9 / 22.2.
+constexpr int kPfTokens = 8, kPfFp8Tokens = 16;      // of a vector of the value cache: 16 bytes
+struct PfCacheWrite {
+  CacheWrite w;
+  int first, fp8;                 // without a write: `first` is beyond the grid
+};
+
 template <typename act_t, int HEAD, bool CTX, int WAVES, int KSW>
 __global__ void __launch_bounds__(WAVES * 64, (HEAD <= 128 && WAVES == 4) ? 2 : 1)
 prefill_attention_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
@@ -109,7 +123,7 @@ prefill_attention_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict_
                          int num_heads, int num_kv_heads, float scale,
                          const float* __restrict__ alibi_slopes, int64_t q_stride, int64_t k_stride,
                          int64_t v_stride, int64_t out_stride, int sliding_window, int num_seqs, int max_seq_len,
-                         PfContext cx) {
+                         PfContext cx, const PfCacheWrite cw) {
   using M = Mfma<act_t>;
   using frag = typename M::frag;
   constexpr int NT = pf_tiles(HEAD);                 // score tiles per stage
@@ -134,6 +148,19 @@ prefill_attention_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict_
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   char* k_img = smem;                                // [kPfBufs][kPfStage][KSTRIDE]
   char* v_img = smem + kPfBufs * kPfStage * KSTRIDE; // [kPfBufs][kPfStage][VSTRIDE]
+
+  if constexpr (!CTX) {
+    if ((int)blockIdx.x >= cw.first) {               // workgroup-uniform
+      const int part = wave / (kRcThreads / 64), tile = ((int)blockIdx.x - cw.first) * (WAVES * 64 / kRcThreads) + part;
+      char* const lds = smem + part * (pf_lds_bytes(HEAD) / (WAVES * 64 / kRcThreads) / 16 * 16);
+      if (cw.fp8) {
+        cache_tile<act_t, true, kPfFp8Tokens>(cw.w, tile, tid % kRcThreads, lds);
+      } else {
+        cache_tile<act_t, false, kPfTokens>(cw.w, tile, tid % kRcThreads, lds);
+      }
+      return;
+    }
+  }
 
   // One workgroup per (query tile, sequence, head), numbered tile-major with the LATEST tiles first: under the
   // causal mask they have the longest key loops, so the launch's last round is made of the short ones.  Within
@@ -794,11 +821,18 @@ context_attention_reduce_kernel(uint16_t* __restrict__ out, const float* __restr
   *reinterpret_cast<uint2*>(out + row * out_stride + (int64_t)head * head_size + d) = make_uint2(lo, hi);
 }
 
+// Tiles of the cache write that are left when heads are taken together: about one for each of the places that the attention leaves.  A
+// workgroup has as much LDS as the attention's, so that few fit on a compute unit, and what each has in flight counts (us, one tile a
+// head / 512 / 256 left: 3 x 773 tokens, 32 heads 55 / 50 / 50; 4 x 700 tokens, 12 heads of 64 into an fp8 cache 31 / 22 / 22; 2 x 700,
+// 8 of 128 into an fp8 cache 45 / 44 / 42; 2 x 2000, 40 heads 180 / 168 / 167).
+constexpr int kPfWriteTiles = 256;
+
 template <typename act_t, int HEAD, bool CTX, int WAVES, int KSW>
 int launch_prefill_w(void* out, const void* q, const void* k, const void* v, const int32_t* seq_starts,
                      const int32_t* seq_lens, int num_seqs, int max_seq_len, int num_heads, int num_kv_heads,
                      float scale, const float* alibi, int64_t q_stride, int64_t k_stride, int64_t v_stride,
-                     int64_t out_stride, int sliding_window, const PfContext& cx, hipStream_t stream) {
+                     int64_t out_stride, int sliding_window, const PfContext& cx, const CacheWrite* write, int fp8,
+                     hipStream_t stream) {
   const int rows_per_wg = WAVES / KSW * kPfRows;
   const int q_tiles = (max_seq_len + rows_per_wg - 1) / rows_per_wg;
   SW_CHECK_ARG((int64_t)q_tiles * num_heads * num_seqs < (int64_t)1 << 31, "prefill attention: %d x %d x %d workgroups",
@@ -809,6 +843,19 @@ int launch_prefill_w(void* out, const void* q, const void* k, const void* v, con
                HEAD, cx.block_size);
   dim3 grid((unsigned)(q_tiles * num_heads * num_seqs), (unsigned)parts);
   const size_t smem = (size_t)pf_lds_bytes(HEAD);
+  PfCacheWrite cw{{}, 0x7fffffff, fp8};
+  if (!CTX && write != nullptr) {
+    constexpr int kTiles = WAVES * 64 / kRcThreads;            // of a workgroup
+    const int vt = fp8 ? kPfFp8Tokens : kPfTokens;
+    const size_t lds = smem / kTiles / 16 * 16;
+    SW_CHECK_ARG(rc_lds(vt, HEAD, 2) <= lds, "prefill attention: a tile of the cache write does not fit");
+    cw.w = *write;
+    cw.first = (int)grid.x;
+    cache_merge(cw.w, vt, 2, kPfWriteTiles, lds);
+    const int64_t more = ((int64_t)cw.w.tiles() + kTiles - 1) / kTiles;
+    SW_CHECK_ARG(cw.first + more < (int64_t)1 << 31, "prefill attention: %d + %lld workgroups", cw.first, (long long)more);
+    grid.x += (unsigned)more;
+  }
   auto kern = prefill_attention_kernel<act_t, HEAD, CTX, WAVES, KSW>;
 
   if (smem > 64 * 1024)
@@ -817,7 +864,7 @@ int launch_prefill_w(void* out, const void* q, const void* k, const void* v, con
   kern<<<grid, WAVES * 64, smem, stream>>>(
       static_cast<uint16_t*>(out), static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
       static_cast<const uint16_t*>(v), seq_starts, seq_lens, num_heads, num_kv_heads, scale, alibi, q_stride,
-      k_stride, v_stride, out_stride, sliding_window, num_seqs, max_seq_len, cx);
+      k_stride, v_stride, out_stride, sliding_window, num_seqs, max_seq_len, cx, cw);
   SW_CHECK_LAUNCH();
   if (parts > 1) {
     const unsigned col_groups = (unsigned)((num_heads * (HEAD / 4) + 255) / 256);
@@ -845,7 +892,8 @@ template <typename act_t, int HEAD, bool CTX>
 int launch_prefill(void* out, const void* q, const void* k, const void* v, const int32_t* seq_starts,
                    const int32_t* seq_lens, int num_seqs, int max_seq_len, int num_heads, int num_kv_heads,
                    float scale, const float* alibi, int64_t q_stride, int64_t k_stride, int64_t v_stride,
-                   int64_t out_stride, int sliding_window, const PfContext& cx, hipStream_t stream) {
+                   int64_t out_stride, int sliding_window, const PfContext& cx, const CacheWrite* write, int fp8,
+                   hipStream_t stream) {
   int wide = !CTX && HEAD <= 128 && max_seq_len >= kPfWideFrom &&
              (int64_t)((max_seq_len + 8 * kPfRows - 1) / (8 * kPfRows)) * num_heads * num_seqs >= kPfWideWorkgroups;
   // Launches of few workgroups wait for their longest key loop: waves in pairs that split every stage's keys
@@ -859,24 +907,24 @@ int launch_prefill(void* out, const void* q, const void* k, const void* v, const
     if (wide)
       return launch_prefill_w<act_t, HEAD, CTX, 8, 1>(out, q, k, v, seq_starts, seq_lens, num_seqs, max_seq_len, num_heads,
                                                       num_kv_heads, scale, alibi, q_stride, k_stride, v_stride, out_stride,
-                                                      sliding_window, cx, stream);
+                                                      sliding_window, cx, write, fp8, stream);
   }
   if constexpr (pf_tiles(HEAD) == 2) {
     if (pairs)
       return launch_prefill_w<act_t, HEAD, CTX, kPfWaves, 2>(out, q, k, v, seq_starts, seq_lens, num_seqs, max_seq_len,
                                                              num_heads, num_kv_heads, scale, alibi, q_stride, k_stride,
-                                                             v_stride, out_stride, sliding_window, cx, stream);
+                                                             v_stride, out_stride, sliding_window, cx, write, fp8, stream);
   }
   return launch_prefill_w<act_t, HEAD, CTX, kPfWaves, 1>(out, q, k, v, seq_starts, seq_lens, num_seqs, max_seq_len,
                                                          num_heads, num_kv_heads, scale, alibi, q_stride, k_stride,
-                                                         v_stride, out_stride, sliding_window, cx, stream);
+                                                         v_stride, out_stride, sliding_window, cx, write, fp8, stream);
 }
 
 int prefill_entry(void* out, const void* query, const void* key, const void* value, const int32_t* seq_starts,
                   const int32_t* seq_lens, int num_seqs, int max_seq_len, int num_heads, int num_kv_heads,
                   int head_size, float scale, const float* alibi_slopes, int64_t q_stride, int64_t k_stride,
                   int64_t v_stride, int64_t out_stride, int sliding_window, int act_dtype, const PfContext* cx,
-                  void* stream) {
+                  const CacheWrite* write, int fp8, void* stream) {
   if (num_seqs == 0 || max_seq_len == 0) return SW_OK;
   SW_CHECK_ARG(num_seqs > 0 && max_seq_len > 0 && num_heads > 0 && num_kv_heads > 0 &&
                    num_heads % num_kv_heads == 0, "prefill_attention: bad shape");
@@ -895,10 +943,10 @@ int prefill_entry(void* out, const void* query, const void* key, const void* val
 #define SW_PF_T(T, HEAD)                                                                                        \
   return cx ? launch_prefill<T, HEAD, true>(out, query, key, value, seq_starts, seq_lens, num_seqs, max_seq_len, \
                                             num_heads, num_kv_heads, scale, alibi_slopes, q_stride, k_stride,   \
-                                            v_stride, out_stride, sliding_window, *cx, s)                       \
+                                            v_stride, out_stride, sliding_window, *cx, write, fp8, s)                       \
             : launch_prefill<T, HEAD, false>(out, query, key, value, seq_starts, seq_lens, num_seqs,            \
                                              max_seq_len, num_heads, num_kv_heads, scale, alibi_slopes,         \
-                                             q_stride, k_stride, v_stride, out_stride, sliding_window, none, s)
+                                             q_stride, k_stride, v_stride, out_stride, sliding_window, none, write, fp8, s)
 #define SW_PF(HEAD)                        \
   if (act_dtype == SW_BF16) {              \
     SW_PF_T(bf16_t, HEAD);                 \
@@ -930,7 +978,29 @@ extern "C" int sw_prefill_attention(void* out, const void* query, const void* ke
                                     int sliding_window, int act_dtype, void* stream) {
   return sw::prefill_entry(out, query, key, value, seq_starts, seq_lens, num_seqs, max_seq_len, num_heads,
                            num_kv_heads, head_size, scale, alibi_slopes, q_stride, k_stride, v_stride, out_stride,
-                           sliding_window, act_dtype, nullptr, stream);
+                           sliding_window, act_dtype, nullptr, nullptr, 0, stream);
+}
+
+extern "C" int sw_prefill_attention_and_cache(void* out, const void* query, const void* key, const void* value,
+                                              const int32_t* seq_starts, const int32_t* seq_lens, int num_seqs, int max_seq_len,
+                                              int num_heads, int num_kv_heads, int head_size, float scale,
+                                              const float* alibi_slopes, int64_t q_stride, int64_t k_stride, int64_t v_stride,
+                                              int64_t out_stride, int sliding_window, int act_dtype, void* key_cache,
+                                              void* value_cache, const int64_t* slot_mapping, int num_tokens, int block_size, int x,
+                                              int cache_dtype, void* stream) {
+  using namespace sw;
+  const bool fp8 = cache_dtype == SW_FP8_E5M2;
+  SW_CHECK_ARG(num_seqs > 0 && max_seq_len > 0 && num_tokens > 0 && num_kv_heads > 0 && block_size > 0,
+               "prefill_attention_and_cache: nothing to do for one of the two");
+  SW_CHECK_ARG(act_dtype == SW_F16 || act_dtype == SW_BF16, "Unsupported data type of key/value: %d", act_dtype);
+  SW_CHECK_ARG(fp8 || cache_dtype == act_dtype, "Unsupported data type of kv cache: %d", cache_dtype);
+  SW_CHECK_ARG(x == (fp8 ? 16 : 8) && head_size % x == 0 && block_size % (fp8 ? kPfFp8Tokens : kPfTokens) == 0,
+               "prefill_attention_and_cache: x %d, heads of %d, blocks of %d", x, head_size, block_size);
+  const CacheWrite write = cache_write(key, value, key_cache, value_cache, slot_mapping, num_tokens, num_kv_heads, head_size,
+                                       block_size, k_stride, v_stride, 2);
+  return prefill_entry(out, query, key, value, seq_starts, seq_lens, num_seqs, max_seq_len, num_heads,
+                       num_kv_heads, head_size, scale, alibi_slopes, q_stride, k_stride, v_stride, out_stride,
+                       sliding_window, act_dtype, nullptr, &write, fp8, stream);
 }
 
 static int context_attention_entry(void* out, const void* query, const void* key, const void* value,
@@ -975,7 +1045,7 @@ static int context_attention_entry(void* out, const void* query, const void* key
   }
   return prefill_entry(out, query, key, value, seq_starts, new_lens, num_seqs, max_new_len, num_heads, num_kv_heads,
                        head_size, scale, alibi_slopes, q_stride, k_stride, v_stride, out_stride, sliding_window,
-                       act_dtype, &cx, stream);
+                       act_dtype, &cx, nullptr, 0, stream);
 }
 
 extern "C" int64_t sw_context_attention_split_workspace_bytes(int num_parts, int64_t total_rows, int num_heads,

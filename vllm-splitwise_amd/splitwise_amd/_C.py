@@ -55,6 +55,8 @@ _SIGNATURES = {
     "sw_prefill_attention": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int,
                              _c_int, _c_int, _c_int, _c_float, _c_void_p, _c_i64, _c_i64, _c_i64, _c_i64,
                              _c_int, _c_int, _c_void_p],
+    "sw_prefill_attention_and_cache": [_c_void_p] * 6 + [_c_int] * 5 + [ctypes.c_float, _c_void_p] + [_c_i64] * 4
+                                      + [_c_int] * 2 + [_c_void_p] * 3 + [_c_int] * 4 + [_c_void_p],
     "sw_rms_norm": [_c_void_p, _c_void_p, _c_void_p, _c_float, _c_i64, _c_int, _c_i64, _c_int, _c_void_p],
     "sw_fused_add_rms_norm": [_c_void_p, _c_void_p, _c_void_p, _c_float, _c_i64, _c_int, _c_i64, _c_int,
                               _c_void_p],
@@ -107,7 +109,7 @@ def library_path() -> str:
     return _LIB_PATH
 
 
-ABI_VERSION = 7                # SW_ABI_VERSION of include/splitwise_hip.h this binding was written against
+ABI_VERSION = 8                # SW_ABI_VERSION of include/splitwise_hip.h this binding was written against
 
 
 def load_library() -> ctypes.CDLL:
@@ -407,6 +409,50 @@ def prefill_attention(out: torch.Tensor, query: torch.Tensor, key: torch.Tensor,
             query.shape[2], float(scale), alibi_slopes.data_ptr() if alibi_slopes is not None else None,
             query.stride(0), key.stride(0), value.stride(0), out.stride(0),
             int(sliding_window) if sliding_window else 0, act, _stream(query)))
+
+
+def prefill_attention_and_cache(out: torch.Tensor, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
+                                seq_starts: torch.Tensor, seq_lens: torch.Tensor, max_seq_len: int, scale: float,
+                                alibi_slopes: Optional[torch.Tensor], sliding_window: Optional[int], key_cache: torch.Tensor,
+                                value_cache: torch.Tensor, slot_mapping: torch.Tensor, kv_cache_dtype: str) -> bool:
+    """``reshape_and_cache`` of a prompt run's keys and values and ``prefill_attention`` over them in one launch.  False: not in
+    this form, nothing has been done and the two are to be called one after the other (which also word the refusals)."""
+    if alibi_slopes is None:
+        status = _native.prefill_attention_and_cache(out, query, key, value, seq_starts, seq_lens, max_seq_len, scale, alibi_slopes,
+                                                     sliding_window, key_cache, value_cache, slot_mapping, kv_cache_dtype)
+        if status is not None:
+            return _done(status)
+    tensors = (out, query, key, value, seq_starts, seq_lens, key_cache, value_cache, slot_mapping)
+    if not all(t.is_cuda and t.device == query.device for t in tensors):
+        return False
+    if query.dtype not in (torch.float16, torch.bfloat16) or key.dtype != query.dtype or kv_cache_dtype not in ("auto", "fp8_e5m2"):
+        return False
+    if (seq_starts.dtype != torch.int32 or seq_lens.dtype != torch.int32 or slot_mapping.dtype != torch.int64
+            or key_cache.dim() != 5):
+        return False
+    if any(t.dim() != 3 or t.stride(2) != 1 or t.stride(1) != t.shape[2] for t in (out, query, key, value)):
+        return False
+    if key.shape != value.shape or key.shape[2] != query.shape[2] or out.dtype != query.dtype or value.dtype != key.dtype:
+        return False
+    act = _act_dtype(query)
+    if alibi_slopes is not None and not alibi_slopes.is_cuda:
+        alibi_slopes = alibi_slopes.to(query.device)
+    with _on_device_of(query):
+        return _done(load_library().sw_prefill_attention_and_cache(
+            out.data_ptr(), query.data_ptr(), key.data_ptr(), value.data_ptr(), seq_starts.data_ptr(),
+            seq_lens.data_ptr(), seq_lens.numel(), int(max_seq_len), query.shape[1], key.shape[1],
+            query.shape[2], float(scale), alibi_slopes.data_ptr() if alibi_slopes is not None else None,
+            query.stride(0), key.stride(0), value.stride(0), out.stride(0),
+            int(sliding_window) if sliding_window else 0, act, key_cache.data_ptr(), value_cache.data_ptr(),
+            slot_mapping.data_ptr(), key.shape[0], key_cache.shape[3], key_cache.shape[4],
+            _cache_dtype(kv_cache_dtype, act), _stream(query)))
+
+
+def _done(status: int) -> bool:
+    if status == -1:               # SW_ERR_INVALID
+        return False
+    _check(status)
+    return True
 
 
 def context_attention_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, k_cache: torch.Tensor,
@@ -836,6 +882,7 @@ ops = SimpleNamespace(
     paged_attention_v2=paged_attention_v2,
     paged_attention_v2_static=paged_attention_v2_static,
     prefill_attention=prefill_attention,
+    prefill_attention_and_cache=prefill_attention_and_cache,
     context_attention_fwd=context_attention_fwd,
     rms_norm=rms_norm,
     fused_add_rms_norm=fused_add_rms_norm,

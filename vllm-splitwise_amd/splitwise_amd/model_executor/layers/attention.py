@@ -186,7 +186,20 @@ class Attention(nn.Module):
         if self.alibi_slopes is not None and self.alibi_slopes.device != query.device:
             self.alibi_slopes = self.alibi_slopes.to(query.device)
 
-        if key_cache is not None and value_cache is not None and not fused_cache_write:
+        tables = input_metadata.block_tables
+        writes_cache = key_cache is not None and value_cache is not None and not fused_cache_write
+        if (writes_cache and input_metadata.is_prompt and (tables is None or tables.numel() == 0)
+                and not (input_metadata.blocks_to_nw and self.kvcache_comm_manager is not None)):
+            # a plain prompt run: both in one launch, where that has a form for the call
+            output = torch.empty_like(query)
+            slots = input_metadata.slot_mapping
+            if _C.ops.prefill_attention_and_cache(output, query, key, value, input_metadata.start_loc,
+                                                  input_metadata.prompt_lens, input_metadata.max_seq_len, self.scale,
+                                                  self.alibi_slopes, self.sliding_window, key_cache, value_cache,
+                                                  slots if slots.dim() == 1 else slots.flatten(),
+                                                  input_metadata.kv_cache_dtype):
+                return output.view(out_shape[:-1] + (self.num_heads * self.head_size,))
+        if writes_cache:
             PagedAttentionImpl.reshape_and_cache(key, value, key_cache, value_cache, input_metadata)
 
         if input_metadata.is_prompt:
@@ -204,7 +217,6 @@ class Attention(nn.Module):
                     for sem_id, runs in input_metadata.blocks_to_nw.items():
                         for block_start, num_blocks in runs:
                             comm.put(sem_id, self.layer_id, block_start, num_blocks)
-            tables = input_metadata.block_tables
             if key_cache is not None and tables is not None and tables.numel() > 0:
                 # some prompt of the step continues a prefix that is in the cache already: the new tokens
                 # attend to the paged context and to each other (backends/xformers.py:166-177)
