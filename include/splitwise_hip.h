@@ -52,7 +52,7 @@ const char* sw_last_error(void);
  * 6: sw_kv_push_mapped added.
  * 7: sw_context_attention_split, sw_context_attention_split_parts, sw_context_attention_split_workspace_bytes
  *    added. */
-#define SW_ABI_VERSION 8
+#define SW_ABI_VERSION 9
 int sw_abi_version(void);
 
 /* csrc/cuda_utils_kernels.cu:16-35 get_max_shared_memory_per_block_device_attribute:
@@ -134,6 +134,19 @@ int sw_paged_attention_v2(void* out, float* exp_sums, float* max_logits,
                           const float* alibi_slopes, int64_t q_stride,
                           int64_t kv_block_stride, int64_t kv_head_stride,
                           int act_dtype, int cache_dtype, void* stream);
+
+/* sw_reshape_and_cache of a decode step's keys and values ([num_tokens] rows) and paged attention over the caches after it, in one
+ * launch (two where the context is split: tmp_out, exp_sums and max_logits as in sw_paged_attention_v2; NULL: unsplit).  For few
+ * tokens and sequences (16 of each, and tokens x sequences x num_kv_heads x head_size up to 327680), contiguous caches; refuses others before anything is launched. */
+int sw_paged_attention_and_cache(void* out, float* exp_sums, float* max_logits, void* tmp_out, const void* query,
+                                 const void* key, const void* value, void* key_cache, void* value_cache,
+                                 const int64_t* slot_mapping, int num_tokens, int x, int num_seqs, int num_heads,
+                                 int num_kv_heads, int head_size, float scale, const int32_t* block_tables,
+                                 const int32_t* context_lens, int block_size, int max_context_len,
+                                 int max_num_blocks_per_seq, const float* alibi_slopes, int64_t q_stride,
+                                 int64_t key_stride, int64_t value_stride, int64_t kv_block_stride,
+                                 int64_t kv_head_stride, int act_dtype, int cache_dtype, void* stream);
+
 
 /* No counterpart in the reference (whose caller allocates the three temporaries on every call,
  * vllm/model_executor/layers/attention/ops/paged_attn.py:83-93).  For callers that cannot

@@ -23,7 +23,7 @@
 namespace {
 
 #define STEP_OPS(X)                                                                                                     \
-  X(sw_reshape_and_cache) X(sw_paged_attention_v1) X(sw_prefill_attention) X(sw_prefill_attention_and_cache) X(swm_causal_conv) X(swm_gated_delta)        \
+  X(sw_reshape_and_cache) X(sw_paged_attention_v1) X(sw_prefill_attention) X(sw_prefill_attention_and_cache) X(sw_paged_attention_and_cache) X(swm_causal_conv) X(swm_gated_delta)        \
   X(swm_gated_delta_chunked) X(swm_gated_delta_chunked_workspace_floats) X(swm_head_norm_gate_act) X(swm_group_pairs)   \
   X(swm_expert_up_weighted) X(swm_expert_down_weighted) X(swm_masked_attention) X(swm_sink_attention)                   \
   X(swm_masked_attention_workspace_floats) X(swm_gla) X(swm_gla_workspace_floats) X(swm_lightning) X(swm_retention)     \
@@ -244,6 +244,33 @@ STEP_OP(paged_attention_v1) {
                                       (int)query.size(1), kv_heads, (int)query.size(2), scale, ptr<int32_t>(tables),
                                       ptr<int32_t>(lens), block_size, longest, (int)tables.stride(0), nullptr, query.stride(0),
                                       kc.stride(0), kc.stride(1), act, cache, stream);
+    }));
+  });
+}
+
+STEP_OP(paged_attention_and_cache) {
+  return call([&] {
+    const Args c(args, nargs, 17);
+    take(sw_paged_attention_and_cache_at != nullptr && args[16] == Py_None);
+    const Tensor &out = c.tensor(0), &query = c.tensor(4), &key = c.tensor(5), &value = c.tensor(6), &kc = c.tensor(7), &vc = c.tensor(8),
+                 &slots = c.tensor(9), &tables = c.tensor(11), &lens = c.tensor(12);
+    const Tensor *sums = c.optional(1), *most = c.optional(2), *tmp = c.optional(3);
+    const int longest = c.i32(13);
+    const float scale = c.f32(10);
+    const int act = hip_act(query), cache = cache_dtype(args[14], act), kv_heads = c.i32(15);
+    take(query.dim() == 3 && key.dim() == 3 && kc.dim() == 5 && vc.dim() == 4 && kc.is_contiguous() && vc.is_contiguous()
+         && slots.scalar_type() == at::kLong && tables.dim() == 2 && tables.scalar_type() == at::kInt && tables.stride(1) == 1
+         && lens.scalar_type() == at::kInt && key.scalar_type() == query.scalar_type() && value.scalar_type() == query.scalar_type()
+         && out.scalar_type() == query.scalar_type() && value.sizes() == key.sizes() && key.size(1) == kv_heads
+         && key.size(2) == query.size(2) && vc.size(3) == kc.size(3));
+    for (const Tensor* t : {&query, &key, &value}) take(t->stride(2) == 1 && t->stride(1) == t->size(2));
+    void* stream = c.stream();
+    return PyLong_FromLong(unlocked([&] {
+      return sw_paged_attention_and_cache_at(
+          ptr<void>(out), ptr(sums), ptr(most), ptr<void>(tmp), ptr<void>(query), ptr<void>(key), ptr<void>(value), ptr<void>(kc),
+          ptr<void>(vc), ptr<int64_t>(slots), (int)key.size(0), (int)kc.size(4), (int)query.size(0), (int)query.size(1), kv_heads,
+          (int)query.size(2), scale, ptr<int32_t>(tables), ptr<int32_t>(lens), (int)kc.size(3), longest, (int)tables.stride(0), nullptr,
+          query.stride(0), key.stride(0), value.stride(0), kc.stride(0), kc.stride(1), act, cache, stream);
     }));
   });
 }
@@ -592,7 +619,7 @@ PyObject* bind(PyObject*, PyObject* table) {
 #define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr},
 PyMethodDef kMethods[] = {
     METHOD(reshape_and_cache) METHOD(paged_attention_v1) METHOD(prefill_attention) METHOD(causal_conv) METHOD(gated_delta)
-    METHOD(prefill_attention_and_cache)
+    METHOD(prefill_attention_and_cache) METHOD(paged_attention_and_cache)
     METHOD(head_norm_gate) METHOD(gla) METHOD(lightning) METHOD(retention) METHOD(group_pairs) METHOD(expert_ffn)
     METHOD(capped_attention) {"bind", bind, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -29,8 +29,11 @@
 
 namespace sw {
 
-constexpr int kPaThreads = 256;
-constexpr int kPaWaves = 4;
+// Launches of up to this many workgroups have 8 waves each, not 4: a workgroup's chain is half as long where the GPU has room for the waves
+// (us, 4 / 8 waves, the write below included: 32 heads of 128, 2 x 700 tokens 15.8 / 13.0, 8 x 700 24.2 / 20.3, 8 x 2000 62.3 / 55.5).  Twice
+// as many where a token is 128 bytes of a head's keys (fp8 of 128, 16 bits of 64): 40 heads of 128, fp8, 8 x 1300 29.7 / 24.8, 8 x 1800
+// 50.2 / 38.3, but 32 of 128, bf16, 10 x 2500 97.3 / 101.9.
+constexpr int pa_wide_up_to(int key_bytes) { return key_bytes <= 128 ? 512 : 256; }
 constexpr int kPaLeanUpTo = 4096;     // workgroups: launches up to this size take the vector kernel's LEAN form
 constexpr int kPartitionSize = 512;   // vllm/.../ops/paged_attn.py:12 _PARTITION_SIZE
 
@@ -122,23 +125,89 @@ __device__ __forceinline__ void cache_pairs(const uint32_t* w, uint32_t* out) {
 template <typename act_t, bool FP8> struct PackedPath { static constexpr bool value = Dot2<act_t>::kAvailable && !FP8; };
 template <> struct PackedPath<f16_t, true> { static constexpr bool value = true; };
 
+// A decode step's new tokens on their way into the cache, beside the attention over it.  Every workgroup writes the new keys and values of
+// its kv head, of ALL the call's tokens, before it reads the cache: what it then reads is what a launch in front of it would have left,
+// whatever blocks the sequences share, and no workgroup waits for another (they write the same bytes to the same places).  That is
+// (tokens x sequences) times the write, so it is for few tokens: kPaWriteUpTo, and kPaWriteElements of keys in all.
+// Measured, a layer's decode step in a stream of calls, two launches / one (us): 32 heads of 128, 2 x 700 tokens 18.3 / 15.8, 1 x 4000 (split)
+// 25.9 / 19.7; 64 on 8, fp8, 2 x 700 14.7 / 12.0; 12 of 64, 16 x 300 14.5 / 11.8; but 32 of 128, 16 x 700 44.3 / 47.0.
+struct PaWrite {
+  const void *key, *value;
+  void *k_cache, *v_cache;
+  const int64_t* slots;
+  int64_t key_stride, value_stride;                // elements
+  int tokens;                                      // 0: the cache is as it should be
+};
+constexpr int kPaWriteUpTo = 16;
+constexpr int64_t kPaWriteElements = 8 * 8 * 40 * 128;
+// The caches' pointers of a kernel that writes them are not __restrict__: its loads stay behind the stores.
+template <bool WRITE> struct PaCachePtr { using type = const void* __restrict__; };
+template <> struct PaCachePtr<true> { using type = const void*; };
+
+template <typename act_t, bool FP8, int HEAD, int BS, int THREADS>
+__device__ __forceinline__ void pa_write(const PaWrite& w, int kv_head, int64_t kv_block_stride, int64_t kv_head_stride) {
+  using T = CacheTraits<act_t, FP8>;
+  using S = typename T::S;
+  constexpr int ES = T::ES, CS = T::CS, X = T::X, NCH = HEAD / X, DW = X * ES / 16;
+  const int tid = threadIdx.x;
+  auto tile = [&](int64_t slot) { return (slot / BS * kv_block_stride + (int64_t)kv_head * kv_head_stride) * CS; };
+  // keys: 16 bytes of the cache a thread
+  for (int p = tid; p < w.tokens * NCH; p += THREADS) {
+    const int t = p / NCH, c = p - t * NCH;
+    const int64_t slot = w.slots[t];
+    const uint4* src = reinterpret_cast<const uint4*>(static_cast<const S*>(w.key) + t * w.key_stride + (int64_t)kv_head * HEAD + c * X);
+    union {
+      uint4 q[DW];
+      S e[X];
+    } in;
+#pragma unroll
+    for (int i = 0; i < DW; ++i) in.q[i] = src[i];
+    union {
+      uint4 q;
+      uint8_t b[16];
+    } to;
+    if constexpr (FP8) {
+#pragma unroll
+      for (int i = 0; i < X; ++i) to.b[i] = Conv<act_t>::to_e5m2(in.e[i]);
+    } else {
+      to.q = in.q[0];
+    }
+    if (slot >= 0) *reinterpret_cast<uint4*>(static_cast<char*>(w.k_cache) + tile(slot) + (c * BS + (int)(slot % BS)) * 16) = to.q;
+  }
+  // values: an element a thread
+  for (int e = tid; e < w.tokens * HEAD; e += THREADS) {
+    const int t = e / HEAD, d = e - t * HEAD;
+    const int64_t slot = w.slots[t];
+    const S v = static_cast<const S*>(w.value)[t * w.value_stride + (int64_t)kv_head * HEAD + d];
+    if (slot < 0) continue;
+    char* to = static_cast<char*>(w.v_cache) + tile(slot) + (int64_t)(d * BS + (int)(slot % BS)) * CS;
+    if constexpr (FP8) {
+      *reinterpret_cast<uint8_t*>(to) = Conv<act_t>::to_e5m2(v);
+    } else {
+      *reinterpret_cast<S*>(to) = v;
+    }
+  }
+}
+
 // LEAN: the group's block-table entries are read once (the P.V phase takes block b's entry from lane b * BS of
 // the Q.K phase's read instead of reading the table again in front of every block's loads) and the wave index
 // is handed to the compiler as uniform, which moves the P.V address arithmetic to the scalar unit.  Faster
 // wherever a wave's chain of dependent loads shows -- launches of a few thousand workgroups or fewer (8 x 1024
 // tokens 24.5 -> 22 us, 4 x 1024 20.8 -> 16.6, 128 x 860 311 -> 306) and every fp8 launch (256 x 860: 325 ->
 // 305 us) -- and 0.4-1.6 % slower on the largest 16-bit launches, which keep the plain form.
-template <typename act_t, bool FP8, int HEAD, int BS, int QG, bool LEAN>
-__global__ void __launch_bounds__(kPaThreads)
+// WRITE: the call's tokens go into the cache first (pa_write).
+// NW: waves, which take the context's 64-token groups in turn.
+template <typename act_t, bool FP8, int HEAD, int BS, int QG, bool LEAN, bool WRITE, int NW>
+__global__ void __launch_bounds__(NW * 64)
 paged_attention_kernel(void* __restrict__ out_,            // v1: [S,H,HEAD]; v2: tmp_out [S,H,P,HEAD]
                        float* __restrict__ exp_sums,       // v2 only [S,H,P]
                        float* __restrict__ max_logits,     // v2 only [S,H,P]
-                       const void* __restrict__ q_, const void* __restrict__ k_cache_,
-                       const void* __restrict__ v_cache_, int num_heads, int num_kv_heads,
+                       const void* __restrict__ q_, typename PaCachePtr<WRITE>::type k_cache_,
+                       typename PaCachePtr<WRITE>::type v_cache_, int num_heads, int num_kv_heads,
                        float scale, const int32_t* __restrict__ block_tables,
                        const int32_t* __restrict__ context_lens, int max_num_blocks_per_seq,
                        const float* __restrict__ alibi_slopes, int64_t q_stride,
-                       int64_t kv_block_stride, int64_t kv_head_stride, int partitioned) {
+                       int64_t kv_block_stride, int64_t kv_head_stride, int partitioned, const PaWrite w) {
   using T = CacheTraits<act_t, FP8>;
   using S = typename T::S;
   constexpr int ES = T::ES, CS = T::CS, X = T::X;
@@ -158,9 +227,9 @@ paged_attention_kernel(void* __restrict__ out_,            // v1: [S,H,HEAD]; v2
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* q_s = reinterpret_cast<float*>(smem);                              // [QG][HEAD]
-  S* p_s = reinterpret_cast<S*>(smem + QG * HEAD * 4);                      // [4][QG][64]
-  float* red_s = reinterpret_cast<float*>(smem + QG * HEAD * 4 + kPaWaves * QG * 64 * ES);
-  // red_s: [4][QG][HEAD] acc, then [4][QG] m, then [4][QG] l
+  S* p_s = reinterpret_cast<S*>(smem + QG * HEAD * 4);                      // [NW][QG][64]
+  float* red_s = reinterpret_cast<float*>(smem + QG * HEAD * 4 + NW * QG * 64 * ES);
+  // red_s: [NW][QG][HEAD] acc, then [NW][QG] m, then [NW][QG] l
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -197,6 +266,8 @@ paged_attention_kernel(void* __restrict__ out_,            // v1: [S,H,HEAD]; v2
   const int kv_head = hx / wg_per_kv;
   const int head0 = kv_head * groups_per_kv + (hx - kv_head * wg_per_kv) * QG;
 
+  if constexpr (WRITE) pa_write<act_t, FP8, HEAD, BS, NW * 64>(w, kv_head, kv_block_stride, kv_head_stride);
+
   const int ctx = context_lens[seq];
   const int tok_begin = partitioned ? part_idx * kPartitionSize : 0;
   if (partitioned && tok_begin >= ctx) return;              // uniform: whole workgroup leaves
@@ -210,12 +281,12 @@ paged_attention_kernel(void* __restrict__ out_,            // v1: [S,H,HEAD]; v2
     if constexpr (PACKED) {
       uint32_t* dst = reinterpret_cast<uint32_t*>(smem);
       const uint32_t* src = reinterpret_cast<const uint32_t*>(q);          // 4-byte aligned: checked on the host
-      for (int i = tid; i < QG * HEAD / 2; i += kPaThreads) dst[i] = src[i];
+      for (int i = tid; i < QG * HEAD / 2; i += NW * 64) dst[i] = src[i];
     } else {
-      for (int i = tid; i < QG * HEAD; i += kPaThreads) q_s[i] = Conv<act_t>::to_float(q[i]);
+      for (int i = tid; i < QG * HEAD; i += NW * 64) q_s[i] = Conv<act_t>::to_float(q[i]);
     }
   }
-  __syncthreads();
+  __syncthreads();                                          // the query, and what was written to the cache
 
   const char* k_cache = reinterpret_cast<const char*>(k_cache_);
   const char* v_cache = reinterpret_cast<const char*>(v_cache_);
@@ -239,7 +310,7 @@ paged_attention_kernel(void* __restrict__ out_,            // v1: [S,H,HEAD]; v2
   const int blk_in_group = lane / BS;
   const int off_in_blk = lane % BS;
 
-  for (int g = wave; g < n_groups; g += kPaWaves) {
+  for (int g = wave; g < n_groups; g += NW) {
     const int g_tok0 = tok_begin + (g << 6);
     const int token = g_tok0 + lane;
     const bool valid = token < tok_end;
@@ -420,9 +491,9 @@ paged_attention_kernel(void* __restrict__ out_,            // v1: [S,H,HEAD]; v2
 #pragma unroll
       for (int it = 0; it < NIT; ++it) Dot2<act_t>::settle(acc[h][it]);
   }
-  float* acc_s = red_s;                                     // [4][QG][HEAD]
-  float* m_s = red_s + kPaWaves * QG * HEAD;                // [4][QG]
-  float* l_s = m_s + kPaWaves * QG;                         // [4][QG]
+  float* acc_s = red_s;                                     // [NW][QG][HEAD]
+  float* m_s = red_s + NW * QG * HEAD;                // [NW][QG]
+  float* l_s = m_s + NW * QG;                         // [NW][QG]
 #pragma unroll
   for (int h = 0; h < QG; ++h) {
     const float l = wave_sum(l_lane[h]);
@@ -441,15 +512,15 @@ paged_attention_kernel(void* __restrict__ out_,            // v1: [S,H,HEAD]; v2
   }
   __syncthreads();
 
-  for (int i = tid; i < QG * HEAD; i += kPaThreads) {
+  for (int i = tid; i < QG * HEAD; i += NW * 64) {
     const int h = i / HEAD;
     const int d = i - h * HEAD;
     float m = -FLT_MAX;
 #pragma unroll
-    for (int w = 0; w < kPaWaves; ++w) m = fmaxf(m, m_s[w * QG + h]);
+    for (int w = 0; w < NW; ++w) m = fmaxf(m, m_s[w * QG + h]);
     float l = 0.f, o = 0.f;
 #pragma unroll
-    for (int w = 0; w < kPaWaves; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float f = __expf(m_s[w * QG + h] - m);
       l = fmaf(l_s[w * QG + h], f, l);
       o = fmaf(acc_s[(w * QG + h) * HEAD + d], f, o);
@@ -527,6 +598,7 @@ struct PaArgs {
   int block_size, max_context_len, max_num_blocks_per_seq;
   const float* alibi; int64_t q_stride, kv_block_stride, kv_head_stride;
   int partitioned; hipStream_t stream;
+  PaWrite write;
 };
 
 template <typename act_t, bool FP8, int HEAD, int BS, int QG>
@@ -535,16 +607,21 @@ int launch_pa(const PaArgs& a) {
   const int g = a.num_heads / a.num_kv_heads;
   const int parts = a.partitioned ? (a.max_context_len + kPartitionSize - 1) / kPartitionSize : 1;
   dim3 grid(a.num_kv_heads * (g / QG), a.num_seqs, parts);
-  const size_t smem = (size_t)QG * HEAD * 4 + (size_t)kPaWaves * QG * 64 * T::ES +
-                      (size_t)kPaWaves * QG * HEAD * 4 + 2 * kPaWaves * QG * 4;
   // fp8 caches always take the lean form (there is no other instantiation for them)
-  const bool lean = FP8 || (int64_t)grid.x * grid.y * grid.z <= kPaLeanUpTo;
-  auto kernel = lean ? paged_attention_kernel<act_t, FP8, HEAD, BS, QG, true>
-                     : paged_attention_kernel<act_t, FP8, HEAD, BS, QG, FP8>;
-  kernel<<<grid, kPaThreads, smem, a.stream>>>(
+  const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
+  const bool lean = FP8 || wgs <= kPaLeanUpTo, wide = lean && wgs <= pa_wide_up_to(HEAD * T::CS);
+  SW_CHECK_ARG(lean || a.write.tokens == 0, "paged_attention_and_cache: too large a launch");
+  const int nw = wide ? 8 : 4;
+  const size_t smem = (size_t)QG * HEAD * 4 + (size_t)nw * QG * 64 * T::ES + (size_t)nw * QG * HEAD * 4 + 2 * nw * QG * 4;
+  auto kernel = a.write.tokens > 0 ? (wide ? paged_attention_kernel<act_t, FP8, HEAD, BS, QG, true, true, 8>
+                                           : paged_attention_kernel<act_t, FP8, HEAD, BS, QG, true, true, 4>)
+                : wide             ? paged_attention_kernel<act_t, FP8, HEAD, BS, QG, true, false, 8>
+                : lean             ? paged_attention_kernel<act_t, FP8, HEAD, BS, QG, true, false, 4>
+                                   : paged_attention_kernel<act_t, FP8, HEAD, BS, QG, FP8, false, 4>;
+  kernel<<<grid, nw * 64, smem, a.stream>>>(
       a.partitioned ? a.tmp_out : a.out, a.exp_sums, a.max_logits, a.q, a.k, a.v, a.num_heads,
       a.num_kv_heads, a.scale, a.block_tables, a.context_lens, a.max_num_blocks_per_seq, a.alibi,
-      a.q_stride, a.kv_block_stride, a.kv_head_stride, a.partitioned);
+      a.q_stride, a.kv_block_stride, a.kv_head_stride, a.partitioned, a.write);
   SW_CHECK_LAUNCH();
   if (a.partitioned) {
     dim3 rgrid(a.num_heads, a.num_seqs);
@@ -562,7 +639,8 @@ namespace sw {
 template <typename act_t, bool FP8, int HEAD, int BS, int NW>
 int launch_pa_mfma_nw(const PaArgs& a, int qg, dim3 grid) {
   const size_t smem = (size_t)NW * kPaMfmaHeads * kPaMfmaPRow * 2 + (size_t)NW * qg * HEAD * 4 + 2 * NW * qg * 4;
-  auto kernel = paged_attention_mfma_kernel<act_t, FP8, HEAD, BS, NW>;
+  auto kernel = a.write.tokens > 0 ? paged_attention_mfma_kernel<act_t, FP8, HEAD, BS, NW, true>
+                                   : paged_attention_mfma_kernel<act_t, FP8, HEAD, BS, NW, false>;
   if (smem > 64 * 1024) {
     // on every launch: the attribute belongs to the function ON THE CURRENT DEVICE, and a process may drive
     // several devices from several threads; the call costs well under a microsecond
@@ -572,7 +650,7 @@ int launch_pa_mfma_nw(const PaArgs& a, int qg, dim3 grid) {
   kernel<<<grid, NW * 64, smem, a.stream>>>(
       a.partitioned ? a.tmp_out : a.out, a.exp_sums, a.max_logits, a.q, a.k, a.v, a.num_heads, a.num_kv_heads,
       a.scale, a.block_tables, a.context_lens, a.max_num_blocks_per_seq, a.alibi, a.q_stride, a.kv_block_stride,
-      a.kv_head_stride, a.partitioned, qg);
+      a.kv_head_stride, a.partitioned, qg, a.write);
   SW_CHECK_LAUNCH();
   return SW_OK;
 }

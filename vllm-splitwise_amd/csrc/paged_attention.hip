@@ -77,7 +77,7 @@ int sw_paged_attention_v1(void* out, const void* query, const void* key_cache,
   sw::PaArgs a{out, nullptr, nullptr, nullptr, query, key_cache, value_cache, num_seqs, num_heads,
                num_kv_heads, head_size, scale, block_tables, context_lens, block_size,
                max_context_len, max_num_blocks_per_seq, alibi_slopes, q_stride, kv_block_stride,
-               kv_head_stride, 0, static_cast<hipStream_t>(stream)};
+               kv_head_stride, 0, static_cast<hipStream_t>(stream), {}};
   return sw::run_paged_attention(a, act_dtype, cache_dtype);
 }
 
@@ -91,7 +91,37 @@ int sw_paged_attention_v2(void* out, float* exp_sums, float* max_logits, void* t
   sw::PaArgs a{out, exp_sums, max_logits, tmp_out, query, key_cache, value_cache, num_seqs,
                num_heads, num_kv_heads, head_size, scale, block_tables, context_lens, block_size,
                max_context_len, max_num_blocks_per_seq, alibi_slopes, q_stride, kv_block_stride,
-               kv_head_stride, 1, static_cast<hipStream_t>(stream)};
+               kv_head_stride, 1, static_cast<hipStream_t>(stream), {}};
+  return sw::run_paged_attention(a, act_dtype, cache_dtype);
+}
+
+int sw_paged_attention_and_cache(void* out, float* exp_sums, float* max_logits, void* tmp_out, const void* query,
+                                 const void* key, const void* value, void* key_cache, void* value_cache,
+                                 const int64_t* slot_mapping, int num_tokens, int x, int num_seqs, int num_heads,
+                                 int num_kv_heads, int head_size, float scale, const int32_t* block_tables,
+                                 const int32_t* context_lens, int block_size, int max_context_len,
+                                 int max_num_blocks_per_seq, const float* alibi_slopes, int64_t q_stride, int64_t key_stride,
+                                 int64_t value_stride, int64_t kv_block_stride, int64_t kv_head_stride, int act_dtype,
+                                 int cache_dtype, void* stream) {
+  const bool fp8 = cache_dtype == SW_FP8_E5M2;
+  const int es = sw::dtype_size(act_dtype), cs = fp8 ? 1 : es;
+  SW_CHECK_ARG(num_seqs > 0 && num_tokens > 0 && num_kv_heads > 0 && block_size > 0 &&
+                   (act_dtype == SW_F32 || act_dtype == SW_F16 || act_dtype == SW_BF16),
+               "paged_attention_and_cache: nothing to do for one of the two");
+  SW_CHECK_ARG(num_tokens <= sw::kPaWriteUpTo && num_seqs <= sw::kPaWriteUpTo &&
+                   (int64_t)num_tokens * num_seqs * num_kv_heads * head_size <= sw::kPaWriteElements,
+               "paged_attention_and_cache: %d tokens of %d sequences",
+               num_tokens, num_seqs);
+  SW_CHECK_ARG(x == 16 / cs && head_size % x == 0 && (head_size * es) % 16 == 0 && (key_stride * es) % 16 == 0 &&
+                   (value_stride * es) % 16 == 0 && reinterpret_cast<uintptr_t>(key) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(value) % 16 == 0,
+               "paged_attention_and_cache: key/value rows must be 16-byte aligned");
+  SW_CHECK_ARG(kv_head_stride == (int64_t)head_size * block_size && kv_block_stride == kv_head_stride * num_kv_heads,
+               "paged_attention_and_cache: the caches must be contiguous");
+  sw::PaArgs a{out, exp_sums, max_logits, tmp_out, query, key_cache, value_cache, num_seqs, num_heads, num_kv_heads, head_size, scale,
+               block_tables, context_lens, block_size, max_context_len, max_num_blocks_per_seq, alibi_slopes, q_stride,
+               kv_block_stride, kv_head_stride, tmp_out != nullptr, static_cast<hipStream_t>(stream),
+               {key, value, key_cache, value_cache, slot_mapping, key_stride, value_stride, num_tokens}};
   return sw::run_paged_attention(a, act_dtype, cache_dtype);
 }
 
@@ -129,7 +159,7 @@ int sw_paged_attention_v2_static(void* out, const void* query, const void* key_c
   sw::PaArgs a{out, exp_sums, max_logits, tmp_out, query, key_cache, value_cache, num_seqs,
                num_heads, num_kv_heads, head_size, scale, block_tables, context_lens, block_size,
                max_context_len, max_num_blocks_per_seq, alibi_slopes, q_stride, kv_block_stride,
-               kv_head_stride, 1, static_cast<hipStream_t>(stream)};
+               kv_head_stride, 1, static_cast<hipStream_t>(stream), {}};
   return sw::run_paged_attention(a, act_dtype, cache_dtype);
 }
 

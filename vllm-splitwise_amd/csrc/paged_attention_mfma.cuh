@@ -65,14 +65,14 @@ constexpr int kPaMfmaPRow = 72;         // 16-bit elements per row of the probab
 // NW waves per workgroup share one (sequence, head group[, partition]): 64-token groups go to the waves
 // round robin.  A launch of few workgroups takes more waves each, so that every SIMD of the chip
 // still has a wave streaming (the launcher picks 4 or 8).
-template <typename act_t, bool FP8, int HEAD, int BS, int NW>
+template <typename act_t, bool FP8, int HEAD, int BS, int NW, bool WRITE>
 __global__ void __launch_bounds__(NW * 64)
 paged_attention_mfma_kernel(void* __restrict__ out_, float* __restrict__ exp_sums, float* __restrict__ max_logits,
-                            const void* __restrict__ q_, const void* __restrict__ k_cache_,
-                            const void* __restrict__ v_cache_, int num_heads, int num_kv_heads, float scale,
+                            const void* __restrict__ q_, typename PaCachePtr<WRITE>::type k_cache_,
+                            typename PaCachePtr<WRITE>::type v_cache_, int num_heads, int num_kv_heads, float scale,
                             const int32_t* __restrict__ block_tables, const int32_t* __restrict__ context_lens,
                             int max_num_blocks_per_seq, const float* __restrict__ alibi_slopes, int64_t q_stride,
-                            int64_t kv_block_stride, int64_t kv_head_stride, int partitioned, int qg) {
+                            int64_t kv_block_stride, int64_t kv_head_stride, int partitioned, int qg, const PaWrite w) {
   using S = uint16_t;
   constexpr bool F16M = FP8 || std::is_same<act_t, f16_t>::value;        // element type of the products
   constexpr bool REEXPRESS = FP8 && std::is_same<act_t, bf16_t>::value;  // bf16 values carried as f16
@@ -130,6 +130,11 @@ paged_attention_mfma_kernel(void* __restrict__ out_, float* __restrict__ exp_sum
   const int wg_per_kv = groups_per_kv / qg;
   const int kv_head = hx / wg_per_kv;
   const int head0 = kv_head * groups_per_kv + (hx - kv_head * wg_per_kv) * qg;
+
+  if constexpr (WRITE) {
+    pa_write<act_t, FP8, HEAD, BS, NW * 64>(w, kv_head, kv_block_stride, kv_head_stride);
+    __syncthreads();
+  }
 
   const int ctx = context_lens[seq];
   const int tok_begin = partitioned ? part_idx * kPartitionSize : 0;

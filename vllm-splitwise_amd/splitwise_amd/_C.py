@@ -55,6 +55,8 @@ _SIGNATURES = {
     "sw_prefill_attention": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int,
                              _c_int, _c_int, _c_int, _c_float, _c_void_p, _c_i64, _c_i64, _c_i64, _c_i64,
                              _c_int, _c_int, _c_void_p],
+    "sw_paged_attention_and_cache": [_c_void_p] * 10 + [_c_int] * 6 + [_c_float] + [_c_void_p] * 2 + [_c_int] * 3 + [_c_void_p]
+                                    + [_c_i64] * 5 + [_c_int] * 2 + [_c_void_p],
     "sw_prefill_attention_and_cache": [_c_void_p] * 6 + [_c_int] * 5 + [ctypes.c_float, _c_void_p] + [_c_i64] * 4
                                       + [_c_int] * 2 + [_c_void_p] * 3 + [_c_int] * 4 + [_c_void_p],
     "sw_rms_norm": [_c_void_p, _c_void_p, _c_void_p, _c_float, _c_i64, _c_int, _c_i64, _c_int, _c_void_p],
@@ -109,7 +111,7 @@ def library_path() -> str:
     return _LIB_PATH
 
 
-ABI_VERSION = 8                # SW_ABI_VERSION of include/splitwise_hip.h this binding was written against
+ABI_VERSION = 9                # SW_ABI_VERSION of include/splitwise_hip.h this binding was written against
 
 
 def load_library() -> ctypes.CDLL:
@@ -359,6 +361,50 @@ def paged_attention_v2(out: torch.Tensor, exp_sums: torch.Tensor, max_logits: to
             block_size, int(max_context_len), block_tables.stride(0),
             alibi_slopes.data_ptr() if alibi_slopes is not None else None, query.stride(0),
             key_cache.stride(0), key_cache.stride(1), act, cache, _stream(query)))
+
+
+def paged_attention_and_cache(out: torch.Tensor, exp_sums: Optional[torch.Tensor], max_logits: Optional[torch.Tensor],
+                              tmp_out: Optional[torch.Tensor], query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
+                              key_cache: torch.Tensor, value_cache: torch.Tensor, slot_mapping: torch.Tensor, scale: float,
+                              block_tables: torch.Tensor, context_lens: torch.Tensor, max_context_len: int,
+                              kv_cache_dtype: str, num_kv_heads: int, alibi_slopes: Optional[torch.Tensor]) -> bool:
+    """``reshape_and_cache`` of a decode step's keys and values and ``paged_attention_v1`` (``v2`` with temporaries) over the caches
+    in one launch, for few tokens.  False: not in this form, nothing has been done and the two are to be called one after the
+    other (which also word the refusals)."""
+    if alibi_slopes is None:
+        status = _native.paged_attention_and_cache(out, exp_sums, max_logits, tmp_out, query, key, value, key_cache, value_cache,
+                                                   slot_mapping, scale, block_tables, context_lens, max_context_len,
+                                                   kv_cache_dtype, num_kv_heads, alibi_slopes)
+        if status is not None:
+            return _done(status)
+    tensors = (out, query, key, value, key_cache, value_cache, slot_mapping, block_tables, context_lens)
+    if not all(t.is_cuda and t.device == query.device for t in tensors):
+        return False
+    if (query.dtype not in (torch.float32, torch.float16, torch.bfloat16) or kv_cache_dtype not in ("auto", "fp8_e5m2")
+            or not query.dtype == key.dtype == value.dtype == out.dtype):
+        return False
+    if (slot_mapping.dtype != torch.int64 or block_tables.dtype != torch.int32 or context_lens.dtype != torch.int32
+            or block_tables.dim() != 2 or block_tables.stride(1) != 1):
+        return False
+    if (key_cache.dim() != 5 or value_cache.dim() != 4 or not key_cache.is_contiguous() or not value_cache.is_contiguous()
+            or key_cache.shape[3] != value_cache.shape[3]):
+        return False
+    if any(t.dim() != 3 or t.stride(2) != 1 or t.stride(1) != t.shape[2] for t in (query, key, value)):
+        return False
+    if key.shape != value.shape or key.shape[1] != num_kv_heads or key.shape[2] != query.shape[2]:
+        return False
+    act = _act_dtype(query)
+    if alibi_slopes is not None and not alibi_slopes.is_cuda:
+        alibi_slopes = alibi_slopes.to(query.device)
+    at = lambda t: t.data_ptr() if t is not None else None      # noqa: E731
+    with _on_device_of(query):
+        return _done(load_library().sw_paged_attention_and_cache(
+            out.data_ptr(), at(exp_sums), at(max_logits), at(tmp_out), query.data_ptr(), key.data_ptr(), value.data_ptr(),
+            key_cache.data_ptr(), value_cache.data_ptr(), slot_mapping.data_ptr(), key.shape[0], key_cache.shape[4],
+            query.shape[0], query.shape[1], num_kv_heads, query.shape[2], float(scale), block_tables.data_ptr(),
+            context_lens.data_ptr(), key_cache.shape[3], int(max_context_len), block_tables.stride(0), at(alibi_slopes),
+            query.stride(0), key.stride(0), value.stride(0), key_cache.stride(0), key_cache.stride(1), act,
+            _cache_dtype(kv_cache_dtype, act), _stream(query)))
 
 
 def paged_attention_v2_static(out: torch.Tensor, query: torch.Tensor, key_cache: torch.Tensor,
@@ -881,6 +927,7 @@ ops = SimpleNamespace(
     paged_attention_v1=paged_attention_v1,
     paged_attention_v2=paged_attention_v2,
     paged_attention_v2_static=paged_attention_v2_static,
+    paged_attention_and_cache=paged_attention_and_cache,
     prefill_attention=prefill_attention,
     prefill_attention_and_cache=prefill_attention_and_cache,
     context_attention_fwd=context_attention_fwd,

@@ -19,6 +19,7 @@ from ... import _C
 from ..input_metadata import InputMetadata
 
 _PARTITION_SIZE = 512          # must match the partition size of sw_paged_attention_v2
+_WRITES_BESIDE_ATTENTION = 16, 327680      # what sw_paged_attention_and_cache takes: tokens and sequences, key elements over both
 _SUPPORTED_HEAD_SIZES = [64, 80, 96, 112, 128, 256]
 
 
@@ -81,13 +82,18 @@ class PagedAttentionImpl:
             # the matrix-core kernel (8 waves per workgroup below 256 workgroups): unpartitioned from 128
             # workgroups, and for short contexts whatever the launch size
             return workgroups >= 128 or max_context_len <= 2 * _PARTITION_SIZE
+        # the vector kernels, 8 waves per workgroup up to 256 (us, unpartitioned / partitioned, 32 heads of 128: 1 x 814 tokens
+        # 9.8 / 10.8, 1 x 1176 15.6 / 13.3, 3 x 1578 20.0 / 21.4, 4 x 2185 26.1 / 28.4, 4 x 3035 46.8 / 42.7, 6 x 2185 44.6 / 47.1; 12
+        # heads of 64: 8 x 1578 16.7 / 15.4, 12 x 1578 19.5 / 20.4, 20 x 2216 27.3 / 29.2, 20 x 3078 42.6 / 40.2)
         if workgroups >= 512:
             return True
         if workgroups >= 256:
             return max_context_len < 4096
+        if workgroups >= 160:
+            return max_context_len <= 5 * _PARTITION_SIZE
         if workgroups >= 128:
-            return max_context_len <= _PARTITION_SIZE + _PARTITION_SIZE // 2
-        return workgroups >= 16 and max_context_len <= 2 * _PARTITION_SIZE
+            return max_context_len <= 7 * _PARTITION_SIZE // 2
+        return max_context_len <= 2 * _PARTITION_SIZE
 
     @staticmethod
     def forward_prefix(query, key, value, key_cache, value_cache, input_metadata: InputMetadata,
@@ -104,7 +110,8 @@ class PagedAttentionImpl:
 
     @staticmethod
     def forward_decode(query, key_cache, value_cache, input_metadata: InputMetadata, num_kv_heads: int,
-                       scale: float, alibi_slopes: Optional[torch.Tensor], workspace=None) -> torch.Tensor:
+                       scale: float, alibi_slopes: Optional[torch.Tensor], workspace=None, key=None, value=None) -> torch.Tensor:
+        """key / value: of the step's tokens, which are not in the cache yet.  A few go there in the attention's own launch."""
         output = torch.empty_like(query)
         block_size = value_cache.shape[3]
         num_seqs, num_heads, head_size = query.shape
@@ -117,16 +124,28 @@ class PagedAttentionImpl:
         else:
             unpartitioned = PagedAttentionImpl.use_v1(num_seqs, num_heads, num_kv_heads, max_ctx, width,
                                                       getattr(input_metadata, "mean_context_len", None))
-        if unpartitioned:
-            _C.ops.paged_attention_v1(output, query, key_cache, value_cache, num_kv_heads, scale,
-                                      input_metadata.block_tables, input_metadata.context_lens, block_size,
-                                      max_ctx, alibi_slopes, input_metadata.kv_cache_dtype)
-        else:
+        tmp_output = exp_sums = max_logits = None
+        if not unpartitioned:
             parts = (max_ctx + _PARTITION_SIZE - 1) // _PARTITION_SIZE
             tmp_output = torch.empty((num_seqs, num_heads, parts, head_size), dtype=output.dtype,
                                      device=output.device)
             exp_sums = torch.empty((num_seqs, num_heads, parts), dtype=torch.float32, device=output.device)
             max_logits = torch.empty_like(exp_sums)
+        if key is not None:
+            few, elements = _WRITES_BESIDE_ATTENTION
+            if num_seqs <= few and key.shape[0] <= few and num_seqs * key.numel() <= elements:
+                slots = input_metadata.slot_mapping
+                if _C.ops.paged_attention_and_cache(output, exp_sums, max_logits, tmp_output, query, key, value, key_cache,
+                                                    value_cache, slots if slots.dim() == 1 else slots.flatten(), scale,
+                                                    input_metadata.block_tables, input_metadata.context_lens, max_ctx,
+                                                    input_metadata.kv_cache_dtype, num_kv_heads, alibi_slopes):
+                    return output
+            PagedAttentionImpl.reshape_and_cache(key, value, key_cache, value_cache, input_metadata)
+        if unpartitioned:
+            _C.ops.paged_attention_v1(output, query, key_cache, value_cache, num_kv_heads, scale,
+                                      input_metadata.block_tables, input_metadata.context_lens, block_size,
+                                      max_ctx, alibi_slopes, input_metadata.kv_cache_dtype)
+        else:
             _C.ops.paged_attention_v2(output, exp_sums, max_logits, tmp_output, query, key_cache, value_cache,
                                       num_kv_heads, scale, input_metadata.block_tables,
                                       input_metadata.context_lens, block_size, max_ctx, alibi_slopes,
@@ -199,7 +218,7 @@ class Attention(nn.Module):
                                                   slots if slots.dim() == 1 else slots.flatten(),
                                                   input_metadata.kv_cache_dtype):
                 return output.view(out_shape[:-1] + (self.num_heads * self.head_size,))
-        if writes_cache:
+        if writes_cache and input_metadata.is_prompt:
             PagedAttentionImpl.reshape_and_cache(key, value, key_cache, value_cache, input_metadata)
 
         if input_metadata.is_prompt:
@@ -229,7 +248,8 @@ class Attention(nn.Module):
                                          self.alibi_slopes, self.sliding_window)
         else:
             output = PagedAttentionImpl.forward_decode(query, key_cache, value_cache, input_metadata,
-                                                       self.num_kv_heads, self.scale, self.alibi_slopes)
+                                                       self.num_kv_heads, self.scale, self.alibi_slopes,
+                                                       key=key if writes_cache else None, value=value if writes_cache else None)
         return output.view(out_shape[:-1] + (self.num_heads * self.head_size,))
 
 
