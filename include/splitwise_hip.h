@@ -136,8 +136,9 @@ int sw_paged_attention_v2(void* out, float* exp_sums, float* max_logits,
                           int act_dtype, int cache_dtype, void* stream);
 
 /* sw_reshape_and_cache of a decode step's keys and values ([num_tokens] rows) and paged attention over the caches after it, in one
- * launch (two where the context is split: tmp_out, exp_sums and max_logits as in sw_paged_attention_v2; NULL: unsplit).  For few
- * tokens and sequences (16 of each, and tokens x sequences x num_kv_heads x head_size up to 327680), contiguous caches; refuses others before anything is launched. */
+ * launch (two where the context is split: tmp_out, exp_sums and max_logits as in sw_paged_attention_v2; NULL: unsplit).  For up to 128
+ * tokens, no more than sequences, and num_seqs x num_kv_heads up to 1024 (or up to 16 tokens with tokens x num_seqs x num_kv_heads x
+ * head_size up to 327680), and contiguous caches; refuses others before anything is launched. */
 int sw_paged_attention_and_cache(void* out, float* exp_sums, float* max_logits, void* tmp_out, const void* query,
                                  const void* key, const void* value, void* key_cache, void* value_cache,
                                  const int64_t* slot_mapping, int num_tokens, int x, int num_seqs, int num_heads,

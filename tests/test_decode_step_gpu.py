@@ -57,24 +57,25 @@ def _both(case, cache, split, slopes=None):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("heads,kv_heads,dim,block", [(32, 32, 128, 16), (64, 8, 128, 32), (12, 12, 64, 16), (6, 3, 96, 8), (4, 4, 256, 32)])
 def test_one_launch_is_the_two(heads, kv_heads, dim, block, dtype, cache, split):
-    for ctx in ([1], [15, 16, 17, 1040], [513] * 3 + [100] * 5):
+    for ctx in ([1], [15, 16, 17, 1040], [513] * 3 + [100] * 5, [40 + 31 * i for i in range(25)]):
         _both(_case(heads, kv_heads, dim, ctx, dtype, cache, block), cache, split)
     slopes = torch.rand(heads, device=DEV)
     _both(_case(heads, kv_heads, dim, [70, 530], dtype, cache, block), cache, split, slopes)
 
 
 @pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("seqs", [14, 17, 98])               # all tokens written by everyone; those that are looked up
 @pytest.mark.parametrize("heads,kv_heads,dim", [(8, 8, 128), (16, 2, 128), (6, 3, 80)])
-def test_sequences_that_read_each_others_tokens(heads, kv_heads, dim, split):
+def test_sequences_that_read_each_others_tokens(heads, kv_heads, dim, seqs, split):
     """Every sequence's table also holds the others' newest blocks, one token has no slot, and one goes into the middle of a block that
     all of them read."""
-    ctx = [700, 650, 600, 530, 33, 48, 16, 90, 700, 700, 20, 5, 64, 129]
+    ctx = ([700, 650, 600, 530, 33, 48, 16, 90, 700, 700, 20, 5, 64, 129] * 7)[:seqs]
     case = _case(heads, kv_heads, dim, ctx, torch.bfloat16, "auto", 16)
     q, k, v, caches, slots, tables, lens = case
     newest = (slots // 16).to(torch.int32)
     for i, c in enumerate(ctx):
-        held = -(-c // 16)
-        tables[i, :min(held - 1, len(ctx))] = newest[:min(held - 1, len(ctx))]
+        held = min(-(-c // 16) - 1, len(ctx))
+        tables[i, :held] = newest.roll(i)[:held]
     slots[3] = -1
     slots[5] = int(newest[0]) * 16 + 2
     _both(case, "auto", split)
@@ -92,8 +93,11 @@ def test_what_is_left_to_the_two_calls():
         return done
     small = lambda: _case(4, 4, 64, [20, 40], torch.float16, "auto", 16)      # noqa: E731
     assert call(small())
-    assert not call(_case(4, 4, 64, [20] * 17, torch.float16, "auto", 16))                 # tokens
-    assert not call(_case(40, 40, 128, [20] * 9, torch.float16, "auto", 16))               # tokens x sequences x elements
+    assert call(_case(4, 4, 64, [20] * 128, torch.float16, "auto", 16))
+    assert not call(_case(4, 4, 64, [20] * 129, torch.float16, "auto", 16))                # tokens
+    assert not call(_case(32, 32, 64, [20] * 33, torch.float16, "auto", 16))               # sequences x heads
+    q, k, v, caches, slots, tables, lens = _case(4, 4, 64, [20] * 40, torch.float16, "auto", 16)
+    assert not call((q[:39], k, v, caches, slots, tables[:39], lens[:39]))                 # more tokens than sequences, and too many for all
     case = small()
     assert not call(case, slots=case[4].int())
     assert not call(case, k=case[1].transpose(0, 1).contiguous().transpose(0, 1))

@@ -126,34 +126,65 @@ template <typename act_t, bool FP8> struct PackedPath { static constexpr bool va
 template <> struct PackedPath<f16_t, true> { static constexpr bool value = true; };
 
 // A decode step's new tokens on their way into the cache, beside the attention over it.  Every workgroup writes the new keys and values of
-// its kv head, of ALL the call's tokens, before it reads the cache: what it then reads is what a launch in front of it would have left,
-// whatever blocks the sequences share, and no workgroup waits for another (they write the same bytes to the same places).  That is
-// (tokens x sequences) times the write, so it is for few tokens: kPaWriteUpTo, and kPaWriteElements of keys in all.
-// Measured, a layer's decode step in a stream of calls, two launches / one (us): 32 heads of 128, 2 x 700 tokens 18.3 / 15.8, 1 x 4000 (split)
-// 25.9 / 19.7; 64 on 8, fp8, 2 x 700 14.7 / 12.0; 12 of 64, 16 x 300 14.5 / 11.8; but 32 of 128, 16 x 700 44.3 / 47.0.
+// its kv head before it reads the cache: those of its own sequence's token, and of every other token that goes into a block of the part of
+// the context that it reads.  What it then reads is what a launch in front of it would have left, whatever blocks the sequences share, and
+// no workgroup waits for another (they write the same bytes to the same places).  With few tokens it writes all of them; else it looks the
+// tokens' blocks up among its own, in a bit map of their numbers (a token that only looks like one of them is written once too often).
 struct PaWrite {
   const void *key, *value;
   void *k_cache, *v_cache;
   const int64_t* slots;
   int64_t key_stride, value_stride;                // elements
   int tokens;                                      // 0: the cache is as it should be
+  int all;
 };
-constexpr int kPaWriteUpTo = 16;
-constexpr int64_t kPaWriteElements = 8 * 8 * 40 * 128;
+// Tokens, and sequences x kv heads: beyond, what every workgroup looks up costs more than the launch (us in a stream of calls, two launches /
+// one: 32 heads of 128, 2 x 700 tokens 16.8 / 14.2, 16 x 700 45.4 / 43.4, 32 x 300 41.4 / 39.5, 64 x 100 33.1 / 33.4, 251 x 857 626 / 698;
+// 32 on 8, 32 x 700 25.0 / 22.1, 60 x 326 20.9 / 19.1, 250 x 1000 206 / 216; 64 on 8, fp8, 61 x 2011 58.6 / 56.5; 12 of 64, 61 x 700
+// 35.4 / 34.4, 200 x 300 into fp8 34.3 / 41.1; 16 on 2, 100 x 500 17.5 / 15.0, 250 x 3000, fp8, 85.0 / 85.8).
+constexpr int kPaWriteUpTo = 128, kPaWriteHeadsUpTo = 1024;
+constexpr int kPaWriteAllUpTo = 16;
+constexpr int64_t kPaWriteAllElements = 8 * 8 * 40 * 128;      // tokens x sequences x elements of a token's keys
+constexpr int kPaSeenBits = 8192;
 // The caches' pointers of a kernel that writes them are not __restrict__: its loads stay behind the stores.
 template <bool WRITE> struct PaCachePtr { using type = const void* __restrict__; };
 template <> struct PaCachePtr<true> { using type = const void*; };
 
+// first .. last: the entries of the block table that the workgroup reads
 template <typename act_t, bool FP8, int HEAD, int BS, int THREADS>
-__device__ __forceinline__ void pa_write(const PaWrite& w, int kv_head, int64_t kv_block_stride, int64_t kv_head_stride) {
+__device__ __forceinline__ void pa_write(const PaWrite& w, int seq, int kv_head, const int32_t* table, int first, int last,
+                                         int64_t kv_block_stride, int64_t kv_head_stride) {
   using T = CacheTraits<act_t, FP8>;
   using S = typename T::S;
   constexpr int ES = T::ES, CS = T::CS, X = T::X, NCH = HEAD / X, DW = X * ES / 16;
+  __shared__ uint32_t seen[kPaSeenBits / 32];
+  __shared__ int list[kPaWriteUpTo], listed;
   const int tid = threadIdx.x;
+  int count = w.tokens;
+  if (!w.all) {                                    // uniform over the launch
+    for (int i = tid; i < kPaSeenBits / 32; i += THREADS) seen[i] = 0;
+    if (tid == 0) {
+      list[0] = seq;
+      listed = seq < w.tokens ? 1 : 0;
+    }
+    __syncthreads();
+    for (int b = first + tid; b < last; b += THREADS) {
+      const uint32_t bit = (uint32_t)table[b] % kPaSeenBits;
+      atomicOr(&seen[bit / 32], 1u << (bit % 32));
+    }
+    __syncthreads();
+    for (int t = tid; t < w.tokens; t += THREADS) {
+      const int64_t slot = w.slots[t];
+      const uint32_t bit = (uint32_t)(slot / BS) % kPaSeenBits;
+      if (t != seq && slot >= 0 && (seen[bit / 32] >> (bit % 32) & 1)) list[atomicAdd(&listed, 1)] = t;
+    }
+    __syncthreads();
+    count = listed;
+  }
   auto tile = [&](int64_t slot) { return (slot / BS * kv_block_stride + (int64_t)kv_head * kv_head_stride) * CS; };
   // keys: 16 bytes of the cache a thread
-  for (int p = tid; p < w.tokens * NCH; p += THREADS) {
-    const int t = p / NCH, c = p - t * NCH;
+  for (int p = tid; p < count * NCH; p += THREADS) {
+    const int n = p / NCH, c = p - n * NCH, t = w.all ? n : list[n];
     const int64_t slot = w.slots[t];
     const uint4* src = reinterpret_cast<const uint4*>(static_cast<const S*>(w.key) + t * w.key_stride + (int64_t)kv_head * HEAD + c * X);
     union {
@@ -175,8 +206,8 @@ __device__ __forceinline__ void pa_write(const PaWrite& w, int kv_head, int64_t 
     if (slot >= 0) *reinterpret_cast<uint4*>(static_cast<char*>(w.k_cache) + tile(slot) + (c * BS + (int)(slot % BS)) * 16) = to.q;
   }
   // values: an element a thread
-  for (int e = tid; e < w.tokens * HEAD; e += THREADS) {
-    const int t = e / HEAD, d = e - t * HEAD;
+  for (int e = tid; e < count * HEAD; e += THREADS) {
+    const int n = e / HEAD, d = e - n * HEAD, t = w.all ? n : list[n];
     const int64_t slot = w.slots[t];
     const S v = static_cast<const S*>(w.value)[t * w.value_stride + (int64_t)kv_head * HEAD + d];
     if (slot < 0) continue;
@@ -266,13 +297,17 @@ paged_attention_kernel(void* __restrict__ out_,            // v1: [S,H,HEAD]; v2
   const int kv_head = hx / wg_per_kv;
   const int head0 = kv_head * groups_per_kv + (hx - kv_head * wg_per_kv) * QG;
 
-  if constexpr (WRITE) pa_write<act_t, FP8, HEAD, BS, NW * 64>(w, kv_head, kv_block_stride, kv_head_stride);
-
   const int ctx = context_lens[seq];
   const int tok_begin = partitioned ? part_idx * kPartitionSize : 0;
-  if (partitioned && tok_begin >= ctx) return;              // uniform: whole workgroup leaves
   const int tok_end = partitioned ? min(tok_begin + kPartitionSize, ctx) : ctx;
   const int num_ctx_blocks = (ctx + BS - 1) / BS;
+  const int32_t* block_table = block_tables + (int64_t)seq * max_num_blocks_per_seq;
+  if constexpr (WRITE) {
+    if (tok_begin < ctx || part_idx == 0)                   // uniform; a sequence's first partition writes in any case
+      pa_write<act_t, FP8, HEAD, BS, NW * 64>(w, seq, kv_head, block_table, tok_begin / BS, (tok_end + BS - 1) / BS, kv_block_stride,
+                                              kv_head_stride);
+  }
+  if (partitioned && tok_begin >= ctx) return;              // uniform: whole workgroup leaves
 
   // ---- query -> LDS as fp32, pre-multiplied by nothing (scale is applied to the dot)
   const uint32_t* q_p = reinterpret_cast<const uint32_t*>(smem);           // packed path: [QG][HEAD/2] pairs
@@ -290,7 +325,6 @@ paged_attention_kernel(void* __restrict__ out_,            // v1: [S,H,HEAD]; v2
 
   const char* k_cache = reinterpret_cast<const char*>(k_cache_);
   const char* v_cache = reinterpret_cast<const char*>(v_cache_);
-  const int32_t* block_table = block_tables + (int64_t)seq * max_num_blocks_per_seq;
 
   float slope[QG];
 #pragma unroll

@@ -131,15 +131,17 @@ paged_attention_mfma_kernel(void* __restrict__ out_, float* __restrict__ exp_sum
   const int kv_head = hx / wg_per_kv;
   const int head0 = kv_head * groups_per_kv + (hx - kv_head * wg_per_kv) * qg;
 
-  if constexpr (WRITE) {
-    pa_write<act_t, FP8, HEAD, BS, NW * 64>(w, kv_head, kv_block_stride, kv_head_stride);
-    __syncthreads();
-  }
-
   const int ctx = context_lens[seq];
   const int tok_begin = partitioned ? part_idx * kPartitionSize : 0;
-  if (partitioned && tok_begin >= ctx) return;
   const int tok_end = partitioned ? min(tok_begin + kPartitionSize, ctx) : ctx;
+  const int32_t* block_table = block_tables + (int64_t)seq * max_num_blocks_per_seq;
+  if constexpr (WRITE) {
+    if (tok_begin < ctx || part_idx == 0)
+      pa_write<act_t, FP8, HEAD, BS, NW * 64>(w, seq, kv_head, block_table, tok_begin / BS, (tok_end + BS - 1) / BS, kv_block_stride,
+                                              kv_head_stride);
+    __syncthreads();
+  }
+  if (partitioned && tok_begin >= ctx) return;
   const int num_ctx_blocks = (ctx + BS - 1) / BS;
 
   // ---- Q^T fragments: lane (head r, dims 32 ks + 8 kq ..+7); zero for the unused head columns
@@ -183,7 +185,6 @@ paged_attention_mfma_kernel(void* __restrict__ out_, float* __restrict__ exp_sum
 
   const char* k_cache = reinterpret_cast<const char*>(k_cache_);
   const char* v_cache = reinterpret_cast<const char*>(v_cache_);
-  const int32_t* block_table = block_tables + (int64_t)seq * max_num_blocks_per_seq;
   const int64_t head_off = (int64_t)kv_head * kv_head_stride * CS;
   const int64_t block_bytes = kv_block_stride * CS;
 

@@ -19,7 +19,7 @@ from ... import _C
 from ..input_metadata import InputMetadata
 
 _PARTITION_SIZE = 512          # must match the partition size of sw_paged_attention_v2
-_WRITES_BESIDE_ATTENTION = 16, 327680      # what sw_paged_attention_and_cache takes: tokens and sequences, key elements over both
+_WRITES_BESIDE_ATTENTION = 128, 1024       # of sw_paged_attention_and_cache: tokens, sequences x kv heads
 _SUPPORTED_HEAD_SIZES = [64, 80, 96, 112, 128, 256]
 
 
@@ -132,8 +132,8 @@ class PagedAttentionImpl:
             exp_sums = torch.empty((num_seqs, num_heads, parts), dtype=torch.float32, device=output.device)
             max_logits = torch.empty_like(exp_sums)
         if key is not None:
-            few, elements = _WRITES_BESIDE_ATTENTION
-            if num_seqs <= few and key.shape[0] <= few and num_seqs * key.numel() <= elements:
+            tokens, heads = _WRITES_BESIDE_ATTENTION
+            if key.shape[0] <= tokens and num_seqs * num_kv_heads <= heads:
                 slots = input_metadata.slot_mapping
                 if _C.ops.paged_attention_and_cache(output, exp_sums, max_logits, tmp_output, query, key, value, key_cache,
                                                     value_cache, slots if slots.dim() == 1 else slots.flatten(), scale,
