@@ -51,7 +51,9 @@ const char* sw_last_error(void);
  *    grew from 2304 to 2560 bytes, which moves the status word at its end.
  * 6: sw_kv_push_mapped added.
  * 7: sw_context_attention_split, sw_context_attention_split_parts, sw_context_attention_split_workspace_bytes
- *    added. */
+ *    added.
+ * 8: sw_prefill_attention_and_cache added.
+ * 9: sw_paged_attention_and_cache added. */
 #define SW_ABI_VERSION 9
 int sw_abi_version(void);
 

@@ -5,7 +5,8 @@
 // checks, data pointers and the device guard the rest, so that a decode step of two conversations waited for the host (21 us
 // a layer, 12.6 on the GPU).  Measured, us a pass of calls, before / now: cache write + attention of a decode step 20.9 /
 // 16.6, of a prompt of 40 tokens 21.0 / 15.7; the delta rule with its convolution and norm 34.9 / 23.4; experts 27.4 / 21.9;
-// gated linear attention 28.7 / 21.3; the mixers' attention 15.3 / 8.3.
+// gated linear attention 28.7 / 21.3; the mixers' attention 15.3 / 8.3.  (Cache write and attention are one call where their launches
+// are: prefill_attention_and_cache, paged_attention_and_cache.)
 //
 // A function takes a call only if every argument is of the plain kind (exact tensors on the current device, Python numbers)
 // and passes every check; otherwise it returns None before anything happened and the Python function goes on, which knows

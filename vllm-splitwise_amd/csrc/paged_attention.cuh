@@ -139,9 +139,9 @@ struct PaWrite {
   int all;
 };
 // Tokens, and sequences x kv heads: beyond, what every workgroup looks up costs more than the launch (us in a stream of calls, two launches /
-// one: 32 heads of 128, 2 x 700 tokens 16.8 / 14.2, 16 x 700 45.4 / 43.4, 32 x 300 41.4 / 39.5, 64 x 100 33.1 / 33.4, 251 x 857 626 / 698;
-// 32 on 8, 32 x 700 25.0 / 22.1, 60 x 326 20.9 / 19.1, 250 x 1000 206 / 216; 64 on 8, fp8, 61 x 2011 58.6 / 56.5; 12 of 64, 61 x 700
-// 35.4 / 34.4, 200 x 300 into fp8 34.3 / 41.1; 16 on 2, 100 x 500 17.5 / 15.0, 250 x 3000, fp8, 85.0 / 85.8).
+// one: 32 heads of 128, 16 x 700 45.4 / 42.6, 32 x 300 41.4 / 39.1, 64 x 100 33.1 / 32.9, 251 x 857 626 / 698; 32 on 8, 32 x 700 25.0 / 21.7,
+// 60 x 326 20.9 / 18.7, 250 x 1000 206 / 216; 64 on 8, fp8, 61 x 2011 56.8 / 54.4; 12 of 64, 61 x 700 35.4 / 34.0, 200 x 300 into fp8
+// 34.3 / 41.1; 16 on 2, 100 x 500 17.5 / 14.4, 250 x 3000, fp8, 85.0 / 85.8).
 constexpr int kPaWriteUpTo = 128, kPaWriteHeadsUpTo = 1024;
 constexpr int kPaWriteAllUpTo = 16;
 constexpr int64_t kPaWriteAllElements = 8 * 8 * 40 * 128;      // tokens x sequences x elements of a token's keys
@@ -162,6 +162,10 @@ __device__ __forceinline__ void pa_write(const PaWrite& w, int seq, int kv_head,
   const int tid = threadIdx.x;
   int count = w.tokens;
   if (!w.all) {                                    // uniform over the launch
+    static_assert(kPaWriteUpTo <= THREADS, "a thread per token");
+    // a thread's token and its first table entry are asked for together, in front of the barriers
+    const int64_t slot = tid < w.tokens ? w.slots[tid] : -1;
+    const int entry = first + tid < last ? table[first + tid] : 0;
     for (int i = tid; i < kPaSeenBits / 32; i += THREADS) seen[i] = 0;
     if (tid == 0) {
       list[0] = seq;
@@ -169,14 +173,13 @@ __device__ __forceinline__ void pa_write(const PaWrite& w, int seq, int kv_head,
     }
     __syncthreads();
     for (int b = first + tid; b < last; b += THREADS) {
-      const uint32_t bit = (uint32_t)table[b] % kPaSeenBits;
+      const uint32_t bit = (uint32_t)(b == first + tid ? entry : table[b]) % kPaSeenBits;
       atomicOr(&seen[bit / 32], 1u << (bit % 32));
     }
     __syncthreads();
-    for (int t = tid; t < w.tokens; t += THREADS) {
-      const int64_t slot = w.slots[t];
+    if (slot >= 0 && tid != seq) {
       const uint32_t bit = (uint32_t)(slot / BS) % kPaSeenBits;
-      if (t != seq && slot >= 0 && (seen[bit / 32] >> (bit % 32) & 1)) list[atomicAdd(&listed, 1)] = t;
+      if (seen[bit / 32] >> (bit % 32) & 1) list[atomicAdd(&listed, 1)] = tid;
     }
     __syncthreads();
     count = listed;

@@ -3,7 +3,8 @@
 Order of operations restated from the reference's backends
 (vllm/model_executor/layers/attention/backends/xformers.py:70-191, flash_attn.py:77-125):
   1. reshape_and_cache of the step's keys / values (skipped during the profiling run,
-     where no cache exists yet);
+     where no cache exists yet); in the launch of step 3 where that takes it: plain prompt runs, and decode runs of up
+     to 128 sequences (``prefill_attention_and_cache``, ``paged_attention_and_cache``);
   2. prompt run on a prompt-pool worker: for every hand-off slot and block run in
      ``blocks_to_nw``, push this layer's K and V blocks to the paired token worker
      (ordered after step 1 on the same stream, before the layer's attention finishes);
