@@ -106,6 +106,7 @@ def test_what_is_left_to_the_two_calls():
     assert not call(_case(4, 4, 64, [20, 40], torch.float16, "auto", 4))                   # blocks that the attention refuses
 
 
+@torch.inference_mode()                                      # (as the workers capture theirs)
 def test_layer_in_a_graph():
     """The layer's decode step as it is called, captured and replayed on other inputs, for a split and an unsplit context."""
     from splitwise_amd.model_executor.input_metadata import InputMetadata

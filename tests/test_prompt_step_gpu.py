@@ -79,6 +79,7 @@ def test_what_is_left_to_the_two_calls():
     assert not caches[0].any() and not caches[1].any()
 
 
+@torch.inference_mode()                                      # (as the workers capture theirs)
 def test_layer_in_a_graph():
     """The layer's prompt step as it is called, captured and replayed on other inputs."""
     from splitwise_amd.model_executor.input_metadata import InputMetadata
