@@ -1,0 +1,51 @@
+"""Which launches a step of the Llama path's attention module asks for: the operators are stood in for by recorders."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from splitwise_amd import _C
+from splitwise_amd.model_executor.input_metadata import InputMetadata
+from splitwise_amd.model_executor.layers.attention import Attention
+
+
+class _Calls(list):
+    def __init__(self, monkeypatch):
+        super().__init__()
+        def entry(name, answer=None):
+            return lambda *args: (self.append(name), answer)[1]
+        ops = {n: entry(n) for n in ("paged_attention_v1", "paged_attention_v2", "prefill_attention", "rotary_embedding_and_cache")}
+        ops |= {n: entry(n, True) for n in ("prefill_attention_and_cache", "paged_attention_and_cache")}
+        monkeypatch.setattr(_C, "ops", SimpleNamespace(**ops))
+        monkeypatch.setattr(_C, "cache_ops", SimpleNamespace(reshape_and_cache=entry("reshape_and_cache")))
+
+
+def _meta(*shape, dtype=torch.bfloat16):
+    return torch.empty(shape, dtype=dtype, device="meta")
+
+
+def _step(calls, heads, kv_heads, dim, rows, md, **kw):
+    calls.clear()
+    Attention(heads, dim, 1.0, kv_heads)(_meta(rows, heads * dim), _meta(rows, kv_heads * dim), _meta(rows, kv_heads * dim),
+                                         _meta(9, kv_heads, dim // 8, 16, 8), _meta(9, kv_heads, dim, 16), md, **kw)
+    return list(calls)
+
+
+def _prompt(lens, cache):
+    return InputMetadata(is_prompt=True, slot_mapping=_meta(sum(lens)), prompt_lens=_meta(len(lens)), max_seq_len=max(lens),
+                         start_loc=_meta(len(lens)), max_context_len=None, context_lens=None, block_tables=None, use_cuda_graph=False,
+                         kv_cache_dtype=cache)
+
+
+ONE, TWO = ["prefill_attention_and_cache"], ["reshape_and_cache", "prefill_attention"]
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,lens,auto,fp8", [
+    (32, 32, 128, [17], ONE, ONE), (32, 32, 128, [773] * 3, ONE, TWO), (32, 32, 128, [1000], ONE, ONE), (32, 32, 128, [2000] * 2, ONE, TWO),
+    (32, 32, 128, [2049] * 8, TWO, TWO), (32, 32, 128, [773] * 8, TWO, TWO), (32, 32, 128, [120] * 32, ONE, TWO), (32, 32, 128, [4100], TWO, TWO),
+    (32, 32, 128, [33] * 64, TWO, TWO), (32, 32, 128, [33] * 8, ONE, TWO), (64, 8, 128, [300] * 2, ONE, ONE), (64, 8, 128, [2049] * 8, TWO, TWO),
+    (16, 16, 256, [120] * 32, ONE, TWO), (12, 12, 64, [700] * 4, ONE, ONE), (16, 2, 128, [33] * 64, ONE, ONE), (16, 2, 128, [4095], ONE, ONE)])
+def test_prompt_steps(heads, kv_heads, dim, lens, auto, fp8, monkeypatch):
+    calls = _Calls(monkeypatch)
+    assert _step(calls, heads, kv_heads, dim, sum(lens), _prompt(lens, "auto")) == auto
+    assert _step(calls, heads, kv_heads, dim, sum(lens), _prompt(lens, "fp8_e5m2")) == fp8

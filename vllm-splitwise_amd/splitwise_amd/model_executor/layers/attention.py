@@ -97,6 +97,25 @@ class PagedAttentionImpl:
         return max_context_len <= 2 * _PARTITION_SIZE
 
     @staticmethod
+    def writes_beside_prompt(rows: int, prompts: int, longest: int, num_heads: int, num_kv_heads: int, head_size: int,
+                             kv_cache_dtype: str) -> bool:
+        """Whether a prompt run's cache write goes into the attention's launch.  The write's workgroups have the attention's LDS, so
+        that two of them at most run on a compute unit where the write alone has eight: it is ahead while they fill places that the
+        attention leaves empty, and behind once they come after it.  An fp8 cache, for which they convert, needs the places more.
+
+        Over 936 steps into a 16-bit cache (1 to 64 prompts of 33 to 8000 tokens, up to 17000 in all; 8 to 64 heads of 64 to 256) one
+        launch takes 0.83 of the two's time where this says so (648 of them, at most 1.055) and 1.01 elsewhere; over 792 into an fp8
+        cache 0.79 (407, at most 1.03) and 1.04.  Two launches / one, us, 32 heads of 128: 3 x 773 tokens 54.6 / 47.1, 2 x 2000 124.4 /
+        118.3, 1 x 4100 196.3 / 199.9, 8 x 2049 506 / 544; fp8: 1 x 400 19.0 / 13.8, 1 x 1000 34.2 / 30.9, 32 x 120 64.4 / 75.0, 8 x 773
+        133.9 / 149.3, 8 x 2049 518 / 588; 8 heads of 128, 64 x 33 14.4 / 15.7."""
+        written = rows * num_kv_heads * head_size
+        # query rows that a key of an average prompt is read for
+        readers = rows * num_heads // (max(prompts, 1) * num_kv_heads)
+        if kv_cache_dtype == "auto":
+            return rows * num_heads * head_size <= 20 << 20 and longest < 4096 and (written <= 2 << 20 or readers >= 64)
+        return written <= 8 << 20 and longest < 4096 and (written <= 1 << 20 or readers >= 300)
+
+    @staticmethod
     def forward_prefix(query, key, value, key_cache, value_cache, input_metadata: InputMetadata,
                        alibi_slopes=None):
         """Prompt attention of new tokens over a prefix that is already in the cache
@@ -209,8 +228,11 @@ class Attention(nn.Module):
         tables = input_metadata.block_tables
         writes_cache = key_cache is not None and value_cache is not None and not fused_cache_write
         if (writes_cache and input_metadata.is_prompt and (tables is None or tables.numel() == 0)
-                and not (input_metadata.blocks_to_nw and self.kvcache_comm_manager is not None)):
-            # a plain prompt run: both in one launch, where that has a form for the call
+                and not (input_metadata.blocks_to_nw and self.kvcache_comm_manager is not None)
+                and PagedAttentionImpl.writes_beside_prompt(query.shape[0], input_metadata.prompt_lens.numel(),
+                                                            input_metadata.max_seq_len, self.num_heads, self.num_kv_heads,
+                                                            self.head_size, input_metadata.kv_cache_dtype)):
+            # a plain prompt run: both in one launch, where that is the faster and has a form for the call
             output = torch.empty_like(query)
             slots = input_metadata.slot_mapping
             if _C.ops.prefill_attention_and_cache(output, query, key, value, input_metadata.start_loc,
