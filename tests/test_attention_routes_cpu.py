@@ -49,3 +49,24 @@ def test_prompt_steps(heads, kv_heads, dim, lens, auto, fp8, monkeypatch):
     calls = _Calls(monkeypatch)
     assert _step(calls, heads, kv_heads, dim, sum(lens), _prompt(lens, "auto")) == auto
     assert _step(calls, heads, kv_heads, dim, sum(lens), _prompt(lens, "fp8_e5m2")) == fp8
+
+
+def _decode(seqs, ctx, cache):
+    return InputMetadata(is_prompt=False, slot_mapping=_meta(seqs), prompt_lens=None, max_seq_len=None, start_loc=None, max_context_len=ctx,
+                         context_lens=_meta(seqs), block_tables=_meta(seqs, 9), use_cuda_graph=False, kv_cache_dtype=cache)
+
+
+BESIDE, SPLIT, UNSPLIT = ["paged_attention_and_cache"], ["reshape_and_cache", "paged_attention_v2"], ["reshape_and_cache", "paged_attention_v1"]
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,seqs,ctx,auto,fp8", [
+    (32, 32, 128, 2, 700, BESIDE, BESIDE), (32, 32, 128, 32, 700, BESIDE, UNSPLIT), (32, 32, 128, 16, 700, BESIDE, BESIDE),
+    (32, 32, 128, 33, 700, UNSPLIT, UNSPLIT), (32, 32, 128, 2, 4096, BESIDE, BESIDE), (32, 32, 128, 3, 4096, SPLIT, SPLIT),
+    (32, 32, 128, 8, 15000, SPLIT, SPLIT), (64, 8, 128, 64, 2011, BESIDE, BESIDE), (64, 8, 128, 65, 2011, UNSPLIT, UNSPLIT),
+    (64, 8, 128, 12, 2875, SPLIT, SPLIT), (64, 8, 128, 2, 2875, BESIDE, BESIDE), (16, 2, 128, 24, 3000, BESIDE, BESIDE),
+    (16, 2, 128, 24, 28000, SPLIT, SPLIT), (32, 32, 128, 1, 16384, BESIDE, BESIDE), (32, 32, 128, 1, 16385, SPLIT, SPLIT), (12, 12, 64, 128, 300, UNSPLIT, UNSPLIT), (4, 4, 64, 128, 300, BESIDE, BESIDE),
+    (4, 4, 64, 129, 300, UNSPLIT, UNSPLIT)])
+def test_decode_steps(heads, kv_heads, dim, seqs, ctx, auto, fp8, monkeypatch):
+    calls = _Calls(monkeypatch)
+    assert _step(calls, heads, kv_heads, dim, seqs, _decode(seqs, ctx, "auto")) == auto
+    assert _step(calls, heads, kv_heads, dim, seqs, _decode(seqs, ctx, "fp8_e5m2")) == fp8
