@@ -81,6 +81,12 @@ def test_sequences_that_read_each_others_tokens(heads, kv_heads, dim, seqs, spli
     _both(case, "auto", split)
 
 
+@pytest.mark.parametrize("split", [False, True])
+def test_lds_just_under_64_kb(split):
+    """Eleven query heads a kv head, eight waves: 64192 bytes of LDS, and tokens that are looked up (in some of them)."""
+    _both(_case(22, 2, 128, [40 + 31 * i for i in range(25)], torch.bfloat16, "auto", 16), "auto", split)
+
+
 def test_what_is_left_to_the_two_calls():
     from splitwise_amd import _C
     def call(case, cache="auto", **other):

@@ -146,19 +146,21 @@ constexpr int kPaWriteUpTo = 128, kPaWriteHeadsUpTo = 1024;
 constexpr int kPaWriteAllUpTo = 16;
 constexpr int64_t kPaWriteAllElements = 8 * 8 * 40 * 128;      // tokens x sequences x elements of a token's keys
 constexpr int kPaSeenBits = 8192;
+struct PaSeen {                                    // LDS of the lookup
+  uint32_t bits[kPaSeenBits / 32];
+  int list[kPaWriteUpTo], listed;
+};
 // The caches' pointers of a kernel that writes them are not __restrict__: its loads stay behind the stores.
 template <bool WRITE> struct PaCachePtr { using type = const void* __restrict__; };
 template <> struct PaCachePtr<true> { using type = const void*; };
 
-// first .. last: the entries of the block table that the workgroup reads
+// first .. last: the entries of the block table that the workgroup reads; s: free until the workgroup's next barrier
 template <typename act_t, bool FP8, int HEAD, int BS, int THREADS>
-__device__ __forceinline__ void pa_write(const PaWrite& w, int seq, int kv_head, const int32_t* table, int first, int last,
+__device__ __forceinline__ void pa_write(const PaWrite& w, PaSeen& s, int seq, int kv_head, const int32_t* table, int first, int last,
                                          int64_t kv_block_stride, int64_t kv_head_stride) {
   using T = CacheTraits<act_t, FP8>;
   using S = typename T::S;
   constexpr int ES = T::ES, CS = T::CS, X = T::X, NCH = HEAD / X, DW = X * ES / 16;
-  __shared__ uint32_t seen[kPaSeenBits / 32];
-  __shared__ int list[kPaWriteUpTo], listed;
   const int tid = threadIdx.x;
   int count = w.tokens;
   if (!w.all) {                                    // uniform over the launch
@@ -166,28 +168,28 @@ __device__ __forceinline__ void pa_write(const PaWrite& w, int seq, int kv_head,
     // a thread's token and its first table entry are asked for together, in front of the barriers
     const int64_t slot = tid < w.tokens ? w.slots[tid] : -1;
     const int entry = first + tid < last ? table[first + tid] : 0;
-    for (int i = tid; i < kPaSeenBits / 32; i += THREADS) seen[i] = 0;
+    for (int i = tid; i < kPaSeenBits / 32; i += THREADS) s.bits[i] = 0;
     if (tid == 0) {
-      list[0] = seq;
-      listed = seq < w.tokens ? 1 : 0;
+      s.list[0] = seq;
+      s.listed = seq < w.tokens ? 1 : 0;
     }
     __syncthreads();
     for (int b = first + tid; b < last; b += THREADS) {
       const uint32_t bit = (uint32_t)(b == first + tid ? entry : table[b]) % kPaSeenBits;
-      atomicOr(&seen[bit / 32], 1u << (bit % 32));
+      atomicOr(&s.bits[bit / 32], 1u << (bit % 32));
     }
     __syncthreads();
     if (slot >= 0 && tid != seq) {
       const uint32_t bit = (uint32_t)(slot / BS) % kPaSeenBits;
-      if (seen[bit / 32] >> (bit % 32) & 1) list[atomicAdd(&listed, 1)] = tid;
+      if (s.bits[bit / 32] >> (bit % 32) & 1) s.list[atomicAdd(&s.listed, 1)] = tid;
     }
     __syncthreads();
-    count = listed;
+    count = s.listed;
   }
   auto tile = [&](int64_t slot) { return (slot / BS * kv_block_stride + (int64_t)kv_head * kv_head_stride) * CS; };
   // keys: 16 bytes of the cache a thread
   for (int p = tid; p < count * NCH; p += THREADS) {
-    const int n = p / NCH, c = p - n * NCH, t = w.all ? n : list[n];
+    const int n = p / NCH, c = p - n * NCH, t = w.all ? n : s.list[n];
     const int64_t slot = w.slots[t];
     const uint4* src = reinterpret_cast<const uint4*>(static_cast<const S*>(w.key) + t * w.key_stride + (int64_t)kv_head * HEAD + c * X);
     union {
@@ -210,7 +212,7 @@ __device__ __forceinline__ void pa_write(const PaWrite& w, int seq, int kv_head,
   }
   // values: an element a thread
   for (int e = tid; e < count * HEAD; e += THREADS) {
-    const int n = e / HEAD, d = e - n * HEAD, t = w.all ? n : list[n];
+    const int n = e / HEAD, d = e - n * HEAD, t = w.all ? n : s.list[n];
     const int64_t slot = w.slots[t];
     const S v = static_cast<const S*>(w.value)[t * w.value_stride + (int64_t)kv_head * HEAD + d];
     if (slot < 0) continue;
@@ -306,8 +308,9 @@ paged_attention_kernel(void* __restrict__ out_,            // v1: [S,H,HEAD]; v2
   const int num_ctx_blocks = (ctx + BS - 1) / BS;
   const int32_t* block_table = block_tables + (int64_t)seq * max_num_blocks_per_seq;
   if constexpr (WRITE) {
+    __shared__ PaSeen seen;                                 // (beside the query, which goes to LDS behind it without a barrier)
     if (tok_begin < ctx || part_idx == 0)                   // uniform; a sequence's first partition writes in any case
-      pa_write<act_t, FP8, HEAD, BS, NW * 64>(w, seq, kv_head, block_table, tok_begin / BS, (tok_end + BS - 1) / BS, kv_block_stride,
+      pa_write<act_t, FP8, HEAD, BS, NW * 64>(w, seen, seq, kv_head, block_table, tok_begin / BS, (tok_end + BS - 1) / BS, kv_block_stride,
                                               kv_head_stride);
   }
   if (partitioned && tok_begin >= ctx) return;              // uniform: whole workgroup leaves

@@ -136,9 +136,11 @@ paged_attention_mfma_kernel(void* __restrict__ out_, float* __restrict__ exp_sum
   const int tok_end = partitioned ? min(tok_begin + kPartitionSize, ctx) : ctx;
   const int32_t* block_table = block_tables + (int64_t)seq * max_num_blocks_per_seq;
   if constexpr (WRITE) {
+    // in the strips' LDS, which nobody uses before the barrier: the launch's check of 64 KB counts all there is
+    static_assert(sizeof(PaSeen) <= NW * kPaMfmaHeads * kPaMfmaPRow * 2, "the lookup must fit the strips");
     if (tok_begin < ctx || part_idx == 0)
-      pa_write<act_t, FP8, HEAD, BS, NW * 64>(w, seq, kv_head, block_table, tok_begin / BS, (tok_end + BS - 1) / BS, kv_block_stride,
-                                              kv_head_stride);
+      pa_write<act_t, FP8, HEAD, BS, NW * 64>(w, *reinterpret_cast<PaSeen*>(smem), seq, kv_head, block_table, tok_begin / BS,
+                                              (tok_end + BS - 1) / BS, kv_block_stride, kv_head_stride);
     __syncthreads();
   }
   if (partitioned && tok_begin >= ctx) return;
