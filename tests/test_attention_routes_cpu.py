@@ -70,3 +70,12 @@ def test_decode_steps(heads, kv_heads, dim, seqs, ctx, auto, fp8, monkeypatch):
     calls = _Calls(monkeypatch)
     assert _step(calls, heads, kv_heads, dim, seqs, _decode(seqs, ctx, "auto")) == auto
     assert _step(calls, heads, kv_heads, dim, seqs, _decode(seqs, ctx, "fp8_e5m2")) == fp8
+
+
+def test_decode_steps_that_rotate(monkeypatch):
+    """A model that hands its rotary module over (the Llama models): rotation and cache write in one launch, the attention in the next."""
+    calls = _Calls(monkeypatch)
+    rotary = SimpleNamespace(fusable_with_cache_write=lambda dtype: True, cos_sin_cache=None, is_neox_style=True)
+    kw = dict(rotary=rotary, positions=_meta(2))
+    assert _step(calls, 32, 32, 128, 2, _decode(2, 700, "auto"), **kw) == ["rotary_embedding_and_cache", "paged_attention_v1"]
+    assert _step(calls, 32, 32, 128, 3, _decode(3, 4096, "auto"), **kw) == ["rotary_embedding_and_cache", "paged_attention_v2"]

@@ -82,6 +82,50 @@ def test_sequences_that_read_each_others_tokens(heads, kv_heads, dim, seqs, spli
 
 
 @pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(1, 1, 64), (4, 1, 64)])        # the vector kernel, the matrix cores
+def test_blocks_that_look_alike(heads, kv_heads, dim, split):
+    """Block numbers beyond the lookup's 8192 bits: sequence i reads blocks whose numbers differ by 8192 from those that the others' tokens
+    go to, the one above or the one below, and two of the others' own."""
+    ctx = [700 - 16 * (i % 7) for i in range(24)]
+    q, k, v, _, _, tables, lens = _case(heads, kv_heads, dim, ctx, torch.bfloat16, "auto", 16)
+    blocks = 3 * 8192
+    g = torch.Generator(device=DEV).manual_seed(1)
+    caches = [torch.randn(blocks, kv_heads, *shape, generator=g, device=DEV).to(torch.bfloat16) for shape in ((dim // 8, 16, 8), (dim, 16))]
+    newest = [8192 + 100 + 5 * i if i % 2 else 2 * 8192 + 100 + 5 * i for i in range(24)]
+    for i, c in enumerate(ctx):
+        row = [(b + 8192) % blocks for b in newest[:i] + newest[i + 1:]] + [newest[i - 1], newest[i - 2]] + list(range(20 * i, 20 * i + 20))
+        last = (c - 1) // 16
+        tables[i, :last] = torch.tensor(row[:last], dtype=torch.int32)
+        tables[i, last] = newest[i]
+    slots = torch.tensor([newest[i] * 16 + (c - 1) % 16 for i, c in enumerate(ctx)], device=DEV)
+    _both((q, k, v, caches, slots, tables, lens), "auto", split)
+
+
+@torch.inference_mode()
+@pytest.mark.parametrize("heads,kv_heads", [(8, 8), (8, 2)])
+def test_layer_with_rotary(heads, kv_heads):
+    """A layer that is handed the rotary module rotates and writes the cache in a launch of its own: the same bits as rotating first and
+    then the layer without it, which writes the cache in the attention's."""
+    from splitwise_amd.model_executor.input_metadata import InputMetadata
+    from splitwise_amd.model_executor.layers.attention import Attention
+    from splitwise_amd.model_executor.layers.basic import RotaryEmbedding
+    dim, ctx = 128, [40, 700, 1100]
+    q, k, v, caches, slots, tables, lens = _case(heads, kv_heads, dim, ctx, torch.bfloat16, "auto", 16)
+    layer, rotary = Attention(heads, dim, dim ** -0.5, kv_heads), RotaryEmbedding(dim, dim, 2048, 10000.0, True, torch.bfloat16).to(DEV)
+    md = InputMetadata(is_prompt=False, slot_mapping=slots, prompt_lens=None, max_seq_len=None, start_loc=None, max_context_len=max(ctx),
+                       context_lens=lens, block_tables=tables, use_cuda_graph=False, kv_cache_dtype="auto")
+    positions, results = lens.long() - 1, []
+    for handed_over in (True, False):
+        a, b, c, to = q.flatten(1).clone(), k.flatten(1).clone(), v.flatten(1), [t.clone() for t in caches]
+        if handed_over:
+            out = layer(a, b, c, *to, md, rotary=rotary, positions=positions)
+        else:
+            out = layer(*rotary(positions, a, b), c, *to, md)
+        results.append([out, a, *to])
+    assert all(torch.equal(x, y) for x, y in zip(*results)) and not torch.equal(results[0][2], caches[0])
+
+
+@pytest.mark.parametrize("split", [False, True])
 def test_lds_just_under_64_kb(split):
     """Eleven query heads a kv head, eight waves: 64192 bytes of LDS, and tokens that are looked up (in some of them)."""
     _both(_case(22, 2, 128, [40 + 31 * i for i in range(25)], torch.bfloat16, "auto", 16), "auto", split)

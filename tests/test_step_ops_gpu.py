@@ -85,7 +85,19 @@ def _call(name, step):
         out = torch.zeros(len(lens), H, D, device="cuda", dtype=BF)
         return _C, name, (out, q3[:len(lens)], kc, vc, KVH, D ** -0.5, b.block_tables, b.ctx_len + 1, 16, max(ctx) + 1, None,
                           "auto"), {}, [out]
+    if name.startswith("paged_attention_and_cache"):
+        few, longest = len(lens), max(ctx) + 1 + (600 if name.endswith("split") else 0)      # (two parts)
+        out, temporaries = torch.zeros(few, H, D, device="cuda", dtype=BF), [None] * 3
+        if name.endswith("split"):
+            sums = torch.zeros(few, H, 2, device="cuda")
+            temporaries = [sums, torch.zeros_like(sums), torch.zeros(few, H, 2, D, device="cuda", dtype=BF)]
+        return _C, "paged_attention_and_cache", (out, *temporaries, q3[:few], k3[:few], v3[:few], kc, vc,
+                                                 (b.ctx_len + b.block_tables[:, 0] * 16).long(), D ** -0.5, b.block_tables, b.ctx_len + 1, longest,
+                                                 "auto", KVH, None), {}, [out, kc, vc]
     out = torch.zeros(rows, H, D, device="cuda", dtype=BF)
+    if name == "prefill_attention_and_cache":
+        return _C, name, (out, q3, k3, v3, b.q_start[:-1], torch.tensor(lens, dtype=torch.int32, device="cuda"), max(lens), D ** -0.5,
+                          None, 8, kc, vc, torch.arange(rows, device="cuda"), "auto"), {}, [out, kc, vc]
     return _C, name, (out, q3, k3, v3, b.q_start[:-1], torch.tensor(lens, dtype=torch.int32, device="cuda"), max(lens), D ** -0.5,
                       None, 8), {}, [out]
 
@@ -108,7 +120,8 @@ class _None:
 
 
 NAMES = ["causal_conv", "gated_delta", "head_norm_gate", "gla", "lightning", "retention", "expert_ffn", "capped_attention",
-         "reshape_and_cache", "paged_attention_v1", "prefill_attention"]
+         "reshape_and_cache", "paged_attention_v1", "prefill_attention", "prefill_attention_and_cache", "paged_attention_and_cache",
+         "paged_attention_and_cache split"]
 
 
 @pytest.mark.parametrize("step", list(STEPS))
@@ -217,7 +230,7 @@ def test_nothing_is_taken_that_python_refuses(name, monkeypatch):
             if asked:
                 taken += 1
                 assert not recorder.calls and plain(asked, known) == alone
-            elif alone is None:
+            elif not alone:                   # (an exception, or the answer that the call is for other functions)
                 refused += 1
     finally:
         native.bind(real)
