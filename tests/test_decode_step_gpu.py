@@ -125,6 +125,13 @@ def test_layer_with_rotary(heads, kv_heads):
     assert all(torch.equal(x, y) for x, y in zip(*results)) and not torch.equal(results[0][2], caches[0])
 
 
+@pytest.mark.parametrize("longest", [256, 257])
+@pytest.mark.parametrize("seqs", [5, 24])                    # all tokens written by everyone; those that are looked up
+def test_waves_of_short_contexts(seqs, longest):
+    """On either side of the length from which a launch has 8 waves whatever it writes."""
+    _both(_case(12, 12, 64, ([longest, 1, 64, 65, 200, 255] * 4)[:seqs], torch.float16, "auto", 16), "auto", False)
+
+
 @pytest.mark.parametrize("split", [False, True])
 def test_lds_just_under_64_kb(split):
     """Eleven query heads a kv head, eight waves: 64192 bytes of LDS, and tokens that are looked up (in some of them)."""

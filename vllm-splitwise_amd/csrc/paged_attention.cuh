@@ -24,16 +24,12 @@
 #pragma once
 
 #include "common.cuh"
+#include "paged_plan.h"
 #include <float.h>
 #include <stdlib.h>
 
 namespace sw {
 
-// Launches of up to this many workgroups have 8 waves each, not 4: a workgroup's chain is half as long where the GPU has room for the waves
-// (us, 4 / 8 waves, the write below included: 32 heads of 128, 2 x 700 tokens 15.8 / 13.0, 8 x 700 24.2 / 20.3, 8 x 2000 62.3 / 55.5).  Twice
-// as many where a token is 128 bytes of a head's keys (fp8 of 128, 16 bits of 64): 40 heads of 128, fp8, 8 x 1300 29.7 / 24.8, 8 x 1800
-// 50.2 / 38.3, but 32 of 128, bf16, 10 x 2500 97.3 / 101.9.
-constexpr int pa_wide_up_to(int key_bytes) { return key_bytes <= 128 ? 512 : 256; }
 constexpr int kPaLeanUpTo = 4096;     // workgroups: launches up to this size take the vector kernel's LEAN form
 constexpr int kPartitionSize = 512;   // vllm/.../ops/paged_attn.py:12 _PARTITION_SIZE
 
@@ -649,7 +645,7 @@ int launch_pa(const PaArgs& a) {
   dim3 grid(a.num_kv_heads * (g / QG), a.num_seqs, parts);
   // fp8 caches always take the lean form (there is no other instantiation for them)
   const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
-  const bool lean = FP8 || wgs <= kPaLeanUpTo, wide = lean && wgs <= pa_wide_up_to(HEAD * T::CS);
+  const bool lean = FP8 || wgs <= kPaLeanUpTo, wide = lean && pa_wide(wgs, HEAD * T::CS, a.max_context_len, a.write.tokens > 0 && a.write.all);
   SW_CHECK_ARG(lean || a.write.tokens == 0, "paged_attention_and_cache: too large a launch");
   const int nw = wide ? 8 : 4;
   const size_t smem = (size_t)QG * HEAD * 4 + (size_t)nw * QG * 64 * T::ES + (size_t)nw * QG * HEAD * 4 + 2 * nw * QG * 4;
