@@ -62,8 +62,8 @@ BESIDE, SPLIT, UNSPLIT = ["paged_attention_and_cache"], ["reshape_and_cache", "p
 @pytest.mark.parametrize("heads,kv_heads,dim,seqs,ctx,auto,fp8", [
     (32, 32, 128, 2, 700, BESIDE, BESIDE), (32, 32, 128, 32, 700, BESIDE, UNSPLIT), (32, 32, 128, 16, 700, BESIDE, BESIDE),
     (32, 32, 128, 33, 700, UNSPLIT, UNSPLIT), (32, 32, 128, 2, 4096, BESIDE, BESIDE), (32, 32, 128, 3, 4096, SPLIT, SPLIT),
-    (32, 32, 128, 8, 15000, SPLIT, SPLIT), (64, 8, 128, 64, 2011, BESIDE, BESIDE), (64, 8, 128, 65, 2011, UNSPLIT, UNSPLIT),
-    (64, 8, 128, 12, 2875, SPLIT, SPLIT), (64, 8, 128, 2, 2875, BESIDE, BESIDE), (16, 2, 128, 24, 3000, BESIDE, BESIDE),
+    (32, 32, 128, 8, 15000, SPLIT, SPLIT), (64, 8, 128, 64, 2011, BESIDE, BESIDE), (64, 8, 128, 65, 2011, BESIDE, UNSPLIT), (64, 8, 128, 65, 2049, UNSPLIT, UNSPLIT), (64, 8, 128, 128, 2048, BESIDE, UNSPLIT),
+    (64, 8, 128, 12, 2875, BESIDE, BESIDE), (64, 8, 128, 12, 7000, SPLIT, SPLIT), (64, 8, 128, 2, 2875, BESIDE, BESIDE), (16, 2, 128, 24, 3000, BESIDE, BESIDE),
     (16, 2, 128, 24, 28000, SPLIT, SPLIT), (32, 32, 128, 1, 16384, BESIDE, BESIDE), (32, 32, 128, 1, 16385, SPLIT, SPLIT), (12, 12, 64, 128, 300, UNSPLIT, UNSPLIT), (4, 4, 64, 128, 300, BESIDE, BESIDE),
     (4, 4, 64, 129, 300, UNSPLIT, UNSPLIT)])
 def test_decode_steps(heads, kv_heads, dim, seqs, ctx, auto, fp8, monkeypatch):

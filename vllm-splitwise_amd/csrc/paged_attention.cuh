@@ -139,8 +139,9 @@ struct PaWrite {
 // 60 x 326 20.9 / 18.7, 250 x 1000 206 / 216; 64 on 8, fp8, 61 x 2011 56.8 / 54.4; 12 of 64, 61 x 700 35.4 / 34.0, 200 x 300 into fp8
 // 34.3 / 41.1; 16 on 2, 100 x 500 17.5 / 14.4, 250 x 3000, fp8, 85.0 / 85.8).
 constexpr int kPaWriteUpTo = 128, kPaWriteHeadsUpTo = 1024;
-constexpr int kPaWriteAllUpTo = 16;
-constexpr int64_t kPaWriteAllElements = 8 * 8 * 40 * 128;      // tokens x sequences x elements of a token's keys
+// Few tokens are taken whatever their sequences: more than there are sequences, or of more sequences x kv heads.
+constexpr int kPaWriteFewTokens = 16;
+constexpr int64_t kPaWriteFewElements = 327680;                // tokens x sequences x elements of a token's keys
 constexpr int kPaSeenBits = 8192;
 struct PaSeen {                                    // LDS of the lookup
   uint32_t bits[kPaSeenBits / 32];

@@ -108,9 +108,8 @@ int sw_paged_attention_and_cache(void* out, float* exp_sums, float* max_logits, 
   SW_CHECK_ARG(num_seqs > 0 && num_tokens > 0 && num_kv_heads > 0 && block_size > 0 &&
                    (act_dtype == SW_F32 || act_dtype == SW_F16 || act_dtype == SW_BF16),
                "paged_attention_and_cache: nothing to do for one of the two");
-  const bool all = num_tokens <= sw::kPaWriteAllUpTo &&
-                   (int64_t)num_tokens * num_seqs * num_kv_heads * head_size <= sw::kPaWriteAllElements;
-  SW_CHECK_ARG(all || (num_tokens <= num_seqs && num_tokens <= sw::kPaWriteUpTo &&
+  const bool few = num_tokens <= sw::kPaWriteFewTokens && (int64_t)num_tokens * num_seqs * num_kv_heads * head_size <= sw::kPaWriteFewElements;
+  SW_CHECK_ARG(few || (num_tokens <= num_seqs && num_tokens <= sw::kPaWriteUpTo &&
                        (int64_t)num_seqs * num_kv_heads <= sw::kPaWriteHeadsUpTo),
                "paged_attention_and_cache: %d tokens of %d sequences", num_tokens, num_seqs);
   SW_CHECK_ARG(x == 16 / cs && head_size % x == 0 && (head_size * es) % 16 == 0 && (key_stride * es) % 16 == 0 &&
@@ -122,7 +121,8 @@ int sw_paged_attention_and_cache(void* out, float* exp_sums, float* max_logits, 
   sw::PaArgs a{out, exp_sums, max_logits, tmp_out, query, key_cache, value_cache, num_seqs, num_heads, num_kv_heads, head_size, scale,
                block_tables, context_lens, block_size, max_context_len, max_num_blocks_per_seq, alibi_slopes, q_stride,
                kv_block_stride, kv_head_stride, tmp_out != nullptr, static_cast<hipStream_t>(stream),
-               {key, value, key_cache, value_cache, slot_mapping, key_stride, value_stride, num_tokens, all}};
+               {key, value, key_cache, value_cache, slot_mapping, key_stride, value_stride, num_tokens,
+                sw::pa_writes_all(num_tokens, num_seqs)}};
   return sw::run_paged_attention(a, act_dtype, cache_dtype);
 }
 

@@ -115,21 +115,25 @@ class PagedAttentionImpl:
         return written <= 8 << 20 and longest < 4096 and (written <= 1 << 20 or readers >= 300)
 
     @staticmethod
-    def writes_beside_decode(tokens: int, num_seqs: int, num_kv_heads: int, workgroups: int, parts: int, matrix_cores: bool) -> bool:
+    def writes_beside_decode(tokens: int, num_seqs: int, longest: int, num_kv_heads: int, head_size: int, workgroups: int, parts: int,
+                             matrix_cores: bool, fp8: bool) -> bool:
         """Whether a decode run's cache write goes into the attention's launch, of which every workgroup then writes what it may read
-        (all of up to 16 tokens; else its own sequence's and those that it finds among its blocks).  ``workgroups``: of one part of
+        (all of up to 4 tokens; else its own sequence's and those that it finds among its blocks).  ``workgroups``: of one part of
         the contexts; ``parts``: 0 where they are not split.
 
-        Not split: up to 1024 sequences x kv heads, 512 on the matrix cores (us, two launches / one: 64 heads on 8, fp8, 64 x 1600
-        tokens 47.0 / 45.0, 128 x 500 38.5 / 39.6, 128 x 2300 120.3 / 122.8; bf16 over fp8, 32 heads, 16 x 800 28 / 25, 24 x 800 42.2 /
-        42.7).  Split, every part's workgroups write the same over again (not those of a part that the sequence does not reach): up to
-        1024 workgroups, and of those that write all of them 2048 tokens in all.  Over 370 such launches 1.8 us ahead on average, never
-        behind; with 2600 to 4700 tokens written 0.6 ahead but up to 13 % behind, with 6000 to 9000 1.6 behind (32 heads of 128: 2 x 2300
-        25 / 23, 1 x 28000 over fp8 54 / 57, 8 x 12000 154 / 197; 64 on 8, fp8, 12 x 2300 25 / 29; 16 on 2, 16 x 28000 104 / 121)."""
-        if tokens > 128 or num_seqs * num_kv_heads > (512 if matrix_cores else 1024):
+        Not split: up to 1024 sequences x kv heads, 512 on the matrix cores over an fp8 cache or from 2048 tokens on (us, two launches /
+        one, 64 heads on 8: 64 x 1500 tokens 83.6 / 81.0, 128 x 100 21.0 / 19.5, 128 x 1500 154.1 / 153.6, 128 x 2300 230 / 236; over fp8
+        64 x 1500 47.5 / 45.8, 128 x 700 49.5 / 50.0; bf16 over fp8, 32 heads, 16 x 700 25.9 / 23.2, 24 x 700 40.6 / 41.7).
+
+        Split, every part's workgroups write the same over again (not those of a part that the sequence does not reach): up to 1024
+        workgroups of heads of 128, and of those that write all of them 2048 tokens in all; as much of other heads.  Over 848 such steps
+        of 1 to 32 sequences and 1200 to 28000 tokens one launch takes 0.89 of the two's time where this says so (610 of them, at most
+        1.024) and 1.03 elsewhere (32 heads of 128: 2 x 2000 21.5 / 19.7, 1 x 28000 over fp8 55.8 / 59.1, 8 x 12000 155 / 188; 40 over fp8
+        5 x 2800 39.5 / 45.4; 64 on 8, fp8, 12 x 2000 21.7 / 19.4, 12 x 7000 51.5 / 53.8)."""
+        if tokens > 128 or num_seqs * num_kv_heads > (512 if matrix_cores and (fp8 or longest > 2048) else 1024):
             return False
-        launch = workgroups * parts
-        return launch <= 1024 and launch * (tokens if tokens <= 16 else 1) <= 2048
+        elements = workgroups * parts * head_size
+        return elements <= 1024 * 128 and elements * (tokens if tokens <= 4 else 1) <= 2048 * 128
 
     @staticmethod
     def forward_prefix(query, key, value, key_cache, value_cache, input_metadata: InputMetadata,
@@ -170,8 +174,10 @@ class PagedAttentionImpl:
             max_logits = torch.empty_like(exp_sums)
         if key is not None:
             # (the matrix cores' kernel is the one for 4 and more query heads, and for bf16 over an fp8 cache)
-            matrix = width >= 4 or (query.dtype == torch.bfloat16 and input_metadata.kv_cache_dtype == "fp8_e5m2")
-            if PagedAttentionImpl.writes_beside_decode(key.shape[0], num_seqs, num_kv_heads, num_seqs * num_heads // width, parts, matrix):
+            fp8 = input_metadata.kv_cache_dtype == "fp8_e5m2"
+            matrix = width >= 4 or (query.dtype == torch.bfloat16 and fp8)
+            if PagedAttentionImpl.writes_beside_decode(key.shape[0], num_seqs, max_ctx, num_kv_heads, head_size,
+                                                       num_seqs * num_heads // width, parts, matrix, fp8):
                 slots = input_metadata.slot_mapping
                 if _C.ops.paged_attention_and_cache(output, exp_sums, max_logits, tmp_output, query, key, value, key_cache,
                                                     value_cache, slots if slots.dim() == 1 else slots.flatten(), scale,
