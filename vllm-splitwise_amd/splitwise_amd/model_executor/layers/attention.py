@@ -3,8 +3,9 @@
 Order of operations restated from the reference's backends
 (vllm/model_executor/layers/attention/backends/xformers.py:70-191, flash_attn.py:77-125):
   1. reshape_and_cache of the step's keys / values (skipped during the profiling run,
-     where no cache exists yet); in the launch of step 3 where that takes it: plain prompt runs, and decode runs of up
-     to 128 sequences (``prefill_attention_and_cache``, ``paged_attention_and_cache``);
+     where no cache exists yet); in the launch of step 3 where that is the faster: plain prompt runs (``writes_beside_prompt``)
+     and decode runs of up to 128 sequences (``writes_beside_decode``).  Not in decode runs of models that hand their rotary
+     module over (the Llama models): those rotate and write in a launch of their own (``rotary_embedding_and_cache``);
   2. prompt run on a prompt-pool worker: for every hand-off slot and block run in
      ``blocks_to_nw``, push this layer's K and V blocks to the paired token worker
      (ordered after step 1 on the same stream, before the layer's attention finishes);
@@ -63,10 +64,10 @@ class PagedAttentionImpl:
         """The unpartitioned kernel launches one workgroup per (sequence, group of ``query_group``
         query heads); it fills the 256 CUs only with enough of them, below that the context is
         split into 512-token partitions (v2).  Thresholds measured on MI355X for MHA, GQA and fp8
-        shapes (1..256 sequences, 768..16384 tokens; within 1 % of the better kernel summed over that sweep,
-        at most 18 % off in any one case).  (The reference's rule, ops/paged_attn.py:62-63,
-        is tuned for 128-thread blocks per query head and a shared-memory cap that does not exist
-        here.)"""
+        shapes (1..256 sequences, 768..16384 tokens, 624 steps; 0.4 % behind the better kernel summed over that
+        sweep, at most 16 % in any one: 32 heads of 128, bf16 over fp8, 4 x 2048 tokens 18.3 us where one part
+        takes 15.8).  (The reference's rule, ops/paged_attn.py:62-63, is tuned for 128-thread blocks per query
+        head and a shared-memory cap that does not exist here.)"""
         if max_context_len <= _PARTITION_SIZE:
             return True
         workgroups = num_seqs * num_heads // max(query_group, 1)
@@ -82,9 +83,10 @@ class PagedAttentionImpl:
             # the matrix-core kernel (8 waves per workgroup below 256 workgroups): unpartitioned from 128
             # workgroups, and for short contexts whatever the launch size
             return workgroups >= 128 or max_context_len <= 2 * _PARTITION_SIZE
-        # the vector kernels, 8 waves per workgroup up to 256 (us, unpartitioned / partitioned, 32 heads of 128: 1 x 814 tokens
-        # 9.8 / 10.8, 1 x 1176 15.6 / 13.3, 3 x 1578 20.0 / 21.4, 4 x 2185 26.1 / 28.4, 4 x 3035 46.8 / 42.7, 6 x 2185 44.6 / 47.1; 12
-        # heads of 64: 8 x 1578 16.7 / 15.4, 12 x 1578 19.5 / 20.4, 20 x 2216 27.3 / 29.2, 20 x 3078 42.6 / 40.2)
+        # the vector kernels, 8 waves per workgroup up to 256 of them, 512 where a token is 128 bytes of a head's keys (csrc/paged_plan.h;
+        # us, unpartitioned / partitioned, 32 heads of 128: 1 x 814 tokens 9.8 / 10.8, 1 x 1176 15.6 / 13.3, 3 x 1578 20.0 / 21.4, 4 x 2185
+        # 26.1 / 28.4, 4 x 3035 46.8 / 42.7, 6 x 2185 44.6 / 47.1; 12 heads of 64: 8 x 1578 16.7 / 15.4, 12 x 1578 19.5 / 20.4, 20 x 2216
+        # 27.3 / 29.2, 20 x 3078 42.6 / 40.2)
         if workgroups >= 512:
             return True
         if workgroups >= 256:
