@@ -79,3 +79,27 @@ def test_decode_steps_that_rotate(monkeypatch):
     kw = dict(rotary=rotary, positions=_meta(2))
     assert _step(calls, 32, 32, 128, 2, _decode(2, 700, "auto"), **kw) == ["rotary_embedding_and_cache", "paged_attention_v1"]
     assert _step(calls, 32, 32, 128, 3, _decode(3, 4096, "auto"), **kw) == ["rotary_embedding_and_cache", "paged_attention_v2"]
+
+
+class _Held(torch.Tensor):
+    """A CPU tensor that says that it is on the GPU, for the operators' checks in front of the library."""
+    is_cuda = property(lambda self: True)
+
+
+@pytest.mark.parametrize("dtype,taken", [(torch.float32, True), (torch.bfloat16, False), (torch.float64, False)])
+def test_slopes_of_another_type_are_left_to_the_two_calls(dtype, taken, monkeypatch):
+    """The kernel reads the slopes as fp32; paged attention alone refuses others, and so the one launch may not take them."""
+    from contextlib import nullcontext
+    calls = []
+    monkeypatch.setattr(_C, "load_library", lambda: SimpleNamespace(sw_paged_attention_and_cache=lambda *args: calls.append(args) or 0))
+    monkeypatch.setattr(_C, "_on_device_of", lambda t: nullcontext())
+    monkeypatch.setattr(_C, "_stream", lambda t: None)
+    held = lambda *shape, dtype=torch.bfloat16: torch.zeros(shape, dtype=dtype).as_subclass(_Held)      # noqa: E731
+    q, k, v, slopes = held(2, 4, 64), held(2, 4, 64), held(2, 4, 64), held(4, dtype=dtype)
+    kc, vc, tables, lens = held(5, 4, 8, 16, 8), held(5, 4, 64, 16), held(2, 2, dtype=torch.int32), held(2, dtype=torch.int32)
+    assert _C.paged_attention_and_cache(held(2, 4, 64), None, None, None, q, k, v, kc, vc, held(2, dtype=torch.int64), 0.125, tables, lens, 20,
+                                        "auto", 4, slopes) is taken
+    assert len(calls) == taken
+    if not taken:
+        with pytest.raises(RuntimeError, match="alibi_slopes must be float32"):
+            _C.paged_attention_v1(held(2, 4, 64), q, kc, vc, 4, 0.125, tables, lens, 16, 20, slopes, "auto")

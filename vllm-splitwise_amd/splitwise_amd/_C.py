@@ -393,6 +393,8 @@ def paged_attention_and_cache(out: torch.Tensor, exp_sums: Optional[torch.Tensor
         return False
     if key.shape != value.shape or key.shape[1] != num_kv_heads or key.shape[2] != query.shape[2]:
         return False
+    if alibi_slopes is not None and alibi_slopes.dtype != torch.float32:
+        return False
     act = _act_dtype(query)
     if alibi_slopes is not None and not alibi_slopes.is_cuda:
         alibi_slopes = alibi_slopes.to(query.device)
