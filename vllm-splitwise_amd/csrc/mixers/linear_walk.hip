@@ -26,7 +26,9 @@
 // taken twice, from nothing and from their true states, with a scan between (560 workgroups on 512 places: the second round
 // nearly empty); 46 us prologue and 136 us walk with one wave per 32 coordinates for state and outputs, operands in rows and stores
 // under a condition; 45 and 78 here.  Of the walk's 1.0 us a chunk the products are 0.5 (38 of 32 cycles), the rest the exchange and
-// its barrier, and 37 KB of operands through the L1.  The prologue's time is the exponentials' (52 us with expf and divisions).
+// its barrier, and 37 KB of operands through the L1.  The prologue's bytes (135 MB) would take
+// 27; the rest is vector work: the exponentials (52 us with expf and divisions), and 48 row addresses, uniform over the wave, that do
+// not fit the scalar registers and travel through the lanes of vector registers (226 of them spilled).
 // Relative error of the end states against 64 bits: 1.3e-7 here, 2.2e-7 in segments taken twice.
 // One run of 16000 tokens, 4 heads of 128, decays per channel / per head: 448 / 468 us in one piece, 138 / 140 in 8 segments (415 /
 // 300 in segments of 128 tokens); of 32000 tokens, 16 heads: 1120 and 1015 in 2.
