@@ -24,10 +24,10 @@ def _meta(*shape, dtype=torch.bfloat16):
     return torch.empty(shape, dtype=dtype, device="meta")
 
 
-def _step(calls, heads, kv_heads, dim, rows, md, **kw):
+def _step(calls, heads, kv_heads, dim, rows, md, block=16, **kw):
     calls.clear()
     Attention(heads, dim, 1.0, kv_heads)(_meta(rows, heads * dim), _meta(rows, kv_heads * dim), _meta(rows, kv_heads * dim),
-                                         _meta(9, kv_heads, dim // 8, 16, 8), _meta(9, kv_heads, dim, 16), md, **kw)
+                                         _meta(9, kv_heads, dim // 8, block, 8), _meta(9, kv_heads, dim, block), md, **kw)
     return list(calls)
 
 
@@ -49,6 +49,13 @@ def test_prompt_steps(heads, kv_heads, dim, lens, auto, fp8, monkeypatch):
     calls = _Calls(monkeypatch)
     assert _step(calls, heads, kv_heads, dim, sum(lens), _prompt(lens, "auto")) == auto
     assert _step(calls, heads, kv_heads, dim, sum(lens), _prompt(lens, "fp8_e5m2")) == fp8
+
+
+@pytest.mark.parametrize("block,auto,fp8", [(8, ONE, TWO), (16, ONE, ONE), (32, ONE, ONE)])
+def test_prompt_steps_do_not_ask_for_a_launch_that_refuses_their_blocks(block, auto, fp8, monkeypatch):
+    calls = _Calls(monkeypatch)
+    assert _step(calls, 12, 12, 64, 40, _prompt([40], "auto"), block) == auto
+    assert _step(calls, 12, 12, 64, 40, _prompt([40], "fp8_e5m2"), block) == fp8
 
 
 def _decode(seqs, ctx, cache):

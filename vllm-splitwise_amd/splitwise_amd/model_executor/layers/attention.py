@@ -99,7 +99,7 @@ class PagedAttentionImpl:
 
     @staticmethod
     def writes_beside_prompt(rows: int, prompts: int, longest: int, num_heads: int, num_kv_heads: int, head_size: int,
-                             kv_cache_dtype: str) -> bool:
+                             block_size: int, kv_cache_dtype: str) -> bool:
         """Whether a prompt run's cache write goes into the attention's launch.  The write's workgroups have the attention's LDS, so
         that two of them at most run on a compute unit where the write alone has eight: it is ahead while they fill places that the
         attention leaves empty, and behind once they come after it.  An fp8 cache, for which they convert, needs the places more.
@@ -108,7 +108,12 @@ class PagedAttentionImpl:
         launch takes 0.83 of the two's time where this says so (648 of them, at most 1.055) and 1.01 elsewhere; over 792 into an fp8
         cache 0.79 (407, at most 1.03) and 1.04.  Two launches / one, us, 32 heads of 128: 3 x 773 tokens 54.6 / 47.1, 2 x 2000 124.4 /
         118.3, 1 x 4100 196.3 / 199.9, 8 x 2049 506 / 544; fp8: 1 x 400 19.0 / 13.8, 1 x 1000 34.2 / 30.9, 32 x 120 64.4 / 75.0, 8 x 773
-        133.9 / 149.3, 8 x 2049 518 / 588; 8 heads of 128, 64 x 33 14.4 / 15.7."""
+        133.9 / 149.3, 8 x 2049 518 / 588; 8 heads of 128, 64 x 33 14.4 / 15.7.
+
+        The one launch writes values 16 bytes at a time and refuses an fp8 cache in blocks of 8 tokens; to ask it all the same costs
+        the host 1.7 us (a 40-token prompt 12.5, 10.7 without asking)."""
+        if kv_cache_dtype != "auto" and block_size % 16 != 0:
+            return False
         written = rows * num_kv_heads * head_size
         # query rows that a key of an average prompt is read for
         readers = rows * num_heads // (max(prompts, 1) * num_kv_heads)
@@ -257,7 +262,8 @@ class Attention(nn.Module):
                 and not (input_metadata.blocks_to_nw and self.kvcache_comm_manager is not None)
                 and PagedAttentionImpl.writes_beside_prompt(query.shape[0], input_metadata.prompt_lens.numel(),
                                                             input_metadata.max_seq_len, self.num_heads, self.num_kv_heads,
-                                                            self.head_size, input_metadata.kv_cache_dtype)):
+                                                            self.head_size, value_cache.shape[3],
+                                                            input_metadata.kv_cache_dtype)):
             # a plain prompt run: both in one launch, where that is the faster and has a form for the call
             output = torch.empty_like(query)
             slots = input_metadata.slot_mapping
